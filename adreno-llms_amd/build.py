@@ -9,7 +9,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libmi_linear.so")
-SOURCES = ["runtime.hip", "gemv.hip", "gemm.hip", "argmax.hip", "decode.hip", "probe.hip", "quantize.cpp", "bundle.cpp"]
+SOURCES = ["runtime.hip", "gemv.hip", "gemm.hip", "argmax.hip", "decode.hip", "attention.hip", "probe.hip", "quantize.cpp", "bundle.cpp"]
 
 # -ffp-contract=off: the kernels spell every fused multiply-add as fmaf(); nothing else
 # may be fused, or results stop being bit-identical to the reference evaluation order.
@@ -23,6 +23,10 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unus
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-fhip-fp32-correctly-rounded-divide-sqrt", "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
+# (attention.hip takes every result of a matrix product through the vector units at once: with the
+#  accumulators in the general registers a key tile of its main loop loses 116 register moves)
+PER_SOURCE = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+
 
 def build(verbose=True, extra=()):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -32,7 +36,7 @@ def build(verbose=True, extra=()):
         obj = os.path.join(CSRC, os.path.splitext(src)[0] + ".o")
         cmd = [hipcc, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
         if src.endswith(".hip"):
-            cmd[1:1] = DEVICE
+            cmd[1:1] = DEVICE + PER_SOURCE.get(src, [])
         else:
             cmd[1:1] = ["-x", "c++"]
         if verbose:

@@ -1,0 +1,319 @@
+// Causal attention of a prompt on the matrix cores: rows pos0 .. pos0 + M - 1 of a sequence against
+// cache rows 0 .. their own position, softmax(q k / sqrt(D)) v per query head, key/value heads shared by
+// n_heads / n_kv_heads query heads (QW/kernels/attention.cl gqa_attn_scores, gqa_softmax, gqa_attn_out).
+//
+// The kernels of decode.hip that keep the reference's order of operations are bound by that order: one
+// chain of additions over the keys per output element and per denominator, on the vector units.  Where
+// the caller has the projections run on the matrix cores, the sums run in another order anyway, and this
+// kernel takes their place: fp16 products, fp32 sums, scores and exponentials kept in fp32 (the reference
+// order rounds both to fp16), probabilities rounded to fp16 once, before they meet the values.
+#include "common.h"
+#include "device_math.h"
+
+namespace mi {
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kKeys = 64;                        // keys per tile
+constexpr int kRows = 16;                        // queries per wavefront (of one head)
+constexpr float kNone = -3.402823466e+38f;       // the score of a key that the query does not see
+constexpr float kStart = -1.0e30f;               // the running maximum of a query that has seen no key
+constexpr float kSlack = 8.0f;                   // see the main loop
+
+// The greater of a lane's value and those of the lanes 16, 32 and 48 away.
+__device__ __forceinline__ float max_of_groups(float a) {
+    unsigned u = __float_as_uint(a);
+    auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    u = __float_as_uint(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+    r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{a, b}, half2v));
+}
+
+constexpr size_t tile_bytes(int D) { return static_cast<size_t>(kKeys) * (2 * D + 16) + static_cast<size_t>(D) * (2 * kKeys + 8); }
+constexpr size_t merge_bytes(int D) { return static_cast<size_t>(D / 4 + 2) * 64 * 4; }     // a wavefront's sums, see the end of the kernel
+constexpr size_t flash_lds(int D, int KS) { return 2 * KS * tile_bytes(D); }
+
+// A wavefront owns 16 queries of one head ("a set"), KS wavefronts of the block share them, wavefront k of
+// the KS taking key tiles k, k + KS, ...; the block's WAVES / KS sets belong to one key/value head and share
+// its tiles, KS of them at a time, in LDS.
+//
+// Scores are computed transposed (A = keys, B = queries), so that lane (query i = lane % 16, group g =
+// lane / 16) ends up with keys 4 g .. 4 g + 3 of every 16 keys for its query: maximum and sum are taken
+// inside the lane and across the four groups (two register swaps), and two such quadruples are, as they
+// stand, the B operand of the product with the values (k = 8 values per lane; which keys they are does
+// not matter as long as the A operand brings the same ones), so probabilities never go through LDS.  The
+// values are transposed on their way into LDS, 4 keys x 4 elements per thread in registers.
+// LDS pitches: key rows 2 D + 16 bytes (16-byte reads of 16 consecutive rows), value rows (one element,
+// 64 keys) 136 bytes (8-byte reads of 16 consecutive rows): either spreads over all banks.
+//
+// What bounds it: a wavefront alone on its SIMD takes 0.8 us per tile, of which the matrix cores work a
+// sixth; the reads from LDS (16 KB per wavefront and tile), the exponentials and the waits between the
+// phases are the rest, and they overlap only across wavefronts.  14 heads over 2 key/value heads, 2048
+// rows: 433 us in the reference's order (attention_group_kernel), 24.3 us here (0.31 of the rate a large
+// matrix product reaches, causal half counted); 300 rows at position 900: 96 -> 13.2 us.  Requesting tiles
+// two ahead, forming the next tile's scores under the current tile's exponentials, and two sets per
+// wavefront (27.9 us) were no faster.
+template <int D, int WAVES, int KS>
+__global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* __restrict__ QR, const uint16_t* __restrict__ kc,
+                                                         const uint16_t* __restrict__ vc, uint16_t* __restrict__ out, int M,
+                                                         int pos0, int n_heads, int n_kv_heads, float scale_log2, int mirror) {
+    constexpr int kThreads = 64 * WAVES, kSets = WAVES / KS;                            // sets of queries per block
+    constexpr int kKPitch = 2 * D + 16, kVPitch = 2 * kKeys + 8;
+    constexpr int kKTile = kKeys * kKPitch, kVTile = D * kVPitch;
+    constexpr int kKPieces = KS * kKeys * (D / 8) / kThreads;  // 16-byte pieces of KS key tiles per thread
+    constexpr int kVBlocks = KS * (kKeys / 4) * (D / 4) / kThreads;   // 4 x 4 blocks of KS value tiles per thread
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    uint8_t* const kbuf = lds;                                 // [2][KS][kKTile]
+    uint8_t* const vbuf = lds + 2 * KS * kKTile;               // [2][KS][kVTile]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int slice = wave % KS;
+    const int nrep = n_heads / n_kv_heads, kvd = n_kv_heads * D, qd = n_heads * D;
+    const int sets = (M + kRows - 1) / kRows * nrep;           // of a key/value head
+    const int per_head = (sets + kSets - 1) / kSets;
+    // Longest rows first.  (mirror > 0: the blocks from number `mirror` on, one CU's worth, are taken from
+    // the short end: they share a CU with the longest ones.)
+    int rank = blockIdx.x;
+    if (mirror && rank >= mirror) rank = per_head * n_kv_heads - 1 - (rank - mirror);
+    const int kvh = rank % n_kv_heads, b = per_head - 1 - rank / n_kv_heads;
+    const int last_set = (b + 1) * kSets < sets ? (b + 1) * kSets - 1 : sets - 1;
+    const int q_end = last_set / nrep * kRows + kRows;         // one past the block's last query
+    const int keys = pos0 + (q_end < M ? q_end : M);           // keys the block reads
+    const int tiles = (keys + kKeys - 1) / kKeys, steps = (tiles + KS - 1) / KS;
+    // (a set past the last and rows past M: computed as the last ones, not stored)
+    const int set = b * kSets + wave / KS < sets ? b * kSets + wave / KS : sets - 1;
+    const int q0 = set / nrep * kRows, head = kvh * nrep + set % nrep;
+    const bool live = b * kSets + wave / KS < sets && q0 + i < M;
+    const int row = q0 + i < M ? q0 + i : M - 1, my_pos = pos0 + row;
+    half8 q[D / 32];
+    #pragma unroll
+    for (int j = 0; j < D / 32; ++j)
+        q[j] = *reinterpret_cast<const half8*>(QR + static_cast<size_t>(row) * qd + head * D + 8 * g + 32 * j);
+
+    // Tiles travel memory -> registers -> LDS.  A request's address is a scalar base per tile plus a thread's
+    // constant offset.  Keys past the last are read as the last one and masked: 0 x a number, never 0 x what
+    // lies there; past the last tile that one is read again.
+    struct Regs { u32x4 k[kKPieces]; u32x2 v[kVBlocks][4]; };
+    const uint32_t row_bytes = static_cast<uint32_t>(kvd) * 2;
+    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(kc + kvh * D);
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(vc + kvh * D);
+    const int row_last = keys - 1 - (steps - 1) * KS * kKeys;  // the last key's row in the last step's tiles
+    uint32_t koff[2][kKPieces], voff[2][kVBlocks][4];          // of any step, of the last
+    #pragma unroll
+    for (int p = 0; p < kKPieces; ++p) {
+        const int r = (tid + kThreads * p) / (D / 8), c = 16 * ((tid + kThreads * p) % (D / 8));
+        koff[0][p] = r * row_bytes + c;
+        koff[1][p] = (r < row_last ? r : row_last) * row_bytes + c;
+    }
+    #pragma unroll
+    for (int p = 0; p < kVBlocks; ++p)
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 4 * ((tid + kThreads * p) / (D / 4)) + e, c = 8 * ((tid + kThreads * p) % (D / 4));
+            voff[0][p][e] = r * row_bytes + c;
+            voff[1][p][e] = (r < row_last ? r : row_last) * row_bytes + c;
+        }
+    auto fetch = [&](Regs& R, int step) {
+        const int t = step < steps ? step : steps - 1;
+        const bool last = t == steps - 1;
+        const size_t at = static_cast<size_t>(t) * KS * kKeys * row_bytes;
+        const uint8_t *kb = kbase + at, *vb = vbase + at;
+        #pragma unroll
+        for (int p = 0; p < kKPieces; ++p) R.k[p] = *reinterpret_cast<const u32x4*>(kb + (last ? koff[1][p] : koff[0][p]));
+        #pragma unroll
+        for (int p = 0; p < kVBlocks; ++p)
+            #pragma unroll
+            for (int e = 0; e < 4; ++e) R.v[p][e] = *reinterpret_cast<const u32x2*>(vb + (last ? voff[1][p][e] : voff[0][p][e]));
+    };
+    auto stash = [&](const Regs& R, int buf) {
+        #pragma unroll
+        for (int p = 0; p < kKPieces; ++p) {
+            const int idx = tid + kThreads * p;
+            *reinterpret_cast<u32x4*>(kbuf + buf * KS * kKTile + idx / (D / 8) * kKPitch + 16 * (idx % (D / 8))) = R.k[p];
+        }
+        #pragma unroll
+        for (int p = 0; p < kVBlocks; ++p) {
+            const int idx = tid + kThreads * p, k4 = idx / (D / 4);          // 4 keys
+            uint8_t* dst = vbuf + (buf * KS + k4 / (kKeys / 4)) * kVTile + 4 * (idx % (D / 4)) * kVPitch + 8 * (k4 % (kKeys / 4));
+            const u32x2 (&v)[4] = R.v[p];
+            #pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+                *reinterpret_cast<u32x2*>(dst + e * kVPitch) =
+                    u32x2{__builtin_amdgcn_perm(v[1][e / 2], v[0][e / 2], sel), __builtin_amdgcn_perm(v[3][e / 2], v[2][e / 2], sel)};
+            }
+        }
+    };
+
+    floatx4 acc[D / 16];
+    #pragma unroll
+    for (int d = 0; d < D / 16; ++d) acc[d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    // running maximum of the query's scores, times scale_log2; sum of the probabilities (as they meet the values, rounded
+    // to fp16: a row of ones beside the values' rows, the same number in every register)
+    float base = kStart;
+    floatx4 l = {0.0f, 0.0f, 0.0f, 0.0f};
+    half8 ones;
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = static_cast<_Float16>(1.0f);
+    auto multiply = [&](int buf, int k0) {
+        const uint8_t* ktile = kbuf + (buf * KS + slice) * kKTile + i * kKPitch + 16 * g;
+        const uint8_t* vtile = vbuf + (buf * KS + slice) * kVTile + i * kVPitch + 8 * g;
+        floatx4 s[4];
+        #pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            s[kt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            #pragma unroll
+            for (int j = 0; j < D / 32; ++j)
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8*>(ktile + 16 * kt * kKPitch + 64 * j), q[j], s[kt], 0, 0, 0);
+        }
+        if (k0 + kKeys - 1 > pos0 + q0) {                      // (keys up to the set's first query need no mask)
+            #pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (k0 + 16 * kt + 4 * g + r > my_pos) s[kt][r] = kNone;
+        }
+        // A score may exceed the running maximum by 2^kSlack before the sums are rescaled: exponentials up to
+        // that are as good in fp16 as those up to 1, and the test needs the lane's own keys only.
+        float top = kNone;
+        #pragma unroll
+        for (int kt = 0; kt < 4; ++kt) top = fmaxf(top, fmaxf(fmaxf(s[kt][0], s[kt][1]), fmaxf(s[kt][2], s[kt][3])));
+        top *= scale_log2;
+        if (__any(top > base + kSlack)) {
+            top = fmaxf(base, max_of_groups(top));
+            const float alpha = __builtin_amdgcn_exp2f(base - top);
+            l *= alpha;
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d) acc[d] *= alpha;
+            base = top;
+        }
+        // (a query without a key so far: every score is kNone, and its exponentials must be 0)
+        const float sub = base == kStart ? 0.0f : base;
+        uint32_t p[4][2];
+        #pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            float e[4];
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) e[r] = __builtin_amdgcn_exp2f(fmaf(s[kt][r], scale_log2, -sub));
+            p[kt][0] = pack2(e[0], e[1]);
+            p[kt][1] = pack2(e[2], e[3]);
+        }
+        #pragma unroll
+        for (int kp = 0; kp < 2; ++kp) {
+            const half8 pb = __builtin_bit_cast(half8, u32x4{p[2 * kp][0], p[2 * kp][1], p[2 * kp + 1][0], p[2 * kp + 1][1]});
+            l = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb, l, 0, 0, 0);
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d) {
+                const u32x2 lo = *reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp);
+                const u32x2 hi = *reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp + 32);
+                acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, u32x4{lo.x, lo.y, hi.x, hi.y}), pb, acc[d], 0, 0, 0);
+            }
+        }
+    };
+    const int w_last = pos0 + (q0 + kRows < M ? q0 + kRows : M) - 1;       // the set's last query
+    Regs R;
+    fetch(R, 0);
+    for (int t = 0; t < steps; ++t) {
+        // registers -> LDS, the next tiles requested, one barrier (a buffer is written again two barriers after it
+        // was last read), the wavefront's tile multiplied unless its queries end before it
+        stash(R, t & 1);
+        fetch(R, t + 1);
+        __syncthreads();
+        const int k0 = (t * KS + slice) * kKeys;
+        if (k0 <= w_last) multiply(t & 1, k0);
+    }
+    float sum = l[0];
+    if constexpr (KS > 1) {
+        // the KS wavefronts' sums meet in LDS: slices 1 .. KS - 1 leave theirs, slice 0 merges them in order
+        __syncthreads();
+        float* mine = reinterpret_cast<float*>(lds) + wave * static_cast<int>(merge_bytes(D) / 4) + lane;
+        if (slice > 0) {
+            mine[0] = base;
+            mine[64] = sum;
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) mine[(2 + 4 * d + r) * 64] = acc[d][r];
+        }
+        __syncthreads();
+        if (slice > 0) return;
+        #pragma unroll
+        for (int z = 1; z < KS; ++z) {
+            const float* other = mine + z * static_cast<int>(merge_bytes(D) / 4);
+            const float bz = other[0], lz = other[64];
+            const float top = fmaxf(base, bz);                 // (slice 0 always has key 0: top is of a score)
+            const float a = __builtin_amdgcn_exp2f(base - top), c = __builtin_amdgcn_exp2f(bz - top);
+            sum = sum * a + lz * c;
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) acc[d][r] = acc[d][r] * a + other[(2 + 4 * d + r) * 64] * c;
+            base = top;
+        }
+    }
+    if (!live) return;
+    const float inv = __fdiv_rn(1.0f, sum);
+    uint16_t* dst = out + static_cast<size_t>(row) * qd + head * D + 4 * g;
+    #pragma unroll
+    for (int d = 0; d < D / 16; ++d)
+        *reinterpret_cast<u32x2*>(dst + 16 * d) = u32x2{pack2(acc[d][0] * inv, acc[d][1] * inv), pack2(acc[d][2] * inv, acc[d][3] * inv)};
+}
+
+// Blocks of a launch of WAVES wavefronts per block, KS per set.
+inline int flash_blocks(int M, int n_heads, int n_kv_heads, int WAVES, int KS) {
+    const int sets = (M + kRows - 1) / kRows * (n_heads / n_kv_heads), per_block = WAVES / KS;
+    return (sets + per_block - 1) / per_block * n_kv_heads;
+}
+
+template <int D, int WAVES, int KS>
+bool launch_flash(hipStream_t s, const uint16_t* QR, const uint16_t* kc, const uint16_t* vc, uint16_t* out, int M, int pos0,
+                  int n_heads, int n_kv_heads, float scale) {
+    constexpr size_t lds = flash_lds(D, KS);
+    static_assert(lds <= 160 * 1024 && (KS == 1 || WAVES * merge_bytes(D) <= lds), "tiles and merge buffer fit");
+    auto* kern = flash_rows_kernel<D, WAVES, KS>;
+    if (lds > 65536 &&
+        !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  static_cast<int>(lds)))))
+        return false;
+    const int total = flash_blocks(M, n_heads, n_kv_heads, WAVES, KS), cus = device_info().cus;
+    hipLaunchKernelGGL(kern, dim3(total), dim3(64 * WAVES), lds, s, QR, kc, vc, out, M, pos0, n_heads, n_kv_heads,
+                       scale * 1.44269504088896341f, total > cus && total <= 2 * cus ? cus : 0);
+    return MI_HIP_OK(hipGetLastError());
+}
+
+}  // namespace
+
+bool attention_prompt_supported(int head_dim) { return head_dim == 64 || head_dim == 128; }
+
+bool launch_attention_prompt(hipStream_t s, const uint16_t* QR, const uint16_t* kc, const uint16_t* vc, uint16_t* out, int M,
+                             int pos0, int n_heads, int n_kv_heads, int head_dim, float scale) {
+#define MI_FLASH(D, WAVES, KS) return launch_flash<D, WAVES, KS>(s, QR, kc, vc, out, M, pos0, n_heads, n_kv_heads, scale)
+    // A set's chain of tiles bounds the launch (0.8 us per tile while a wavefront has its SIMD to itself), so the
+    // keys of a set go over several wavefronts, and as many of those share a CU as there are blocks for.  Measured
+    // at 14 heads over 2 (head width 64), us, eight wavefronts / 2 per set, 4 / 2, 8 / 4:
+    //   2048 rows 24.3 / 31.6 / 41.2, 1000 rows 13.3 / 13.4 / 17.2: enough blocks of 8 / 2 for the chip;
+    //   300 rows at 900 15.2 / 14.3 / 13.2, 40 at 1500 17.4 / 17.0 / 14.9: few blocks, long chains;
+    //   100 rows 5.2 / 4.7 / 6.0, 40 at 300 7.2 / 6.7 / 7.5: a tile or a few per wavefront either way.
+    const int cus = device_info().cus;
+    if (head_dim == 64) {
+        if (flash_blocks(M, n_heads, n_kv_heads, 8, 2) * 4 >= cus * 3) MI_FLASH(64, 8, 2);
+        if (pos0 + M <= 512) MI_FLASH(64, 4, 2);
+        MI_FLASH(64, 8, 4);
+    }
+    // (head width 128, 16 heads over 4, four wavefronts, 1 / 2 per set: 2048 rows 52.6 / 83.4, 300 at 900 29.6 / 24.6)
+    if (flash_blocks(M, n_heads, n_kv_heads, 4, 1) >= cus) MI_FLASH(128, 4, 1);
+    MI_FLASH(128, 4, 2);
+#undef MI_FLASH
+}
+
+}  // namespace mi

@@ -118,6 +118,13 @@ bool launch_argmax_f16(hipStream_t s, const void* logits, int N, int num_partial
 bool launch_argmax_finish(hipStream_t s, const float* cand_v, const int* cand_i, int count, int N, int num_partials,
                           void* token_out, int* token_copy, int* counter);
 
+// attention.hip: causal attention of M prompt rows (queries QR [M, n_heads * head_dim] after bias and rotary
+// embedding, at positions pos0 ..) against the cache rows of one layer, on the matrix cores.  Within the
+// GEMM's tolerance of the reference-order kernels, not bit for bit.
+bool attention_prompt_supported(int head_dim);
+bool launch_attention_prompt(hipStream_t s, const uint16_t* QR, const uint16_t* kc, const uint16_t* vc, uint16_t* out, int M,
+                             int pos0, int n_heads, int n_kv_heads, int head_dim, float scale);
+
 // gemm.hip: out[M,N] = x[M,K] W^T on MFMA with the dequant fused into the tile load.
 // Shapes and pointers the GEMM kernels take (M >= 2, K a multiple of 64, 16-byte aligned x and W).
 bool gemm_supported(WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale);

@@ -734,7 +734,8 @@ __global__ void swiglu_kernel(uint16_t* __restrict__ gate, const uint16_t* __res
 // operations of the single-token kernels above in the same order, so that a prompt gives the
 // same cache rows and logits as M single-token steps wherever the projections do (they do bit
 // for bit when the M > 1 projections run as rows of GEMV, and within the GEMM's tolerance when
-// they run on the matrix cores).
+// they run on the matrix cores; the attention then runs there too, attention.hip, and the two
+// attention kernels below serve the rows of GEMV and the head widths that kernel does not take).
 
 // H[r][c] = embed[tokens[r]][c]   (QW/kernels/embedding.cl)
 __global__ void embed_rows_kernel(const uint16_t* __restrict__ embed, const int* __restrict__ tokens,
@@ -1671,6 +1672,9 @@ int mi_decoder_prefill(void* dec, void* stream, const int* tokens, int n_tokens,
                                                       256 * 2 * (1 + kPromptTile) + kMaxPositions * 6))))
             return 0;
     }
+    // Attention on the matrix cores unless the projections run as rows of GEMV (then the whole prompt keeps
+    // the reference's order, bit for bit).
+    const bool matrix_attention = M > 1 && gemm_mode(s) != 1 && attention_prompt_supported(D);
     // one block per key/value head and row where the group's scores fit the LDS of a CU (160 KB, less
     // the kernel's few static bytes)
     constexpr size_t kGroupLdsMost = 160 * 1024 - 256;
@@ -1722,7 +1726,9 @@ int mi_decoder_prefill(void* dec, void* stream, const int* tokens, int n_tokens,
                            static_cast<const uint16_t*>(d->bk[l]), static_cast<const uint16_t*>(d->bv[l]), d->cosT, d->sinT,
                            kc, vc, QR, pos0, c.n_heads, c.n_kv_heads, D, ldq, ldkv);
         if (!launched()) return 0;
-        if (grouped && D == 64)
+        if (matrix_attention) {
+            if (!launch_attention_prompt(s, QR, kc, vc, ATT, M, pos0, c.n_heads, c.n_kv_heads, D, scale)) return 0;
+        } else if (grouped && D == 64)
             hipLaunchKernelGGL(attention_group_kernel<64>, dim3(c.n_kv_heads, M), dim3(256), grp_lds, s, QR, kc, vc, ATT, pos0,
                                grp_cap, c.n_heads, c.n_kv_heads, scale);
         else if (grouped)
