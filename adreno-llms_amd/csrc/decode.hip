@@ -256,39 +256,46 @@ __global__ __launch_bounds__(256) void rope_attention_kernel(const uint16_t* __r
     }
 }
 
-// The same launch for head widths known at compile time (64 and 128), laid out for latency: a
-// decode step at a short context is a chain of memory round trips, so everything that does not
-// depend on an earlier result is requested at once.  256 threads; the first kTileRows rows of the
-// group's key and value cache are requested in 16-byte pieces, in passes of 256 pieces (rows past
-// the current position too: the caches hold max_pos rows, and what is not older than the current
-// position is never used; the passes above it are neither waited for nor kept), and between the
-// first pass and the others the projections, biases and the rotary row (which the step's first
-// launch has set aside, so that its address does not wait for the position); keys and values wait
-// in LDS tiles (rows padded by 16 bytes against bank conflicts) while q, k and v of the current
-// position are prepared.  Scores: one thread per key from the tile; values: one thread per
-// output element, keys in index order from the tile.  Longer contexts take further tiles the
-// same way, each requested while the one before it is used.  The arithmetic and its order are those of
-// rope_attention_kernel.
-// The two serial chains the order of operations leaves (the sum of the exponentials by one lane, an
-// output element's sum over the keys by one lane each) run in batches of kBatch positions: all LDS
-// reads of a batch are asked for together and the dependent additions follow as they arrive, so a
-// batch costs one LDS round trip and not one per position.  The last batch is filled up with
-// zeros (exponentials past the last key, probabilities from the current position on, value rows
-// from the current position on), which leaves a sum as it is: x + 0 = x and fma(0, 0, x) = x for
-// every x but -0, and a sum that starts at +0 never becomes -0.  The current position's
-// probability is kept aside (pc) and meets the current value row after the tiles, as before.
-// Dynamic LDS: 6 D bytes, 6 bytes per position (positions rounded up to kBatch), 16 bytes, then two
-// tiles of kTileRows x (2 D + 16) bytes.
-constexpr int kTileRows = 128;
+// The same launch for head widths known at compile time (64 and 128): one block of 512 threads per query
+// head, the arithmetic and its order those of rope_attention_kernel.
+//
+// What bounds it at a long context are the two serial chains that order leaves: the sum of the exponentials
+// and, per output element, the sum over the keys.  A dependent addition takes 8 shader cycles (3.55 ns)
+// whatever else the CU does, so the launch cannot be faster than 7.1 ns per position.  Everything else is kept off
+// the chains' path:
+//  * scores, exponentials and probabilities are spread over all eight wavefronts (a key per thread, from a
+//    tile of key rows in LDS; the next tile is requested while one is worked on);
+//  * the sum's terms and the probabilities are read from LDS sixteen bytes at a time, a batch ahead;
+//  * the values reach the chain transposed, eight keys of one element per 16-byte read, and are multiplied as
+//    fp16 straight out of the pair they lie in (v_fma_mix_f32): one instruction per key.  Wavefronts 4 to 7 fill
+//    the ring of value tiles (4 keys x 4 elements per thread, turned in registers) while wavefront 0 (and 1 at
+//    head width 128) runs down the chain.
+// us per launch, 256 threads with everything but the scores in the first wavefront -> this: 14 heads at position 1900
+// 47.6 -> 25.3 (the two chains are 13.5 of it), 9 heads at 210 8.75 -> 7.24, 14 heads at 40 4.64 -> 4.63.
+//
+// At a short context (up to kShort keys, all of them in the first tiles) the launch is a chain of memory
+// round trips and barriers instead, so everything that does not depend on an earlier result is requested at once
+// (the first kShort rows of both caches before the position is known; rows that turn out not to be needed
+// arrive unused), and wavefront 0 does the softmax and, at head width 64, the rest alone, without barriers.
+//
+// The current position's key and value take their places in the tiles as rows like the others.  Sums run in
+// whole batches of kBatch positions: exponentials and probabilities past the last key are zeros, and so are
+// value rows, which leaves a sum as it is: x + 0 = x and fma(0, 0, x) = x for every x but -0, and a sum that
+// starts at +0 never becomes -0.
+constexpr int kAttnThreads = 512;
+constexpr int kShort = 128;
 constexpr int kBatch = 32;
-static_assert(kTileRows % kBatch == 0, "whole batches in a tile");
 __host__ __device__ inline int padded_positions(int max_pos) { return (max_pos + kBatch - 1) / kBatch * kBatch; }
 constexpr int kMaxPositions = 8192;                      // longest context a decoder is created for
+// Bytes of LDS for tiles: a tile of key rows (padded by 16 bytes against bank conflicts), later two value tiles; at a
+// short context kShort rows of either.
+constexpr int kTileData = 65536;
+constexpr size_t tile_area(int D) { return static_cast<size_t>(kTileData) / (2 * D) * (2 * D + 16); }
 
 template <int D>
 // (Arguments in the order of need: the first 14 dwords arrive in registers with the wavefront, and the
 //  first thing the kernel does is ask for the cache tiles and the position.)
-__global__ __launch_bounds__(256) void rope_attention_tiled(uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
+__global__ __launch_bounds__(kAttnThreads) void rope_attention_tiled(uint16_t* __restrict__ kc, uint16_t* __restrict__ vc,
                                       const State* __restrict__ st, int n_heads, int n_kv_heads, int max_pos,
                                       float scale, const uint16_t* __restrict__ q_raw, const uint16_t* __restrict__ k_raw,
                                       const uint16_t* __restrict__ v_raw, const uint16_t* __restrict__ bq,
@@ -296,130 +303,163 @@ __global__ __launch_bounds__(256) void rope_attention_tiled(uint16_t* __restrict
                                       const uint16_t* __restrict__ rope_now,
                                       uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
                                       uint16_t* __restrict__ v_out, uint16_t* __restrict__ out) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    constexpr int kRowH = D + 8;                           // tile row stride in halves
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kRowH = D + 8;                           // halves between key rows in LDS
     constexpr int kPieces = D / 8;                         // 16-byte pieces per row
-    constexpr int kPasses = kTileRows * kPieces / 256;     // pieces per thread and tile
-    static_assert(kTileRows * kPieces % 256 == 0, "whole passes");
+    constexpr int kPassRows = kAttnThreads / kPieces;      // key rows that 512 threads request at once
+    constexpr int kKeyRows = kTileData / (2 * D);          // key rows per tile (512 / 256)
+    constexpr int kPasses = kKeyRows / kPassRows;
+    constexpr int kShortPasses = kShort / kPassRows;
+    constexpr int kValueRows = kKeyRows / 2;               // value rows per tile of the ring
+    constexpr int kDG = D / 4;                             // groups of 4 elements
+    constexpr int kShortBlocks = kShort / 4 * kDG / kAttnThreads;         // 4 x 4 blocks per thread, short context
+    constexpr int kRingThreads = 256;                                      // wavefronts 4 .. 7 fill the ring
+    constexpr int kRingBlocks = kValueRows / 4 * kDG / kRingThreads;
+    constexpr int kChainWaves = D / 64;
     extern __shared__ __attribute__((aligned(16))) uint16_t qv[];
-    uint16_t* kcur = qv + D;
-    uint16_t* vcur = kcur + D;
+    uint16_t* vcur = qv + D;
     const int mp = padded_positions(max_pos);
-    float* ex = reinterpret_cast<float*>(vcur + D);                        // [mp] exponentials, 16-byte aligned
-    uint16_t* sc = reinterpret_cast<uint16_t*>(ex + mp);                   // [mp] scores, 16-byte aligned
-    uint16_t* pc = sc + mp;                                                // the current position's probability
-    uint16_t* ktile = pc + 8;                                              // 16-byte aligned
-    uint16_t* vtile = ktile + kTileRows * kRowH;
+    float* ex = reinterpret_cast<float*>(vcur + D);                        // [mp] exponentials, then probabilities; 16-byte aligned
+    uint16_t* sc = reinterpret_cast<uint16_t*>(ex + mp);                   // [mp] scores
+    float* red = reinterpret_cast<float*>(sc + mp);                        // [8] maxima of the wavefronts
+    uint16_t* ktile = reinterpret_cast<uint16_t*>(red + 8);                // 16-byte aligned
+    uint8_t* vring = reinterpret_cast<uint8_t*>(ktile);                    // [2][kValueRows / 8][D][8 keys], where the keys were
+    uint8_t* vshort = reinterpret_cast<uint8_t*>(ktile + kShort * kRowH);
     const int nrep = n_heads / n_kv_heads;
     const int qh = blockIdx.x, kvd = n_kv_heads * D, kvh = qh / nrep, hd2 = D / 2;
     const bool writer = qh % nrep == 0;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // piece p of this thread in a tile: row (tid + 256 p) / kPieces, 16-byte piece (tid + 256 p) % kPieces;
-    // pass p of all threads is rows p kPassRows .. (p + 1) kPassRows - 1.  Passes are asked for in
-    // row order, keys and values alternating, and loads return in the order of the requests: a
-    // short context waits for its first passes only and leaves the rest to arrive unused.
-    constexpr int kPassRows = 256 / kPieces;
-    auto request = [&](const uint16_t* cache, int row0, int p) {
-        const int idx = tid + 256 * p, row = idx / kPieces, piece = idx % kPieces;
-        const int tk = row0 + row < max_pos ? row0 + row : max_pos - 1;
-        return *reinterpret_cast<const u32x4*>(cache + static_cast<size_t>(tk) * kvd + kvh * D + 8 * piece);
+    // piece p of this thread in a key tile: row tid / kPieces + p kPassRows, 16-byte piece tid % kPieces
+    const int krow = tid / kPieces, kpiece = tid % kPieces;
+    auto request_keys = [&](int row0, int p) {
+        const int at = row0 + krow + p * kPassRows, tk = at < max_pos ? at : max_pos - 1;
+        return *reinterpret_cast<const u32x4*>(kc + static_cast<size_t>(tk) * kvd + kvh * D + 8 * kpiece);
     };
-    u32x4 kreg[kPasses], vreg[kPasses];
-    auto request_tiles = [&](int row0, int first_pass) {
+    // 4 keys x 4 elements of the values
+    struct VBlock { u32x2 r[4]; };
+    auto request_values = [&](int key0, int dg) {
+        VBlock b;
         #pragma unroll
-        for (int p = first_pass; p < kPasses; ++p) {
-            kreg[p] = request(kc, row0, p);
-            vreg[p] = request(vc, row0, p);
-            asm volatile("" ::: "memory");                 // in this order: the compiler would sort them by cache
+        for (int e = 0; e < 4; ++e) {
+            const int tk = key0 + e < max_pos ? key0 + e : max_pos - 1;
+            b.r[e] = *reinterpret_cast<const u32x2*>(vc + static_cast<size_t>(tk) * kvd + kvh * D + 4 * dg);
         }
+        return b;
     };
-    // the passes that hold rows below `rows` (of kBatch; the value sums run in whole batches) go to
-    // LDS; value rows from row `valid` of the tile on are stored as zeros
-    auto keep = [&](uint16_t* tile, const u32x4 (&r)[kPasses], int rows, int valid) {
-        #pragma unroll
-        for (int p = 0; p < kPasses; ++p) {
-            if (p * kPassRows < rows) {
-                const int idx = tid + 256 * p, row = idx / kPieces, piece = idx % kPieces;
-                const u32x4 zero = {0u, 0u, 0u, 0u};
-                *reinterpret_cast<u32x4*>(tile + row * kRowH + 8 * piece) = row < valid ? r[p] : zero;
-            }
-        }
-    };
-    // rows of the tile at row0 that anybody reads: the keys below the current position, in whole batches
-    auto tile_rows = [&](int row0, int pos) {
-        const int n = pos - row0 < kTileRows ? pos - row0 : kTileRows;
-        return (n + kBatch - 1) / kBatch * kBatch;
-    };
-    // The tiles' first passes are asked for first: their addresses need nothing but the arguments that
-    // arrive in registers.  What the current position needs (projections, biases, the rotary row: a few
-    // bytes per thread, behind pointers that have to be fetched) is asked for next, ahead of the other
-    // passes, and arrives ahead of them, so that q, k and v are prepared while the tiles come in.  Wavefront 0 prepares q, 1 k, 2 and 3 v; every thread loads from a valid
-    // address whether it has an element or not, so the number of loads in flight is the same for all.
+    u32x4 kreg[kPasses];
+    VBlock vreg[kRingBlocks];
     int pos = st->pos;
-    kreg[0] = request(kc, 0, 0);
-    vreg[0] = request(vc, 0, 0);
+    kreg[0] = request_keys(0, 0);
     asm volatile("" ::: "memory");
-    const int role = tid >> 6, lane = tid & 63;
-    const int i = role < 2 ? (lane < hd2 ? lane : hd2 - 1) : (tid - 128 < D ? tid - 128 : D - 1);
+    // What the current position needs (projections, biases, the rotary row: a few bytes per thread, behind pointers that
+    // have to be fetched) is asked for next, ahead of the other rows.  Wavefront 0 prepares q, 1 k, 2 and 3 v; every
+    // thread loads from a valid address whether it has an element or not, so the number of loads in flight is the same.
+    const int role = wave < 3 ? wave : 2;
+    const int i = role < 2 ? (lane < hd2 ? lane : hd2 - 1) : (tid >= 128 && tid - 128 < D ? tid - 128 : D - 1);
     const int i2 = role < 2 ? i + hd2 : i;
     const uint16_t* buf = role == 0 ? q_raw + qh * D : role == 1 ? k_raw + kvh * D : v_raw + kvh * D;
     const uint16_t* bias = role == 0 ? bq + qh * D : role == 1 ? bk + kvh * D : bv + kvh * D;
     const uint16_t raw1 = buf[i], raw2 = buf[i2], bias1 = bias[i], bias2 = bias[i2];
     const uint16_t cos_i = rope_now[role < 2 ? i : 0], sin_i = rope_now[D + (role < 2 ? i : 0)];   // embed_kernel's row
     asm volatile("" ::: "memory");                             // these first
-    request_tiles(0, 1);
+    #pragma unroll
+    for (int p = 1; p < kShortPasses; ++p) kreg[p] = request_keys(0, p);
+    #pragma unroll
+    for (int p = 0; p < kShortBlocks; ++p) vreg[p] = request_values(4 * ((tid + kAttnThreads * p) / kDG), (tid + kAttnThreads * p) % kDG);
     __builtin_amdgcn_sched_barrier(0);                         // and nothing that waits for one of them in between
 
     pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
-    const int seq_k = pos + 1;
+    const int seq_k = pos + 1, padded = (seq_k + kBatch - 1) / kBatch * kBatch;
+    const bool is_short = seq_k <= kShort;
+    if (!is_short) {
+        #pragma unroll
+        for (int p = kShortPasses; p < kPasses; ++p) kreg[p] = request_keys(0, p);
+    }
     // (computed by every thread, stored by those that have an element: a load that is only used under a
     //  condition would be moved there, behind the tiles)
     const float c = h_f(cos_i), sn = h_f(sin_i);
     const float x1 = h_f(f_h(h_f(raw1) + h_f(bias1)));
     const float x2 = h_f(f_h(h_f(raw2) + h_f(bias2)));
     const uint16_t r1 = f_h(fmaf(x1, c, -(x2 * sn))), r2 = f_h(fmaf(x2, c, x1 * sn));
-    const bool has_pair = role < 2 && lane < hd2, has_v = role >= 2 && tid - 128 < D;
+    const bool has_pair = wave < 2 && lane < hd2, has_v = tid >= 128 && tid - 128 < D;
     const uint16_t rv = f_h(x1);                               // fp16(v + bias), rounded once
-    if (has_pair) {
-        uint16_t* dst = role == 0 ? qv : kcur;
-        dst[i] = r1;
-        dst[i + hd2] = r2;
+    if (has_pair && wave == 0) {
+        qv[i] = r1;
+        qv[i + hd2] = r2;
     } else if (has_v) {
         vcur[tid - 128] = rv;
     }
-    keep(ktile, kreg, tile_rows(0, pos), kTileRows);
-    keep(vtile, vreg, tile_rows(0, pos), pos);
-    // (the stores to memory after the tiles are in LDS: a store in flight counts like a load that has not
-    //  arrived, and would make the waits above wait for later passes than they need)
-    if (has_pair) {
-        if (role == 0) {
-            q_out[qh * D + i] = r1;
-            q_out[qh * D + i + hd2] = r2;
-        } else if (writer) {
-            uint16_t* dst = kc + static_cast<size_t>(pos) * kvd + kvh * D;
-            dst[i] = r1;
-            dst[i + hd2] = r2;
-            k_out[kvh * D + i] = r1;
-            k_out[kvh * D + i + hd2] = r2;
+    // A tile's key rows from registers to LDS; the current position's row comes from its wavefront (k above).
+    auto keep_keys = [&](int row0, int p) {
+        const int row = krow + p * kPassRows;
+        if (row0 + row != pos) *reinterpret_cast<u32x4*>(ktile + row * kRowH + 8 * kpiece) = kreg[p];
+    };
+    auto keep_current_key = [&](int row0) {
+        if (wave == 1 && lane < hd2 && pos >= row0 && pos < row0 + kKeyRows) {
+            ktile[(pos - row0) * kRowH + i] = r1;
+            ktile[(pos - row0) * kRowH + i + hd2] = r2;
         }
-    } else if (has_v && writer) {
-        const int e = tid - 128;
-        vc[static_cast<size_t>(pos) * kvd + kvh * D + e] = rv;
-        v_out[kvh * D + e] = rv;
-    }
-    if (pos > kTileRows) request_tiles(kTileRows, 0);          // the second tiles, one tile ahead of their use
-    __syncthreads();
-
-    // scores: tile rows by threads 0 .. kTileRows - 1, the current position by thread kTileRows
-    auto score = [&](const uint16_t* krow) {
-        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-        const u16x4* kv = reinterpret_cast<const u16x4*>(krow);
-        const u16x4* qq = reinterpret_cast<const u16x4*>(qv);
+    };
+    // Four keys of four elements, transposed, into a value tile [8 keys each][cell][8 keys], zeros past the last key.
+    // Cell c is element 4 (c % kDG) + c / kDG: the threads of a wavefront then write next to each other (element
+    // order had eight of them on the same banks: 3.4 us per launch at position 1900). vcur must be in LDS (the block that holds the
+    // current position takes its row from there).
+    auto keep_values = [&](uint8_t* tile, const VBlock& b, int key0, int kg, int dg) {
+        u32x2 v[4];
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = key0 + e < pos ? b.r[e] : u32x2{0u, 0u};
+        if (key0 <= pos && pos < key0 + 4) {
+            const u32x2 own = *reinterpret_cast<const u32x2*>(vcur + 4 * dg);
+            #pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (key0 + e == pos) v[e] = own;
+        }
+        uint8_t* dst = tile + ((kg / 2) * D + dg) * 16 + (kg & 1) * 8;
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+            *reinterpret_cast<u32x2*>(dst + e * kDG * 16) =
+                u32x2{__builtin_amdgcn_perm(v[1][e / 2], v[0][e / 2], sel), __builtin_amdgcn_perm(v[3][e / 2], v[2][e / 2], sel)};
+        }
+    };
+    // The outputs a caller may inspect and the cache rows (after the first tile is in LDS: a store in flight counts
+    // like a load that has not arrived, and would make the waits above wait for later requests than they need).
+    auto store_current = [&]() {
+        if (has_pair) {
+            if (wave == 0) {
+                q_out[qh * D + i] = r1;
+                q_out[qh * D + i + hd2] = r2;
+            } else if (writer) {
+                uint16_t* dst = kc + static_cast<size_t>(pos) * kvd + kvh * D;
+                dst[i] = r1;
+                dst[i + hd2] = r2;
+                k_out[kvh * D + i] = r1;
+                k_out[kvh * D + i + hd2] = r2;
+            }
+        } else if (has_v && writer) {
+            const int e = tid - 128;
+            vc[static_cast<size_t>(pos) * kvd + kvh * D + e] = rv;
+            v_out[kvh * D + e] = rv;
+        }
+    };
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    struct Query { u16x4 v[D / 4]; };
+    auto read_query = [&]() {
+        Query q;
+        #pragma unroll
+        for (int d4 = 0; d4 < D / 4; ++d4) q.v[d4] = reinterpret_cast<const u16x4*>(qv)[d4];
+        return q;
+    };
+    auto score = [&](const uint16_t* row, const Query& q) {
+        const u16x4* kv = reinterpret_cast<const u16x4*>(row);
         float acc = 0.0f;
         #pragma unroll
         for (int d4 = 0; d4 < D / 4; ++d4) {
-            const u16x4 a = qq[d4], b = kv[d4];
+            const u16x4 a = q.v[d4], b = kv[d4];
             float t = h_f(a[0]) * h_f(b[0]);
             t = fmaf(h_f(a[1]), h_f(b[1]), t);
             t = fmaf(h_f(a[2]), h_f(b[2]), t);
@@ -428,94 +468,195 @@ __global__ __launch_bounds__(256) void rope_attention_tiled(uint16_t* __restrict
         }
         return f_h(acc * scale);
     };
-    if (tid == kTileRows) sc[pos] = score(kcur);
-    for (int row0 = 0; row0 < pos; row0 += kTileRows) {
-        if (row0 > 0) {
-            __syncthreads();                               // the previous tile's scores are done
-            keep(ktile, kreg, tile_rows(row0, pos), kTileRows);
-            if (row0 + kTileRows < pos) {
-                #pragma unroll
-                for (int p = 0; p < kPasses; ++p) kreg[p] = request(kc, row0 + kTileRows, p);
+    // sum of ex[0 .. padded) in index order, by every lane of the wavefront (the same reads, the same sum)
+    auto sum_in_order = [&]() {
+        const f32x4* e4 = reinterpret_cast<const f32x4*>(ex);
+        f32x4 t[2][kBatch / 4];
+        auto read = [&](f32x4 (&b)[kBatch / 4], int c0) {
+            #pragma unroll
+            for (int j = 0; j < kBatch / 4; ++j) b[j] = e4[c0 / 4 + j];
+            asm volatile("" ::: "memory");                     // asked for here, not where it is used
+        };
+        float sum = 0.0f;
+        auto add = [&](const f32x4 (&b)[kBatch / 4]) {
+            #pragma unroll
+            for (int j = 0; j < kBatch / 4; ++j) {
+                sum = sum + b[j][0];
+                sum = sum + b[j][1];
+                sum = sum + b[j][2];
+                sum = sum + b[j][3];
             }
-            __syncthreads();
+        };
+        // (the batch behind the last is the last again: with a request for every addition made the number in flight is a
+        //  constant, and only then does the wait for one batch leave the next one in flight)
+        read(t[0], 0);
+        for (int c0 = 0;;) {
+            read(t[1], c0 + kBatch < padded ? c0 + kBatch : c0);
+            add(t[0]);
+            c0 += kBatch;
+            if (c0 >= padded) break;
+            read(t[0], c0 + kBatch < padded ? c0 + kBatch : c0);
+            add(t[1]);
+            c0 += kBatch;
+            if (c0 >= padded) break;
         }
-        if (tid < kTileRows && row0 + tid < pos) sc[row0 + tid] = score(ktile + tid * kRowH);
-    }
-    __syncthreads();
-    // softmax by the first wavefront alone: its LDS accesses are ordered, so the steps need no
-    // barrier between them (a short context is all barrier otherwise)
-    if (tid < 64) {
-        float m = -3.402823466e+38f;                       // maximum: any order gives the same value
-        for (int c = tid; c < seq_k; c += 64) m = fmaxf(m, h_f(sc[c]));
-        const float maxv = wave_max(m);
-        for (int c = tid; c < seq_k; c += 64) {
-            const float e = exp_poly(h_f(sc[c]) - maxv);
-            ex[c] = e;
-            sc[c] = f_h(e);
-        }
-        const int padded = (seq_k + kBatch - 1) / kBatch * kBatch;
-        if (tid < padded - seq_k) ex[seq_k + tid] = 0.0f;      // kBatch <= 64 lanes
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // lane 0 reads what the other lanes wrote
-        __builtin_amdgcn_wave_barrier();
-        float inv = 0.0f;
-        if (tid == 0) {
-            typedef float f32x4 __attribute__((ext_vector_type(4)));
-            const f32x4* e4 = reinterpret_cast<const f32x4*>(ex);
-            float sum = 0.0f;
-            for (int c = 0; c < padded; c += kBatch) {
-                f32x4 t[kBatch / 4];
-                #pragma unroll
-                for (int j = 0; j < kBatch / 4; ++j) t[j] = e4[c / 4 + j];
-                #pragma unroll
-                for (int j = 0; j < kBatch / 4; ++j) {
-                    sum = sum + t[j][0];
-                    sum = sum + t[j][1];
-                    sum = sum + t[j][2];
-                    sum = sum + t[j][3];
-                }
+        return sum;
+    };
+    // acc + sum over keys 0 .. n - 1 (n a multiple of kBatch) of a value tile, in index order; p: the probabilities from
+    // the tile's first key on, as fp32 (an fp16 first factor makes the compiler put a wait state of 4 cycles behind each
+    // v_fma_mix_f32: 5.1 instead of 3.5 ns per key); e: the cell
+    auto chain = [&](float acc, const uint8_t* tile, const float* p, int e, int n) {
+        u32x4 v[2][kBatch / 8];
+        f32x4 q[2][kBatch / 4];
+        auto read = [&](int b, int r0) {
+            #pragma unroll
+            for (int j = 0; j < kBatch / 8; ++j) {
+                v[b][j] = *reinterpret_cast<const u32x4*>(tile + ((r0 / 8 + j) * D + e) * 16);
+                q[b][2 * j] = *reinterpret_cast<const f32x4*>(p + r0 + 8 * j);
+                q[b][2 * j + 1] = *reinterpret_cast<const f32x4*>(p + r0 + 8 * j + 4);
             }
-            inv = rcp_rn(sum + 1e-20f);
+            asm volatile("" ::: "memory");                     // asked for here, not where it is used
+        };
+        auto run = [&](int b) {
+            #pragma unroll
+            for (int j = 0; j < kBatch / 4; ++j) {
+                const uint32_t v01 = v[b][j / 2][2 * (j % 2)], v23 = v[b][j / 2][2 * (j % 2) + 1];
+                acc = fmaf(q[b][j][0], h_f(static_cast<uint16_t>(v01 & 0xffffu)), acc);
+                acc = fmaf(q[b][j][1], h_f(static_cast<uint16_t>(v01 >> 16)), acc);
+                acc = fmaf(q[b][j][2], h_f(static_cast<uint16_t>(v23 & 0xffffu)), acc);
+                acc = fmaf(q[b][j][3], h_f(static_cast<uint16_t>(v23 >> 16)), acc);
+            }
+        };
+        read(0, 0);
+        for (int r0 = 0;;) {                                   // (requests as in sum_in_order)
+            read(1, r0 + kBatch < n ? r0 + kBatch : r0);
+            run(0);
+            r0 += kBatch;
+            if (r0 >= n) break;
+            read(0, r0 + kBatch < n ? r0 + kBatch : r0);
+            run(1);
+            r0 += kBatch;
+            if (r0 >= n) break;
         }
-        inv = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(inv)));
-        // probabilities of the older keys; zeros from the current position to the end of its batch
-        for (int c = tid; c < padded; c += 64) {
-            const uint16_t pr = f_h(h_f(sc[c]) * inv);
-            if (c == pos) pc[0] = pr;
-            sc[c] = c < pos ? pr : static_cast<uint16_t>(0);
+        return acc;
+    };
+
+    const int element = 4 * (tid % kDG) + tid / kDG;           // of the thread's cell (tid < D)
+    if (is_short) {
+        #pragma unroll
+        for (int p = 0; p < kShortPasses; ++p)
+            if (p * kPassRows < seq_k) keep_keys(0, p);
+        keep_current_key(0);
+        __syncthreads();                                       // (vcur is read by whoever holds the current position's block)
+        #pragma unroll
+        for (int p = 0; p < kShortBlocks; ++p) {
+            const int kg = (tid + kAttnThreads * p) / kDG, dg = (tid + kAttnThreads * p) % kDG;
+            if (4 * kg < padded) keep_values(vshort, vreg[p], 4 * kg, kg, dg);
+        }
+        store_current();
+        if (tid < seq_k) sc[tid] = score(ktile + tid * kRowH, read_query());
+        __syncthreads();
+        // softmax by the first wavefront alone: its LDS accesses are ordered, so the steps need no
+        // barrier between them (a short context is all barrier otherwise)
+        if (wave == 0) {
+            float m = -3.402823466e+38f;                       // maximum: any order gives the same value
+            for (int k = tid; k < seq_k; k += 64) m = fmaxf(m, h_f(sc[k]));
+            const float maxv = wave_max(m);
+            for (int k = tid; k < padded; k += 64) ex[k] = k < seq_k ? exp_poly(h_f(sc[k]) - maxv) : 0.0f;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // every lane reads what the others wrote
+            __builtin_amdgcn_wave_barrier();
+            const float inv = rcp_rn(sum_in_order() + 1e-20f);
+            for (int k = tid; k < padded; k += 64) ex[k] = h_f(f_h(h_f(f_h(ex[k])) * inv));     // probabilities, rounded to fp16
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        }
+        if constexpr (kChainWaves > 1) __syncthreads();
+        if (wave < kChainWaves) out[qh * D + element] = f_h(chain(0.0f, vshort, ex, tid, padded));
+        return;
+    }
+
+    // scores, tile by tile; a thread keeps the greatest of its own
+    float m = -3.402823466e+38f;
+    {
+        #pragma unroll
+        for (int p = 0; p < kPasses; ++p) keep_keys(0, p);
+        keep_current_key(0);
+        store_current();
+        __syncthreads();                                       // q and the first tile are in LDS
+        const Query query = read_query();
+        for (int row0 = 0; row0 < seq_k; row0 += kKeyRows) {
+            if (row0 + kKeyRows < seq_k) {
+                #pragma unroll
+                for (int p = 0; p < kPasses; ++p) kreg[p] = request_keys(row0 + kKeyRows, p);
+            }
+            if (row0 > 0) __syncthreads();                     // the tile is in LDS
+            if (tid < kKeyRows && row0 + tid < seq_k) {
+                const uint16_t s = score(ktile + tid * kRowH, query);
+                sc[row0 + tid] = s;
+                m = fmaxf(m, h_f(s));
+            }
+            if (row0 + kKeyRows < seq_k) {
+                __syncthreads();                               // and has been used
+                #pragma unroll
+                for (int p = 0; p < kPasses; ++p) keep_keys(row0 + kKeyRows, p);
+                keep_current_key(row0 + kKeyRows);
+            }
         }
     }
-    __syncthreads();
-    // output element e by thread e: older keys in index order from the tiles, then the current one
+    // wavefronts 4 .. 7 keep value tiles coming: tile u of the ring holds keys u kValueRows ..
+    const bool feeds = wave >= 4;
+    const int rt = tid - (kAttnThreads - kRingThreads);
+    auto request_tile = [&](int u) {
+        #pragma unroll
+        for (int p = 0; p < kRingBlocks; ++p)
+            vreg[p] = request_values(u * kValueRows + 4 * ((rt + kRingThreads * p) / kDG), (rt + kRingThreads * p) % kDG);
+    };
+    auto keep_tile = [&](int u) {
+        #pragma unroll
+        for (int p = 0; p < kRingBlocks; ++p) {
+            const int kg = (rt + kRingThreads * p) / kDG, dg = (rt + kRingThreads * p) % kDG;
+            keep_values(vring + (u & 1) * (kValueRows * D * 2), vreg[p], u * kValueRows + 4 * kg, kg, dg);
+        }
+    };
+    const int vtiles = (seq_k + kValueRows - 1) / kValueRows;
+    if (feeds) request_tile(0);
+    m = wave_max(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();                                           // scores and maxima are in LDS, the key tile has been used
+    m = fmaxf(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])), fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7])));
+    for (int k = tid; k < padded; k += kAttnThreads) ex[k] = k < seq_k ? exp_poly(h_f(sc[k]) - m) : 0.0f;
+    __syncthreads();                                           // exponentials
+    if (feeds) {
+        keep_tile(0);
+        if (vtiles > 1) { request_tile(1); keep_tile(1); }
+        if (vtiles > 2) request_tile(2);
+    } else if (wave == 0) {
+        const float inv = rcp_rn(sum_in_order() + 1e-20f);
+        if (tid == 0) red[0] = inv;
+    }
+    __syncthreads();                                           // the sum
+    {
+        const float inv = red[0];
+        for (int k = tid; k < padded; k += kAttnThreads) ex[k] = h_f(f_h(h_f(f_h(ex[k])) * inv));
+    }
+    __syncthreads();                                           // probabilities and the first two value tiles
     float acc = 0.0f;
-    for (int row0 = 0; row0 < pos; row0 += kTileRows) {
-        if (row0 > 0) {
-            __syncthreads();                               // the previous tile has been used up
-            keep(vtile, vreg, tile_rows(row0, pos), pos - row0);
-            if (row0 + kTileRows < pos) {
-                #pragma unroll
-                for (int p = 0; p < kPasses; ++p) vreg[p] = request(vc, row0 + kTileRows, p);
+    for (int u = 0; u < vtiles; ++u) {
+        if (wave < kChainWaves) {
+            const int n = padded - u * kValueRows < kValueRows ? padded - u * kValueRows : kValueRows;
+            acc = chain(acc, vring + (u & 1) * (kValueRows * D * 2), ex + u * kValueRows, tid, n);
+        }
+        if (u + 2 < vtiles) {
+            __syncthreads();                                   // tile u has been used; tile u + 1 is behind an earlier barrier
+            if (feeds) {
+                keep_tile(u + 2);
+                if (u + 3 < vtiles) request_tile(u + 3);
             }
+        } else if (u + 1 < vtiles) {
             __syncthreads();
         }
-        if (tid < D) {
-            typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-            const int n = pos - row0 < kTileRows ? pos - row0 : kTileRows;
-            for (int r0 = 0; r0 < n; r0 += kBatch) {
-                u16x8 p[kBatch / 8];
-                uint16_t v[kBatch];
-                #pragma unroll
-                for (int j = 0; j < kBatch / 8; ++j) p[j] = *reinterpret_cast<const u16x8*>(sc + row0 + r0 + 8 * j);
-                #pragma unroll
-                for (int u = 0; u < kBatch; ++u) v[u] = vtile[(r0 + u) * kRowH + tid];
-                #pragma unroll
-                for (int u = 0; u < kBatch; ++u) acc = fmaf(h_f(p[u / 8][u % 8]), h_f(v[u]), acc);
-            }
-        }
     }
-    if (tid < D) {
-        acc = fmaf(h_f(pc[0]), h_f(vcur[tid]), acc);
-        out[qh * D + tid] = f_h(acc);
-    }
+    if (wave < kChainWaves) out[qh * D + element] = f_h(acc);
 }
 
 // ---- attention with the keys of a head split over several blocks (an arithmetic mode, not the default) ----
@@ -1168,10 +1309,9 @@ __global__ void swiglu_stacked_kernel(const uint16_t* __restrict__ GU, uint16_t*
 // last prompt position and advance it
 __global__ void set_pos_kernel(State* st, int pos) { st->pos = pos; }
 
-// Dynamic LDS of rope_attention_tiled<D>.
+// Dynamic LDS of rope_attention_tiled<D>: q and v of the current position, exponentials and scores, eight maxima, tiles.
 inline size_t tiled_attention_lds(int D, int max_pos) {
-    const size_t head = static_cast<size_t>(3 * D + 3 * padded_positions(max_pos) + 8) * 2;
-    return head + 2 * static_cast<size_t>(kTileRows) * (D + 8) * 2;
+    return static_cast<size_t>(2 * D) * 2 + 6 * static_cast<size_t>(padded_positions(max_pos)) + 32 + tile_area(D);
 }
 
 __global__ void advance_kernel(State* st) {
@@ -1504,11 +1644,11 @@ int mi_decoder_step(void* dec, void* stream) {
         } else if (D == 64 || D == 128) {
             const size_t lds = tiled_attention_lds(D, c.max_pos);
             if (D == 64)
-                hipLaunchKernelGGL(rope_attention_tiled<64>, dim3(c.n_heads), dim3(256), lds, s, kc, vc, d->st, c.n_heads,
+                hipLaunchKernelGGL(rope_attention_tiled<64>, dim3(c.n_heads), dim3(kAttnThreads), lds, s, kc, vc, d->st, c.n_heads,
                                    c.n_kv_heads, c.max_pos, scale, d->q, d->k, d->v, bq, bk, bv, d->rope_now, d->qr, d->kr,
                                    d->vr, d->attn);
             else
-                hipLaunchKernelGGL(rope_attention_tiled<128>, dim3(c.n_heads), dim3(256), lds, s, kc, vc, d->st, c.n_heads,
+                hipLaunchKernelGGL(rope_attention_tiled<128>, dim3(c.n_heads), dim3(kAttnThreads), lds, s, kc, vc, d->st, c.n_heads,
                                    c.n_kv_heads, c.max_pos, scale, d->q, d->k, d->v, bq, bk, bv, d->rope_now, d->qr, d->kr,
                                    d->vr, d->attn);
         } else {

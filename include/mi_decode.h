@@ -94,7 +94,7 @@ int   mi_decoder_read(void* decoder, void* stream, int* pos, int* token);
 /* An arithmetic mode of the attention inside mi_decoder_step, for long contexts.  0 or 1 (default): the
  * launch that keeps the reference's order of operations (QW/kernels/attention.cl: one work-group per
  * head, the sum of the exponentials and every output element's sum over the keys in key order), bit
- * for bit; its time grows by about 24 ns per position and layer.  2..32: the keys of a head are taken
+ * for bit; its time grows by about 11 ns per position and layer.  2..32: the keys of a head are taken
  * by that many blocks, each with its own maximum and sums, and a second launch merges them: the same
  * real numbers summed in another order, without the fp16 roundings of the probabilities, within
  * max-abs/rel 1e-3 and cosine 0.9999 of the default, not bit-identical; one launch more per layer.
