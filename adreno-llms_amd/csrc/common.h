@@ -141,5 +141,11 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
 // slices and park fp32 partial sums there; calls on one stream are ordered, so they can share it.
 bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x,
                  const void* W, const void* scale, void* out, void* workspace, size_t workspace_bytes);
+// The first of n projections of one x (M >= 2, the first accepted by gemm_supported) in one launch, where one
+// exists that gives what launch_gemm gives for each: returns how many it took, 0 for none (nothing was launched),
+// -1 on an error.  No output may overlap x or another output.
+struct GemmMat { const void* W; const void* scale; void* out; int N; };
+int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat, int M, int K, const void* x, void* workspace,
+                      size_t workspace_bytes);
 
 }  // namespace mi

@@ -58,11 +58,34 @@ __device__ __forceinline__ uint32_t q4x2_to_h2(uint32_t v, __half2 s2) {
     return __builtin_bit_cast(uint32_t, __hmul2(__hadd2(__builtin_bit_cast(__half2, h), k), s2));
 }
 
+// Further matrices of one launch that multiply the same x (q | k | v, gate | up): tile `first` and up along N
+// belong to the next one.  A block (in the streaming kernel a wavefront) finds its matrix from its tile and does
+// from there on what it does in a launch of that matrix alone, so the results are those of separate launches bit
+// for bit.  What it is for: a launch of a small matrix takes 4 to 9 us whatever its size (one block's serial K, the
+// chip mostly idle), and k and v of a layer are 128 to 320 rows.
+// Measured: the seven int8 projections of a layer with 896 / 4864 channels, given together, at 16 rows 34.6 -> 26.6 us (q | k | v
+// and gate | up in one streaming launch each), at 2048 rows 121.7 -> 106.7 us; a launch of one matrix as before.
+struct MoreMats {
+    int n = 0, tiles = 0;                                    // further matrices; tiles along N of all of them (n > 0)
+    struct { const uint8_t* W; const uint16_t* scale; uint16_t* out; int N, first; } m[kMaxSegments - 1] = {};
+};
+__device__ __forceinline__ void pick_matrix(const MoreMats& mm, int& tile, const uint8_t* __restrict__& W,
+                                            const uint16_t* __restrict__& scale, uint16_t* __restrict__& out, int& N) {
+    int first = 0;
+    #pragma unroll
+    for (int q = 0; q < kMaxSegments - 1; ++q)
+        if (q < mm.n && tile >= mm.m[q].first) {
+            W = mm.m[q].W; scale = mm.m[q].scale; out = mm.m[q].out; N = mm.m[q].N; first = mm.m[q].first;
+        }
+    tile -= first;
+}
+
 template <int BM, int BN, int WM, int WN, int KIND>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restrict__ X,
                                                         const uint8_t* __restrict__ W,
                                                         const uint16_t* __restrict__ scale,
-                                                        uint16_t* __restrict__ out, int M, int N, int K) {
+                                                        uint16_t* __restrict__ out, int M, int N, int K,
+                                                        MoreMats more) {
     static_assert((BM / WM) * (BN / WN) == 4, "four wavefronts per block");
     constexpr int TM = WM / 32, TN = WN / 32;
     constexpr int A_CHUNKS = BM * (kKT / 8) / kThreads;                      // 16-byte chunks of x per thread
@@ -79,7 +102,9 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restri
 
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int wm = wave / (BN / WN), wn = wave % (BN / WN);
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    int tile_n = blockIdx.x;
+    pick_matrix(more, tile_n, W, scale, out, N);
+    const int m0 = blockIdx.y * BM, n0 = tile_n * BN;
     const int gk = lane / 32, li = lane % 32;
 
     floatx16 acc[TM][TN];
@@ -289,7 +314,7 @@ __global__ __launch_bounds__(256) void gemm_wide(const uint16_t* __restrict__ X,
                                                    const uint8_t* __restrict__ W,
                                                    const uint16_t* __restrict__ scale,
                                                    uint16_t* __restrict__ out, int M, int N, int K,
-                                                   float* __restrict__ partial, int splits) {
+                                                   float* __restrict__ partial, int splits, MoreMats more) {
     constexpr int BM = 32 * TM;
     constexpr int kXStage = BM * 128;                    // bytes of x (fp16) per stage
     constexpr bool Q4 = KIND == WK_Q4, F16 = KIND == WK_F16;
@@ -316,7 +341,8 @@ __global__ __launch_bounds__(256) void gemm_wide(const uint16_t* __restrict__ X,
     // sums its slice only and leaves fp32 partial sums for reduce_partials.
     int tile_m, tile_n, split;
     {
-        const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + kBN - 1) / kBN, tiles = tiles_m * tiles_n;
+        const int tiles_m = (M + BM - 1) / BM, tiles_n = more.n ? more.tiles : (N + kBN - 1) / kBN;
+        const int tiles = tiles_m * tiles_n;
         const int total = tiles * splits;
         const int per_xcd = (total + 7) / 8;
         int l = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -329,6 +355,7 @@ __global__ __launch_bounds__(256) void gemm_wide(const uint16_t* __restrict__ X,
         const int in_band = l - band * kBand * tiles_m;
         tile_m = in_band / width;
         tile_n = band * kBand + in_band % width;
+        pick_matrix(more, tile_n, W, scale, out, N);
     }
     const int m0 = tile_m * BM, n0 = tile_n * kBN;
     const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)lds));
@@ -742,9 +769,9 @@ __global__ __launch_bounds__(256) void reduce_partials(const float* __restrict__
 
 template <int TM, int KIND, int TERMS>
 bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out,
-            float* partial, size_t partial_bytes, int splits) {
+            float* partial, size_t partial_bytes, int splits, const MoreMats& more) {
     // the kernel writes splits x M x N fp32 partial sums and gives every slice at least two K-stages
-    if (splits < 1 || (splits > 1 && (!partial || K / 64 < 2 * splits ||
+    if (splits < 1 || (splits > 1 && (more.n || !partial || K / 64 < 2 * splits ||
                                       static_cast<double>(splits) * M * N * 4 > static_cast<double>(partial_bytes)))) {
         MI_ERROR_FMT("gemm: %d slices of K do not fit (M=%d N=%d K=%d, %zu bytes of workspace)", splits, M, N, K,
                      partial_bytes);
@@ -756,11 +783,11 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
         return false;
-    const long total = static_cast<long>((N + kBN - 1) / kBN) * ((M + 32 * TM - 1) / (32 * TM)) * splits;
+    const long total = static_cast<long>(more.n ? more.tiles : (N + kBN - 1) / kBN) * ((M + 32 * TM - 1) / (32 * TM)) * splits;
     const dim3 grid(static_cast<unsigned>(8 * ((total + 7) / 8)), 1, 1);      // see the block -> tile map in the kernel
     hipLaunchKernelGGL(kern, grid, dim3(256), lds_bytes, s, static_cast<const uint16_t*>(x),
                        static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
-                       static_cast<uint16_t*>(out), M, N, K, splits > 1 ? partial : nullptr, splits);
+                       static_cast<uint16_t*>(out), M, N, K, splits > 1 ? partial : nullptr, splits, more);
     if (!MI_HIP_OK(hipGetLastError())) return false;
     if (splits > 1) {
         const long MN = static_cast<long>(M) * N;
@@ -843,13 +870,13 @@ inline void pick_shape(int kind, int terms, int M, int N, int K, int cus, size_t
 
 template <int KIND, int TERMS>
 bool launch_any(int tm, hipStream_t s, int M, int N, int K, const void* x, const void* W,
-                const void* scale, void* out, float* partial, size_t partial_bytes, int splits) {
+                const void* scale, void* out, float* partial, size_t partial_bytes, int splits, const MoreMats& more) {
     switch (tm) {
-        case 1: return launch<1, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits);
-        case 2: return launch<2, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits);
-        case 3: return launch<3, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits);
-        case 4: return launch<4, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits);
-        default: return launch<5, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits);
+        case 1: return launch<1, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more);
+        case 2: return launch<2, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more);
+        case 3: return launch<3, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more);
+        case 4: return launch<4, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more);
+        default: return launch<5, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more);
     }
 }
 
@@ -1154,7 +1181,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
                                                            const uint8_t* __restrict__ W,
                                                            const uint16_t* __restrict__ scale,
                                                            uint16_t* __restrict__ out, int M, int N, int K, int ks,
-                                                           int logical_blocks, float* __restrict__ partial) {
+                                                           int logical_blocks, float* __restrict__ partial,
+                                                           MoreMats more) {
     constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
     constexpr int WV = F16 ? 2 : 1;                       // 16-byte loads of W per lane, strip and iteration
     constexpr int kWB = F16 ? 2 : 1;                      // bytes of a row of W per 64 bytes of an iteration's weights / 64
@@ -1209,10 +1237,16 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
         xp[t] = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(m) * K * 2 + c * (16 * XE);
     }
     const uint32_t xl = (16u * 0 + i) * xrow + c * (16u * XE);  // with XL: this lane's row of the first x tile in LDS
-    const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+    const uint8_t* const W0 = W;
+    const uint16_t* const scale0 = scale;
+    uint16_t* const out0 = out;
+    const int N0 = N;
 
     for (int lb = blockIdx.x; lb < logical_blocks; lb += gridDim.x) {     // (the same trips for the whole block)
-        const int group = lb * (kWaves / ks) + wave / ks;                 // group: SW consecutive strips
+        int group = lb * (kWaves / ks) + wave / ks;                       // group: SW consecutive strips
+        W = W0; scale = scale0; out = out0; N = N0;
+        pick_matrix(more, group, W, scale, out, N);
+        const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
         const uint8_t* wp[SW];
         [[maybe_unused]] const uint16_t* sp[SW];                          // Q4: the row's block scales, this lane's first
         #pragma unroll
@@ -1490,9 +1524,9 @@ inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspa
 
 template <int KIND, int MT, int SW, bool XL, int TERMS>
 bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-                float* partial) {
+                float* partial, const MoreMats& more) {
     const int ks = sh.ks;
-    const long groups = ((N + 15) / 16 + SW - 1) / SW, per_block = kWaves / ks;
+    const long groups = more.n ? more.tiles : ((N + 15) / 16 + SW - 1) / SW, per_block = kWaves / ks;
     const long logical = (groups + per_block - 1) / per_block;
     const size_t lds = lds_bytes(MT, K, XL, ks);
     auto* kern = gemm_skinny<KIND, MT, SW, XL, TERMS>;
@@ -1509,7 +1543,8 @@ bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W
     }
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid), static_cast<unsigned>(sh.kb)), dim3(64 * kWaves), lds, s,
                        static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
-                       static_cast<uint16_t*>(out), M, N, K, ks, static_cast<int>(logical), sh.kb > 1 ? partial : nullptr);
+                       static_cast<uint16_t*>(out), M, N, K, ks, static_cast<int>(logical), sh.kb > 1 ? partial : nullptr,
+                       more);
     if (!MI_HIP_OK(hipGetLastError())) return false;
     if (sh.kb > 1) {
         const long MN = static_cast<long>(M) * N;
@@ -1523,16 +1558,16 @@ bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W
 
 template <int KIND, int MT, int TERMS>
 bool launch_mt(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-               float* partial) {
-    return sh.xl ? launch_one<KIND, MT, 1, true, TERMS>(s, M, N, K, x, W, scale, out, sh, partial)
-                 : launch_one<KIND, MT, 1, false, TERMS>(s, M, N, K, x, W, scale, out, sh, partial);
+               float* partial, const MoreMats& more) {
+    return sh.xl ? launch_one<KIND, MT, 1, true, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more)
+                 : launch_one<KIND, MT, 1, false, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more);
 }
 
 template <int KIND, int TERMS>
 bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-            void* workspace, size_t workspace_bytes) {
+            void* workspace, size_t workspace_bytes, const MoreMats& more) {
     if (M < 1 || M > kMaxM || !(sh.ks == 1 || sh.ks == 2 || sh.ks == 4 || sh.ks == 8) ||
-        lds_bytes((M + 15) / 16, K, sh.xl, sh.ks) > kLdsLimit || sh.kb < 1 || (sh.kb > 1 && sh.xl) ||
+        lds_bytes((M + 15) / 16, K, sh.xl, sh.ks) > kLdsLimit || sh.kb < 1 || (sh.kb > 1 && (sh.xl || more.n)) ||
         (sh.kb > 1 && (!workspace || static_cast<double>(sh.kb) * M * N * 4 > static_cast<double>(workspace_bytes)))) {
         MI_ERROR_FMT("gemm: the streaming kernel takes up to %d rows of x, 1, 2, 4 or 8 slices of K per block, %zu bytes of LDS "
                      "and a workspace for slices over blocks (M=%d K=%d, %d slices, x in LDS %d, %d slices over blocks, %zu bytes)",
@@ -1541,10 +1576,10 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
     }
     auto* partial = static_cast<float*>(workspace);
     switch ((M + 15) / 16) {
-        case 1: return launch_mt<KIND, 1, TERMS>(s, M, N, K, x, W, scale, out, sh, partial);
-        case 2: return launch_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, sh, partial);
-        case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial);
-        default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial);
+        case 1: return launch_mt<KIND, 1, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more);
+        case 2: return launch_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more);
+        case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more);
+        default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more);
     }
 }
 
@@ -1552,8 +1587,8 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
 
 template <int BM, int BN, int WM, int WN>
 bool launch_tile(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W,
-                 const void* scale, void* out) {
-    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, 1);
+                 const void* scale, void* out, const MoreMats& more) {
+    const dim3 grid(more.n ? more.tiles : (N + BN - 1) / BN, (M + BM - 1) / BM, 1);
     const auto* xp = static_cast<const uint16_t*>(x);
     const auto* wp = static_cast<const uint8_t*>(W);
     const auto* sp = static_cast<const uint16_t*>(scale);
@@ -1566,14 +1601,14 @@ bool launch_tile(hipStream_t s, WeightKind kind, int M, int N, int K, const void
             !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
             return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K);
+        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
     } else {
         auto* kern = gemm_kernel<BM, BN, WM, WN, WK_F16>;
         if (lds_bytes > 65536 &&
             !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
             return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K);
+        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
     }
     return MI_HIP_OK(hipGetLastError());
 }
@@ -1701,6 +1736,42 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
     return p;
 }
 
+namespace {
+
+bool launch_planned(hipStream_t s, const GemmPlan& p, WeightKind kind, int M, int N, int K, const void* x, const void* W,
+                    const void* scale, void* out, void* workspace, size_t ws_bytes, const MoreMats& more) {
+    auto* partial = static_cast<float*>(workspace);
+    switch (p.kernel) {
+        case 1: {
+            const int tm = p.tile_rows / 32, ks = p.k_slices;
+            if (kind == WK_Q4)
+                return p.terms == 1 ? wide::launch_any<WK_Q4, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, ks, more)
+                                    : wide::launch_any<WK_Q4, 2>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, ks, more);
+            if (kind == WK_F16) return wide::launch_any<WK_F16, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, ks, more);
+            return wide::launch_any<WK_I8, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, ks, more);
+        }
+        case 4:
+        {
+            const skinny::Shape sh = skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes);
+            if (kind == WK_Q4)
+                return p.terms == 1 ? skinny::launch<WK_Q4, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more)
+                                    : skinny::launch<WK_Q4, 2>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more);
+            return kind == WK_F16 ? skinny::launch<WK_F16, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more)
+                                  : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more);
+        }
+        case 5: return quad::launch(s, M, N, K, x, W, scale, out);
+        case 2: return launch_tile<64, 64, 32, 32>(s, kind, M, N, K, x, W, scale, out, more);
+        case 3: return launch_tile<128, 128, 64, 64>(s, kind, M, N, K, x, W, scale, out, more);
+        default:
+            MI_ERROR_FMT("gemm: mode %d has no kernel for kind=%d M=%d N=%d K=%d (Q4 weights have no tile kernel; the "
+                         "streaming kernel takes up to 64 rows of x; the wide kernel's 32-bit offsets reach 4 GiB of x and "
+                         "of W)", gemm_mode(s), static_cast<int>(kind), M, N, K);
+            return false;
+    }
+}
+
+}  // namespace
+
 bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W,
                  const void* scale, void* out, void* workspace, size_t workspace_bytes) {
     if (!gemm_supported(kind, M, N, K, x, W, scale)) {
@@ -1709,35 +1780,52 @@ bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void
         return false;
     }
     const size_t ws_bytes = workspace ? workspace_bytes : 0;
-    const GemmPlan p = plan_gemm(s, kind, M, N, K, ws_bytes);
-    auto* partial = static_cast<float*>(workspace);
-    switch (p.kernel) {
-        case 1: {
-            const int tm = p.tile_rows / 32;
-            if (kind == WK_Q4)
-                return p.terms == 1 ? wide::launch_any<WK_Q4, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, p.k_slices)
-                                    : wide::launch_any<WK_Q4, 2>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, p.k_slices);
-            if (kind == WK_F16) return wide::launch_any<WK_F16, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, p.k_slices);
-            return wide::launch_any<WK_I8, 1>(tm, s, M, N, K, x, W, scale, out, partial, ws_bytes, p.k_slices);
+    return launch_planned(s, plan_gemm(s, kind, M, N, K, ws_bytes), kind, M, N, K, x, W, scale, out, workspace, ws_bytes,
+                          MoreMats{});
+}
+
+// One launch serves the leading matrices whose own plans sum K in the same order, so that each result is what
+// launch_gemm gives: the same kernel and number of slices, none of them over blocks (their partial sums meet in one
+// workspace).  The wide kernel's tile height does not enter a sum: where the library chooses it, it is chosen for
+// all matrices side by side.
+int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat, int M, int K, const void* x, void* workspace,
+                      size_t workspace_bytes) {
+    const size_t ws_bytes = workspace ? workspace_bytes : 0;
+    const int cus = device_info().cus;
+    GemmPlan p = plan_gemm(s, kind, M, mat[0].N, K, ws_bytes);
+    skinny::Shape sh{};
+    if (p.kernel == 4) sh = skinny::pick_shape(kind, M, mat[0].N, K, cus, ws_bytes);
+    if (!(p.kernel == 2 || p.kernel == 3 || (p.kernel == 1 && p.k_slices == 1) || (p.kernel == 4 && sh.kb == 1))) return 0;
+    const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : 16;
+    auto tiles_of = [&](int N) { return N / width + (N % width != 0); };
+    MoreMats more;
+    more.tiles = tiles_of(mat[0].N);
+    int g = 1;
+    for (; g < n && g < kMaxSegments; ++g) {
+        const GemmMat& c = mat[g];
+        if (!gemm_supported(kind, M, c.N, K, x, c.W, c.scale)) break;
+        const GemmPlan q = plan_gemm(s, kind, M, c.N, K, ws_bytes);
+        if (q.kernel != p.kernel || q.terms != p.terms || q.k_slices != p.k_slices) break;
+        if (p.kernel == 4) {
+            const skinny::Shape t = skinny::pick_shape(kind, M, c.N, K, cus, ws_bytes);
+            if (t.ks != sh.ks || t.xl != sh.xl || t.kb != 1) break;
         }
-        case 4:
-        {
-            const skinny::Shape sh = skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes);
-            if (kind == WK_Q4)
-                return p.terms == 1 ? skinny::launch<WK_Q4, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes)
-                                    : skinny::launch<WK_Q4, 2>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes);
-            return kind == WK_F16 ? skinny::launch<WK_F16, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes)
-                                  : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes);
-        }
-        case 5: return quad::launch(s, M, N, K, x, W, scale, out);
-        case 2: return launch_tile<64, 64, 32, 32>(s, kind, M, N, K, x, W, scale, out);
-        case 3: return launch_tile<128, 128, 64, 64>(s, kind, M, N, K, x, W, scale, out);
-        default:
-            MI_ERROR_FMT("gemm: mode %d has no kernel for kind=%d M=%d N=%d K=%d (Q4 weights have no tile kernel; the "
-                         "streaming kernel takes up to 64 rows of x; the wide kernel's 32-bit offsets reach 4 GiB of x and "
-                         "of W)", gemm_mode(s), static_cast<int>(kind), M, N, K);
-            return false;
+        if (static_cast<long>(more.tiles) + tiles_of(c.N) > 65535) break;
+        more.m[g - 1].W = static_cast<const uint8_t*>(c.W);
+        more.m[g - 1].scale = static_cast<const uint16_t*>(c.scale);
+        more.m[g - 1].out = static_cast<uint16_t*>(c.out);
+        more.m[g - 1].N = c.N;
+        more.m[g - 1].first = more.tiles;
+        more.tiles += tiles_of(c.N);
+        more.n = g;
     }
+    if (g == 1) return 0;
+    if (p.kernel == 1 && (gemm_mode(s) == 0 || gemm_mode(s) == 4)) {
+        int tm = 1, splits = 1;
+        wide::pick_shape(kind, p.terms, M, more.tiles * wide::kBN, K, cus, 0, &tm, &splits, nullptr);
+        p.tile_rows = 32 * tm;
+    }
+    return launch_planned(s, p, kind, M, mat[0].N, K, x, mat[0].W, mat[0].scale, mat[0].out, workspace, ws_bytes, more) ? g : -1;
 }
 
 }  // namespace mi
