@@ -141,6 +141,12 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
 // slices and park fp32 partial sums there; calls on one stream are ordered, so they can share it.
 bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x,
                  const void* W, const void* scale, void* out, void* workspace, size_t workspace_bytes);
+// out[M, N / 2] = swiglu of the gate and up columns of x W^T, W interleaved by 16 rows: 1 = launched,
+// 0 = no kernel with this epilogue for the call (nothing was launched), -1 = an error.
+int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
+                    void* out, void* workspace, size_t workspace_bytes);
+// runtime.hip: the same for a registered W where mi_linear would run the GEMM
+int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out);
 // The first of n projections of one x (M >= 2, the first accepted by gemm_supported) in one launch, where one
 // exists that gives what launch_gemm gives for each: returns how many it took, 0 for none (nothing was launched),
 // -1 on an error.  No output may overlap x or another output.

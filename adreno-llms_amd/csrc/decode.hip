@@ -863,9 +863,7 @@ inline size_t split_attention_lds(int D, int chunk_cap) {
 // gate[i] = fp16((g * sigmoid(g)) * up[i])   (QW/kernels/mlp.cl swiglu_inplace)
 __global__ void swiglu_kernel(uint16_t* __restrict__ gate, const uint16_t* __restrict__ up, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const float g = h_f(gate[i]), u = h_f(up[i]);
-        const float sig = rcp_rn(1.0f + exp_poly(-g));
-        gate[i] = f_h((g * sig) * u);
+        gate[i] = swiglu_h(gate[i], up[i]);
     }
 }
 
@@ -1277,30 +1275,26 @@ __global__ void swiglu_rows_kernel(uint16_t* __restrict__ gate, const uint16_t* 
         const u16x4 u4 = *reinterpret_cast<const u16x4*>(up + 4 * i);
         #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float g = h_f(g4[e]), u = h_f(u4[e]);
-            const float sig = rcp_rn(1.0f + exp_poly(-g));
-            g4[e] = f_h((g * sig) * u);
+            g4[e] = swiglu_h(g4[e], u4[e]);
         }
         *reinterpret_cast<u16x4*>(gate + 4 * i) = g4;
     }
 }
 
-// out[r][c] = swiglu(GU[r][c], GU[r][inter + c]): rows of a stacked gate|up projection ([M, 2 inter]),
-// four columns per thread and step (inter a multiple of 4); swiglu_kernel's operations per element
-__global__ void swiglu_stacked_kernel(const uint16_t* __restrict__ GU, uint16_t* __restrict__ out, int inter, long n4) {
+// out[r][c] = swiglu of column c of a stacked gate | up projection ([M, 2 inter]), four columns per thread and step:
+// `run` gate columns, the same up columns, and so on (run = inter: one matrix behind the other; run and inter are
+// multiples of 4); swiglu_kernel's operations per element
+__global__ void swiglu_stacked_kernel(const uint16_t* __restrict__ GU, uint16_t* __restrict__ out, int inter, int run, long n4) {
     typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
     const int c4n = inter >> 2;
     for (long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n4; i += static_cast<long>(gridDim.x) * blockDim.x) {
         const long r = i / c4n;
         const int c = static_cast<int>(i - r * c4n) * 4;
-        u16x4 g4 = *reinterpret_cast<const u16x4*>(GU + r * 2 * inter + c);
-        const u16x4 u4 = *reinterpret_cast<const u16x4*>(GU + r * 2 * inter + inter + c);
+        const uint16_t* src = GU + r * 2 * inter + c + c / run * run;
+        u16x4 g4 = *reinterpret_cast<const u16x4*>(src);
+        const u16x4 u4 = *reinterpret_cast<const u16x4*>(src + run);
         #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float g = h_f(g4[e]), u = h_f(u4[e]);
-            const float sig = rcp_rn(1.0f + exp_poly(-g));
-            g4[e] = f_h((g * sig) * u);
-        }
+        for (int e = 0; e < 4; ++e) g4[e] = swiglu_h(g4[e], u4[e]);
         *reinterpret_cast<u16x4*>(out + r * inter + c) = g4;
     }
 }
@@ -1672,8 +1666,9 @@ int mi_decoder_step(void* dec, void* stream) {
 }
 
 // Rows of n matrices of one kind and K (and their scales) copied into one matrix, registered like
-// its parts.  Null when the parts are not of one kind or memory is short; *failed on a HIP error.
-static void* stack_weights(Decoder* d, hipStream_t s, int n, const void* const* W, const int* N, int K, bool* failed) {
+// its parts: one behind the other, or (run > 0; parts of one N, a multiple of run) `run` rows of each in turn.  Null
+// when the parts are not of one kind or memory is short; *failed on a HIP error.
+static void* stack_weights(Decoder* d, hipStream_t s, int n, const void* const* W, const int* N, int K, int run, bool* failed) {
     WeightKind kind = WK_F16, k0 = WK_F16;
     const void* scale[4] = {nullptr, nullptr, nullptr, nullptr};
     int total = 0;
@@ -1694,11 +1689,16 @@ static void* stack_weights(Decoder* d, hipStream_t s, int n, const void* const* 
     }
     size_t at = 0;
     for (int i = 0; i < n; ++i) {
-        bool ok = MI_HIP_OK(hipMemcpyAsync(static_cast<char*>(w) + at * row, W[i], row * N[i], hipMemcpyDeviceToDevice, s));
-        if (ok && srow)
-            ok = MI_HIP_OK(hipMemcpyAsync(static_cast<char*>(sc) + at * srow, scale[i], srow * N[i], hipMemcpyDeviceToDevice, s));
-        if (!ok) { *failed = true; return nullptr; }
-        at += N[i];
+        // pieces of `len` rows, n pieces apart in the stack
+        const size_t len = run > 0 ? run : N[i], pieces = N[i] / len;
+        auto append = [&](void* dst, const void* src, size_t row_bytes) {
+            char* to = static_cast<char*>(dst) + at * row_bytes;
+            return MI_HIP_OK(run > 0 ? hipMemcpy2DAsync(to, n * len * row_bytes, src, len * row_bytes, len * row_bytes, pieces,
+                                                        hipMemcpyDeviceToDevice, s)
+                                     : hipMemcpyAsync(to, src, len * row_bytes, hipMemcpyDeviceToDevice, s));
+        };
+        if (!append(w, W[i], row) || (srow && !append(sc, scale[i], srow))) { *failed = true; return nullptr; }
+        at += len;
     }
     const int reg = k0 == WK_I8 ? mi_register_int8_weight(w, sc, total, K) : k0 == WK_Q4 ? mi_register_q4_weight(w, sc, total, K) : 1;
     return reg ? w : nullptr;
@@ -1728,6 +1728,10 @@ static bool ensure_prompt_rows(Decoder* d, hipStream_t s, int M) {
     return true;
 }
 
+// Rows of the gate matrix, then of the up matrix, that take turns in their stack: 16, as launch_gemm_glu takes them,
+// or, where the width is no multiple of 16, 0: one matrix behind the other.
+static int glu_run(int inter) { return inter % 16 == 0 ? 16 : 0; }
+
 // Every layer's q | k | v and gate | up matrices stacked into one registered matrix each, once.
 static bool ensure_stacked(Decoder* d, hipStream_t s) {
     if (d->stacked_built) return true;
@@ -1739,10 +1743,10 @@ static bool ensure_stacked(Decoder* d, hipStream_t s) {
     for (int l = 0; l < c.n_layers && !failed; ++l) {
         const void* const W3[3] = {d->wq[l], d->wk[l], d->wv[l]};
         const int N3[3] = {qd, kvd, kvd};
-        d->wqkv[l] = stack_weights(d, s, 3, W3, N3, Hd, &failed);
+        d->wqkv[l] = stack_weights(d, s, 3, W3, N3, Hd, 0, &failed);
         const void* const W2[2] = {d->wgate[l], d->wup[l]};
         const int N2[2] = {I, I};
-        if (!failed && I % 4 == 0) d->wgu[l] = stack_weights(d, s, 2, W2, N2, Hd, &failed);
+        if (!failed && I % 4 == 0) d->wgu[l] = stack_weights(d, s, 2, W2, N2, Hd, glu_run(I), &failed);
     }
     if (failed) {
         // nothing half-built stays behind: the next prompt starts over, and no registry entry
@@ -1882,8 +1886,10 @@ int mi_decoder_prefill(void* dec, void* stream, const int* tokens, int n_tokens,
         if (!add_then_norm(d->post_norm[l])) return 0;
         const uint16_t* act;                      // swiglu(gate, up), [M, inter]
         if (d->wgu[l]) {
-            if (!mi_linear(stream, M, 2 * I, Hd, XN, d->wgu[l], GU)) return 0;
-            hipLaunchKernelGGL(swiglu_stacked_kernel, dim3(gI), dim3(256), 0, s, GU, G2, I, nI / 4);
+            const int run = glu_run(I), fused = run ? linear_glu(s, M, 2 * I, Hd, XN, d->wgu[l], G2) : 0;
+            if (fused < 0 || (!fused && !mi_linear(stream, M, 2 * I, Hd, XN, d->wgu[l], GU))) return 0;
+            if (!fused)
+                hipLaunchKernelGGL(swiglu_stacked_kernel, dim3(gI), dim3(256), 0, s, GU, G2, I, run ? run : I, nI / 4);
             act = G2;
         } else {
             uint16_t *G = GU, *U = GU + static_cast<size_t>(cap) * I;

@@ -71,4 +71,15 @@ __device__ __forceinline__ float exp_poly(float x) {
     return ldexpf(p, static_cast<int>(n));
 }
 
+// fp16((g * sigmoid(g)) * u) of two fp16 values (QW/kernels/mlp.cl swiglu_inplace)
+__device__ __forceinline__ uint16_t swiglu_h(uint16_t gate, uint16_t up) {
+    const float g = h_f(gate), u = h_f(up);
+    const float sig = __fdiv_rn(1.0f, 1.0f + exp_poly(-g));
+    return f_h((g * sig) * u);
+}
+__device__ __forceinline__ uint32_t swiglu_h2(uint32_t gate, uint32_t up) {       // two of them
+    return swiglu_h(static_cast<uint16_t>(gate & 0xffffu), static_cast<uint16_t>(up & 0xffffu)) |
+           (static_cast<uint32_t>(swiglu_h(static_cast<uint16_t>(gate >> 16), static_cast<uint16_t>(up >> 16))) << 16);
+}
+
 }  // namespace mi

@@ -622,3 +622,15 @@ int mi_unpack_q4_to_int8(void* stream, const void* W, int N, int K, void* w8) {
 }
 
 }  // extern "C"
+
+namespace mi {
+
+int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out) {
+    if (!ensure_init()) return -1;
+    Entry e;
+    if (!resolve("mi_decoder_prefill", W, N, K, &e)) return -1;
+    if (!takes_gemm(s, e, M, N, K, x, W)) return 0;
+    return launch_gemm_glu(s, e.kind, M, N, K, x, W, e.scale, out, workspace_of(s), kWorkspaceBytes);
+}
+
+}  // namespace mi
