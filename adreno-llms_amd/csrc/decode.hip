@@ -683,8 +683,8 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float* sc = sm;                                            // [chunk_cap] scores, then exponentials
     float* red = sc + chunk_cap;                               // [8] block reductions
-    float* osum = red + 8;                                     // [wavefronts][D] partial outputs
-    uint16_t* qv = reinterpret_cast<uint16_t*>(osum + kSplitThreads / 64 * D);   // [D] q, [D] k, [D] v of the current position
+    float* osum = red + 8;                                     // [kSplitThreads / D][D] partial outputs
+    uint16_t* qv = reinterpret_cast<uint16_t*>(osum + kSplitThreads);   // [D] q, [D] k, [D] v of the current position
     uint16_t* kcur = qv + D;
     uint16_t* vcur = kcur + D;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -703,14 +703,10 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
     }
     const bool has_current = k1 == seq_k;                      // the block whose run ends with the current position
     // Everything the block reads from memory is asked for now, behind the position alone: the row of the
-    // thread's first key, its eight elements of the values of its first kAhead keys, and (below) the current
+    // thread's first key, the first kAhead values of the thread's output element, and (below) the current
     // position's q, k and v; the arithmetic then waits for one round trip, not for four in a row.
-    // Values: D / 8 neighbouring threads take a row, 16 bytes each, and the block kVKeys rows at a time, so that
-    // kAhead loads per thread are the first 256 keys (D = 64) of the run.  (Before, a thread took one element of every
-    // fourth row: 2 bytes per load, and keys past the 128th in batches of eight with a trip to memory each.  Steps of the
-    // 14-head model: position 3701 in 16 splits 674 -> 594 us, 2400 in 8 splits 714 -> 612 us, 300 in 8 splits 556 -> 538 us.)
-    constexpr int kVLanes = D / 8, kVKeys = kSplitThreads / kVLanes, kAhead = 8;
-    const int vl = tid % kVLanes, vg = tid / kVLanes;
+    constexpr int kGroups = kSplitThreads / D, kAhead = 32;
+    const int d = tid % D, grp = tid / D;
     const int c_first = k0 + tid;
     u32x4 kr_first[D / 8];
     // (a thread without such a key reads row 0 instead and does not use it: loads under a condition of
@@ -721,12 +717,11 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
         #pragma unroll
         for (int i = 0; i < D / 8; ++i) kr_first[i] = row[i];
     }
-    const uint16_t* const vbase = vc + kvh * D + 8 * vl;       // (16-byte aligned: D is a multiple of 64)
-    u32x4 v_first[kAhead];
+    uint16_t v_first[kAhead];
     #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-        const int c = k0 + vg + i * kVKeys;
-        v_first[i] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(c < k1 && c != pos ? c : 0) * kvd);
+        const int c = k0 + grp + i * kGroups;
+        v_first[i] = vc[static_cast<size_t>(c < k1 && c != pos ? c : 0) * kvd + kvh * D + d];
     }
     // q of the head (every block), k and v of the current position (the block that needs them); the block of
     // the group's first head also writes them to the caches and to the buffers a caller may inspect
@@ -804,46 +799,26 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
     for (int sft = 32; sft > 0; sft >>= 1) l += __shfl_xor(l, sft, 64);
     if (lane == 0) red[4 + wave] = l;
     __syncthreads();                                           // exponentials and the waves' sums are in LDS
-    // o: thread (vg, vl) sums elements 8 vl .. of the keys k0 + vg, k0 + vg + kVKeys, ..., then the threads of a
-    // wavefront with the same vl add theirs, then the wavefronts
-    float o[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    auto add_value = [&](int c, u32x4 v) {
-        if (c == pos) v = reinterpret_cast<const u32x4*>(vcur)[vl];
-        const float e = sc[c - k0];
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-        #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            o[2 * j] = fmaf(e, h_f(static_cast<uint16_t>(w[j] & 0xffffu)), o[2 * j]);
-            o[2 * j + 1] = fmaf(e, h_f(static_cast<uint16_t>(w[j] >> 16)), o[2 * j + 1]);
-        }
-    };
+    // o[d]: kSplitThreads / D groups of D threads, group g takes the keys k0 + g, k0 + g + groups, ...
+    float o = 0.0f;
     #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-        const int c = k0 + vg + i * kVKeys;
-        if (c < k1) add_value(c, v_first[i]);
+        const int c = k0 + grp + i * kGroups;
+        if (c < k1) o = fmaf(sc[c - k0], h_f(c == pos ? vcur[d] : v_first[i]), o);
     }
-    for (int c0 = k0 + vg + kAhead * kVKeys; c0 < k1; c0 += 4 * kVKeys) {
-        u32x4 v[4];
-        #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int c = c0 + u * kVKeys;
-            v[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(c < k1 && c != pos ? c : 0) * kvd);
-        }
-        #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (c0 + u * kVKeys < k1) add_value(c0 + u * kVKeys, v[u]);
+    #pragma unroll 8
+    for (int c = k0 + grp + kAhead * kGroups; c < k1; c += kGroups) {
+        const uint16_t v = c == pos ? vcur[d] : vc[static_cast<size_t>(c) * kvd + kvh * D + d];
+        o = fmaf(sc[c - k0], h_f(v), o);
     }
-    #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        #pragma unroll
-        for (int sft = 32; sft >= kVLanes; sft >>= 1) o[e] += __shfl_xor(o[e], sft, 64);
-    }
-    if (lane < kVLanes) {
-        #pragma unroll
-        for (int e = 0; e < 8; ++e) osum[wave * D + 8 * vl + e] = o[e];
-    }
+    osum[grp * D + d] = o;
     __syncthreads();
-    if (tid < D) mine[2 + tid] = (osum[tid] + osum[D + tid]) + (osum[2 * D + tid] + osum[3 * D + tid]);
+    if (tid < D) {
+        float t = osum[tid];
+        #pragma unroll
+        for (int g2 = 1; g2 < kGroups; ++g2) t += osum[g2 * D + tid];
+        mine[2 + tid] = t;
+    }
     if (tid == 0) {
         mine[0] = m;
         mine[1] = (red[4] + red[5]) + (red[6] + red[7]);
@@ -882,7 +857,7 @@ __global__ __launch_bounds__(D) void attention_merge_kernel(const float* __restr
 }
 
 inline size_t split_attention_lds(int D, int chunk_cap) {
-    return static_cast<size_t>(chunk_cap + 8 + kSplitThreads / 64 * D) * 4 + 3 * static_cast<size_t>(D) * 2;
+    return static_cast<size_t>(chunk_cap + 8 + kSplitThreads) * 4 + 3 * static_cast<size_t>(D) * 2;
 }
 
 // gate[i] = fp16((g * sigmoid(g)) * up[i])   (QW/kernels/mlp.cl swiglu_inplace)
