@@ -1,6 +1,7 @@
 // Host layer behind the C ABI: device plumbing, the weight registry and the
 // `pytorch_linear` dispatcher (QW/src/utils.cpp:758-823, LF/src/utils.cpp:1263-1374).
 #include "../../include/mi_linear.h"
+#include "batch_rule.h"
 #include "common.h"
 
 #include <atomic>
@@ -460,31 +461,25 @@ int mi_linear_argmax_static(void* stream, int N, int K, const void* x, const voi
     return launch_argmax_f16(as_stream(stream), logits, N, num_partials, token_out, ws) ? 1 : 0;
 }
 
-// True when [a, a+na) and [b, b+nb) share a byte.
-static bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
-    const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-    return pa < pb + nb && pb < pa + na;
-}
-
 int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
     if (!ensure_init()) return 0;
     if (!calls || n < 0) { MI_ERROR_FMT("mi_linear_batch: bad argument"); return 0; }
     // Consecutive calls that read the same x with the same M, K and weight kind, and whose outputs
-    // touch neither that x nor each other, cannot observe one another: they go out as one launch
-    // (q/k/v and gate/up do), GEMV calls always and GEMM calls where launch_gemm_group has a launch for
-    // them.  Everything else is enqueued call by call, in order.
+    // touch neither what one of them reads (x, weights, scales) nor each other, cannot observe one another:
+    // they go out as one launch (q/k/v and gate/up do), GEMV calls always and GEMM calls where
+    // launch_gemm_group has a launch for them.  Everything else is enqueued call by call, in order.
     const hipStream_t s = as_stream(stream);
     int i = 0;
     while (i < n) {
         const mi_linear_call& c0 = calls[i];
         GemvCall group[kMaxSegments];
+        CallMemory memory[kMaxSegments];
         int g = 0;
         bool gemm = false;
         Entry e0;
         if (c0.M >= 1 && c0.N > 0 && c0.K > 0 && c0.x && c0.W && c0.out &&
             resolve("mi_linear_batch", c0.W, c0.N, c0.K, &e0)) {
             gemm = takes_gemm(s, e0, c0.M, c0.N, c0.K, c0.x, c0.W);
-            const size_t xbytes = static_cast<size_t>(c0.M) * c0.K * 2;
             while ((gemm || c0.M < 16) && i + g < n && g < kMaxSegments) {
                 const mi_linear_call& c = calls[i + g];
                 Entry e;
@@ -494,10 +489,9 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
                     if (e.kind != e0.kind || e.N != c.N || e.K != c.K) break;
                     if (gemm && !takes_gemm(s, e, c.M, c.N, c.K, c.x, c.W)) break;
                 } else e = e0;
-                const size_t obytes = static_cast<size_t>(c.M) * c.N * 2;
-                bool clash = overlaps(c.out, obytes, c0.x, xbytes);
-                for (int j = 0; j < g && !clash; ++j)
-                    clash = overlaps(c.out, obytes, group[j].y, static_cast<size_t>(group[j].M) * group[j].N * 2);
+                memory[g] = call_memory(e.kind, c.M, c.N, c.K, c.x, c.W, e.scale, c.out);
+                bool clash = writes_what_reads(memory[g], memory[g]);
+                for (int j = 0; j < g && !clash; ++j) clash = !independent(memory[j], memory[g]);
                 if (clash) break;
                 GemvCall& d = group[g];
                 d.x = c.x; d.W = c.W; d.scale = e.scale; d.y = c.out;
@@ -515,7 +509,7 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
         } else if (g > 0 && !launch_gemv_group(s, group, g)) {
             return i;
         }
-        if (g == 0) {                                   // no launch for several: out aliases x, or a GEMM of its own
+        if (g == 0) {                                   // no launch for several: out aliases an operand, or a GEMM of its own
             if (!mi_linear(stream, c0.M, c0.N, c0.K, c0.x, c0.W, c0.out)) return i;
             g = 1;
         }
