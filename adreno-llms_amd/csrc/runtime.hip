@@ -467,7 +467,8 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
     // Consecutive calls that read the same x with the same M, K and weight kind, and whose outputs
     // touch neither what one of them reads (x, weights, scales) nor each other, cannot observe one another:
     // they go out as one launch (q/k/v and gate/up do), GEMV calls always and GEMM calls where
-    // launch_gemm_group has a launch for them.  Everything else is enqueued call by call, in order.
+    // launch_gemm_group has a launch for them (a call that mi_linear would send to the other of the two
+    // ends the run).  Everything else is enqueued call by call, in order.
     const hipStream_t s = as_stream(stream);
     int i = 0;
     while (i < n) {
@@ -487,7 +488,7 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
                     if (c.x != c0.x || c.K != c0.K || c.M != c0.M || c.N <= 0 || !c.W || !c.out) break;
                     if (!lookup(c.W, &e)) e = Entry{WK_F16, nullptr, c.N, c.K};
                     if (e.kind != e0.kind || e.N != c.N || e.K != c.K) break;
-                    if (gemm && !takes_gemm(s, e, c.M, c.N, c.K, c.x, c.W)) break;
+                    if (gemm != takes_gemm(s, e, c.M, c.N, c.K, c.x, c.W)) break;
                 } else e = e0;
                 memory[g] = call_memory(e.kind, c.M, c.N, c.K, c.x, c.W, e.scale, c.out);
                 bool clash = writes_what_reads(memory[g], memory[g]);

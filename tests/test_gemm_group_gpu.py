@@ -24,29 +24,47 @@ def _weights(kind, n, k, seed, keep):
     return qb
 
 
+def _together_as_one_by_one(queue, kind, rows, k, widths):
+    keep = []
+    x = mil.Buffer.from_host(mil.synth_normal_f16(5 + rows, 1.0, (rows, k)))
+    ws = [_weights(kind, n, k, 100 + j, keep) for j, n in enumerate(widths)]
+    fill = np.full(1, 0x7bff, np.uint16)
+    one = [mil.Buffer.from_host(np.repeat(fill, rows * n)) for n in widths]
+    many = [mil.Buffer.from_host(np.repeat(fill, rows * n)) for n in widths]
+    print(f"{kind} rows {rows} K {k} N {widths}", flush=True)
+    for n, w, o in zip(widths, ws, one):
+        assert mil.pytorch_linear(queue, rows, n, k, x, w, o)
+    calls = mil.make_calls([(rows, n, k, x, w, o) for n, w, o in zip(widths, ws, many)])
+    assert mil.linear_batch(queue, calls) == len(widths)
+    queue.finish()
+    for n, a, b in zip(widths, one, many):
+        assert np.array_equal(a.read(np.uint16, (rows, n)), b.read(np.uint16, (rows, n))), (rows, k, n)
+
+
 @pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
 @pytest.mark.parametrize("rows,mode", [(2, 5), (15, 5), (15, 3), (16, 0), (17, 0), (48, 0), (65, 0), (129, 0), (300, 0), (1025, 0)])
 def test_together_as_one_by_one(kind, rows, mode):
-    """Mode 0: the library's own choice of kernel, which below 16 rows may be the GEMV; 5 and 3 name the streaming
-    and the wide kernel."""
+    """Mode 0: the library's own choice of kernel; 5 and 3 name the streaming and the wide kernel."""
     assert mil.lib().mi_init(0) == 1
     queue = mil.Queue()
     assert mil.lib().mi_stream_set_modes(queue.handle, -1, mode if mode else -1)
     for k, widths in SHAPES:
-        keep = []
-        x = mil.Buffer.from_host(mil.synth_normal_f16(5 + rows, 1.0, (rows, k)))
-        ws = [_weights(kind, n, k, 100 + j, keep) for j, n in enumerate(widths)]
-        fill = np.full(1, 0x7bff, np.uint16)
-        one = [mil.Buffer.from_host(np.repeat(fill, rows * n)) for n in widths]
-        many = [mil.Buffer.from_host(np.repeat(fill, rows * n)) for n in widths]
-        print(f"{kind} rows {rows} K {k} N {widths}", flush=True)
-        for n, w, o in zip(widths, ws, one):
-            assert mil.pytorch_linear(queue, rows, n, k, x, w, o)
-        calls = mil.make_calls([(rows, n, k, x, w, o) for n, w, o in zip(widths, ws, many)])
-        assert mil.linear_batch(queue, calls) == len(widths)
-        queue.finish()
-        for n, a, b in zip(widths, one, many):
-            assert np.array_equal(a.read(np.uint16, (rows, n)), b.read(np.uint16, (rows, n)))
+        _together_as_one_by_one(queue, kind, rows, k, widths)
+    assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
+
+
+@pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
+@pytest.mark.parametrize("rows", [2, 4, 7, 12, 15])
+def test_together_where_gemv_and_gemm_meet(kind, rows):
+    """Below 16 rows a matrix goes to the GEMV or to the GEMM by its size: a neighbour of the other kind does not
+    change which, whichever of the two comes first.  (Q4 rows of GEMV in their exact mode: the throughput order is
+    chosen by the rows of a launch, and so not alike for one matrix and for several.)"""
+    assert mil.lib().mi_init(0) == 1
+    queue = mil.Queue()
+    assert mil.lib().mi_stream_set_modes(queue.handle, 0, -1)
+    for k, widths in [(896, [128, 896, 4864]), (896, [4864, 896, 128]), (576, [64, 576, 64, 1536]), (4864, [64, 896]), (104, [64, 896])]:
+        if kind != "q4" or k % 32 == 0:
+            _together_as_one_by_one(queue, kind, rows, k, widths)
     assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
 
 
