@@ -101,8 +101,8 @@ __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* 
         q[j] = *reinterpret_cast<const half8*>(QR + static_cast<size_t>(row) * qd + head * D + 8 * g + 32 * j);
 
     // Tiles travel memory -> registers -> LDS.  A request's address is a scalar base per tile plus a thread's
-    // constant offset.  Keys past the last are read as the last one and masked: 0 x a number, never 0 x what
-    // lies there; past the last tile that one is read again.
+    // constant offset.  Keys past the block's last are read as the last one, never what lies there, and masked; past
+    // the last tile that one is read again.
     struct Regs { u32x4 k[kKPieces]; u32x2 v[kVBlocks][4]; };
     const uint32_t row_bytes = static_cast<uint32_t>(kvd) * 2;
     const uint8_t* kbase = reinterpret_cast<const uint8_t*>(kc + kvh * D);
@@ -176,7 +176,8 @@ __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* 
             for (int j = 0; j < D / 32; ++j)
                 s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8*>(ktile + 16 * kt * kKPitch + 64 * j), q[j], s[kt], 0, 0, 0);
         }
-        if (k0 + kKeys - 1 > pos0 + q0) {                      // (keys up to the set's first query need no mask)
+        const bool masked = k0 + kKeys - 1 > pos0 + q0;        // (keys up to the set's first query need no mask)
+        if (masked) {
             #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
                 #pragma unroll
@@ -208,15 +209,59 @@ __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* 
             p[kt][0] = pack2(e[0], e[1]);
             p[kt][1] = pack2(e[2], e[3]);
         }
+        half8 pb[2];
         #pragma unroll
         for (int kp = 0; kp < 2; ++kp) {
-            const half8 pb = __builtin_bit_cast(half8, u32x4{p[2 * kp][0], p[2 * kp][1], p[2 * kp + 1][0], p[2 * kp + 1][1]});
-            l = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb, l, 0, 0, 0);
+            pb[kp] = __builtin_bit_cast(half8, u32x4{p[2 * kp][0], p[2 * kp][1], p[2 * kp + 1][0], p[2 * kp + 1][1]});
+            l = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb[kp], l, 0, 0, 0);
+        }
+        // `from` + the tile's product for elements 16 d ..; `keep` takes the 4 values of the lane's keys 16 n + 4 g ..
+        auto product = [&](int d, floatx4 from, auto keep) {
             #pragma unroll
-            for (int d = 0; d < D / 16; ++d) {
-                const u32x2 lo = *reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp);
-                const u32x2 hi = *reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp + 32);
-                acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, u32x4{lo.x, lo.y, hi.x, hi.y}), pb, acc[d], 0, 0, 0);
+            for (int kp = 0; kp < 2; ++kp) {
+                const u32x2 lo = keep(*reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp), 2 * kp);
+                const u32x2 hi = keep(*reinterpret_cast<const u32x2*>(vtile + 16 * d * kVPitch + 64 * kp + 32), 2 * kp + 1);
+                from = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, u32x4{lo.x, lo.y, hi.x, hi.y}), pb[kp], from, 0, 0, 0);
+            }
+            return from;
+        };
+        auto all = [](u32x2 v, int) { return v; };
+        if (!masked) {
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d) acc[d] = product(d, acc[d], all);
+            return;
+        }
+        // A masked key has probability 0, but 0 x inf and 0 x NaN are NaN: where a NaN comes up, the tile is multiplied
+        // once more per query of the set, with the values that query does not see as zeros, and the query's column kept.
+        floatx4 sums[D / 16];
+        bool nan = false;
+        #pragma unroll
+        for (int d = 0; d < D / 16; ++d) {
+            sums[d] = product(d, acc[d], all);
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) nan |= sums[d][r] != sums[d][r];
+        }
+        if (!__any(nan)) {
+            #pragma unroll
+            for (int d = 0; d < D / 16; ++d) acc[d] = sums[d];
+        } else {
+            #pragma unroll 1
+            for (int j = 0; j < kRows; ++j) {
+                asm volatile("" ::: "memory");     // (read again per query: kept, the values take the registers of the CU's second block)
+                const int seen = pos0 + q0 + j + 1 - k0 - 4 * g;           // of the keys 4 g .. of the tile, this many
+                auto own = [&](u32x2 v, int n) {
+                    #pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int left = seen - 16 * n - 2 * h;
+                        v[h] = left >= 2 ? v[h] : left == 1 ? v[h] & 0xffffu : 0u;
+                    }
+                    return v;
+                };
+                #pragma unroll
+                for (int d = 0; d < D / 16; ++d) {
+                    const floatx4 mine = product(d, acc[d], own);
+                    if (i == j) acc[d] = mine;
+                }
             }
         }
     };
