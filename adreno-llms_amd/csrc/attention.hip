@@ -307,7 +307,7 @@ __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* 
         }
     }
     if (!live) return;
-    const float inv = __fdiv_rn(1.0f, sum);
+    const float inv = __fdiv_rn(1.0f, sum + 1e-20f);           // (the reference's: 0 where every score is -inf)
     uint16_t* dst = out + static_cast<size_t>(row) * qd + head * D + 4 * g;
     #pragma unroll
     for (int d = 0; d < D / 16; ++d)

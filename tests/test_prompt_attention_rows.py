@@ -56,8 +56,9 @@ def _exact(q, k, v, pos0, n_heads, n_kv, head):
     s[unseen] = -np.inf
     size = np.where(unseen, 0.0, np.abs(np.nan_to_num(qh, posinf=0, neginf=0)) @ np.abs(np.nan_to_num(kh, posinf=0, neginf=0)).T) / np.sqrt(d)
     with np.errstate(invalid="ignore"):
-        p = np.exp(s - np.max(s, axis=1, keepdims=True))
+        p = np.exp(s - np.max(s, axis=1, keepdims=True))         # NaN where a row has no weight at all
         p /= np.sum(p, axis=1, keepdims=True)
+    p[np.all(s == -np.inf, axis=1)] = 0.0                    # no key at all: the reference's sum + 1e-20 makes that 0
     fin = np.where(np.isfinite(vh), vh, 0.0)
     o = p @ fin
     t = p @ np.abs(fin) + np.abs(o)                          # >= sum P |v - o|
@@ -132,3 +133,20 @@ def test_values_that_are_not_finite_stay_behind_the_mask(d, n_heads, n_kv, rows,
             v[last - back, (11 * i) % (n_kv * d)] = what
     k[last - min(3, rows - 1), d * (n_kv - 1)] = np.nan
     _compare(_launch(queue, q, k, v, pos0, n_heads, n_kv), q, k, v, pos0, n_heads, n_kv)
+
+
+@pytest.mark.parametrize("d,n_heads,n_kv,rows,pos0", SHAPES)
+def test_scores_of_minus_infinity(d, n_heads, n_kv, rows, pos0):
+    """Every other key has a score of -inf, or every key of the first tiles, or every key: no weight, and where no key
+    has any the output is 0 (QW/kernels/attention.cl gqa_softmax divides by the sum + 1e-20)."""
+    assert mil.lib().mi_init(0) == 1
+    queue = mil.Queue()
+    rng = np.random.default_rng(rows + pos0)
+    keys = np.arange(pos0 + rows)
+    for what in (keys % 2 == 0, keys < 150, keys >= 0):
+        q, k, v = _operands(rng, d, n_heads, n_kv, rows, pos0, np.zeros(pos0 + rows))
+        for head in range(n_heads):
+            q[:, head * d] = np.abs(q[:, head * d]) + np.float16(0.5)
+        for head in range(n_kv):
+            k[what, head * d] = -np.inf
+        _compare(_launch(queue, q, k, v, pos0, n_heads, n_kv), q, k, v, pos0, n_heads, n_kv)
