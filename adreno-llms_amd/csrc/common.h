@@ -147,6 +147,8 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
                     void* out, void* workspace, size_t workspace_bytes);
 // runtime.hip: the same for a registered W where mi_linear would run the GEMM
 int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out);
+// whether mi_linear would run the GEMM (and not rows of GEMV) for the call
+bool linear_takes_gemm(hipStream_t s, int M, int N, int K, const void* x, const void* W);
 // The first of n projections of one x (M >= 2, the first accepted by gemm_supported) in one launch, where one
 // exists that gives what launch_gemm gives for each: returns how many it took, 0 for none (nothing was launched),
 // -1 on an error.  No output may overlap x or another output.

@@ -1816,9 +1816,18 @@ int mi_decoder_prefill(void* dec, void* stream, const int* tokens, int n_tokens,
                                                       256 * 2 * (1 + kPromptTile) + kMaxPositions * 6))))
             return 0;
     }
-    // Attention on the matrix cores unless the projections run as rows of GEMV (then the whole prompt keeps
-    // the reference's order, bit for bit).
-    const bool matrix_attention = M > 1 && gemm_mode(s) != 1 && attention_prompt_supported(D);
+    // A layer's attention runs on the matrix cores where any of its projections does.  Where all of them run as rows
+    // of GEMV (mode 1; in the default mode a few rows, whose weights mi_linear keeps on the GEMV) the layer keeps
+    // the reference's order, and a prompt of such layers leaves the cache rows and logits of single-token steps bit for bit.
+    auto matrix_attention = [&](int l) {
+        if (M < 2 || gemm_mode(s) == 1 || !attention_prompt_supported(D)) return false;
+        auto gemm = [&](int N, int K, const void* x, const void* W) { return linear_takes_gemm(s, M, N, K, x, W); };
+        return (d->wqkv[l] ? gemm(qd + 2 * kvd, Hd, XN, d->wqkv[l])
+                           : gemm(qd, Hd, XN, d->wq[l]) || gemm(kvd, Hd, XN, d->wk[l]) || gemm(kvd, Hd, XN, d->wv[l])) ||
+               gemm(Hd, qd, ATT, d->wo[l]) ||
+               (d->wgu[l] ? gemm(2 * I, Hd, XN, d->wgu[l]) : gemm(I, Hd, XN, d->wgate[l]) || gemm(I, Hd, XN, d->wup[l])) ||
+               gemm(Hd, I, d->wgu[l] ? G2 : GU, d->wdown[l]);
+    };
     // one block per key/value head and row where the group's scores fit the LDS of a CU (160 KB, less
     // the kernel's few static bytes)
     constexpr size_t kGroupLdsMost = 160 * 1024 - 256;
@@ -1870,7 +1879,7 @@ int mi_decoder_prefill(void* dec, void* stream, const int* tokens, int n_tokens,
                            static_cast<const uint16_t*>(d->bk[l]), static_cast<const uint16_t*>(d->bv[l]), d->cosT, d->sinT,
                            kc, vc, QR, pos0, c.n_heads, c.n_kv_heads, D, ldq, ldkv);
         if (!launched()) return 0;
-        if (matrix_attention) {
+        if (matrix_attention(l)) {
             if (!launch_attention_prompt(s, QR, kc, vc, ATT, M, pos0, c.n_heads, c.n_kv_heads, D, scale)) return 0;
         } else if (grouped && D == 64)
             hipLaunchKernelGGL(attention_group_kernel<64>, dim3(c.n_kv_heads, M), dim3(256), grp_lds, s, QR, kc, vc, ATT, pos0,

@@ -620,6 +620,12 @@ int mi_unpack_q4_to_int8(void* stream, const void* W, int N, int K, void* w8) {
 
 namespace mi {
 
+bool linear_takes_gemm(hipStream_t s, int M, int N, int K, const void* x, const void* W) {
+    Entry e;
+    if (!lookup(W, &e)) e = Entry{WK_F16, nullptr, N, K};
+    return takes_gemm(s, e, M, N, K, x, W);
+}
+
 int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out) {
     if (!ensure_init()) return -1;
     Entry e;

@@ -236,3 +236,56 @@ def test_prompt_other_geometries_bit_for_bit(name, cfg, n_prompt):
         gd.close()
     finally:
         mil.lib().mi_set_gemm_mode(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["i8", "f16", "q4"])
+@pytest.mark.parametrize("n_heads,n_kv,head_dim,hidden,inter", [(4, 2, 64, 256, 512), (9, 3, 64, 576, 768), (4, 2, 128, 320, 256)])
+def test_default_mode_prompt_on_the_gemv_equals_steps_bit_for_bit(kind, n_heads, n_kv, head_dim, hidden, inter):
+    """The default mode, few rows: where every projection of the prompt is one that mi_linear runs as rows of GEMV, the
+    logits (and those of steps on top of its cache rows) are those of single-token steps bit for bit."""
+    assert mil.lib().mi_init(0) == 1
+    mil.lib().mi_set_gemv_mode(0)
+    try:
+        queue = mil.Queue()
+        cfg = dict(hidden=hidden, inter=inter, n_heads=n_heads, n_kv_heads=n_kv, head_dim=head_dim, n_layers=2, vocab=512,
+                   max_pos=200, rms_eps=1e-6, rope_theta=10000.0)
+        m = Model(cfg, seed=51) if kind == "i8" else KindModel(cfg, kind, seed=51)
+        gd = GpuDecoder(m, queue)
+        qd, kvd = n_heads * head_dim, n_kv * head_dim
+        x, w = mil.Buffer(2 * 16 * max(hidden, inter, qd)), mil.Buffer(2 * max(hidden, inter, qd) * max(qd + 2 * kvd, 2 * inter, hidden))
+        register = {"i8": mil.nnopt_register_int8_weight, "q4": mil.nnopt_register_q4_weight}.get(kind)
+
+        def on_the_gemv(rows):
+            for n, k in ((qd + 2 * kvd, hidden), (hidden, qd), (2 * inter, hidden), (hidden, inter)):
+                if register:
+                    assert register(w, x, n, k)
+                kernel = mil.linear_plan(queue, rows, n, k, x, w)[0]
+                if register:
+                    mil.nnopt_unregister_weight(w)
+                if kernel != 0:
+                    return False
+            return True
+
+        tried = 0
+        for rows in (2, 3, 4, 6, 8, 12):
+            if not on_the_gemv(rows):
+                continue
+            tried += 1
+            for before in (0, 130):
+                ids = _prompt(before + rows, cfg["vocab"], rows + before)
+                want = gd.greedy(ids, 3)
+                logits = gd.logits()
+                if before:
+                    assert gd.greedy(ids[:before], 1)
+                assert gd.dec.prefill(queue, ids[before:], before)
+                got = [gd.dec.read(queue)[1]]
+                for _ in range(2):
+                    assert gd.dec.step(queue)
+                    got.append(gd.dec.read(queue)[1])
+                print(f"{kind} {hidden} {rows} rows at {before}", flush=True)
+                assert got == want and np.array_equal(gd.logits(), logits)
+        assert tried
+        gd.close()
+    finally:
+        mil.lib().mi_set_gemv_mode(1)
