@@ -81,8 +81,8 @@ __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* 
     const int nrep = n_heads / n_kv_heads, kvd = n_kv_heads * D, qd = n_heads * D;
     const int sets = (M + kRows - 1) / kRows * nrep;           // of a key/value head
     const int per_head = (sets + kSets - 1) / kSets;
-    // Longest rows first.  (mirror > 0: the blocks from number `mirror` on, one CU's worth, are taken from
-    // the short end: they share a CU with the longest ones.)
+    // Longest rows first.  (mirror > 0: the blocks from number `mirror` on, the second of their CU, are taken from
+    // the short end: they share it with the longest ones.)
     int rank = blockIdx.x;
     if (mirror && rank >= mirror) rank = per_head * n_kv_heads - 1 - (rank - mirror);
     const int kvh = rank % n_kv_heads, b = per_head - 1 - rank / n_kv_heads;
@@ -330,9 +330,14 @@ bool launch_flash(hipStream_t s, const uint16_t* QR, const uint16_t* kc, const u
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                   static_cast<int>(lds)))))
         return false;
+    // More blocks than CUs and at most two per CU, all resident at once: a CU's second block is one of the shortest where
+    // its first is one of the longest.  us with / without, 2048 rows: 14 heads over 2 22.7 / 24.6, 15 over 5 23.0 / 24.9,
+    // 9 over 3 21.1 / 21.6, width 128, 16 over 4 49.5 / 54.0.  Where LDS holds one block, the second round has to go on
+    // with the long ones (width 128 in two slices at 1000 rows 29.0 / 24.4).
     const int total = flash_blocks(M, n_heads, n_kv_heads, WAVES, KS), cus = device_info().cus;
+    const bool mirror = 2 * lds <= 160 * 1024 && total > cus && total <= 2 * cus;
     hipLaunchKernelGGL(kern, dim3(total), dim3(64 * WAVES), lds, s, QR, kc, vc, out, M, pos0, n_heads, n_kv_heads,
-                       scale * 1.44269504088896341f, total > cus && total <= 2 * cus ? cus : 0);
+                       scale * 1.44269504088896341f, mirror ? cus : 0);
     return MI_HIP_OK(hipGetLastError());
 }
 
