@@ -4,9 +4,15 @@
 //
 // The kernels of decode.hip that keep the reference's order of operations are bound by that order: one
 // chain of additions over the keys per output element and per denominator, on the vector units.  Where
-// the caller has the projections run on the matrix cores, the sums run in another order anyway, and this
-// kernel takes their place: fp16 products, fp32 sums, scores and exponentials kept in fp32 (the reference
-// order rounds both to fp16), probabilities rounded to fp16 once, before they meet the values.
+// a layer's projections run on the matrix cores, the sums run in another order anyway, and this
+// kernel takes their place: fp16 products, fp32 sums, scores kept in fp32 (the reference order rounds them
+// to fp16), exponentials rounded to fp16 once, before they are summed and before they meet the values (the
+// reference order sums them in fp32 and rounds exponential and probability).  The denominator takes the rounded
+// ones too because an error of one then moves the output by that key's distance from it only.  Error of an fp16
+// output against fp64 in a numpy model of the roundings (37 to 2048 keys, scores of standard deviation 0.3 to 4,
+// values of mean 0 to 3), 2-norm: reference order 1.9e-4 to 1.5e-3, this order 1.9e-4 to 3.2e-4, with unrounded
+// terms in the denominator up to 2 % more.  Logits after 8 layers, 37 to 2048 rows, against an fp64 model: 1.2e-3 to
+// 3.2e-3 either way (mean of 14 prompts 2.1e-3).
 #include "common.h"
 #include "device_math.h"
 
@@ -53,15 +59,16 @@ constexpr size_t flash_lds(int D, int KS) { return 2 * KS * tile_bytes(D); }
 // not matter as long as the A operand brings the same ones), so probabilities never go through LDS.  The
 // values are transposed on their way into LDS, 4 keys x 4 elements per thread in registers.
 // LDS pitches: key rows 2 D + 16 bytes (16-byte reads of 16 consecutive rows), value rows (one element,
-// 64 keys) 136 bytes (8-byte reads of 16 consecutive rows): either spreads over all banks.
+// 64 keys) 136 bytes (8-byte reads of 16 consecutive rows): the addresses of either spread over all banks (the counters
+// below show conflicts all the same; the value rows' writes, four rows apart, meet two to a bank).
 //
-// What bounds it: a wavefront alone on its SIMD takes 0.8 us per tile, of which the matrix cores work a
-// sixth; the reads from LDS (16 KB per wavefront and tile), the exponentials and the waits between the
-// phases are the rest, and they overlap only across wavefronts.  14 heads over 2 key/value heads, 2048
-// rows: 433 us in the reference's order (attention_group_kernel), 24.3 us here (0.31 of the rate a large
-// matrix product reaches, causal half counted); 300 rows at position 900: 96 -> 13.2 us.  Requesting tiles
-// two ahead, forming the next tile's scores under the current tile's exponentials, and two sets per
-// wavefront (27.9 us) were no faster.
+// What bounds it: a wavefront alone on its SIMD takes 0.8 us per tile; the reads from LDS (16 KB per wavefront and
+// tile), the exponentials and the waits between the phases overlap only across wavefronts.  Counters at 2048 rows,
+// 14 heads over 2: matrix cores busy 17 % of the SIMD-cycles, LDS 52 % of the CU-cycles (38 % of that bank conflicts).
+// us per launch, launches back to back: 433 in the reference's order (attention_group_kernel), 22.7 here (0.33
+// PFLOP/s, causal half counted; a large matrix product reaches 1.5); 300 rows at position 900: 96 -> 11.4.
+// Requesting tiles two ahead, forming the next tile's scores under the current tile's exponentials, and two sets
+// per wavefront were no faster.
 template <int D, int WAVES, int KS>
 __global__ __launch_bounds__(64 * WAVES) void flash_rows_kernel(const uint16_t* __restrict__ QR, const uint16_t* __restrict__ kc,
                                                          const uint16_t* __restrict__ vc, uint16_t* __restrict__ out, int M,
@@ -349,18 +356,22 @@ bool launch_attention_prompt(hipStream_t s, const uint16_t* QR, const uint16_t* 
                              int pos0, int n_heads, int n_kv_heads, int head_dim, float scale) {
 #define MI_FLASH(D, WAVES, KS) return launch_flash<D, WAVES, KS>(s, QR, kc, vc, out, M, pos0, n_heads, n_kv_heads, scale)
     // A set's chain of tiles bounds the launch (0.8 us per tile while a wavefront has its SIMD to itself), so the
-    // keys of a set go over several wavefronts, and as many of those share a CU as there are blocks for.  Measured
-    // at 14 heads over 2 (head width 64), us, eight wavefronts / 2 per set, 4 / 2, 8 / 4:
-    //   2048 rows 24.3 / 31.6 / 41.2, 1000 rows 13.3 / 13.4 / 17.2: enough blocks of 8 / 2 for the chip;
-    //   300 rows at 900 15.2 / 14.3 / 13.2, 40 at 1500 17.4 / 17.0 / 14.9: few blocks, long chains;
-    //   100 rows 5.2 / 4.7 / 6.0, 40 at 300 7.2 / 6.7 / 7.5: a tile or a few per wavefront either way.
+    // keys of a set go over several wavefronts, and as many of those share a CU as there are blocks for.  us, launches
+    // back to back, eight wavefronts / 2 per set, 4 / 2, 8 / 4, head width 64, at 14 heads over 2 (15 over 5 within 0.3
+    // of it) and 9 over 3:
+    //   2048 rows 22.2 / 28.9 / 37.4, 21.1 / 21.9 / 25.8; 1000 rows 12.2 / 12.2 / 14.7, 11.9 / 11.7 / 10.3 (8 / 4 by
+    //   the rule): enough blocks of 8 / 2 for the chip;
+    //   300 rows at 900 14.2 / 13.4 / 11.4, 14.1 / 13.4 / 11.3; 40 at 1500 16.9 / 16.4 / 13.8, 16.7 / 16.3 / 13.8: few
+    //   blocks, long chains (in between, 600 rows, 8.9 / 8.6 / 10.0 and 8.8 / 8.2 / 8.4, the line is not at its best);
+    //   100 rows 4.7 / 4.0 / 5.5, 40 at 300 6.8 / 6.1 / 6.9: a tile or a few per wavefront either way.
     const int cus = device_info().cus;
     if (head_dim == 64) {
         if (flash_blocks(M, n_heads, n_kv_heads, 8, 2) * 4 >= cus * 3) MI_FLASH(64, 8, 2);
         if (pos0 + M <= 512) MI_FLASH(64, 4, 2);
         MI_FLASH(64, 8, 4);
     }
-    // (head width 128, 16 heads over 4, four wavefronts, 1 / 2 per set: 2048 rows 52.6 / 83.4, 300 at 900 29.6 / 24.6)
+    // (head width 128, 16 heads over 4, four wavefronts, 1 / 2 per set: 2048 rows 49.5 / 77.2, 1000 rows 25.9 / 24.4,
+    //  300 at 900 29.9 / 23.0)
     if (flash_blocks(M, n_heads, n_kv_heads, 4, 1) >= cus) MI_FLASH(128, 4, 1);
     MI_FLASH(128, 4, 2);
 #undef MI_FLASH

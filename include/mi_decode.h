@@ -70,10 +70,11 @@ int   mi_decoder_step(void* decoder, void* stream);
  * writes their KV rows (rows below pos0 are read as they are), leaves the greedy token after the
  * last one as the device token and pos0 + n_tokens as the device position: the state n_tokens
  * calls of mi_decoder_step with the tokens forced would leave.  The cache rows and the logits
- * are those of such steps bit for bit when the M > 1 projections run as rows of GEMV
- * (mi_set_gemm_mode(1), the reference's quantised prefill, LF/src/model.cpp:243-250), and within
- * the GEMM's tolerance of them on the matrix cores, where the attention of head widths 64 and 128 runs too
- * (fp16 products, fp32 scores, exponentials and sums).  pos0 + n_tokens <= max_pos.  The first prompt
+ * are those of such steps bit for bit when the M > 1 projections all run as rows of GEMV
+ * (mi_set_gemm_mode(1), the reference's quantised prefill, LF/src/model.cpp:243-250; in the default mode a few
+ * tokens, where mi_linear keeps them there), and within the GEMM's tolerance of them on the matrix cores, where
+ * the attention of head widths 64 and 128 runs too (fp16 products, fp32 scores and sums; an exponential is rounded
+ * to fp16 before it is summed and before it meets the values).  pos0 + n_tokens <= max_pos.  The first prompt
  * makes device copies of every layer's q, k, v and gate, up matrices stacked into one matrix each
  * (the reference's stacked qkv, QW/src/layers/attention.cpp:414; as much memory again as those
  * matrices), so that the projections of one input are one GEMM; it, and any longer prompt later,
@@ -99,7 +100,7 @@ int   mi_decoder_read(void* decoder, void* stream, int* pos, int* token);
  * real numbers summed in another order, without the fp16 roundings of the probabilities, within
  * max-abs/rel 1e-3 and cosine 0.9999 of the default, not bit-identical; one launch more per layer.
  * head_dim 64 or 128.  Measured on Qwen2.5-0.5B shapes: 16 is the fastest up to about 2000 positions, 32 beyond
- * (position 4000: 594 us per step against 659 with 16 and 2723 in the reference's order); below about 150
+ * (position 4000: 623 us per step against 688 with 16 and 1511 in the reference's order); below about 250
  * positions the default is faster.  Allocates once; call it between steps, never under graph capture (a graph
  * captured afterwards keeps the mode it was captured in).  No counterpart in the reference. */
 int   mi_decoder_set_attention_splits(void* decoder, int splits);

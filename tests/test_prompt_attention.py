@@ -2,10 +2,13 @@
 keep the reference's order (mi_set_gemm_mode(1)), which equal the CPU harness bit for bit (test_prefill.py).
 
 Three layers, so that every row's attention reaches the compared residual stream through the keys and values of
-the next layers, not the last row's alone.  Bound: the reference's order rounds scores to fp16, half a step of
-2^-9 at scores up to 8, so the two sides' probabilities differ by up to 2e-3 of themselves, with random signs;
-an attention output, an average over keys, differs by less, and the projections by a fp16 rounding each: 2e-3
-of the residual stream's 2-norm covers three layers of it (measured 3e-4 to 7e-4)."""
+the next layers, not the last row's alone.  What these models bring: scores below 1 nat, nearly even weights, and one
+comparison per prompt, of the last row; single rows, large scores and values that are not finite are
+test_prompt_attention_rows.py's.  Bound: the reference's order rounds scores (half a step of 2^-11 below 1),
+exponentials and probabilities to fp16, the matrix cores' the exponentials, so the two sides' probabilities differ by up
+to 2e-3 of themselves, with random signs; an attention output, an average over keys, differs by less, and the
+projections by a fp16 rounding each: 2e-3 of the residual stream's 2-norm covers three layers of it (measured 3e-4 to
+7e-4)."""
 import numpy as np
 import pytest
 
