@@ -82,6 +82,12 @@ constexpr int kMaxSegments = 4;
 bool launch_gemv(hipStream_t s, const GemvCall& c);
 // n <= kMaxSegments calls that share x, K, M, weight kind and epilogue, as one launch.
 bool launch_gemv_group(hipStream_t s, const GemvCall* calls, int n);
+// n <= kMaxMany EPI_STORE calls of one M and weight kind, each accepted by gemv_many_takes, of any x, K and N, none of
+// which reads or writes what another one writes, as one launch.  run_of: calls of the same run (equal numbers) are
+// computed as launch_gemv_group computes that run.
+constexpr int kMaxMany = 64;
+bool gemv_many_takes(const GemvCall& c);
+bool launch_gemv_many(hipStream_t s, const GemvCall* calls, const int* run_of, int n);
 bool gemv_takes_norm(WeightKind kind, int K);    // GemvCall::norm_w is supported for this kind and K
 bool gemv_takes_swiglu(WeightKind kind, int K);  // EPI_SWIGLU is supported for this kind and K
 // Candidates a launch with GemvCall::am_v writes (one per wavefront of its grid), and their upper bound.

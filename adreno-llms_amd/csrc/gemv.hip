@@ -244,8 +244,9 @@ __device__ __forceinline__ Seg find_segment(const SegList& L, int rb) {
 // multiplies the current one.  Without PIPE a wavefront is expected to own one batch.
 // RB row batches are fetched together, so that narrow rows (Q4, small K) still keep enough
 // bytes in flight per wavefront.
-template <int KIND, int KT, int VL, int EPI, bool PIPE, int RB, bool AM = false>
-__global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegList L) {
+// first: the wavefront's first row batch (its number among the nw wavefronts of the launch), m: its row of x.
+template <int KIND, int KT, int VL, int EPI, bool PIPE, int RB, bool AM>
+__device__ __forceinline__ void fixed_k_rows(MI_HOT_PARAMS, const SegList& L, const int first, const int nw, const int m) {
     using T = WT<KIND>;
     constexpr int LPR = kWave / VL, RPW = VL;
     constexpr int EIT = kWave * T::EPV;                 // elements per K-iteration
@@ -256,11 +257,9 @@ __global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegL
     constexpr int ITB = kWave * T::BPV;                 // weight bytes per row and iteration
 
     const int lane = threadIdx.x % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int g = lane % LPR, r = lane / LPR;
     const int koff = g * VL * T::EPV;
     const Consts cst = make_consts();
-    const int m = blockIdx.y;
     x += static_cast<size_t>(m) * KT;
 
     // One row batch in registers: weights, scales and (EPI_ADD) the residual, all fetched
@@ -307,20 +306,17 @@ __global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegL
         // (last: y's address is the one argument that does not come in registers)
         if constexpr (EPI == EPI_ADD) b.res = b.ybase[rr];
     };
-    const int nw = gridDim.x * kWavesPerBlock;
-    int rb = blockIdx.x * kWavesPerBlock + wave;
-    const int wid = rb;
+    int rb = first;
     const TieRule rule{L.am_chunk};
     Cand top{kArgmaxNone, 0};                                 // AM: best row so far (lanes with g == 0)
     if (rb >= hnbatch) {
         if constexpr (AM) {
-            if (lane == 0) { L.am_v[wid] = kArgmaxNone; L.am_i[wid] = 0; }
+            if (lane == 0) { L.am_v[first] = kArgmaxNone; L.am_i[first] = 0; }
         }
         return;
     }
     constexpr int GB = PIPE ? RB : 1;
     struct Group { Batch b[GB]; };
-    const int first = rb;
     // A wavefront owns batches rb, rb + nw, rb + 2 nw, ...; it takes them GB at a time.  A batch
     // index past the end is replaced by the wavefront's first batch (a cached re-read whose
     // result is dropped), so every fetch issues the same loads.
@@ -503,8 +499,14 @@ __global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegL
     }
     if constexpr (AM) {
         const Cand w = rule.best_of_wave(top);
-        if (lane == 0) { L.am_v[wid] = w.v; L.am_i[wid] = w.i; }
+        if (lane == 0) { L.am_v[first] = w.v; L.am_i[first] = w.i; }
     }
+}
+__device__ __forceinline__ int block_wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
+template <int KIND, int KT, int VL, int EPI, bool PIPE, int RB, bool AM = false>
+__global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegList L) {
+    fixed_k_rows<KIND, KT, VL, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L,
+                                                  blockIdx.x * kWavesPerBlock + block_wave(), gridDim.x * kWavesPerBlock, blockIdx.y);
 }
 
 // ---- Q4, throughput variant --------------------------------------------------------
@@ -521,18 +523,16 @@ __global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegL
 //     block scale multiplies the block sum once.
 // 16 lanes still share a row and a wavefront still streams row batches of 4 rows with the
 // same double-buffered fetch; each lane owns one scale block per K-iteration.
-template <int KT, int EPI, bool PIPE, int RB, bool AM = false>
-__global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegList L) {
+template <int KT, int EPI, bool PIPE, int RB, bool AM>
+__device__ __forceinline__ void q4_fast_rows(MI_HOT_PARAMS, const SegList& L, const int first, const int nw, const int m) {
     constexpr int EIT = 512;                            // elements per K-iteration (16 lanes x 32)
     constexpr int NIT = (KT + EIT - 1) / EIT;
     constexpr int ROWB = KT / 2;
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
     const int lane = threadIdx.x % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int g = lane % 16, r = lane / 16;
     const int koff = g * 32;
-    const int m = blockIdx.y;
     x += static_cast<size_t>(m) * KT;
 
     struct Batch {
@@ -566,14 +566,12 @@ __global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegL
     // The activations are requested first and the first weights right behind them, without a
     // wait in between: loads return in order, so the pairing of x below can run while the
     // weights are still on their way.
-    const int nw = gridDim.x * kWavesPerBlock;
-    int rb = blockIdx.x * kWavesPerBlock + wave;
-    const int wid = rb;
+    int rb = first;
     const TieRule rule{L.am_chunk};
     Cand top{kArgmaxNone, 0};                                 // AM: best row so far (lanes with g == 0)
     if (rb >= hnbatch) {
         if constexpr (AM) {
-            if (lane == 0) { L.am_v[wid] = kArgmaxNone; L.am_i[wid] = 0; }
+            if (lane == 0) { L.am_v[first] = kArgmaxNone; L.am_i[first] = 0; }
         }
         return;
     }
@@ -588,7 +586,6 @@ __global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegL
     }
     struct Group { Batch b[PIPE ? RB : 1]; };
     constexpr int GB = PIPE ? RB : 1;
-    const int first = rb;
     auto fetch_group = [&](Group& gr, int at) {
         #pragma unroll
         for (int u = 0; u < GB; ++u) fetch(gr.b[u], at + u * nw < hnbatch ? at + u * nw : first);
@@ -680,8 +677,87 @@ __global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegL
     }
     if constexpr (AM) {
         const Cand w = rule.best_of_wave(top);
-        if (lane == 0) { L.am_v[wid] = w.v; L.am_i[wid] = w.i; }
+        if (lane == 0) { L.am_v[first] = w.v; L.am_i[first] = w.i; }
     }
+}
+template <int KT, int EPI, bool PIPE, int RB, bool AM = false>
+__global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegList L) {
+    q4_fast_rows<KT, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L,
+                                        blockIdx.x * kWavesPerBlock + block_wave(), gridDim.x * kWavesPerBlock, blockIdx.y);
+}
+
+// Row batches a pipelined wavefront fetches at once: enough for about 3.5 KB of weights.
+constexpr int group_size(int kind, int K, int vl) {
+    const int batch_bytes = vl * (K / (kind == WK_Q4 ? 8 : 4)) * (kind == WK_F16 ? 8 : 4);
+    return batch_bytes <= 1280 ? 4 : (batch_bytes <= 2560 ? 2 : 1);
+}
+
+// ---- many independent GEMVs in one launch --------------------------------------------
+//
+// Calls of a batch that cannot observe one another's results, whatever their x and K (the batch's host code
+// checks that): their row batches stream side by side, so a short matrix no longer has the chip to itself for the
+// 1.6 us that a dependent launch takes at least, and a launch of a few MB no longer ends before the memory
+// system is at its rate (169 int8 calls, 495 MB, in three such launches: 93 us, 5.3 TB/s).  A block works on one call; blocks are dealt out to calls by their bytes (launch_gemv_many),
+// every row's sum is that of the kernels above, in their order.
+struct ManyCalls {
+    int n = 0;
+    uint16_t first[kMaxMany] = {};                       // a call's first block
+    struct Call {
+        const uint16_t* x;
+        const uint8_t* W;
+        const uint16_t* sc;
+        uint16_t* y;
+        int N, nbatch;                                   // rows of W, row batches of many_tile(kind, K) of them
+        int waves;                                       // wavefronts that share the batches
+        int code;                                        // K, or -K for Q4 in the throughput arithmetic
+    } c[kMaxMany] = {};
+};
+static_assert(sizeof(ManyCalls) <= 4096, "kernel arguments");
+
+// Rows per wavefront and load instruction in such a launch: the widest tile, as pick_vl has it for a long stream
+constexpr int many_tile(int kind, int K) {
+    return K == 4608 || K == 4864 ? 1 : kind == WK_Q4 ? 4 : K == 1536 ? 1 : K == 2048 || K == 2560 ? 2 : kind == WK_F16 ? 2 : 4;
+}
+
+template <int KIND>
+__global__ __launch_bounds__(kBlock, 3) void gemv_many(const ManyCalls) {
+    // (the argument is read where it lies: indexed by a run-time number it would be copied to scratch first)
+    const auto* L = (const __attribute__((address_space(4))) ManyCalls*)__builtin_amdgcn_kernarg_segment_ptr();
+    const int lane = threadIdx.x % kWave;
+    static_assert(kMaxMany == kWave, "a lane per call");
+    const int mine = L->first[lane], n = L->n;
+    const int i = __popcll(__ballot(lane < n && static_cast<int>(blockIdx.x) >= mine)) - 1;
+    const uint16_t* x = L->c[i].x;
+    const uint8_t* W = L->c[i].W;
+    const uint16_t* sc = L->c[i].sc;
+    uint16_t* y = L->c[i].y;
+    const int N = L->c[i].N, nbatch = L->c[i].nbatch, waves = L->c[i].waves, code = L->c[i].code;
+    const int wid = (static_cast<int>(blockIdx.x) - L->first[i]) * kWavesPerBlock + block_wave();
+    const SegList none{};
+#define MI_MANY(KT)                                                                                                     \
+    case KT: {                                                                                                          \
+        constexpr int kVL = many_tile(KIND, KT);                                                                        \
+        fixed_k_rows<KIND, KT, kVL, EPI_STORE, KIND != WK_Q4 || KT <= 1536, group_size(KIND, KT, kVL), false>(          \
+            x, N, nbatch, W, sc, nullptr, nullptr, nullptr, y, none, wid, waves, blockIdx.y);                           \
+        break;                                                                                                          \
+    }
+#define MI_MANY_FAST(KT)                                                                                                \
+    case -KT:                                                                                                           \
+        q4_fast_rows<KT, EPI_STORE, KT <= 1536, group_size(WK_Q4, KT, 4), false>(x, N, nbatch, W, sc, nullptr, nullptr, \
+                                                                           nullptr, y, none, wid, waves, blockIdx.y);   \
+        break;
+    switch (code) {
+        MI_MANY(576) MI_MANY(896) MI_MANY(960) MI_MANY(1024) MI_MANY(1536) MI_MANY(2048) MI_MANY(2560) MI_MANY(4608) MI_MANY(4864)
+        default: break;
+    }
+    if constexpr (KIND == WK_Q4) {
+        switch (code) {
+            MI_MANY_FAST(576) MI_MANY_FAST(896) MI_MANY_FAST(960) MI_MANY_FAST(1024) MI_MANY_FAST(1536) MI_MANY_FAST(2048) MI_MANY_FAST(2560)
+            default: break;
+        }
+    }
+#undef MI_MANY
+#undef MI_MANY_FAST
 }
 
 // x (K halves, K % 4 == 0, 8-byte aligned) into LDS by the whole block.  Where K is long a thread
@@ -1004,12 +1080,6 @@ int pick_vl(WeightKind kind, int M, long rows, int K) {
     return narrowest;
 }
 
-// Row batches a pipelined wavefront fetches at once: enough for about 3.5 KB of weights.
-constexpr int group_size(int kind, int K, int vl) {
-    const int batch_bytes = vl * (K / (kind == WK_Q4 ? 8 : 4)) * (kind == WK_F16 ? 8 : 4);
-    return batch_bytes <= 1280 ? 4 : (batch_bytes <= 2560 ? 2 : 1);
-}
-
 struct Plan {
     SegList L;
     dim3 grid;
@@ -1309,6 +1379,80 @@ bool launch_gemv_group(hipStream_t s, const GemvCall* calls, int n) {
 }
 
 bool launch_gemv(hipStream_t s, const GemvCall& c) { return launch_gemv_group(s, &c, 1); }
+
+// The K that gemv_many has an instance for.
+static bool many_k(int K) {
+    return K == 576 || K == 896 || K == 960 || K == 1024 || K == 1536 || K == 2048 || K == 2560 || K == 4608 || K == 4864;
+}
+
+bool gemv_many_takes(const GemvCall& c) {
+    return c.epi == EPI_STORE && !c.norm_w && !c.am_v && many_k(c.K) && c.M >= 1 && c.M <= 65535 && c.N >= 1 && c.x && c.W && c.y &&
+           aligned(c.x, 16) && aligned(c.W, 16) && aligned(c.y, 2) && (c.kind == WK_F16 || (c.scale && aligned(c.scale, 2)));
+}
+
+// A run is what launch_gemv_group would take as one launch (its Q4 arithmetic follows from the rows of the run).
+bool launch_gemv_many(hipStream_t s, const GemvCall* calls, const int* run_of, int n) {
+    if (n < 1 || n > kMaxMany) {
+        MI_ERROR_FMT("gemv: %d calls in one launch (1..%d allowed)", n, kMaxMany);
+        return false;
+    }
+    const WeightKind kind = calls[0].kind;
+    ManyCalls L;
+    L.n = n;
+    double bytes = 0.0;
+    int batch_bytes[kMaxMany];
+    for (int i = 0; i < n; ++i) {
+        const GemvCall& c = calls[i];
+        if (!gemv_many_takes(c) || c.kind != kind || c.M != calls[0].M) {
+            MI_ERROR_FMT("gemv: a call that does not fit a launch of several (M=%d N=%d K=%d)", c.M, c.N, c.K);
+            return false;
+        }
+        const int vl = many_tile(kind, c.K);
+        ManyCalls::Call& d = L.c[i];
+        d.x = static_cast<const uint16_t*>(c.x);
+        d.W = static_cast<const uint8_t*>(c.W);
+        d.sc = static_cast<const uint16_t*>(c.scale);
+        d.y = static_cast<uint16_t*>(c.y);
+        d.N = c.N;
+        d.nbatch = (c.N + vl - 1) / vl;
+        d.code = c.K;
+        if (kind == WK_Q4 && gemv_mode(s) == 1) {
+            long rows = 0;
+            for (int j = 0; j < n; ++j)
+                if (run_of[j] == run_of[i]) rows += calls[j].N;
+            if (pick_vl(kind, c.M, rows, c.K) == 4) d.code = -c.K;      // (every such K has an instance of the throughput kernel)
+        }
+        batch_bytes[i] = vl * (c.K / (kind == WK_Q4 ? 8 : 4)) * (kind == WK_F16 ? 8 : 4);
+        bytes += static_cast<double>(d.nbatch) * batch_bytes[i];
+    }
+    // Every wavefront gets about the same bytes, and all of them, of all rows of x, are resident at once: the bytes per
+    // wavefront grow until the blocks fit (with that many blocks per row of x instead, 15 rows of a 576-wide Q4 layer took
+    // 19.7 us where they now take 17.0 and launches of a run each 18.7; 8 fp16 rows 14.1 against 8 and 17).
+    const int M = calls[0].M;
+    const long cap = resident_waves() / kWavesPerBlock / M;
+    long blocks = 0;
+    for (double share = bytes * M / resident_waves();; share *= 1.05) {
+        blocks = 0;
+        for (int i = 0; i < n; ++i) {
+            const long per_wave = share > batch_bytes[i] ? static_cast<long>(share / batch_bytes[i]) : 1;
+            const long b = ((L.c[i].nbatch + per_wave - 1) / per_wave + kWavesPerBlock - 1) / kWavesPerBlock;
+            L.first[i] = static_cast<uint16_t>(blocks);
+            L.c[i].waves = static_cast<int>(b * kWavesPerBlock);
+            blocks += b;
+        }
+        if (blocks <= cap || blocks <= n) break;
+    }
+    // (a multiple of 8 blocks per row of x: the blocks that read the same weights for different rows then share an XCD's
+    //  L2; the blocks past the last call's find no row batch left)
+    if (M > 1) blocks = (blocks + 7) / 8 * 8;
+    const dim3 grid(static_cast<unsigned>(blocks), M, 1);
+    switch (kind) {
+        case WK_F16: hipLaunchKernelGGL(gemv_many<WK_F16>, grid, dim3(kBlock), 0, s, L); break;
+        case WK_I8:  hipLaunchKernelGGL(gemv_many<WK_I8>, grid, dim3(kBlock), 0, s, L); break;
+        case WK_Q4:  hipLaunchKernelGGL(gemv_many<WK_Q4>, grid, dim3(kBlock), 0, s, L); break;
+    }
+    return MI_HIP_OK(hipGetLastError());
+}
 
 bool launch_gate_up_silu(hipStream_t s, WeightKind kind, int N, int K, const void* x, const void* Wg,
                          const void* sg, const void* Wu, const void* su, void* out) {
