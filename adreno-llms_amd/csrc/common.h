@@ -151,6 +151,17 @@ bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void
 // 0 = no kernel with this epilogue for the call (nothing was launched), -1 = an error.
 int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
                     void* out, void* workspace, size_t workspace_bytes);
+// n calls of one M and weight kind that gemm_many_takes accepts, of any x, K and N, none of which reads or writes what
+// another one writes: in one launch where they fit it, each result what launch_gemm gives.
+bool gemm_many_takes(hipStream_t s, const GemvCall& c, size_t workspace_bytes);
+bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes);
+// A stream's workspace holds kWorkspaceBytes for whatever a launch puts there and, behind them, kSliceCounters
+// counters that are 0 between launches (slices of K that meet inside a launch).
+constexpr size_t kWorkspaceBytes = 16u << 20;
+constexpr int kSliceCounters = 16384;
+inline uint32_t* slice_counters(void* workspace) {
+    return reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kWorkspaceBytes);
+}
 // runtime.hip: the same for a registered W where mi_linear would run the GEMM
 int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out);
 // whether mi_linear would run the GEMM (and not rows of GEMV) for the call

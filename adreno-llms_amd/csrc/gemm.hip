@@ -1254,36 +1254,73 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kMaxM = 64;
 constexpr int kWaves = 8;                // wavefronts per block
 
-// SW strips of W per wavefront: the fragments of x a lane holds are multiplied with SW strips.
+// The sums of a 16 x 16 tile's kb slices of K, each in one wavefront of a block of its own, meet in memory: the
+// wavefront that arrives last takes all of them in slice order (a lane the sums of the lanes of its number) and goes
+// on with their total; the others return false.  Sums and counter travel as agent-scope accesses, which pass the
+// XCDs' own L2s: a store that has been acknowledged (vmcnt) is where every other CU's such load looks for it.  No
+// block waits for another.  The counter starts at 0 (add_workspace) and is left at 0; launches on a stream are ordered.
+// What it replaces is a second launch over 1 KB per tile and slice, which in a prompt or a batch waits for this one and
+// holds up the next: a prompt of 37 fp16 tokens 1618 -> 1576 us in 32 layers (960 x 2560 each); at 64 rows equal.
+__device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ sums, uint32_t* __restrict__ counter, const int by,
+                                            const int kb, const int lane) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    auto* at = reinterpret_cast<uint64_t*>(sums) + lane;                 // [kb][2][64] pairs
+    #pragma unroll
+    for (int h = 0; h < 2; ++h)
+        __hip_atomic_store(at + (by * 2 + h) * 64, __builtin_bit_cast(uint64_t, f32x2{acc[2 * h], acc[2 * h + 1]}),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t before = 0;
+    if (lane == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    before = __builtin_amdgcn_readfirstlane(before);
+    if (before + 1 != static_cast<uint32_t>(kb)) return false;
+    asm volatile("" ::: "memory");
+    if (lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int kMost = 8;                                             // slices over blocks (pick_shape), asked for together
+    f32x2 v[kMost][2];
+    #pragma unroll
+    for (int y = 0; y < kMost; ++y)
+        #pragma unroll
+        for (int h = 0; h < 2; ++h)
+            v[y][h] = __builtin_bit_cast(f32x2, __hip_atomic_load(at + ((y < kb ? y : 0) * 2 + h) * 64, __ATOMIC_RELAXED,
+                                                                  __HIP_MEMORY_SCOPE_AGENT));
+    #pragma unroll
+    for (int y = 0; y < kMost; ++y)
+        if (y < kb) {
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = y == 0 ? v[y][r / 2][r % 2] : acc[r] + v[y][r / 2][r % 2];
+        }
+    return true;
+}
+
 // XL: the block first copies its rows of x into LDS (rows padded by 16 bytes, which spreads the 16
 // rows a 16-byte read touches over all banks) and every wavefront reads its fragments from there;
 // blocks then live long and walk over the strips.  Without XL (x too large for LDS) the fragments
-// come from the caches with the weights, 2 MT / SW bytes per byte of W, and the L1's few requests
+// come from the caches with the weights, 2 MT bytes per byte of W, and the L1's few requests
 // in flight bound the rate: that form only pays for a few rows of x at a long K.
 // Q4 weights: an iteration is 128 values of K, of which a lane holds 32, exactly one scale block (16
 // bytes of nibbles and one scale per lane and iteration); the weights enter the matrix cores as
 // q * scale, exactly, in TERMS = 2 fp16 terms (scale = hi + lo with 7 and 4 significant bits, as in
 // the wide kernel), or rounded to fp16 once with TERMS = 1.
 // GLU: see launch_gemm_glu (an instance of its own: as a switch it cost the plain launch 2 % at 16 rows).
-template <int KIND, int MT, int SW, bool XL, int TERMS, bool GLU>
-__global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __restrict__ X,
-                                                           const uint8_t* __restrict__ W,
-                                                           const uint16_t* __restrict__ scale,
-                                                           uint16_t* __restrict__ out, int M, int N, int K, int ks,
-                                                           int logical_blocks, float* __restrict__ partial,
-                                                           MoreMats more) {
-    static_assert(!GLU || SW == 1, "a strip of gate or up columns per wavefront");
+// bx of gx blocks along N; slice by of kb slices of K, which meet as told at meet_slices.
+template <int KIND, int MT, bool XL, int TERMS, bool GLU>
+__device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
+                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
+                                            const int K, const int ks, const int logical_blocks, float* __restrict__ partial,
+                                            uint32_t* __restrict__ counters, const MoreMats& more, const int bx, const int gx,
+                                            const int by, const int kb) {
     constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
     constexpr int WV = F16 ? 2 : 1;                       // 16-byte loads of W per lane, strip and iteration
     constexpr int kWB = F16 ? 2 : 1;                      // bytes of a row of W per 64 bytes of an iteration's weights / 64
     constexpr int kItK = Q4 ? 128 : 64;                   // values of K per iteration
     constexpr int XE = kItK / 32;                         // 16-byte pieces of x per lane and iteration = MFMAs per x tile and term
-    constexpr int kPerIt = (4 * WV + (Q4 ? 1 : 0)) * SW + (XL ? 0 : 4 * XE * MT);   // registers one iteration's operands take in a buffer
+    constexpr int kPerIt = 4 * WV + (Q4 ? 1 : 0) + (XL ? 0 : 4 * XE * MT);   // registers one iteration's operands take in a buffer
     constexpr int kBudget = F16 ? 40 : 48;                // registers per buffer (with 64 the fp16 instances spill)
     constexpr int kChunk = kBudget / kPerIt < 1 ? 1 : kBudget / kPerIt > 8 ? 8 : kBudget / kPerIt;   // iterations per buffer
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t xrow = XL ? static_cast<uint32_t>(K) * 2u + 16u : 0u;              // bytes per row of x in LDS
-    float* red = reinterpret_cast<float*>(lds + 16u * MT * xrow);                     // [kWaves][MT][4][64]
+    floatx4* red = reinterpret_cast<floatx4*>(lds + 16u * MT * xrow);                 // [kWaves][MT][64]
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1291,10 +1328,9 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
     const int slice = wave % ks;
     const int nit = (K + kItK - 1) / kItK;               // (Q4 at K = 64 mod 128: the upper half of the lanes sits out the last one)
     const size_t wrowb = Q4 ? static_cast<size_t>(K) / 2 : static_cast<size_t>(K) * kWB;   // bytes of a row of W
-    // K is cut over the blocks of the grid's y (then `partial` takes raw sums, one M x N matrix per y,
-    // for reduce_partials) and, inside a block, over ks wavefronts
-    const int b0 = nit * static_cast<int>(blockIdx.y) / static_cast<int>(gridDim.y);
-    const int b1 = nit * (static_cast<int>(blockIdx.y) + 1) / static_cast<int>(gridDim.y);
+    // K is cut over kb blocks (a strip each, one trip through the loop below) and, inside a block, over ks wavefronts
+    const int b0 = nit * by / kb;
+    const int b1 = nit * (by + 1) / kb;
     const int it0 = b0 + (b1 - b0) * slice / ks, it1 = b0 + (b1 - b0) * (slice + 1) / ks;
 
     if constexpr (XL) {
@@ -1332,29 +1368,23 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
     uint16_t* const out0 = out;
     const int N0 = N;
 
-    for (int lb = blockIdx.x; lb < logical_blocks; lb += gridDim.x) {     // (the same trips for the whole block)
-        int group = lb * (kWaves / ks) + wave / ks;                       // group: SW consecutive strips
+    for (int lb = bx; lb < logical_blocks; lb += gx) {     // (the same trips for the whole block)
+        int group = lb * (kWaves / ks) + wave / ks;                       // strip
         if constexpr (!GLU) {
             W = W0; scale = scale0; out = out0; N = N0;
             pick_matrix(more, group, W, scale, out, N);
         }
         const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
-        const uint8_t* wp[SW];
-        [[maybe_unused]] const uint16_t* sp[SW];                          // Q4: the row's block scales, this lane's first
+        const int wr = 16 * group + i < N ? 16 * group + i : N - 1;       // rows past N are read as the last row
+        const uint8_t* wp = W + static_cast<size_t>(wr) * wrowb + c * 16 * WV;
+        [[maybe_unused]] const uint16_t* sp = nullptr;                    // Q4: the row's block scales, this lane's first
+        if constexpr (Q4) sp = scale + static_cast<size_t>(wr) * (K / 32) + c;
+        floatx4 acc[MT];
         #pragma unroll
-        for (int q = 0; q < SW; ++q) {
-            const int row = 16 * (group * SW + q) + i;                    // rows past N are read as the last row
-            wp[q] = W + static_cast<size_t>(row < N ? row : N - 1) * wrowb + c * 16 * WV;
-            if constexpr (Q4) sp[q] = scale + static_cast<size_t>(row < N ? row : N - 1) * (K / 32) + c;
-        }
-        floatx4 acc[SW][MT];
-        #pragma unroll
-        for (int q = 0; q < SW; ++q)
-            #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[q][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-        u32x4 wb[2][kChunk][SW][WV];
-        [[maybe_unused]] uint16_t sb[2][kChunk][SW];
+        u32x4 wb[2][kChunk][WV];
+        [[maybe_unused]] uint16_t sb[2][kChunk];
         [[maybe_unused]] u32x4 xb[2][XL ? 1 : kChunk][XL ? 1 : MT][XE];
         // `full`: kChunk iterations whatever the slice's end (the caller knows they exist); the number
         // of requests is then a constant, and only then can the wait before a buffer is multiplied
@@ -1377,13 +1407,10 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
                                 xp[t] + (mine ? static_cast<ptrdiff_t>(it) * (2 * kItK) : -static_cast<ptrdiff_t>(c) * (16 * XE)))[e];
                 }
                 #pragma unroll
-                for (int q = 0; q < SW; ++q) {
-                    #pragma unroll
-                    for (int v = 0; v < WV; ++v)
-                        wb[b][u][q][v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                            wp[q] + (mine ? static_cast<ptrdiff_t>(it) * 64 * kWB : -static_cast<ptrdiff_t>(c) * 16 * WV)) + v);
-                    if constexpr (Q4) sb[b][u][q] = sp[q][mine ? 4 * it : -c];
-                }
+                for (int v = 0; v < WV; ++v)
+                    wb[b][u][v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                        wp + (mine ? static_cast<ptrdiff_t>(it) * 64 * kWB : -static_cast<ptrdiff_t>(c) * 16 * WV)) + v);
+                if constexpr (Q4) sb[b][u] = sp[mine ? 4 * it : -c];
             }
         };
         auto multiply = [&](int b, int j0) {
@@ -1403,48 +1430,45 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
                             else
                                 xf[t][e] = __builtin_bit_cast(half8, xb[b][u][t][e]);
                         }
-                    #pragma unroll
-                    for (int q = 0; q < SW; ++q) {
-                        half8 a[TERMS][XE];
-                        if constexpr (F16) {
-                            a[0][0] = __builtin_bit_cast(half8, wb[b][u][q][0]);
-                            a[0][1] = __builtin_bit_cast(half8, wb[b][u][q][1]);
-                        } else if constexpr (Q4) {
-                            // a lane that sits the iteration out multiplies by a scale of zero
-                            const uint32_t s1 = mine ? sb[b][u][q] : 0u;
-                            const uint32_t sboth = s1 | (s1 << 16);
-                            __half2 st[TERMS];
-                            if constexpr (TERMS == 2) {
-                                st[0] = __builtin_bit_cast(__half2, sboth & 0xFFF0FFF0u);
-                                st[1] = __hsub2(__builtin_bit_cast(__half2, sboth), st[0]);
-                            } else {
-                                st[0] = __builtin_bit_cast(__half2, sboth);
-                            }
-                            #pragma unroll
-                            for (int e = 0; e < XE; ++e) {
-                                const uint32_t v = wb[b][u][q][0][e];
-                                #pragma unroll
-                                for (int z = 0; z < TERMS; ++z)
-                                    a[z][e] = __builtin_bit_cast(half8, u32x4{q4x2_to_h2<0>(v, st[z]), q4x2_to_h2<1>(v, st[z]),
-                                                                              q4x2_to_h2<2>(v, st[z]), q4x2_to_h2<3>(v, st[z])});
-                            }
+                    half8 a[TERMS][XE];
+                    if constexpr (F16) {
+                        a[0][0] = __builtin_bit_cast(half8, wb[b][u][0]);
+                        a[0][1] = __builtin_bit_cast(half8, wb[b][u][1]);
+                    } else if constexpr (Q4) {
+                        // a lane that sits the iteration out multiplies by a scale of zero
+                        const uint32_t s1 = mine ? sb[b][u] : 0u;
+                        const uint32_t sboth = s1 | (s1 << 16);
+                        __half2 st[TERMS];
+                        if constexpr (TERMS == 2) {
+                            st[0] = __builtin_bit_cast(__half2, sboth & 0xFFF0FFF0u);
+                            st[1] = __hsub2(__builtin_bit_cast(__half2, sboth), st[0]);
                         } else {
-                            uint32_t h[8];
-                            i8x4_to_h4(wb[b][u][q][0].x, h[0], h[1]);
-                            i8x4_to_h4(wb[b][u][q][0].y, h[2], h[3]);
-                            i8x4_to_h4(wb[b][u][q][0].z, h[4], h[5]);
-                            i8x4_to_h4(wb[b][u][q][0].w, h[6], h[7]);
-                            a[0][0] = __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
-                            a[0][1] = __builtin_bit_cast(half8, u32x4{h[4], h[5], h[6], h[7]});
+                            st[0] = __builtin_bit_cast(__half2, sboth);
                         }
                         #pragma unroll
-                        for (int t = 0; t < MT; ++t)
+                        for (int e = 0; e < XE; ++e) {
+                            const uint32_t v = wb[b][u][0][e];
                             #pragma unroll
                             for (int z = 0; z < TERMS; ++z)
-                                #pragma unroll
-                                for (int e = 0; e < XE; ++e)
-                                    acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][e], xf[t][e], acc[q][t], 0, 0, 0);
+                                a[z][e] = __builtin_bit_cast(half8, u32x4{q4x2_to_h2<0>(v, st[z]), q4x2_to_h2<1>(v, st[z]),
+                                                                          q4x2_to_h2<2>(v, st[z]), q4x2_to_h2<3>(v, st[z])});
+                        }
+                    } else {
+                        uint32_t h[8];
+                        i8x4_to_h4(wb[b][u][0].x, h[0], h[1]);
+                        i8x4_to_h4(wb[b][u][0].y, h[2], h[3]);
+                        i8x4_to_h4(wb[b][u][0].z, h[4], h[5]);
+                        i8x4_to_h4(wb[b][u][0].w, h[6], h[7]);
+                        a[0][0] = __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
+                        a[0][1] = __builtin_bit_cast(half8, u32x4{h[4], h[5], h[6], h[7]});
                     }
+                    #pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        #pragma unroll
+                        for (int z = 0; z < TERMS; ++z)
+                            #pragma unroll
+                            for (int e = 0; e < XE; ++e)
+                                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][e], xf[t][e], acc[t], 0, 0, 0);
                 }
             }
         };
@@ -1476,105 +1500,82 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
             multiply(0, j0 + kChunk);
         }
 
-        if (ks > 1) {                                    // (the same for every wavefront of the grid)
+        // The slices' sums meet in LDS; tile t of the strip is then finished by the strip's wavefront t mod ks, which
+        // adds them in slice order (one wavefront for all tiles reads 7 x 16 values one after the other at 64 rows: a
+        // 0.5B layer of such int8 rows 35.5 us against 34.3).
+        if (ks > 1) {                                    // (the same for every wavefront of the block)
+            __syncthreads();                             // the last round's sums have been read
             #pragma unroll
-            for (int q = 0; q < SW; ++q) {               // one strip at a time through the same 4 MT KB per wavefront
-                __syncthreads();                         // the last round's sums have been read
-                if (slice > 0) {
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        #pragma unroll
-                        for (int r = 0; r < 4; ++r) red[((wave * MT + t) * 4 + r) * 64 + lane] = acc[q][t][r];
-                }
-                __syncthreads();
-                if (slice == 0) {
-                    for (int z = 1; z < ks; ++z) {       // slice 0 + slice 1 + ..., in this order
-                        #pragma unroll
-                        for (int t = 0; t < MT; ++t)
-                            #pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[q][t][r] += red[(((wave + z) * MT + t) * 4 + r) * 64 + lane];
-                    }
-                }
-            }
-            if constexpr (GLU) {
-                // odd strips belong to the up matrix, the strip below to the same columns of the gate matrix
-                // (see launch_gemm_glu) and to the wavefronts before these: the up values cross through LDS
-                __syncthreads();                     // the sums have been read
-                const int nq = 16 * group + 4 * c;
-                float s4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-                if constexpr (KIND == WK_I8) {
-                    #pragma unroll
-                    for (int r = 0; r < 4; ++r) s4[r] = h_f(scale[nq + r < N ? nq + r : N - 1]);
-                }
-                uint2 h[MT];
-                #pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    h[t] = uint2{wide::pack_half2(acc[0][t][0] * s4[0], acc[0][t][1] * s4[1]),
-                                 wide::pack_half2(acc[0][t][2] * s4[2], acc[0][t][3] * s4[3])};
-                uint2* cross = reinterpret_cast<uint2*>(red);
-                if (slice == 0 && group % 2) {
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t) cross[(wave * MT + t) * 64 + lane] = h[t];
-                }
-                __syncthreads();
-                if (slice == 0 && group % 2 == 0 && nq < N) {
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t) {
-                        const int m = 16 * t + i;
-                        const uint2 up = cross[((wave + ks) * MT + t) * 64 + lane];
-                        if (m < M)
-                            *reinterpret_cast<uint2*>(out + static_cast<size_t>(m) * (N / 2) + 8 * group + 4 * c) =
-                                uint2{swiglu_h2(h[t].x, up.x), swiglu_h2(h[t].y, up.y)};
-                    }
-                }
-                continue;
-            }
-            if (slice > 0) continue;
+            for (int t = 0; t < MT; ++t) red[(wave * MT + t) * 64 + lane] = acc[t];
+            __syncthreads();
         }
-
+        const int nq = 16 * group + 4 * c;               // first of this lane's 4 output columns
+        float s4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        if constexpr (KIND == WK_I8) {
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) s4[r] = h_f(scale[nq + r < N ? nq + r : N - 1]);
+        }
+        [[maybe_unused]] uint2 h[MT];
         #pragma unroll
-        for (int q = 0; q < SW; ++q) {
-            const int nq = 16 * (group * SW + q) + 4 * c;    // first of this lane's 4 output columns
-            if (nq >= N) continue;
-            float s4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-            if constexpr (KIND == WK_I8) {
-                #pragma unroll
-                for (int r = 0; r < 4; ++r) s4[r] = __half2float(__ushort_as_half(scale[nq + r < N ? nq + r : N - 1]));
-            }
-            if (partial) {
-                float* pout = partial + static_cast<size_t>(blockIdx.y) * M * N;
-                #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const int m = 16 * t + i;
-                    if (m >= M) continue;
-                    float* dst = pout + static_cast<size_t>(m) * N + nq;
-                    if ((N % 4) == 0 && nq + 3 < N) {
-                        *reinterpret_cast<float4*>(dst) = float4{acc[q][t][0], acc[q][t][1], acc[q][t][2], acc[q][t][3]};
-                    } else {
-                        #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (nq + r < N) dst[r] = acc[q][t][r];
-                    }
+        for (int t = 0; t < MT; ++t) {
+            if ((t & (ks - 1)) != slice) continue;
+            if (ks > 1) {
+                acc[t] = red[((wave - slice) * MT + t) * 64 + lane];
+                for (int z = 1; z < ks; ++z) {
+                    const floatx4 v = red[((wave - slice + z) * MT + t) * 64 + lane];
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[t][r] += v[r];
                 }
+            }
+            if (kb > 1 && !meet_slices(acc[t], partial + (static_cast<size_t>(group) * MT + t) * kb * 256, counters + group * MT + t, by, kb, lane))
+                continue;
+            const uint32_t lo = wide::pack_half2(acc[t][0] * s4[0], acc[t][1] * s4[1]);
+            const uint32_t hi = wide::pack_half2(acc[t][2] * s4[2], acc[t][3] * s4[3]);
+            if constexpr (GLU) {
+                h[t] = uint2{lo, hi};
                 continue;
             }
+            const int m = 16 * t + i;
+            if (m >= M || nq >= N) continue;
+            uint16_t* dst = out + static_cast<size_t>(m) * N + nq;
+            if (cols4 && nq + 3 < N) {
+                *reinterpret_cast<uint2*>(dst) = uint2{lo, hi};
+            } else {
+                #pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (nq + r < N) dst[r] = static_cast<uint16_t>((r / 2 ? hi : lo) >> (16 * (r % 2)));
+            }
+        }
+        if constexpr (GLU) {
+            // odd strips belong to the up matrix, the strip below to the same columns of the gate matrix (see
+            // launch_gemm_glu) and to the wavefronts before these: the up values cross through LDS
+            __syncthreads();                             // the sums have been read
+            uint2* cross = reinterpret_cast<uint2*>(red);
+            #pragma unroll
+            for (int t = 0; t < MT; ++t)
+                if ((t & (ks - 1)) == slice && group % 2) cross[(wave * MT + t) * 64 + lane] = h[t];
+            __syncthreads();
             #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 const int m = 16 * t + i;
-                if (m >= M) continue;
-                const uint32_t lo = wide::pack_half2(acc[q][t][0] * s4[0], acc[q][t][1] * s4[1]);
-                const uint32_t hi = wide::pack_half2(acc[q][t][2] * s4[2], acc[q][t][3] * s4[3]);
-                uint16_t* dst = out + static_cast<size_t>(m) * N + nq;
-                if (cols4 && nq + 3 < N) {
-                    *reinterpret_cast<uint2*>(dst) = uint2{lo, hi};
-                } else {
-                    #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (nq + r < N) dst[r] = static_cast<uint16_t>((r / 2 ? hi : lo) >> (16 * (r % 2)));
+                if ((t & (ks - 1)) == slice && group % 2 == 0 && nq < N && m < M) {
+                    const uint2 up = cross[((wave + ks) * MT + t) * 64 + lane];
+                    *reinterpret_cast<uint2*>(out + static_cast<size_t>(m) * (N / 2) + 8 * group + 4 * c) =
+                        uint2{swiglu_h2(h[t].x, up.x), swiglu_h2(h[t].y, up.y)};
                 }
             }
         }
     }
+}
+
+template <int KIND, int MT, bool XL, int TERMS, bool GLU>
+__global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
+                                                           const uint16_t* __restrict__ scale, uint16_t* __restrict__ out,
+                                                           int M, int N, int K, int ks, int logical_blocks,
+                                                           float* __restrict__ partial, uint32_t* __restrict__ counters,
+                                                           MoreMats more) {
+    skinny_rows<KIND, MT, XL, TERMS, GLU>(X, W, scale, out, M, N, K, ks, logical_blocks, partial, counters, more, blockIdx.x,
+                                              gridDim.x, blockIdx.y, gridDim.y);
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -1584,13 +1585,15 @@ inline size_t lds_bytes(int mt, int K, bool xl, int ks) {
            (ks > 1 ? static_cast<size_t>(kWaves) * mt * 4 * 64 * 4 : 0);
 }
 
+// bytes of partial sums that kb slices of K over blocks leave in the workspace (meet_slices)
+inline size_t partial_bytes(int mt, int N, int kb) { return static_cast<size_t>((N + 15) / 16) * kb * mt * 1024; }
+
 struct Shape { int ks; bool xl; int kb; };
 // Slices of K per strip inside a block (1, 2, 4, 8: the fewest that give the chip four wavefronts
 // per CU; measured at 4864 x 896: 4 slices 4.5 us, 8 slices 6.7 us), x in LDS where it fits, and
 // slices of K over blocks (kb) where one block per strip still leaves most CUs idle and what a
 // single CU can pull bounds the launch (896 x 4864: 56 strips): their sums go through the
-// workspace and a second launch adds them in order.  One strip per wavefront: two and four (the
-// kernel's SW) were measured slower at every shape tried (fewer wavefronts; the reads of x they
+// workspace, where the last block to arrive adds them in order.  One strip per wavefront: two and four were measured slower at every shape tried (fewer wavefronts; the reads of x they
 // save are not the bound).
 inline Shape pick_shape(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
     const int mt = (M + 15) / 16;
@@ -1601,8 +1604,8 @@ inline Shape pick_shape(int kind, int M, int N, int K, int cus, size_t workspace
     // (a block whose eight wavefronts share one strip reads every byte of x once either way: no LDS then)
     sh.xl = sh.ks < kWaves && lds_bytes(mt, K, true, sh.ks) <= kLdsLimit;
     if (sh.ks == kWaves) {
-        while (sh.kb < 8 && strips * sh.kb * 2 <= cus && its >= 2 * sh.ks * sh.kb * 2 &&
-               static_cast<double>(sh.kb) * 2 * M * N * 4 <= static_cast<double>(workspace_bytes))
+        while (sh.kb < 8 && strips * sh.kb * 2 <= cus && its >= 2 * sh.ks * sh.kb * 2 && strips * mt <= kSliceCounters &&
+               partial_bytes(mt, N, 2 * sh.kb) <= workspace_bytes)
             sh.kb *= 2;
     }
     return sh;
@@ -1647,51 +1650,91 @@ inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspa
     return q4_us + (sh.xl ? 3.75 + 0.035 * M : xg_us) + w_bytes / 8.0e6;
 }
 
+// ---- calls that share no x, in one launch ----
+//
+// Calls of a batch that cannot observe one another's results (the batch's host code checks that) and that the streaming
+// kernel serves, each as its own plan has it (the same slices of K in the same order: the same bits as a launch of its
+// own), a block per call and group of strips.  A launch of a few hundred rows of W takes 4 to 5 us whatever its size:
+// the seven int8 projections of a 0.5B layer at 16 rows, four launches and one for the slices' sums, 26.6 -> 14.0 us.
+constexpr int kMaxManyGemm = 32;
+struct SkinnyCalls {
+    int n = 0, M = 0;
+    uint16_t first[kMaxManyGemm] = {};                   // a call's first block
+    struct Call {
+        const uint16_t* X;
+        const uint8_t* W;
+        const uint16_t* scale;
+        uint16_t* out;
+        float* partial;
+        uint32_t* counters;
+        int N, K, logical;
+        uint16_t blocks;                                 // blocks along N; kb times as many in all
+        uint8_t ks_xl, kb;                               // slices inside a block, + 16 with x in LDS; slices over blocks
+    } c[kMaxManyGemm] = {};
+};
+static_assert(sizeof(SkinnyCalls) <= 4096, "kernel arguments");
+
+template <int KIND, int MT, int TERMS>
+__global__ __launch_bounds__(64 * kWaves) void gemm_skinny_many(const SkinnyCalls) {
+    // (the argument is read where it lies: indexed by a run-time number it would be copied to scratch first)
+    const auto* L = (const __attribute__((address_space(4))) SkinnyCalls*)__builtin_amdgcn_kernarg_segment_ptr();
+    const int lane = threadIdx.x & 63, n = L->n, b = blockIdx.x;
+    const int mine = L->first[lane < kMaxManyGemm ? lane : 0];
+    const int q = __popcll(__ballot(lane < n && b >= mine)) - 1;
+    const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb, ks_xl = L->c[q].ks_xl, ks = ks_xl & 15;
+    const int by = kb > 1 ? at / blocks : 0;
+    const MoreMats none{};
+    const uint16_t *X = L->c[q].X, *scale = L->c[q].scale;
+    const uint8_t* W = L->c[q].W;
+    uint16_t* out = L->c[q].out;
+    float* partial = L->c[q].partial;
+    uint32_t* counters = L->c[q].counters;
+    const int N = L->c[q].N, K = L->c[q].K, logical = L->c[q].logical, M = L->M;
+    if (ks_xl & 16)
+        skinny_rows<KIND, MT, true, TERMS, false>(X, W, scale, out, M, N, K, ks, logical, nullptr, nullptr, none, at, blocks, 0, 1);
+    else
+        skinny_rows<KIND, MT, false, TERMS, false>(X, W, scale, out, M, N, K, ks, logical, partial, counters, none, at - by * blocks, blocks, by, kb);
+}
+
 // Shapes whose blocks hold a strip of the gate matrix and its strip of the up matrix, and LDS for them to meet in
 inline bool glu_shape(const Shape& sh) { return sh.kb == 1 && (sh.ks == 2 || sh.ks == 4); }
 
-template <int KIND, int MT, int SW, bool XL, int TERMS, bool GLU>
+// Blocks along N for `logical` groups of strips.  With x in LDS a block is worth keeping: as many as fit a CU at once
+// (by LDS; at most 4), each walking over the groups.
+inline long blocks_along_n(bool xl, long logical, size_t lds) {
+    if (!xl) return logical;
+    const long per_cu = lds == 0 ? 4 : static_cast<long>(kLdsLimit / lds) < 4 ? static_cast<long>(kLdsLimit / lds) : 4;
+    const long resident = static_cast<long>(device_info().cus) * (per_cu < 1 ? 1 : per_cu);
+    return logical > resident ? resident : logical;
+}
+
+template <int KIND, int MT, bool XL, int TERMS, bool GLU>
 bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
                 float* partial, const MoreMats& more) {
     const int ks = sh.ks;
-    const long groups = more.n ? more.tiles : ((N + 15) / 16 + SW - 1) / SW, per_block = kWaves / ks;
+    const long groups = more.n ? more.tiles : (N + 15) / 16, per_block = kWaves / ks;
     const long logical = (groups + per_block - 1) / per_block;
     const size_t lds = lds_bytes(MT, K, XL, ks);
-    auto* kern = gemm_skinny<KIND, MT, SW, XL, TERMS, GLU>;
+    auto* kern = gemm_skinny<KIND, MT, XL, TERMS, GLU>;
     if (lds > 65536 &&
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
         return false;
-    // with x in LDS a block is worth keeping: as many as fit a CU at once (by LDS; at most 4), each walking over the strips
-    long grid = logical;
-    if (XL) {
-        const long per_cu = lds == 0 ? 4 : static_cast<long>(kLdsLimit / lds) < 4 ? static_cast<long>(kLdsLimit / lds) : 4;
-        const long resident = static_cast<long>(device_info().cus) * (per_cu < 1 ? 1 : per_cu);
-        if (grid > resident) grid = resident;
-    }
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid), static_cast<unsigned>(sh.kb)), dim3(64 * kWaves), lds, s,
-                       static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
-                       static_cast<uint16_t*>(out), M, N, K, ks, static_cast<int>(logical), sh.kb > 1 ? partial : nullptr,
-                       more);
-    if (!MI_HIP_OK(hipGetLastError())) return false;
-    if (sh.kb > 1) {
-        const long MN = static_cast<long>(M) * N;
-        hipLaunchKernelGGL(wide::reduce_partials, dim3(static_cast<unsigned>((MN / 4 + 256) / 256)), dim3(256), 0, s, partial,
-                           sh.kb, KIND == WK_I8 ? static_cast<const uint16_t*>(scale) : nullptr, static_cast<uint16_t*>(out),
-                           MN, N);
-        if (!MI_HIP_OK(hipGetLastError())) return false;
-    }
-    return true;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks_along_n(XL, logical, lds)), static_cast<unsigned>(sh.kb)),
+                       dim3(64 * kWaves), lds, s, static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W),
+                       static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(out), M, N, K, ks, static_cast<int>(logical),
+                       sh.kb > 1 ? partial : nullptr, sh.kb > 1 ? slice_counters(partial) : nullptr, more);
+    return MI_HIP_OK(hipGetLastError());
 }
 
 template <int KIND, int MT, int TERMS>
 bool launch_mt(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
                float* partial, const MoreMats& more, bool glu) {
     if (glu)
-        return sh.xl ? launch_one<KIND, MT, 1, true, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                     : launch_one<KIND, MT, 1, false, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more);
-    return sh.xl ? launch_one<KIND, MT, 1, true, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                 : launch_one<KIND, MT, 1, false, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
+        return sh.xl ? launch_one<KIND, MT, true, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more)
+                     : launch_one<KIND, MT, false, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more);
+    return sh.xl ? launch_one<KIND, MT, true, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
+                 : launch_one<KIND, MT, false, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
 }
 
 template <int KIND, int TERMS>
@@ -1700,7 +1743,8 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
     if (M < 1 || M > kMaxM || !(sh.ks == 1 || sh.ks == 2 || sh.ks == 4 || sh.ks == 8) ||
         lds_bytes((M + 15) / 16, K, sh.xl, sh.ks) > kLdsLimit || sh.kb < 1 || (sh.kb > 1 && (sh.xl || more.n)) ||
         (glu && !glu_shape(sh)) ||
-        (sh.kb > 1 && (!workspace || static_cast<double>(sh.kb) * M * N * 4 > static_cast<double>(workspace_bytes)))) {
+        (sh.kb > 1 && (sh.ks != kWaves || !workspace || partial_bytes((M + 15) / 16, N, sh.kb) > workspace_bytes ||
+                       (N + 15) / 16 * ((M + 15) / 16) > kSliceCounters))) {
         MI_ERROR_FMT("gemm: the streaming kernel takes up to %d rows of x, 1, 2, 4 or 8 slices of K per block, %zu bytes of LDS "
                      "and a workspace for slices over blocks (M=%d K=%d, %d slices, x in LDS %d, %d slices over blocks, %zu bytes)",
                      kMaxM, kLdsLimit, M, K, sh.ks, static_cast<int>(sh.xl), sh.kb, workspace_bytes);
@@ -1713,6 +1757,102 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
         case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
         default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
     }
+}
+
+// The calls of L as one launch with `lds` bytes per block.
+template <int KIND, int MT, int TERMS>
+bool launch_calls(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_t lds) {
+    auto* kern = gemm_skinny_many<KIND, MT, TERMS>;
+    if (lds > 65536 &&
+        !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
+        return false;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * kWaves), lds, s, L);
+    return MI_HIP_OK(hipGetLastError());
+}
+template <int KIND, int TERMS>
+bool launch_calls_mt(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_t lds) {
+    switch ((L.M + 15) / 16) {
+        case 1: return launch_calls<KIND, 1, TERMS>(s, L, blocks, lds);
+        case 2: return launch_calls<KIND, 2, TERMS>(s, L, blocks, lds);
+        case 3: return launch_calls<KIND, 3, TERMS>(s, L, blocks, lds);
+        default: return launch_calls<KIND, 4, TERMS>(s, L, blocks, lds);
+    }
+}
+
+// n calls of one M <= kMaxM and weight kind in as few launches as hold them.  Calls whose slices meet in memory go
+// first, so that their last blocks' trips run under the others' work.  A launch takes the LDS of the call that needs
+// most, for all its blocks: calls of more than half a CU's (x of many rows in LDS) share launches of their own, with
+// no more blocks than the chip holds at once, dealt out to the calls by their strips: a block is then worth its copy of
+// x (a 0.5B layer's calls at 37 / 64 Q4 rows 34.6 / 39.8 -> 24.4 / 29.5 us; gate and up at 64 fp16 rows with a block per two strips, more
+// than fit at once, made the layer 41.8 us instead of 39.7).
+bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* workspace, size_t workspace_bytes) {
+    const int M = calls[0].M, mt = (M + 15) / 16;
+    const WeightKind kind = calls[0].kind;
+    SkinnyCalls L;
+    long blocks = 0;
+    size_t lds = 0, sums = 0;
+    int counters = 0;
+    auto flush = [&]() {
+        if (L.n == 0) return true;
+        L.M = M;
+        const auto nb = static_cast<unsigned>(blocks);
+        const bool ok = kind == WK_Q4 ? (terms == 1 ? launch_calls_mt<WK_Q4, 1>(s, L, nb, lds) : launch_calls_mt<WK_Q4, 2>(s, L, nb, lds))
+                      : kind == WK_F16 ? launch_calls_mt<WK_F16, 1>(s, L, nb, lds) : launch_calls_mt<WK_I8, 1>(s, L, nb, lds);
+        L = SkinnyCalls{};
+        blocks = 0;
+        lds = sums = 0;
+        counters = 0;
+        return ok;
+    };
+    long crowd = 0;                                      // blocks the calls of much LDS would like
+    auto is_big = [&](size_t need) { return need > kLdsLimit / 2; };
+    for (int i = 0; i < n; ++i) {
+        const Shape sh = pick_shape(kind, M, calls[i].N, calls[i].K, device_info().cus, workspace_bytes);
+        const long strips = (calls[i].N + 15) / 16, per_block = kWaves / sh.ks;
+        if (is_big(lds_bytes(mt, calls[i].K, sh.xl, sh.ks))) crowd += (strips + per_block - 1) / per_block;
+    }
+    for (int pass = 0; pass < 3; ++pass) {               // slices over blocks; the others; those of much LDS
+        if (pass == 2 && !flush()) return false;
+        for (int i = 0; i < n; ++i) {
+            const GemvCall& c = calls[i];
+            const Shape sh = pick_shape(kind, M, c.N, c.K, device_info().cus, workspace_bytes);
+            const size_t need = lds_bytes(mt, c.K, sh.xl, sh.ks);
+            if (pass != (is_big(need) ? 2 : sh.kb > 1 ? 0 : 1)) continue;
+            const int strips = (c.N + 15) / 16, per_block = kWaves / sh.ks, logical = (strips + per_block - 1) / per_block;
+            long along_n = blocks_along_n(sh.xl, logical, need);
+            if (pass == 2 && crowd > device_info().cus) along_n = (static_cast<long>(logical) * device_info().cus + crowd - 1) / crowd;
+            const long nb = along_n * sh.kb;
+            if (need > kLdsLimit || nb > 65535) {
+                MI_ERROR_FMT("gemm: a call beyond a launch of several (M=%d N=%d K=%d)", M, c.N, c.K);
+                return false;
+            }
+            const size_t bytes = sh.kb > 1 ? partial_bytes(mt, c.N, sh.kb) : 0;
+            if (L.n == kMaxManyGemm || blocks + nb > 65535 || sums + bytes > workspace_bytes ||
+                counters + (bytes ? strips * mt : 0) > kSliceCounters) {
+                if (!flush()) return false;
+            }
+            SkinnyCalls::Call& d = L.c[L.n];
+            d.X = static_cast<const uint16_t*>(c.x);
+            d.W = static_cast<const uint8_t*>(c.W);
+            d.scale = static_cast<const uint16_t*>(c.scale);
+            d.out = static_cast<uint16_t*>(c.y);
+            d.N = c.N; d.K = c.K; d.logical = logical;
+            d.blocks = static_cast<uint16_t>(along_n);
+            d.ks_xl = static_cast<uint8_t>(sh.ks + (sh.xl ? 16 : 0));
+            d.kb = static_cast<uint8_t>(sh.kb);
+            if (bytes) {
+                d.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + sums);
+                d.counters = slice_counters(workspace) + counters;
+                sums += bytes;
+                counters += strips * mt;
+            }
+            L.first[L.n++] = static_cast<uint16_t>(blocks);
+            blocks += nb;
+            if (need > lds) lds = need;
+        }
+    }
+    return flush();
 }
 
 }  // namespace skinny
@@ -1978,6 +2118,24 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
         p.tile_rows = 32 * tm;
     }
     return launch_planned(s, p, kind, M, mat[0].N, K, x, mat[0].W, mat[0].scale, mat[0].out, workspace, ws_bytes, more) ? g : -1;
+}
+
+// Calls that the streaming kernel serves, each by its own plan.
+bool gemm_many_takes(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
+    return c.M <= skinny::kMaxM && gemm_supported(c.kind, c.M, c.N, c.K, c.x, c.W, c.scale) && (c.N + 15) / 16 <= 8191 &&
+           plan_gemm(s, c.kind, c.M, c.N, c.K, workspace_bytes).kernel == 4;
+}
+
+bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes) {
+    const size_t ws_bytes = workspace ? workspace_bytes : 0;
+    for (int i = 0; i < n; ++i) {
+        if (calls[i].M != calls[0].M || calls[i].kind != calls[0].kind || !gemm_many_takes(s, calls[i], ws_bytes)) {
+            MI_ERROR_FMT("gemm: a call that does not fit a launch of several (M=%d N=%d K=%d)", calls[i].M, calls[i].N, calls[i].K);
+            return false;
+        }
+    }
+    const GemmPlan p = plan_gemm(s, calls[0].kind, calls[0].M, calls[0].N, calls[0].K, ws_bytes);
+    return skinny::launch_many(s, calls, n, p.terms, workspace, ws_bytes);
 }
 
 }  // namespace mi

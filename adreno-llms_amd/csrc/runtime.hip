@@ -45,7 +45,6 @@ std::mutex g_registry_mu;
 // mi_init: allocated there, never inside a compute call.  Work on one stream is ordered, so the
 // calls of a stream can share its workspace; a stream from elsewhere has none and its GEMMs
 // simply do not slice K.
-constexpr size_t kWorkspaceBytes = 16u << 20;
 std::unordered_map<hipStream_t, void*> g_workspace;
 struct StreamModes { int gemv = -1, gemm = -1; };      // -1: the process default
 std::unordered_map<hipStream_t, StreamModes> g_stream_modes;
@@ -63,8 +62,11 @@ void* workspace_of(hipStream_t s) {
 
 void add_workspace(hipStream_t s) {
     void* p = nullptr;
-    if (hipMalloc(&p, kWorkspaceBytes) != hipSuccess) {
+    // (the counters are cleared on the stream itself, ahead of whatever will use them)
+    if (hipMalloc(&p, kWorkspaceBytes + kSliceCounters * sizeof(uint32_t)) != hipSuccess ||
+        hipMemsetAsync(slice_counters(p), 0, kSliceCounters * sizeof(uint32_t), s) != hipSuccess) {
         (void)hipGetLastError();      // no workspace: that stream's GEMMs run unsliced
+        (void)hipFree(p);
         return;
     }
     std::lock_guard<std::mutex> lk(g_registry_mu);
@@ -499,75 +501,99 @@ static void next_run(hipStream_t s, const mi_linear_call* calls, int n, BatchRun
     }
 }
 
-// The launches of one run: how many of its calls were enqueued, -1 on an error.
-static int launch_run(hipStream_t s, const BatchRun& r) {
-    const GemvCall& c = r.c[0];
-    if (!r.gemm) return launch_gemv_group(s, r.c, r.n) ? r.n : -1;
-    int g = 0;
-    if (r.n > 1) {
-        GemmMat mats[kMaxSegments];
-        for (int j = 0; j < r.n; ++j) mats[j] = GemmMat{r.c[j].W, r.c[j].scale, r.c[j].y, r.c[j].N};
-        g = launch_gemm_group(s, c.kind, r.n, mats, c.M, c.K, c.x, workspace_of(s), kWorkspaceBytes);
+// The launches of one run.
+static bool launch_run(hipStream_t s, const GemvCall* c, int n, bool gemm) {
+    if (!gemm) return launch_gemv_group(s, c, n);
+    for (int i = 0; i < n;) {
+        int g = 0;
+        if (n - i > 1) {
+            GemmMat mats[kMaxSegments];
+            for (int j = i; j < n; ++j) mats[j - i] = GemmMat{c[j].W, c[j].scale, c[j].y, c[j].N};
+            g = launch_gemm_group(s, c->kind, n - i, mats, c->M, c->K, c->x, workspace_of(s), kWorkspaceBytes);
+            if (g < 0) return false;
+        }
+        if (g == 0) {
+            if (!mi_linear(s, c->M, c[i].N, c->K, c->x, c[i].W, c[i].y)) return false;
+            g = 1;
+        }
+        i += g;
     }
-    if (g == 0) g = mi_linear(s, c.M, c.N, c.K, c.x, c.W, c.y) ? 1 : -1;
-    return g;
+    return true;
 }
 
-// Behind a GEMV run, the runs that follow it, whatever their x and K, join its launch as long as they are GEMVs of its
-// M and weight kind that gemv_many has instances for and no call reads or writes what another call of the launch
-// writes: what a launch holds cannot observe the order of its blocks.  One token's projections of SmolLM2-135M in fp16,
-// seven calls of four runs, 16.6 -> 4.8 us; the 169 of Qwen2.5-0.5B in int8, each layer with buffers of its own and so
-// independent, 320 -> 93 us (three launches; a decode step in which attention stands between them has its runs alone).
+// A window: consecutive runs, whatever their x, M, K and weight kind, none of whose calls reads or writes what another
+// call of the window writes.  No order among them can be observed, so the runs of a window that one launch can hold go
+// out together: GEMVs of one M and weight kind (launch_gemv_many), GEMMs of one M and weight kind that the streaming
+// kernel serves (launch_gemm_many); the others as launches of their own.  One token's projections of SmolLM2-135M in
+// fp16, seven calls of four runs, 16.6 -> 4.8 us; of the 0.5B model at 16 int8 rows 26.6 -> 14.0 us; the 169 of Qwen2.5-0.5B in int8, each layer
+// with buffers of its own and so independent, 320 -> 93 us (three launches; a decode step in which attention stands
+// between them has its runs alone).
 int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
     if (!ensure_init()) return 0;
     if (!calls || n < 0) { MI_ERROR_FMT("mi_linear_batch: bad argument"); return 0; }
     const hipStream_t s = as_stream(stream);
-    GemvCall many[kMaxMany];
+    GemvCall held[kMaxMany], some[kMaxMany];
     CallMemory memory[kMaxMany];
+    enum Launch : char { DONE, ALONE, GEMVS, GEMMS };
+    struct { int first, n; Launch how; bool gemm; } run[kMaxMany];
     int run_of[kMaxMany];
     BatchRun r;
-    int i = 0;
     bool have = false;                                   // r is the run at calls[i]
+    int i = 0;
     while (i < n) {
         if (!have) next_run(s, calls + i, n - i, &r);
-        have = false;
-        int held = 0, runs = 0;
-        while (r.n > 0 && !r.gemm && held + r.n <= kMaxMany) {
-            bool joins = true;
-            for (int j = 0; j < r.n && joins; ++j) {
-                joins = gemv_many_takes(r.c[j]) && (held == 0 || (r.c[j].kind == many[0].kind && r.c[j].M == many[0].M));
-                for (int q = 0; q < held && joins; ++q) joins = independent(memory[q], r.memory[j]);
-            }
-            if (!joins) break;
-            for (int j = 0; j < r.n; ++j) {
-                many[held] = r.c[j];
-                memory[held] = r.memory[j];
-                run_of[held++] = runs;
-            }
-            ++runs;
-            have = i + held < n;
-            if (!have) break;
-            next_run(s, calls + i + held, n - i - held, &r);
-        }
-        if (runs > 1) {
-            if (!launch_gemv_many(s, many, run_of, held)) return i;
-            i += held;
-            continue;
-        }
-        if (runs == 1) {                                 // alone: the launch of a run
-            if (!launch_gemv_group(s, many, held)) return i;
-            i += held;
-            continue;
-        }
-        if (r.n == 0) {
+        have = true;
+        if (r.n == 0) {                                  // no launch for several: out aliases an operand, many rows of GEMV, an error
             const mi_linear_call& c = calls[i];
             if (!mi_linear(stream, c.M, c.N, c.K, c.x, c.W, c.out)) return i;
             ++i;
+            have = false;
             continue;
         }
-        const int g = launch_run(s, r);
-        if (g < 0) return i;
-        i += g;
+        int count = 0, runs = 0;
+        while (r.n > 0 && count + r.n <= kMaxMany) {
+            bool apart = true;
+            for (int j = 0; j < r.n && apart; ++j)
+                for (int q = 0; q < count && apart; ++q) apart = independent(memory[q], r.memory[j]);
+            if (!apart) break;
+            bool gemvs = !r.gemm, gemms = r.gemm;
+            for (int j = 0; j < r.n; ++j) {
+                held[count + j] = r.c[j];
+                memory[count + j] = r.memory[j];
+                gemvs = gemvs && gemv_many_takes(r.c[j]);
+                gemms = gemms && gemm_many_takes(s, r.c[j], workspace_of(s) ? kWorkspaceBytes : 0);
+            }
+            run[runs].first = count;
+            run[runs].n = r.n;
+            run[runs].gemm = r.gemm;
+            run[runs++].how = gemvs ? GEMVS : gemms ? GEMMS : ALONE;
+            count += r.n;
+            have = i + count < n;
+            if (!have) break;
+            next_run(s, calls + i + count, n - i - count, &r);
+        }
+        for (int a = 0; a < runs; ++a) {
+            if (run[a].how == DONE) continue;
+            const GemvCall& c = held[run[a].first];
+            int g = 0, members = 0;
+            for (int b = a; b < runs; ++b) {             // the runs that share run a's launch, itself among them
+                const GemvCall& d = held[run[b].first];
+                if (b != a && (run[a].how == ALONE || run[b].how != run[a].how || d.M != c.M || d.kind != c.kind)) continue;
+                for (int j = 0; j < run[b].n; ++j) {
+                    some[g] = held[run[b].first + j];
+                    run_of[g++] = b;
+                }
+                ++members;
+                if (b != a) run[b].how = DONE;
+            }
+            if (members == 1) {
+                if (!launch_run(s, some, g, run[a].gemm)) return i;
+            } else if (!(run[a].how == GEMVS ? launch_gemv_many(s, some, run_of, g)
+                                             : launch_gemm_many(s, some, g, workspace_of(s), kWorkspaceBytes))) {
+                return i;
+            }
+        }
+        i += count;
     }
     return n;
 }
