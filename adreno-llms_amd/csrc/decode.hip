@@ -669,8 +669,19 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_tiled(uint16_t* _
 // The same real numbers as softmax(q k) v, summed in another order and without the fp16 roundings of the
 // probabilities: within the stated tolerance of the reference-order launch, not bit-identical.
 // part: [n_heads][splits][D + 2] floats: m, l, o[D].
+//
+// The launch is a chain of trips to memory: the position, then the block's rows of both caches.  They are asked for
+// at once, 16 bytes per lane (a tile of keys and a tile of values in registers), and turned over to LDS as they are
+// needed: a thread takes the score of a key from the key tile, then one element of the output over every kGroups-th
+// key from the value tile.  14 heads at position 3701 in 16 splits, us per launch: rows read by a thread each and
+// values 2 bytes at a time, 32 in flight, 10.2 -> this 8.7 (6.8 either way at
+// position 2000, where 32 in flight is all there are).  The heads of a group that read the same run put on one XCD: no gain.
 constexpr int kSplitThreads = 256;
 constexpr int kMaxSplits = 32;
+constexpr int split_tile(int D) { return 16384 / D; }          // keys per tile (256 / 128)
+constexpr int split_groups(int D) { return kSplitThreads / D; }
+// Floats of LDS for the exponentials: per group its keys one behind the other, rows of whole 16 bytes
+__host__ __device__ inline int split_group_cap(int D, int chunk_cap) { return ((chunk_cap + split_groups(D) - 1) / split_groups(D) + 3) & ~3; }
 
 template <int D>
 __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
@@ -680,136 +691,153 @@ __global__ __launch_bounds__(kSplitThreads) void attention_split_kernel(
         const uint16_t* __restrict__ bv, const uint16_t* __restrict__ rope_now, uint16_t* __restrict__ q_out,
         uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out, float* __restrict__ part, int chunk_cap) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kTile = split_tile(D), kGroups = split_groups(D);
+    constexpr int kPieces = D / 8, kPassRows = kSplitThreads / kPieces, kPasses = kTile / kPassRows;
+    constexpr int kRowH = D + 8;                               // halves between key rows in LDS (values: D)
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    float* sc = sm;                                            // [chunk_cap] scores, then exponentials
-    float* red = sc + chunk_cap;                               // [8] block reductions
+    const int gcap = split_group_cap(D, chunk_cap);
+    float* ex = sm;                                            // [kGroups][gcap] scores, then exponentials
+    float* red = ex + kGroups * gcap;                          // [8] block reductions
     float* osum = red + 8;                                     // [kSplitThreads / D][D] partial outputs
-    uint16_t* qv = reinterpret_cast<uint16_t*>(osum + kSplitThreads);   // [D] q, [D] k, [D] v of the current position
-    uint16_t* kcur = qv + D;
-    uint16_t* vcur = kcur + D;
+    uint16_t* qv = reinterpret_cast<uint16_t*>(osum + kSplitThreads);   // [D] q
+    uint16_t* tile = qv + D;                                   // [kTile][kRowH] keys, then [kTile][D] values
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int qh = blockIdx.x, sp = blockIdx.y, splits = gridDim.y;
     const int nrep = n_heads / n_kv_heads, kvh = qh / nrep, kvd = n_kv_heads * D, hd2 = D / 2;
     int pos = st->pos;
+    // what the current position needs, a few bytes per thread behind other pointers, rides along with the position:
+    // threads 0 .. D/2 - 1 take a pair of q, 64 .. a pair of k, 128 .. an element of v
+    const int role = tid < 64 ? 0 : tid < 128 ? 1 : 2;
+    const int i = role < 2 ? ((tid & 63) < hd2 ? tid & 63 : hd2 - 1) : (tid - 128 < D ? tid - 128 : D - 1);
+    const int i2 = role < 2 ? i + hd2 : i;
+    const uint16_t* buf = role == 0 ? q_raw + qh * D : role == 1 ? k_raw + kvh * D : v_raw + kvh * D;
+    const uint16_t* bias = role == 0 ? bq + qh * D : role == 1 ? bk + kvh * D : bv + kvh * D;
+    const uint16_t raw1 = buf[i], raw2 = buf[i2], bias1 = bias[i], bias2 = bias[i2];
+    const uint16_t cos_i = rope_now[role < 2 ? i : 0], sin_i = rope_now[D + (role < 2 ? i : 0)];
+
     pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
     const int seq_k = pos + 1;
     const int chunk = (seq_k + splits - 1) / splits;           // <= chunk_cap: the host sizes it for max_pos
-    const int k0 = sp * chunk, k1 = k0 + chunk < seq_k ? k0 + chunk : seq_k;
+    const int k0 = sp * chunk, k1 = k0 + chunk < seq_k ? k0 + chunk : seq_k, n = k1 - k0;
     float* mine = part + (static_cast<size_t>(qh) * splits + sp) * (D + 2);
-    if (k0 >= k1) {                                            // no keys for this block at this position
+    if (n <= 0) {                                              // no keys for this block at this position
         if (tid == 0) { mine[0] = -3.402823466e+38f; mine[1] = 0.0f; }
         if (tid < D) mine[2 + tid] = 0.0f;
         return;
     }
     const bool has_current = k1 == seq_k;                      // the block whose run ends with the current position
-    // Everything the block reads from memory is asked for now, behind the position alone: the row of the
-    // thread's first key, the first kAhead values of the thread's output element, and (below) the current
-    // position's q, k and v; the arithmetic then waits for one round trip, not for four in a row.
-    constexpr int kGroups = kSplitThreads / D, kAhead = 32;
-    const int d = tid % D, grp = tid / D;
-    const int c_first = k0 + tid;
-    u32x4 kr_first[D / 8];
-    // (a thread without such a key reads row 0 instead and does not use it: loads under a condition of
-    //  their own were measured slower, 548 -> 576 us per step at position 2000)
-    {
-        const bool from_cache = c_first < k1 && c_first != pos;
-        const u32x4* row = reinterpret_cast<const u32x4*>(kc + static_cast<size_t>(from_cache ? c_first : 0) * kvd + kvh * D);
+    // piece p of this thread in a tile: row tid / kPieces + p kPassRows, 16-byte piece tid % kPieces; rows past the
+    // run's last key are read as that key's and not used
+    const int prow = tid / kPieces, piece = tid % kPieces;
+    u32x4 kreg[kPasses], vreg[kPasses];
+    auto request = [&](u32x4 (&reg)[kPasses], const uint16_t* cache, int t0) {
         #pragma unroll
-        for (int i = 0; i < D / 8; ++i) kr_first[i] = row[i];
+        for (int p = 0; p < kPasses; ++p)
+            if (t0 + p * kPassRows < n) {                      // (uniform)
+                const int row = t0 + prow + p * kPassRows, c = k0 + (row < n ? row : n - 1);
+                reg[p] = *reinterpret_cast<const u32x4*>(cache + static_cast<size_t>(c) * kvd + kvh * D + 8 * piece);
+            }
+    };
+    auto keep = [&](const u32x4 (&reg)[kPasses], int stride, int t0) {
+        #pragma unroll
+        for (int p = 0; p < kPasses; ++p)
+            if (t0 + p * kPassRows < n) {
+                const int row = prow + p * kPassRows;
+                if (k0 + t0 + row != pos) *reinterpret_cast<u32x4*>(tile + row * stride + 8 * piece) = reg[p];
+            }
+    };
+    request(kreg, kc, 0);
+    request(vreg, vc, 0);
+
+    const float cs = h_f(cos_i), sn = h_f(sin_i);
+    const float x1 = h_f(f_h(h_f(raw1) + h_f(bias1)));
+    const float x2 = h_f(f_h(h_f(raw2) + h_f(bias2)));
+    const uint16_t r1 = f_h(fmaf(x1, cs, -(x2 * sn))), r2 = f_h(fmaf(x2, cs, x1 * sn));
+    const uint16_t rv = f_h(x1);                               // fp16(v + bias), rounded once
+    const bool is_q = tid < hd2, is_k = has_current && tid >= 64 && tid < 64 + hd2, is_v = has_current && tid >= 128 && tid < 128 + D;
+    const int cur = pos - k0;                                  // the current position's row of the run
+    // Scores, tile by tile, a thread per key (key c of the run is thread c % 256's); the current position's key goes
+    // into its tile straight from the threads that made it.
+    float m = -3.402823466e+38f;
+    if (is_q) {
+        qv[i] = r1;
+        qv[i + hd2] = r2;
     }
-    uint16_t v_first[kAhead];
-    #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-        const int c = k0 + grp + i * kGroups;
-        v_first[i] = vc[static_cast<size_t>(c < k1 && c != pos ? c : 0) * kvd + kvh * D + d];
+    for (int t0 = 0; t0 < n; t0 += kTile) {
+        if (t0 > 0) __syncthreads();                           // the last tile has been used
+        keep(kreg, kRowH, t0);
+        if (is_k && cur >= t0 && cur < t0 + kTile) {
+            tile[(cur - t0) * kRowH + i] = r1;
+            tile[(cur - t0) * kRowH + i + hd2] = r2;
+        }
+        __syncthreads();
+        if (t0 + kTile < n) request(kreg, kc, t0 + kTile);
+        const int row = tid - t0 % kSplitThreads;              // (a tile is 256 keys or half of them)
+        if (row >= 0 && row < kTile && t0 + row < n) {
+            float acc = 0.0f;
+            #pragma unroll
+            for (int j = 0; j < D / 8; ++j) {
+                const u32x4 qq = reinterpret_cast<const u32x4*>(qv)[j], kk = *reinterpret_cast<const u32x4*>(tile + row * kRowH + 8 * j);
+                #pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc = fmaf(h_f(static_cast<uint16_t>(qq[e] & 0xffffu)), h_f(static_cast<uint16_t>(kk[e] & 0xffffu)), acc);
+                    acc = fmaf(h_f(static_cast<uint16_t>(qq[e] >> 16)), h_f(static_cast<uint16_t>(kk[e] >> 16)), acc);
+                }
+            }
+            const float sco = h_f(f_h(acc * scale));
+            const int c = t0 + row;
+            ex[(c % kGroups) * gcap + c / kGroups] = sco;
+            m = fmaxf(m, sco);
+        }
     }
-    // q of the head (every block), k and v of the current position (the block that needs them); the block of
-    // the group's first head also writes them to the caches and to the buffers a caller may inspect
-    if (tid < hd2) {
-        const float c = h_f(rope_now[tid]), sn = h_f(rope_now[D + tid]);
-        const float x1 = h_f(f_h(h_f(q_raw[qh * D + tid]) + h_f(bq[qh * D + tid])));
-        const float x2 = h_f(f_h(h_f(q_raw[qh * D + tid + hd2]) + h_f(bq[qh * D + tid + hd2])));
-        const uint16_t r1 = f_h(fmaf(x1, c, -(x2 * sn))), r2 = f_h(fmaf(x2, c, x1 * sn));
-        qv[tid] = r1;
-        qv[tid + hd2] = r2;
-        if (sp == 0) { q_out[qh * D + tid] = r1; q_out[qh * D + tid + hd2] = r2; }
-    } else if (has_current && tid >= 64 && tid < 64 + hd2) {
-        const int i = tid - 64;
-        const float c = h_f(rope_now[i]), sn = h_f(rope_now[D + i]);
-        const float x1 = h_f(f_h(h_f(k_raw[kvh * D + i]) + h_f(bk[kvh * D + i])));
-        const float x2 = h_f(f_h(h_f(k_raw[kvh * D + i + hd2]) + h_f(bk[kvh * D + i + hd2])));
-        const uint16_t r1 = f_h(fmaf(x1, c, -(x2 * sn))), r2 = f_h(fmaf(x2, c, x1 * sn));
-        kcur[i] = r1;
-        kcur[i + hd2] = r2;
-        if (qh % nrep == 0) {
+    // (the outputs a caller may inspect and the cache rows, behind the loads)
+    if (is_q && sp == 0) { q_out[qh * D + i] = r1; q_out[qh * D + i + hd2] = r2; }
+    if (qh % nrep == 0) {
+        if (is_k) {
             uint16_t* dst = kc + static_cast<size_t>(pos) * kvd + kvh * D;
             dst[i] = r1; dst[i + hd2] = r2;
             k_out[kvh * D + i] = r1; k_out[kvh * D + i + hd2] = r2;
+        } else if (is_v) {
+            vc[static_cast<size_t>(pos) * kvd + kvh * D + i] = rv;
+            v_out[kvh * D + i] = rv;
         }
-    } else if (has_current && tid >= 128 && tid < 128 + D) {
-        const int e = tid - 128;
-        const uint16_t r = f_h(h_f(v_raw[kvh * D + e]) + h_f(bv[kvh * D + e]));
-        vcur[e] = r;
-        if (qh % nrep == 0) {
-            vc[static_cast<size_t>(pos) * kvd + kvh * D + e] = r;
-            v_out[kvh * D + e] = r;
-        }
-    }
-    __syncthreads();
-    // scores, a thread per key: the key's row straight from the cache (the current position's from LDS)
-    float m = -3.402823466e+38f;
-    for (int c = c_first; c < k1; c += kSplitThreads) {
-        u32x4 kr[D / 8];
-        if (c == pos) {
-            #pragma unroll
-            for (int i = 0; i < D / 8; ++i) kr[i] = reinterpret_cast<const u32x4*>(kcur)[i];
-        } else if (c == c_first) {
-            #pragma unroll
-            for (int i = 0; i < D / 8; ++i) kr[i] = kr_first[i];
-        } else {
-            const u32x4* row = reinterpret_cast<const u32x4*>(kc + static_cast<size_t>(c) * kvd + kvh * D);
-            #pragma unroll
-            for (int i = 0; i < D / 8; ++i) kr[i] = row[i];
-        }
-        float acc = 0.0f;
-        #pragma unroll
-        for (int i = 0; i < D / 8; ++i) {
-            const u32x4 qq = reinterpret_cast<const u32x4*>(qv)[i];
-            const uint32_t qd[4] = {qq.x, qq.y, qq.z, qq.w}, kd[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-            #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc = fmaf(h_f(static_cast<uint16_t>(qd[j] & 0xffffu)), h_f(static_cast<uint16_t>(kd[j] & 0xffffu)), acc);
-                acc = fmaf(h_f(static_cast<uint16_t>(qd[j] >> 16)), h_f(static_cast<uint16_t>(kd[j] >> 16)), acc);
-            }
-        }
-        const float sco = h_f(f_h(acc * scale));
-        sc[c - k0] = sco;
-        m = fmaxf(m, sco);
     }
     m = wave_max(m);
     if (lane == 0) red[wave] = m;
-    __syncthreads();
+    __syncthreads();                                           // scores and maxima are in LDS, the keys have been used
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     float l = 0.0f;
-    for (int c = k0 + tid; c < k1; c += kSplitThreads) {
-        const float e = exp_poly(sc[c - k0] - m);
-        sc[c - k0] = e;
+    for (int c = tid; c < n; c += kSplitThreads) {
+        float* at = ex + (c % kGroups) * gcap + c / kGroups;
+        const float e = exp_poly(*at - m);
+        *at = e;
         l += e;
     }
     for (int sft = 32; sft > 0; sft >>= 1) l += __shfl_xor(l, sft, 64);
     if (lane == 0) red[4 + wave] = l;
-    __syncthreads();                                           // exponentials and the waves' sums are in LDS
-    // o[d]: kSplitThreads / D groups of D threads, group g takes the keys k0 + g, k0 + g + groups, ...
+    // o[d]: kSplitThreads / D groups of D threads, group g takes the keys g, g + groups, ... of the run
+    const int d = tid % D, grp = tid / D;
+    const float* ep = ex + grp * gcap;
     float o = 0.0f;
-    #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-        const int c = k0 + grp + i * kGroups;
-        if (c < k1) o = fmaf(sc[c - k0], h_f(c == pos ? vcur[d] : v_first[i]), o);
-    }
-    #pragma unroll 8
-    for (int c = k0 + grp + kAhead * kGroups; c < k1; c += kGroups) {
-        const uint16_t v = c == pos ? vcur[d] : vc[static_cast<size_t>(c) * kvd + kvh * D + d];
-        o = fmaf(sc[c - k0], h_f(v), o);
+    for (int t0 = 0; t0 < n; t0 += kTile) {
+        if (t0 > 0) __syncthreads();                           // the last tile has been used
+        keep(vreg, D, t0);
+        if (is_v && cur >= t0 && cur < t0 + kTile) tile[(cur - t0) * D + i] = rv;
+        __syncthreads();                                       // (and the exponentials and the waves' sums are in LDS)
+        if (t0 + kTile < n) request(vreg, vc, t0 + kTile);
+        const int rows = n - t0 < kTile ? n - t0 : kTile, count = (rows - grp + kGroups - 1) / kGroups, i0 = t0 / kGroups;
+        const uint16_t* vp = tile + grp * D + d;
+        int r = 0;
+        for (; r + 8 <= count; r += 8) {                       // eight keys read ahead of their sums
+            const f32x4 e0 = *reinterpret_cast<const f32x4*>(ep + i0 + r), e1 = *reinterpret_cast<const f32x4*>(ep + i0 + r + 4);
+            uint16_t v[8];
+            #pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = vp[(r + u) * kGroups * D];
+            #pragma unroll
+            for (int u = 0; u < 8; ++u) o = fmaf(u < 4 ? e0[u % 4] : e1[u % 4], h_f(v[u]), o);
+        }
+        for (; r < count; ++r) o = fmaf(ep[i0 + r], h_f(vp[r * kGroups * D]), o);
     }
     osum[grp * D + d] = o;
     __syncthreads();
@@ -857,7 +885,8 @@ __global__ __launch_bounds__(D) void attention_merge_kernel(const float* __restr
 }
 
 inline size_t split_attention_lds(int D, int chunk_cap) {
-    return static_cast<size_t>(chunk_cap + 8 + kSplitThreads) * 4 + 3 * static_cast<size_t>(D) * 2;
+    return (static_cast<size_t>(split_groups(D)) * split_group_cap(D, chunk_cap) + 8 + kSplitThreads) * 4 +
+           (static_cast<size_t>(D) + static_cast<size_t>(split_tile(D)) * (D + 8)) * 2;
 }
 
 // gate[i] = fp16((g * sigmoid(g)) * up[i])   (QW/kernels/mlp.cl swiglu_inplace)
