@@ -78,8 +78,7 @@ struct SegList {
 __device__ __forceinline__ float add_residual(float sum, float s, float res, bool scaled, int mode) {
     if (mode == ADD_ROUNDED) return h_f(f_h(scaled ? sum * s : sum)) + res;
     if (mode == ADD_SILU_GATE) {
-        const float sig = __fdiv_rn(1.0f, 1.0f + exp_poly(-res));
-        return (res * sig) * (scaled ? sum * s : sum);
+        return (res * sigmoid_of_half(res)) * (scaled ? sum * s : sum);     // (res is a value of y)
     }
     return scaled ? fmaf(sum, s, res) : sum + res;
 }
@@ -443,8 +442,7 @@ __device__ __forceinline__ void fixed_k_rows(MI_HOT_PARAMS, const SegList& L, co
                 const float sgs = KIND == WK_I8 ? sg_ * h_f(g0.b[0].s[0]) : sg_;
                 const float sus = KIND == WK_I8 ? su_ * h_f(g1.b[0].s[0]) : su_;
                 const float gv = h_f(f_h(sgs)), uv = h_f(f_h(sus));
-                const float sig = __fdiv_rn(1.0f, 1.0f + exp_poly(-gv));
-                g0.b[0].ybase[g0.b[0].yoff] = f_h((gv * sig) * uv);
+                g0.b[0].ybase[g0.b[0].yoff] = f_h((gv * sigmoid_of_half(gv)) * uv);
             }
             rb += nw;
             if (rb >= hnbatch) break;
