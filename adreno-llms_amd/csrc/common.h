@@ -164,6 +164,13 @@ inline uint32_t* slice_counters(void* workspace) {
 }
 // runtime.hip: the same for a registered W where mi_linear would run the GEMM
 int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W, void* out);
+// gemm.hip, runtime.hip: the sums of the K slices of a GEMM that mi_linear would cut into slices, left in the stream's
+// workspace as fp32 [slices][M][N]; *scale: what they are still to be multiplied with per column (null: nothing).  Only
+// for columns that come in whole fours, with their scales at a multiple of 8 bytes.
+// Returns the number of slices, 0 (nothing was launched) or -1 (an error).
+int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
+                       void* workspace, size_t workspace_bytes);
+int linear_slices(hipStream_t s, int M, int N, int K, const void* x, const void* W, const float** sums, const void** scale);
 // whether mi_linear would run the GEMM (and not rows of GEMV) for the call
 bool linear_takes_gemm(hipStream_t s, int M, int N, int K, const void* x, const void* W);
 // The first of n projections of one x (M >= 2, the first accepted by gemm_supported) in one launch, where one

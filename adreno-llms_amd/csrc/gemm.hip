@@ -871,6 +871,7 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
                        static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
                        static_cast<uint16_t*>(out), M, N, K, splits > 1 ? partial : nullptr, splits, more, static_cast<int>(glu));
     if (!MI_HIP_OK(hipGetLastError())) return false;
+    if (splits > 1 && !out) return true;                 // the sums stay where they are (launch_gemm_slices)
     if (splits > 1 && glu) {
         const long MN = static_cast<long>(M) * N;
         hipLaunchKernelGGL(reduce_partials_glu, dim3(static_cast<unsigned>((MN / 8 + 255) / 256)), dim3(256), 0, s, partial, splits,
@@ -2074,6 +2075,17 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
           (p.kernel == 4 && skinny::glu_shape(skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes)))))
         return 0;
     return launch_planned(s, p, kind, M, N, K, x, W, scale, out, workspace, ws_bytes, MoreMats{}, true) ? 1 : -1;
+}
+
+// launch_gemm's own plan for the call where it cuts K into slices, up to their sums: fp32 [slices][M][N] at the start of
+// the workspace, for a launch that adds them in index order and goes on with the result (decode.hip).  Returns the number
+// of slices; 0: the plan has none (nothing was launched); -1: an error.
+int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
+                       void* workspace, size_t workspace_bytes) {
+    if (!workspace || !gemm_supported(kind, M, N, K, x, W, scale)) return 0;
+    const GemmPlan p = plan_gemm(s, kind, M, N, K, workspace_bytes);
+    if (p.kernel != 1 || p.k_slices < 2) return 0;
+    return launch_planned(s, p, kind, M, N, K, x, W, scale, nullptr, workspace, workspace_bytes, MoreMats{}) ? p.k_slices : -1;
 }
 
 // One launch serves the leading matrices whose own plans sum K in the same order, so that each result is what

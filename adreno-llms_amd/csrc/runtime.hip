@@ -713,4 +713,15 @@ int linear_glu(hipStream_t s, int M, int N, int K, const void* x, const void* W,
     return launch_gemm_glu(s, e.kind, M, N, K, x, W, e.scale, out, workspace_of(s), kWorkspaceBytes);
 }
 
+int linear_slices(hipStream_t s, int M, int N, int K, const void* x, const void* W, const float** sums, const void** scale) {
+    if (!ensure_init()) return -1;
+    Entry e;
+    if (!resolve("mi_decoder_prefill", W, N, K, &e)) return -1;
+    void* ws = workspace_of(s);
+    if (!ws || N % 4 || (e.kind == WK_I8 && reinterpret_cast<uintptr_t>(e.scale) % 8) || !takes_gemm(s, e, M, N, K, x, W)) return 0;
+    *sums = static_cast<const float*>(ws);
+    *scale = e.kind == WK_I8 ? e.scale : nullptr;
+    return launch_gemm_slices(s, e.kind, M, N, K, x, W, e.scale, ws, kWorkspaceBytes);
+}
+
 }  // namespace mi
