@@ -114,6 +114,18 @@ bool fused_gemv_kind(const void* W, int N, int K, WeightKind* kind);   // kind W
 // The same with the scales W was registered with (null for fp16 weights).
 bool registered_weight(const void* W, int N, int K, WeightKind* kind, const void** scale);
 
+// What the registry holds for W (kind fp16, no scale: nothing), and a number that every registration and removal raises.
+struct WeightEntry {
+    WeightKind kind = WK_F16;
+    const void* scale = nullptr;
+    int N = 0, K = 0;
+    bool operator==(const WeightEntry& o) const { return kind == o.kind && scale == o.scale && N == o.N && K == o.K; }
+};
+WeightEntry weight_entry(const void* W);
+uint64_t registry_epoch();
+// The workspace of a stream that mi_stream_create made (null: another stream, or no memory was left for one)
+void* own_stream_workspace(hipStream_t s);
+
 // argmax.hip: index of the greatest of N fp16 values, ties as the reference's two argmax kernels break them.
 // scratch: kArgmaxScratchBytes of device memory that belongs to stream s, or null (then one block does all the work).
 constexpr size_t kArgmaxScratchBytes = 512;

@@ -40,6 +40,7 @@ struct Entry {
 };
 std::unordered_map<const void*, Entry> g_registry;
 std::mutex g_registry_mu;
+std::atomic<uint64_t> g_registry_epoch{0};
 
 // One GEMM workspace per stream made by mi_stream_create, and one for the null stream made by
 // mi_init: allocated there, never inside a compute call.  Work on one stream is ordered, so the
@@ -113,6 +114,16 @@ bool registered_weight(const void* W, int N, int K, WeightKind* kind, const void
     *scale = e.scale;
     return true;
 }
+
+WeightEntry weight_entry(const void* W) {
+    Entry e;
+    if (!lookup(W, &e)) return WeightEntry{};
+    return WeightEntry{e.kind, e.scale, e.N, e.K};
+}
+
+uint64_t registry_epoch() { return g_registry_epoch.load(); }
+
+void* own_stream_workspace(hipStream_t s) { return s ? workspace_of(s) : nullptr; }
 
 bool fused_gemv_kind(const void* W, int N, int K, WeightKind* kind) {
     Entry e;
@@ -302,6 +313,7 @@ int mi_register_int8_weight(const void* W, const void* scale, int N, int K) {
     if (!W || !scale || N <= 0 || K <= 0) return 0;          // LF/src/utils.cpp:358
     std::lock_guard<std::mutex> lk(g_registry_mu);
     g_registry[W] = Entry{WK_I8, scale, N, K};
+    g_registry_epoch.fetch_add(1);
     return 1;
 }
 
@@ -314,12 +326,15 @@ int mi_register_q4_weight(const void* W, const void* scale, int N, int K) {
     }
     std::lock_guard<std::mutex> lk(g_registry_mu);
     g_registry[W] = Entry{WK_Q4, scale, N, K};
+    g_registry_epoch.fetch_add(1);
     return 1;
 }
 
 int mi_unregister_weight(const void* W) {
     std::lock_guard<std::mutex> lk(g_registry_mu);
-    return g_registry.erase(W) ? 1 : 0;
+    if (!g_registry.erase(W)) return 0;
+    g_registry_epoch.fetch_add(1);
+    return 1;
 }
 
 int mi_weight_kind(const void* W) {
