@@ -1,7 +1,7 @@
 """Prompts whose projections are cut into slices of K: the launch that adds the slices also adds the residual and norms
 the row (o and down projection), or adds the biases, rotates q and k and fills the cache rows (q | k | v).  The first is
 held bit for bit to the separate launches, which run where a matrix's scales are not 8-byte aligned; both are held to
-the rows of GEMV within the GEMM's tolerance.  Rows around the tiles, 2 to 24 slices, hidden widths with and without a part
+the rows of GEMV within the GEMM's tolerance.  Rows around the tiles, hidden widths with and without a part
 of 256 columns left over, head widths 64 and 128, every weight kind."""
 import numpy as np
 import pytest
@@ -63,19 +63,21 @@ SHAPES = [(896, 4864, 14, 2, 64), (576, 1536, 9, 3, 64), (1024, 2816, 8, 2, 128)
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}")
-@pytest.mark.parametrize("rows", [65, 66, 130, 300])
-def test_sums_residual_and_norm_bit_for_bit(shape, rows):
+@pytest.mark.parametrize("rows", [65, 66, 97])
+@pytest.mark.parametrize("tile,slices", [(1, 2), (2, 3), (1, 4)])
+def test_sums_residual_and_norm_bit_for_bit(shape, rows, tile, slices):
+    """The number of slices pinned: left to itself the library may cut a projection for the one way and not for the other."""
     assert mil.lib().mi_init(0) == 1
     queue = mil.Queue()
     hidden, inter = shape[:2]
-    ids, got, sliced = [(37 * t) % VOCAB for t in range(rows)], [], 0
+    ids, got = [(37 * t) % VOCAB for t in range(rows)], []
+    print(f"{shape} rows {rows} slices {slices}", flush=True)
     for off in (False, True):
         dec, bufs, keep = _decoder(queue, "int8", *shape, off)
-        _, _, slices = mil.linear_plan(queue, rows, hidden, inter, bufs["wdown"][0], bufs["wdown"][0])
-        sliced += slices > 1
+        assert mil.lib().mi_stream_set_modes(queue.handle, -1, 100 * slices + 10 + tile)
+        assert mil.linear_plan(queue, rows, hidden, inter, bufs["wdown"][0], bufs["wdown"][0])[2] == slices
         got.append(_outputs(queue, dec, hidden, ids, 0, 2))
-    print(f"{shape} rows {rows}: {slices} slices", flush=True)
-    assert sliced == 2
+        assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
 
