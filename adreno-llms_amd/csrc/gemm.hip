@@ -81,12 +81,8 @@ __device__ __forceinline__ void pick_matrix(const MoreMats& mm, int& tile, const
     tile -= first;
 }
 
-// The sums over the even and the odd K-tiles are kept apart where TEAMS x SETS = 2 (halves_k), and added at the end: by two teams of
-// four wavefronts, or by one that keeps two sets of accumulators, with the same bits.  A K-tile is a chain (registers ->
-// LDS, barrier, fragments, MFMAs) of 0.5 to 0.6 us whatever the load, and where a CU has one 64 x 64 block only, nothing
-// else runs meanwhile: two teams take half as many steps (times at halves_k).
-template <int BM, int BN, int WM, int WN, int KIND, int TEAMS, int SETS>
-__global__ __launch_bounds__(kThreads * TEAMS) void gemm_kernel(const uint16_t* __restrict__ X,
+template <int BM, int BN, int WM, int WN, int KIND>
+__global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restrict__ X,
                                                         const uint8_t* __restrict__ W,
                                                         const uint16_t* __restrict__ scale,
                                                         uint16_t* __restrict__ out, int M, int N, int K,
@@ -99,22 +95,19 @@ __global__ __launch_bounds__(kThreads * TEAMS) void gemm_kernel(const uint16_t* 
     constexpr int B_CHUNKS = BN * B_CPR / kThreads;
     static_assert(A_CHUNKS >= 1 && B_CHUNKS >= 1, "tile too small for 256 threads");
 
-    // Two LDS stages (x tile then W tile in each) and kAhead register stages: the global
-    // loads of K-tile i + kAhead are issued while tile i is multiplied, which is what hides
+    // Two LDS stages (x tile then W tile in each) and kStages register stages: the global
+    // loads of K-tile i + kStages are issued while tile i is multiplied, which is what hides
     // the HBM / L2 latency (one tile ahead is far too short for it).
-    extern __shared__ __attribute__((aligned(16))) uint16_t lds_all[];
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     constexpr int kStageHalves = (BM + BN) * kLd;
-    constexpr int kAhead = SETS > 1 ? 4 : 3;                                 // register stages (with two sets an even number)
 
-    const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
-    uint16_t* const lds = lds_all + team * 2 * kStageHalves;
-    const int tid = threadIdx.x % kThreads, lane = tid % 64, wave = tid / 64;
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int wm = wave / (BN / WN), wn = wave % (BN / WN);
     // Block -> tile.  Blocks go to the 8 XCDs round-robin, each with an L2 of its own.  In the order of the tiles an XCD
     // keeps to its share of the columns of tiles where their number is even; where it is odd it comes through all of
     // them, and XCD x takes the x-th eighth of a list instead that runs through bands of kBand tiles along N, down M inside
-    // a band.  us, int8, tiles in order / in bands: 15 columns, 2048 x 960 x 960 16.1 / 13.3, 25, 700 x 1600 x 960 13.3 / 12.0, 9,
-    // 1200 x 576 x 1536 15.4 / 13.0; but 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.
+    // a band.  us, int8, tiles in order / in bands: 15 columns, 2048 x 960 x 960 16.2 / 12.2, 25, 700 x 1600 x 960 13.1 / 11.1, 9,
+    // 1200 x 576 x 1536 15.5 / 14.0; but 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.
     int tile_m, tile_n;
     const int tiles_n = more.n ? more.tiles : (N + BN - 1) / BN;
     if (tiles_n % 2 == 0) {                                                  // (a grid of tiles: no divisions)
@@ -136,16 +129,13 @@ __global__ __launch_bounds__(kThreads * TEAMS) void gemm_kernel(const uint16_t* 
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int gk = lane / 32, li = lane % 32;
 
-    floatx16 acc[TM][TN], odd[SETS > 1 ? TM : 1][SETS > 1 ? TN : 1];
+    floatx16 acc[TM][TN];
     #pragma unroll
     for (int t = 0; t < TM; ++t)
         #pragma unroll
         for (int u = 0; u < TN; ++u)
             #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[t][u][r] = 0.0f;
-                if constexpr (SETS > 1) odd[t][u][r] = 0.0f;
-            }
+            for (int r = 0; r < 16; ++r) acc[t][u][r] = 0.0f;
 
     struct Regs { u32x4 a[A_CHUNKS]; u32x4 b[B_CHUNKS]; };
     auto load_tile = [&](Regs& R, int k0) {
@@ -185,7 +175,7 @@ __global__ __launch_bounds__(kThreads * TEAMS) void gemm_kernel(const uint16_t* 
             }
         }
     };
-    auto multiply = [&](const uint16_t* As, const uint16_t* Bs, auto& sum) {
+    auto multiply = [&](const uint16_t* As, const uint16_t* Bs) {
         #pragma unroll
         for (int kk = 0; kk < kKT / 16; ++kk) {
             // lane group gk supplies k = 32 gk + 8 kk .. +7 of the tile, for both operands
@@ -201,83 +191,34 @@ __global__ __launch_bounds__(kThreads * TEAMS) void gemm_kernel(const uint16_t* 
             for (int t = 0; t < TM; ++t)
                 #pragma unroll
                 for (int u = 0; u < TN; ++u)
-                    sum[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t], b[u], sum[t][u], 0, 0, 0);
+                    acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t], b[u], acc[t][u], 0, 0, 0);
         }
     };
 
-    // Step i of a team is K-tile TEAMS i + team; every team takes the same steps (and meets the others at their
-    // barriers), the last of them on the last tile again, not multiplied, where the tiles do not divide evenly.
-    const int nk = K / kKT, steps = (nk + TEAMS - 1) / TEAMS;
-    auto tile_k = [&](int i) { return (TEAMS * i + team < nk ? TEAMS * i + team : nk - 1) * kKT; };
-    Regs R0, R1, R2, R3;
-    load_tile(R0, tile_k(0));
-    load_tile(R1, tile_k(1));
-    load_tile(R2, tile_k(2));
-    if constexpr (kAhead > 3) load_tile(R3, tile_k(3));
-    // One step: its tile goes registers -> LDS stage i % 2; one barrier publishes it (and, being
+    const int nk = K / kKT;
+    Regs R0, R1, R2;
+    load_tile(R0, 0);
+    load_tile(R1, (1 < nk ? 1 : nk - 1) * kKT);
+    load_tile(R2, (2 < nk ? 2 : nk - 1) * kKT);
+    // One step: tile i goes registers -> LDS stage i % 2; one barrier publishes it (and, being
     // the second barrier since stage i % 2 was last read, also guards the overwrite); the
-    // freed registers take the tile of step i + kAhead; the matrix cores run on the tile.
-#define MI_GEMM_STEP(R, SUM)                                                   \
+    // freed registers take tile i + 3; the matrix cores run on tile i.
+#define MI_GEMM_STEP(R)                                                        \
     {                                                                          \
         uint16_t* As = lds + (i & 1) * kStageHalves;                           \
         uint16_t* Bs = As + BM * kLd;                                          \
         store_tile(R, As, Bs);                                                 \
         __syncthreads();                                                       \
-        load_tile(R, tile_k(i + kAhead));                                      \
-        if (TEAMS == 1 || TEAMS * i + team < nk) multiply(As, Bs, SUM);        \
-        if (++i >= steps) break;                                               \
+        load_tile(R, (i + 3 < nk ? i + 3 : nk - 1) * kKT);                     \
+        multiply(As, Bs);                                                      \
+        if (++i >= nk) break;                                                  \
     }
-    if constexpr (SETS > 1) {
-        for (int i = 0;;) {
-            MI_GEMM_STEP(R0, acc)
-            MI_GEMM_STEP(R1, odd)
-            MI_GEMM_STEP(R2, acc)
-            MI_GEMM_STEP(R3, odd)
-        }
-        #pragma unroll
-        for (int t = 0; t < TM; ++t)
-            #pragma unroll
-            for (int u = 0; u < TN; ++u)
-                #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[t][u][r] += odd[t][u][r];
-    } else {
-        for (int i = 0;;) {
-            MI_GEMM_STEP(R0, acc)
-            MI_GEMM_STEP(R1, acc)
-            MI_GEMM_STEP(R2, acc)
-            if constexpr (kAhead > 3) MI_GEMM_STEP(R3, acc)
-        }
+    for (int i = 0;;) {
+        MI_GEMM_STEP(R0)
+        MI_GEMM_STEP(R1)
+        MI_GEMM_STEP(R2)
     }
 #undef MI_GEMM_STEP
-    if constexpr (TEAMS > 1) {
-        static_assert(TEAMS == 2 && 4 * TM * TN * 16 * 64 * 4 <= 4 * kStageHalves * 2, "a team's sums fit the stages");
-        auto* sums = reinterpret_cast<float4*>(lds_all);                   // [wave][TM][TN][4][lane]
-        __syncthreads();                                                   // nobody reads operands from LDS any more
-        if (team == 1) {
-            #pragma unroll
-            for (int t = 0; t < TM; ++t)
-                #pragma unroll
-                for (int u = 0; u < TN; ++u) {
-                    auto* dst = sums + ((wave * TM + t) * TN + u) * 4 * 64 + lane;
-                    #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        dst[r * 64] = float4{acc[t][u][4 * r], acc[t][u][4 * r + 1], acc[t][u][4 * r + 2], acc[t][u][4 * r + 3]};
-                }
-        }
-        __syncthreads();
-        if (team == 1) return;
-        #pragma unroll
-        for (int t = 0; t < TM; ++t)
-            #pragma unroll
-            for (int u = 0; u < TN; ++u) {
-                const auto* src = sums + ((wave * TM + t) * TN + u) * 4 * 64 + lane;
-                #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float4 v = src[r * 64];
-                    acc[t][u][4 * r] += v.x; acc[t][u][4 * r + 1] += v.y; acc[t][u][4 * r + 2] += v.z; acc[t][u][4 * r + 3] += v.w;
-                }
-            }
-    }
 
     // D[i][j]: j = lane % 32 (a W row, i.e. an output column), i = 8 (r / 4) + 4 (lane / 32) + r % 4.
     #pragma unroll
@@ -1005,7 +946,7 @@ inline double estimate_us(int kind, int terms, int tm, int splits, int M, int N,
     //  14.0, 9.8 and 11.8.
     const bool f16_roomy = kind == WK_F16 && splits == 1 && blocks <= cus && tm <= 2 && stages <= 48;
     // (int8, 32-row tiles of 14 or 15 stages: 300 x 4864 x 896 10.0 us, 700 x 2560 x 960 10.5, 2048 x 960 x 960 12.1,
-    //  where the 64 x 64 tiles take 11.6, 11.1 and 12.8)
+    //  where the 64 x 64 tiles take 11.1, 10.2 and 12.2)
     const bool i8_short = kind == WK_I8 && splits == 1 && tm == 1 && blocks > cus / 2 && blocks <= cus && (stages == 14 || stages == 15);
     const bool roomy = splits == 1 && blocks > cus / 2 && blocks <= cus &&
                        (tm == 2 || (tm == 1 && stages >= 16 && stages <= 48));
@@ -1958,7 +1899,7 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
 
 }  // namespace skinny
 
-template <int BM, int BN, int WM, int WN, int TEAMS, int SETS>
+template <int BM, int BN, int WM, int WN>
 bool launch_tile(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W,
                  const void* scale, void* out, const MoreMats& more) {
     const int tiles_n = more.n ? more.tiles : (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM;
@@ -1969,22 +1910,22 @@ bool launch_tile(hipStream_t s, WeightKind kind, int M, int N, int K, const void
     const auto* wp = static_cast<const uint8_t*>(W);
     const auto* sp = static_cast<const uint16_t*>(scale);
     auto* op = static_cast<uint16_t*>(out);
-    constexpr size_t lds_bytes = 2u * TEAMS * (BM + BN) * kLd * sizeof(uint16_t);
+    constexpr size_t lds_bytes = 2u * (BM + BN) * kLd * sizeof(uint16_t);
     // more than 64 KB of LDS per block has to be asked for once per kernel
     if (kind == WK_I8) {
-        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_I8, TEAMS, SETS>;
+        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_I8>;
         if (lds_bytes > 65536 &&
             !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
             return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads * TEAMS), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
+        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
     } else {
-        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_F16, TEAMS, SETS>;
+        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_F16>;
         if (lds_bytes > 65536 &&
             !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
             return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads * TEAMS), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
+        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
     }
     return MI_HIP_OK(hipGetLastError());
 }
@@ -2009,19 +1950,10 @@ bool wide_reaches(WeightKind kind, int M, int N, int K) {     // 32-bit byte off
            static_cast<double>(N) * K * (kind == WK_F16 ? 2 : 1) < 4294967296.0;
 }
 
-// Whether the 64 x 64 blocks keep the sums of even and odd K-tiles apart: where the K loop is worth halving.  Two teams
-// then run a launch of at most one block per CU, one team with two sets of sums the others.  us, int8, one team and one
-// set / two teams: 300 x 1152 x 896 9.1 / 8.7, 700 x 896 x 896 9.3 / 8.8, 300 x 960 x 960 10.4 / 9.4, 700 x 576 x 1536 14.9 /
-// 13.2, fp16 700 x 1152 x 896 10.2 / 9.7; with more blocks two teams are slower (1200 x 1152 x 896, 342 tiles, 11.3 / 11.9,
-// 2048 x 960 x 960 16.1 / 18.9), as both are at a short K (fp16 700 x 960 x 576 8.7 / 9.3; a 135M layer's calls at 150 rows
-// with two sets 28.6 us against 26.4).  Beyond 1024 rows nearly every launch has more blocks than CUs, and one set is
-// the faster by 0.5 to 1 us (2048 x 1152 x 896 15.2 / 16.2).
-bool halves_k(int M, int K) { return K >= 768 && M <= 1024; }
-
 // The 64 x 64 tiles are bound either by one tile's serial K loop (about 0.4 us per K-tile, up to
 // 1.3 times that as the chip fills) or by throughput (1.2 to 1.55 ns per tile and K-tile);
 // fitted to measurements.
-double tiled_estimate_us(WeightKind kind, int M, int N, int K) {
+double tiled_estimate_us(int M, int N, int K) {
     const int nk = K / kKT;
     const long t64 = tiles(M, N, 64, 64);
     const double serial = (0.9 + nk * 0.4) * (1.0 + 0.3 * (t64 < 128 ? t64 / 128.0 : 1.0));
@@ -2032,9 +1964,7 @@ double tiled_estimate_us(WeightKind kind, int M, int N, int K) {
     const long rounds = (t64 + cus - 1) / cus * cus;
     const long counted = t64 <= cus ? t64 : nk >= 20 ? rounds : (t64 + rounds) / 2;
     const double bulk = 3.3 + counted * nk * (nk > 32 ? 0.00155 : 0.0012);
-    // (two teams, int8: 512 x 576 x 1536 10.0 us where three slices take 12.9)
-    const bool teams = kind == WK_I8 && halves_k(M, K) && t64 > 64 && t64 <= cus;
-    return (serial > bulk ? serial : bulk) * (teams ? 0.93 : 1.0);
+    return serial > bulk ? serial : bulk;
 }
 
 }  // namespace
@@ -2048,7 +1978,7 @@ double gemm_estimate_us(WeightKind kind, int M, int N, int K, size_t workspace_b
     if (M <= skinny::kMaxM && skinny::preferred(kind, M, N, K, device_info().cus, workspace_bytes))
         return skinny::estimate_us(kind, M, N, K, device_info().cus, workspace_bytes);
     if (kind == WK_Q4) return wide_us;
-    const double tiled_us = tiled_estimate_us(kind, M, N, K);
+    const double tiled_us = tiled_estimate_us(M, N, K);
     return wide_us < tiled_us ? wide_us : tiled_us;
 }
 
@@ -2109,7 +2039,7 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         wide::pick_shape(kind, 1, M, N, K, cus, mode == 0 ? workspace_bytes : 0, &tm, &splits, &wide_us);
         if (mode >= 11) tm = mode - 10;
         if (pin_splits) splits = pin_splits;
-        if (mode != 0 || wide_us < tiled_estimate_us(kind, M, N, K)) {
+        if (mode != 0 || wide_us < tiled_estimate_us(M, N, K)) {
             p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;
             return p;
         }
@@ -2147,13 +2077,8 @@ bool launch_planned(hipStream_t s, const GemmPlan& p, WeightKind kind, int M, in
                                   : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more, glu);
         }
         case 5: return quad::launch(s, M, N, K, x, W, scale, out);
-        case 2:
-            // (which sums are kept apart follows from M and K alone, so that a matrix has the same bits in any launch)
-            if (!halves_k(M, K)) return launch_tile<64, 64, 32, 32, 1, 1>(s, kind, M, N, K, x, W, scale, out, more);
-            return (more.n ? more.tiles : (N + 63) / 64) * static_cast<long>((M + 63) / 64) <= device_info().cus
-                       ? launch_tile<64, 64, 32, 32, 2, 1>(s, kind, M, N, K, x, W, scale, out, more)
-                       : launch_tile<64, 64, 32, 32, 1, 2>(s, kind, M, N, K, x, W, scale, out, more);
-        case 3: return launch_tile<128, 128, 64, 64, 1, 1>(s, kind, M, N, K, x, W, scale, out, more);
+        case 2: return launch_tile<64, 64, 32, 32>(s, kind, M, N, K, x, W, scale, out, more);
+        case 3: return launch_tile<128, 128, 64, 64>(s, kind, M, N, K, x, W, scale, out, more);
         default:
             MI_ERROR_FMT("gemm: mode %d has no kernel for kind=%d M=%d N=%d K=%d (Q4 weights have no tile kernel; the "
                          "streaming kernel takes up to 64 rows of x; the wide kernel's 32-bit offsets reach 4 GiB of x and "
@@ -2200,8 +2125,8 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
 // adds them in index order and goes on with the result (decode.hip).  As launch_gemm would cut it, or, where that has no
 // slices, as many as pay without the launch that would add them: that launch is counted as 2.5 us in the estimate.
 // Returns the number of slices; 0: none (nothing was launched); -1: an error.  Prompts of 80 / 300 / 600
-// tokens with these launches: int8 0.5B 1472 / 1792 / 2229 -> 1362 / 1671 / 2074 us, Q4 360M 2101 / 2578 / 3063 -> 1855 /
-// 2302 / 2830.
+// tokens without and with these launches: int8 0.5B 1472 / 1802 / 2247 -> 1360 / 1706 / 2116 us, Q4 360M 2112 / 2585 / 3069 ->
+// 1875 / 2329 / 2838.
 int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
                        void* workspace, size_t workspace_bytes) {
     if (!workspace || !gemm_supported(kind, M, N, K, x, W, scale)) return 0;
