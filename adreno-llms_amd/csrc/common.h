@@ -80,6 +80,7 @@ struct GemvCall {
 // gemv.hip
 constexpr int kMaxSegments = 4;
 bool launch_gemv(hipStream_t s, const GemvCall& c);
+bool gemv_accepts(const GemvCall& c);            // false: launch_gemv refuses the call by its shape or an operand
 // n <= kMaxSegments calls that share x, K, M, weight kind and epilogue, as one launch.
 bool launch_gemv_group(hipStream_t s, const GemvCall* calls, int n);
 // n <= kMaxMany EPI_STORE calls of one M and weight kind, each accepted by gemv_many_takes, of any x, K and N, none of
@@ -163,9 +164,12 @@ bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void
 // 0 = no kernel with this epilogue for the call (nothing was launched), -1 = an error.
 int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
                     void* out, void* workspace, size_t workspace_bytes);
-// n calls of one M and weight kind that gemm_many_takes accepts, of any x, K and N, none of which reads or writes what
+// What becomes of a call on its way to the GEMM: launch_gemm refuses it (whatever it refuses before it launches), launches it
+// by itself, or the streaming kernel serves it, which launch_gemm_many can have serve several.
+enum class GemmRoute { kRefused, kAlone, kShares };
+GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes);
+// n calls of one M and weight kind and of GemmRoute::kShares, of any x, K and N, none of which reads or writes what
 // another one writes: in one launch where they fit it, each result what launch_gemm gives.
-bool gemm_many_takes(hipStream_t s, const GemvCall& c, size_t workspace_bytes);
 bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes);
 // A stream's workspace holds kWorkspaceBytes for whatever a launch puts there and, behind them, kSliceCounters
 // counters that are 0 between launches (slices of K that meet inside a launch).

@@ -870,12 +870,15 @@ __global__ __launch_bounds__(256) void reduce_partials_glu(const float* __restri
               swiglu_h2(pack_half2(a.z * s[2], a.w * s[3]), pack_half2(b.z * s[6], b.w * s[7]))};
 }
 
+// the kernel writes splits x M x N fp32 partial sums and gives every slice at least two K-stages
+inline bool slices_fit(int splits, int M, int N, int K, size_t partial_bytes) {
+    return K / 64 >= 2 * splits && static_cast<double>(splits) * M * N * 4 <= static_cast<double>(partial_bytes);
+}
+
 template <int TM, int KIND, int TERMS>
 bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out,
             float* partial, size_t partial_bytes, int splits, const MoreMats& more, bool glu) {
-    // the kernel writes splits x M x N fp32 partial sums and gives every slice at least two K-stages
-    if (splits < 1 || (splits > 1 && (more.n || !partial || K / 64 < 2 * splits ||
-                                      static_cast<double>(splits) * M * N * 4 > static_cast<double>(partial_bytes)))) {
+    if (splits < 1 || (splits > 1 && (more.n || !partial || !slices_fit(splits, M, N, K, partial_bytes)))) {
         MI_ERROR_FMT("gemm: %d slices of K do not fit (M=%d N=%d K=%d, %zu bytes of workspace)", splits, M, N, K,
                      partial_bytes);
         return false;
@@ -990,7 +993,7 @@ inline bool pick_sliced(int kind, int terms, int M, int N, int K, int cus, size_
     *best_us = 1e30;
     for (int tm = 1; tm <= 5 && 32 * (tm - 1) < M; ++tm)
         for (int sp : {2, 3, 4, 6, 8, 12, 16, 24}) {
-            if (K / 64 < 2 * sp || static_cast<double>(sp) * M * N * 4 > static_cast<double>(workspace_bytes)) continue;
+            if (!slices_fit(sp, M, N, K, workspace_bytes)) continue;
             const double t = estimate_us(kind, terms, tm, sp, M, N, K, cus);
             if (t < *best_us) { *best_us = t; *tm_out = tm; *splits_out = sp; }
         }
@@ -2191,16 +2194,21 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
     return launch_planned(s, p, kind, M, mat[0].N, K, x, mat[0].W, mat[0].scale, mat[0].out, workspace, ws_bytes, more) ? g : -1;
 }
 
-// Calls that the streaming kernel serves, each by its own plan.
-bool gemm_many_takes(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
-    return c.M <= skinny::kMaxM && gemm_supported(c.kind, c.M, c.N, c.K, c.x, c.W, c.scale) && (c.N + 15) / 16 <= 8191 &&
-           plan_gemm(s, c.kind, c.M, c.N, c.K, workspace_bytes).kernel == 4;
+GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
+    if (!gemm_supported(c.kind, c.M, c.N, c.K, c.x, c.W, c.scale)) return GemmRoute::kRefused;
+    const int mode = gemm_mode(s);
+    if (c.M > skinny::kMaxM && (mode == 0 || mode == 4))      // (without a plan: only the wide kernel's reach is missing for Q4)
+        return c.kind != WK_Q4 || wide_reaches(c.kind, c.M, c.N, c.K) ? GemmRoute::kAlone : GemmRoute::kRefused;
+    const GemmPlan p = plan_gemm(s, c.kind, c.M, c.N, c.K, workspace_bytes);
+    if (p.kernel < 1 || (p.kernel == 1 && p.k_slices > 1 && !wide::slices_fit(p.k_slices, c.M, c.N, c.K, workspace_bytes)))
+        return GemmRoute::kRefused;
+    return p.kernel == 4 && (c.N + 15) / 16 <= 8191 ? GemmRoute::kShares : GemmRoute::kAlone;
 }
 
 bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes) {
     const size_t ws_bytes = workspace ? workspace_bytes : 0;
     for (int i = 0; i < n; ++i) {
-        if (calls[i].M != calls[0].M || calls[i].kind != calls[0].kind || !gemm_many_takes(s, calls[i], ws_bytes)) {
+        if (calls[i].M != calls[0].M || calls[i].kind != calls[0].kind || gemm_route(s, calls[i], ws_bytes) != GemmRoute::kShares) {
             MI_ERROR_FMT("gemm: a call that does not fit a launch of several (M=%d N=%d K=%d)", calls[i].M, calls[i].N, calls[i].K);
             return false;
         }

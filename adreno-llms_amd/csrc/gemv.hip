@@ -1267,27 +1267,35 @@ bool launch_kind(hipStream_t s, const GemvCall* calls, int n, int vl) {
     return launch_kind_vl<KIND, 1, EPI>(s, calls, n);
 }
 
-bool check_call(const GemvCall& c) {
-    const int epv = c.kind == WK_Q4 ? 32 : 4;               // Q4 needs whole scale blocks
-    if (c.M < 1 || c.N < 1 || c.K < 1 || c.K % epv != 0) {
-        MI_ERROR_FMT("gemv: unsupported shape M=%d N=%d K=%d (K must be a multiple of %d)", c.M, c.N,
-                     c.K, epv);
-        return false;
-    }
-    if (c.K > 32768 || c.M > 65535) {
-        MI_ERROR_FMT("gemv: K=%d or M=%d beyond the supported range", c.K, c.M);
-        return false;
-    }
+constexpr int whole_k(WeightKind kind) { return kind == WK_Q4 ? 32 : 4; }      // Q4 needs whole scale blocks
+
+// What a launch refuses about a call by itself.
+enum class Refusal { kNone, kShape, kRange, kOperand };
+Refusal refusal(const GemvCall& c) {
+    if (c.M < 1 || c.N < 1 || c.K < 1 || c.K % whole_k(c.kind) != 0) return Refusal::kShape;
+    if (c.K > 32768 || c.M > 65535) return Refusal::kRange;
     if (!c.x || !c.W || !c.y || !aligned(c.x, 16) || !aligned(c.W, 16) || !aligned(c.y, 2) ||
         (c.M > 1 && (static_cast<size_t>(c.K) * 2) % 16 != 0) ||
-        (c.kind != WK_F16 && (!c.scale || !aligned(c.scale, 2)))) {
-        MI_ERROR_FMT("gemv: null or misaligned operand (x and W need 16-byte alignment)");
-        return false;
+        (c.kind != WK_F16 && (!c.scale || !aligned(c.scale, 2))))
+        return Refusal::kOperand;
+    return Refusal::kNone;
+}
+
+bool check_call(const GemvCall& c) {
+    switch (refusal(c)) {
+        case Refusal::kShape:
+            MI_ERROR_FMT("gemv: unsupported shape M=%d N=%d K=%d (K must be a multiple of %d)", c.M, c.N,
+                         c.K, whole_k(c.kind));
+            return false;
+        case Refusal::kRange: MI_ERROR_FMT("gemv: K=%d or M=%d beyond the supported range", c.K, c.M); return false;
+        case Refusal::kOperand: MI_ERROR_FMT("gemv: null or misaligned operand (x and W need 16-byte alignment)"); return false;
+        default: return true;
     }
-    return true;
 }
 
 }  // namespace
+
+bool gemv_accepts(const GemvCall& c) { return refusal(c) == Refusal::kNone; }
 
 // Kernels that can leave argmax candidates: the ones that keep x in registers (int8, fp16) and the
 // Q4 throughput kernel where launch_gemv_group would take it.
@@ -1384,8 +1392,7 @@ static bool many_k(int K) {
 }
 
 bool gemv_many_takes(const GemvCall& c) {
-    return c.epi == EPI_STORE && !c.norm_w && !c.am_v && many_k(c.K) && c.M >= 1 && c.M <= 65535 && c.N >= 1 && c.x && c.W && c.y &&
-           aligned(c.x, 16) && aligned(c.W, 16) && aligned(c.y, 2) && (c.kind == WK_F16 || (c.scale && aligned(c.scale, 2)));
+    return c.epi == EPI_STORE && !c.norm_w && !c.am_v && many_k(c.K) && gemv_accepts(c);
 }
 
 // A run is what launch_gemv_group would take as one launch (its Q4 arithmetic follows from the rows of the run).

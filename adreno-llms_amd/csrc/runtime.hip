@@ -481,13 +481,15 @@ int mi_linear_argmax_static(void* stream, int N, int K, const void* x, const voi
 // A run: consecutive calls that read the same x with the same M, K and weight kind, that mi_linear would all send to
 // the GEMV or all to the GEMM, and whose outputs touch neither what one of them reads (x, weights, scales) nor each
 // other, so that they cannot observe one another.  Runs go out as one launch (q/k/v and gate/up do), GEMV runs always
-// and GEMM runs where launch_gemm_group has a launch for them.  n = 0: the call at the head goes to mi_linear (an
-// argument to refuse, an output that aliases an operand, many rows of GEMV).
+// and GEMM runs where launch_gemm_group has a launch for them.  A call that would be refused is in no run: the run in
+// front of it ends there, and so does its window.  n = 0: the call at the head goes to mi_linear (a call to refuse, an
+// output that aliases an operand, many rows of GEMV).
 struct BatchRun {
     GemvCall c[kMaxSegments];
     CallMemory memory[kMaxSegments];
     int n = 0;
     bool gemm = false;
+    bool shares = false;                                 // launch_gemv_many or launch_gemm_many takes every call
 };
 static void next_run(hipStream_t s, const mi_linear_call* calls, int n, BatchRun* r) {
     const mi_linear_call& c0 = calls[0];
@@ -495,6 +497,8 @@ static void next_run(hipStream_t s, const mi_linear_call* calls, int n, BatchRun
     Entry e0;
     if (!(c0.M >= 1 && c0.N > 0 && c0.K > 0 && c0.x && c0.W && c0.out && resolve("mi_linear_batch", c0.W, c0.N, c0.K, &e0))) return;
     r->gemm = takes_gemm(s, e0, c0.M, c0.N, c0.K, c0.x, c0.W);
+    r->shares = true;
+    const size_t ws_bytes = r->gemm && workspace_of(s) ? kWorkspaceBytes : 0;
     while ((r->gemm || c0.M < 16) && r->n < n && r->n < kMaxSegments) {
         const mi_linear_call& c = calls[r->n];
         Entry e;
@@ -509,31 +513,40 @@ static void next_run(hipStream_t s, const mi_linear_call* calls, int n, BatchRun
         for (int j = 0; j < r->n && !clash; ++j) clash = !independent(r->memory[j], mem);
         if (clash) break;
         r->memory[r->n] = mem;
-        GemvCall& d = r->c[r->n++];
+        GemvCall& d = r->c[r->n];
         d = GemvCall{};
         d.x = c.x; d.W = c.W; d.scale = e.scale; d.y = c.out;
         d.M = c.M; d.N = c.N; d.K = c.K; d.kind = e.kind; d.epi = EPI_STORE;
+        if (r->gemm) {
+            const GemmRoute route = gemm_route(s, d, ws_bytes);
+            if (route == GemmRoute::kRefused) break;
+            r->shares = r->shares && route == GemmRoute::kShares;
+        } else {
+            if (!gemv_accepts(d)) break;
+            r->shares = r->shares && gemv_many_takes(d);
+        }
+        ++r->n;
     }
 }
 
-// The launches of one run.
-static bool launch_run(hipStream_t s, const GemvCall* c, int n, bool gemm) {
-    if (!gemm) return launch_gemv_group(s, c, n);
+// The launches of one run: how many of its calls were enqueued (fewer than n: an error).
+static int launch_run(hipStream_t s, const GemvCall* c, int n, bool gemm) {
+    if (!gemm) return launch_gemv_group(s, c, n) ? n : 0;
     for (int i = 0; i < n;) {
         int g = 0;
         if (n - i > 1) {
             GemmMat mats[kMaxSegments];
             for (int j = i; j < n; ++j) mats[j - i] = GemmMat{c[j].W, c[j].scale, c[j].y, c[j].N};
             g = launch_gemm_group(s, c->kind, n - i, mats, c->M, c->K, c->x, workspace_of(s), kWorkspaceBytes);
-            if (g < 0) return false;
+            if (g < 0) return i;
         }
         if (g == 0) {
-            if (!mi_linear(s, c->M, c[i].N, c->K, c->x, c[i].W, c[i].y)) return false;
+            if (!mi_linear(s, c->M, c[i].N, c->K, c->x, c[i].W, c[i].y)) return i;
             g = 1;
         }
         i += g;
     }
-    return true;
+    return n;
 }
 
 // A window: consecutive runs, whatever their x, M, K and weight kind, none of whose calls reads or writes what another
@@ -571,17 +584,14 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
             for (int j = 0; j < r.n && apart; ++j)
                 for (int q = 0; q < count && apart; ++q) apart = independent(memory[q], r.memory[j]);
             if (!apart) break;
-            bool gemvs = !r.gemm, gemms = r.gemm;
             for (int j = 0; j < r.n; ++j) {
                 held[count + j] = r.c[j];
                 memory[count + j] = r.memory[j];
-                gemvs = gemvs && gemv_many_takes(r.c[j]);
-                gemms = gemms && gemm_many_takes(s, r.c[j], workspace_of(s) ? kWorkspaceBytes : 0);
             }
             run[runs].first = count;
             run[runs].n = r.n;
             run[runs].gemm = r.gemm;
-            run[runs++].how = gemvs ? GEMVS : gemms ? GEMMS : ALONE;
+            run[runs++].how = !r.shares ? ALONE : r.gemm ? GEMMS : GEMVS;
             count += r.n;
             have = i + count < n;
             if (!have) break;
@@ -590,23 +600,23 @@ int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
         for (int a = 0; a < runs; ++a) {
             if (run[a].how == DONE) continue;
             const GemvCall& c = held[run[a].first];
+            const Launch how = run[a].how;
             int g = 0, members = 0;
             for (int b = a; b < runs; ++b) {             // the runs that share run a's launch, itself among them
                 const GemvCall& d = held[run[b].first];
-                if (b != a && (run[a].how == ALONE || run[b].how != run[a].how || d.M != c.M || d.kind != c.kind)) continue;
+                if (b != a && (how == ALONE || run[b].how != how || d.M != c.M || d.kind != c.kind)) continue;
                 for (int j = 0; j < run[b].n; ++j) {
                     some[g] = held[run[b].first + j];
                     run_of[g++] = b;
                 }
                 ++members;
-                if (b != a) run[b].how = DONE;
+                run[b].how = DONE;
             }
-            if (members == 1) {
-                if (!launch_run(s, some, g, run[a].gemm)) return i;
-            } else if (!(run[a].how == GEMVS ? launch_gemv_many(s, some, run_of, g)
-                                             : launch_gemm_many(s, some, g, workspace_of(s), kWorkspaceBytes))) {
-                return i;
-            }
+            // (nothing in a run is refused any more: what fails here is the runtime, and the calls in front of run a are enqueued)
+            const int enqueued = members == 1   ? launch_run(s, some, g, run[a].gemm)
+                                 : how == GEMVS ? (launch_gemv_many(s, some, run_of, g) ? g : 0)
+                                                : (launch_gemm_many(s, some, g, workspace_of(s), kWorkspaceBytes) ? g : 0);
+            if (enqueued < g) return i + run[a].first + (members == 1 ? enqueued : 0);
         }
         i += count;
     }
