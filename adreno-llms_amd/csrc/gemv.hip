@@ -33,6 +33,7 @@
 #include <hip/hip_fp16.h>
 #include "device_math.h"
 #include "argmax_rule.h"
+#include "deal_rule.h"
 
 namespace mi {
 namespace {
@@ -695,8 +696,8 @@ constexpr int group_size(int kind, int K, int vl) {
 // Calls of a batch that cannot observe one another's results, whatever their x and K (the batch's host code
 // checks that): their row batches stream side by side, so a short matrix no longer has the chip to itself for the
 // 1.6 us that a dependent launch takes at least, and a launch of a few MB no longer ends before the memory
-// system is at its rate (169 int8 calls, 495 MB, in three such launches: 93 us, 5.3 TB/s).  A block works on one call; blocks are dealt out to calls by their bytes (launch_gemv_many),
-// every row's sum is that of the kernels above, in their order.
+// system is at its rate (169 int8 calls, 495 MB, in three such launches: 93 us, 5.3 TB/s).  A block works on one call,
+// dealt out by bytes (deal_rule.h); every row's sum is that of the kernels above, in their order.
 struct ManyCalls {
     int n = 0;
     uint16_t first[kMaxMany] = {};                       // a call's first block
@@ -730,7 +731,8 @@ __global__ __launch_bounds__(kBlock, 3) void gemv_many(const ManyCalls) {
     const uint16_t* sc = L->c[i].sc;
     uint16_t* y = L->c[i].y;
     const int N = L->c[i].N, nbatch = L->c[i].nbatch, waves = L->c[i].waves, code = L->c[i].code;
-    const int wid = (static_cast<int>(blockIdx.x) - L->first[i]) * kWavesPerBlock + block_wave();
+    const int wid = first_batch(blockIdx.x, block_wave(), L->first[i], waves, kWavesPerBlock);
+    if (wid < 0) return;
     const SegList none{};
 #define MI_MANY(KT)                                                                                                     \
     case KT: {                                                                                                          \
@@ -1404,8 +1406,7 @@ bool launch_gemv_many(hipStream_t s, const GemvCall* calls, const int* run_of, i
     const WeightKind kind = calls[0].kind;
     ManyCalls L;
     L.n = n;
-    double bytes = 0.0;
-    int batch_bytes[kMaxMany];
+    int nbatch[kMaxMany], batch_bytes[kMaxMany], waves[kMaxMany];
     for (int i = 0; i < n; ++i) {
         const GemvCall& c = calls[i];
         if (!gemv_many_takes(c) || c.kind != kind || c.M != calls[0].M) {
@@ -1419,7 +1420,7 @@ bool launch_gemv_many(hipStream_t s, const GemvCall* calls, const int* run_of, i
         d.sc = static_cast<const uint16_t*>(c.scale);
         d.y = static_cast<uint16_t*>(c.y);
         d.N = c.N;
-        d.nbatch = (c.N + vl - 1) / vl;
+        d.nbatch = nbatch[i] = (c.N + vl - 1) / vl;
         d.code = c.K;
         if (kind == WK_Q4 && gemv_mode(s) == 1) {
             long rows = 0;
@@ -1428,28 +1429,10 @@ bool launch_gemv_many(hipStream_t s, const GemvCall* calls, const int* run_of, i
             if (pick_vl(kind, c.M, rows, c.K) == 4) d.code = -c.K;      // (every such K has an instance of the throughput kernel)
         }
         batch_bytes[i] = vl * (c.K / (kind == WK_Q4 ? 8 : 4)) * (kind == WK_F16 ? 8 : 4);
-        bytes += static_cast<double>(d.nbatch) * batch_bytes[i];
     }
-    // Every wavefront gets about the same bytes, and all of them, of all rows of x, are resident at once: the bytes per
-    // wavefront grow until the blocks fit (with that many blocks per row of x instead, 15 rows of a 576-wide Q4 layer took
-    // 19.7 us where they now take 17.0 and launches of a run each 18.7; 8 fp16 rows 14.1 against 8 and 17).
     const int M = calls[0].M;
-    const long cap = resident_waves() / kWavesPerBlock / M;
-    long blocks = 0;
-    for (double share = bytes * M / resident_waves();; share *= 1.05) {
-        blocks = 0;
-        for (int i = 0; i < n; ++i) {
-            const long per_wave = share > batch_bytes[i] ? static_cast<long>(share / batch_bytes[i]) : 1;
-            const long b = ((L.c[i].nbatch + per_wave - 1) / per_wave + kWavesPerBlock - 1) / kWavesPerBlock;
-            L.first[i] = static_cast<uint16_t>(blocks);
-            L.c[i].waves = static_cast<int>(b * kWavesPerBlock);
-            blocks += b;
-        }
-        if (blocks <= cap || blocks <= n) break;
-    }
-    // (a multiple of 8 blocks per row of x: the blocks that read the same weights for different rows then share an XCD's
-    //  L2; the blocks past the last call's find no row batch left)
-    if (M > 1) blocks = (blocks + 7) / 8 * 8;
+    const long blocks = deal_blocks(n, nbatch, batch_bytes, M, resident_waves(), kWavesPerBlock, L.first, waves);
+    for (int i = 0; i < n; ++i) L.c[i].waves = waves[i];
     const dim3 grid(static_cast<unsigned>(blocks), M, 1);
     switch (kind) {
         case WK_F16: hipLaunchKernelGGL(gemv_many<WK_F16>, grid, dim3(kBlock), 0, s, L); break;
