@@ -126,6 +126,15 @@ WeightEntry weight_entry(const void* W);
 uint64_t registry_epoch();
 // The workspace of a stream that mi_stream_create made (null: another stream, or no memory was left for one)
 void* own_stream_workspace(hipStream_t s);
+// While it lives, launches that this thread enqueues on `recording` (a stream of the library's own, under capture) use the
+// workspace and the modes of `s`, the stream that the recording will be replayed on.  One at a time in a thread.
+class StandsFor {
+public:
+    StandsFor(hipStream_t recording, hipStream_t s);
+    ~StandsFor();
+    StandsFor(const StandsFor&) = delete;
+    StandsFor& operator=(const StandsFor&) = delete;
+};
 
 // argmax.hip: index of the greatest of N fp16 values, ties as the reference's two argmax kernels break them.
 // scratch: kArgmaxScratchBytes of device memory that belongs to stream s, or null (then one block does all the work).

@@ -14,6 +14,7 @@
 // lists can be compared for identity), and are launch-bound at batch 1 whatever they do.
 #include "common.h"
 #include "device_math.h"
+#include "step_record.h"
 #include "../../include/mi_decode.h"
 #include "../../include/mi_linear.h"
 
@@ -1501,22 +1502,10 @@ struct Decoder {
     // attention with a head's keys split over blocks (mi_decoder_set_attention_splits): 0 = the reference-order launch
     int splits = 0;
     float* split_part = nullptr;                               // [n_heads][splits][head_dim + 2]
-    // A step's launches recorded as graphs (mi_decoder_step), and the circumstances of the last step
-    struct StepKey {
-        hipStream_t stream = nullptr;
-        void* workspace = nullptr;
-        int gemv_mode = -1, splits = -1, weights = -1;         // weights: weights_version
-        bool operator==(const StepKey& o) const {
-            return stream == o.stream && workspace == o.workspace && gemv_mode == o.gemv_mode && splits == o.splits && weights == o.weights;
-        }
-    };
-    struct Recording { StepKey key; hipGraphExec_t exec; };
-    std::vector<Recording> recordings;
-    StepKey last_step;
+    StepRecordings<hipGraphExec_t> recordings;                 // a step's launches as graphs (mi_decoder_step)
     std::vector<WeightEntry> weights;                          // what the registry held for the decoder's weights ...
     uint64_t weights_epoch = 0;                                // ... at this registry_epoch()
     int weights_version = 0;                                   // raised whenever that turned out to have changed
-    bool record_refused = false;                               // the runtime would not record: plain steps from then on
 };
 
 template <typename T>
@@ -1621,7 +1610,8 @@ int mi_decoder_destroy(void* dec) {
     for (void* w : d->wqkv) if (w) mi_unregister_weight(w);
     for (void* w : d->wgu) if (w) mi_unregister_weight(w);
     for (void* p : d->stacked_mem) (void)hipFree(p);
-    for (auto& r : d->recordings) (void)hipGraphExecDestroy(r.exec);         // (the frees above have waited for their last replay)
+    for (size_t i = 0; i < d->recordings.count(); ++i)
+        (void)hipGraphExecDestroy(d->recordings.exec(i));      // (the frees above have waited for their last replay)
     delete d;
     return 1;
 }
@@ -1849,22 +1839,57 @@ static int enqueue_step(Decoder* d, void* stream) {
 // recorded (0.5 to 2 ms, once) and from then on replayed: a token of SmolLM2-135M in fp16, read back as it comes, 679 ->
 // 497 us, of Qwen2.5-0.5B in int8 602 -> 482 us.
 //
+// It is recorded on a stream that nobody else knows (StandsFor), so that another thread that meanwhile waits for the step's
+// stream, or asks about it, neither fails nor breaks into the recording.
+//
 // Circumstances: the stream and its workspace, the GEMV arithmetic, the attention's splits, and what the registry holds
 // for the decoder's weights (looked up again whenever anything was registered or removed).  All else that the launches refer to
-// belongs to the decoder.  Only on streams of mi_stream_create: they do not synchronise with the null stream, whose use by
-// another thread would break into a recording; not while the caller records (the launches then go into its graph).
+// belongs to the decoder.  Only on streams of mi_stream_create, which have a workspace to name; not while the caller
+// records (the launches then go into its graph).
+namespace {
+struct StepApi {
+    Decoder* d;
+    hipStream_t s;
+    int enqueue() { return enqueue_step(d, s); }
+    int replay(hipGraphExec_t exec) { return MI_HIP_OK(hipGraphLaunch(exec, s)) ? 1 : 0; }
+    Recorded record(hipGraphExec_t* exec) {
+        hipStream_t own = nullptr;
+        if (hipStreamCreateWithFlags(&own, hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
+            return Recorded::kRefused;
+        }
+        Recorded r = Recorded::kRefused;
+        if (hipStreamBeginCapture(own, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+            hipGraph_t graph = nullptr;
+            int launched = 0;
+            {
+                StandsFor same(own, s);
+                launched = enqueue_step(d, own);
+            }
+            if (hipStreamEndCapture(own, &graph) == hipSuccess && graph) {
+                if (!launched) r = Recorded::kLaunchFailed;
+                else if (hipGraphInstantiate(exec, graph, nullptr, nullptr, 0) == hipSuccess) r = Recorded::kYes;
+            }
+            if (graph) (void)hipGraphDestroy(graph);
+        }
+        if (r != Recorded::kYes) (void)hipGetLastError();
+        (void)hipStreamDestroy(own);
+        return r;
+    }
+};
+}  // namespace
+
 int mi_decoder_step(void* dec, void* stream) {
     auto* d = static_cast<Decoder*>(dec);
     if (!d) return 0;
     auto s = static_cast<hipStream_t>(stream);
     void* ws = own_stream_workspace(s);
-    if (!ws || d->record_refused) return enqueue_step(d, stream);
+    if (!ws) return enqueue_step(d, stream);
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return enqueue_step(d, stream);
     }
-    constexpr size_t kMostRecordings = 8;                      // graphs stay until the decoder goes: one may still be running
     const uint64_t epoch = registry_epoch();
     if (d->weights.empty() || epoch != d->weights_epoch) {
         std::vector<WeightEntry> held;
@@ -1875,33 +1900,14 @@ int mi_decoder_step(void* dec, void* stream) {
         d->weights.swap(held);
         d->weights_epoch = epoch;
     }
-    const Decoder::StepKey now{s, ws, gemv_mode(s), d->splits, d->weights_version};
-    const bool again = d->last_step == now;
-    d->last_step = now;
-    if (!again) return enqueue_step(d, stream);
-    for (const auto& r : d->recordings)
-        if (r.key == now) return MI_HIP_OK(hipGraphLaunch(r.exec, s)) ? 1 : 0;
-    if (d->recordings.size() >= kMostRecordings) return enqueue_step(d, stream);
-    // nothing runs while it is recorded: what fails here is enqueued plainly instead
-    if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-        (void)hipGetLastError();
-        d->record_refused = true;
-        return enqueue_step(d, stream);
-    }
-    const int ok = enqueue_step(d, stream);
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    const bool recorded = hipStreamEndCapture(s, &graph) == hipSuccess && graph &&
-                          hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess;
-    if (graph) (void)hipGraphDestroy(graph);
-    if (!ok || !recorded) {
-        (void)hipGetLastError();
-        if (exec) (void)hipGraphExecDestroy(exec);
-        d->record_refused = d->record_refused || !recorded;
-        return ok ? enqueue_step(d, stream) : 0;
-    }
-    d->recordings.push_back(Decoder::Recording{now, exec});
-    return MI_HIP_OK(hipGraphLaunch(exec, s)) ? 1 : 0;
+    StepKey now;
+    now.stream = s;
+    now.workspace = ws;
+    now.gemv_mode = gemv_mode(s);
+    now.splits = d->splits;
+    now.weights = d->weights_version;
+    StepApi api{d, s};
+    return d->recordings.step(api, now);
 }
 
 // Rows of n matrices of one kind and K (and their scales) copied into one matrix, registered like

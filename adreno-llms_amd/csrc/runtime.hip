@@ -55,9 +55,12 @@ static_assert(kStaticScratchBytes >= kArgmaxScratchBytes, "the two-launch argmax
 constexpr int kMaxDevices = 64;
 void* g_static_scratch[kMaxDevices] = {};     // device address of `scratch` per device, set by mi_init
 
+thread_local hipStream_t t_recording = nullptr, t_stands_for = nullptr;      // StandsFor
+hipStream_t stood_for(hipStream_t s) { return s && s == t_recording ? t_stands_for : s; }
+
 void* workspace_of(hipStream_t s) {
     std::lock_guard<std::mutex> lk(g_registry_mu);
-    auto it = g_workspace.find(s);
+    auto it = g_workspace.find(stood_for(s));
     return it == g_workspace.end() ? nullptr : it->second;
 }
 
@@ -125,6 +128,12 @@ uint64_t registry_epoch() { return g_registry_epoch.load(); }
 
 void* own_stream_workspace(hipStream_t s) { return s ? workspace_of(s) : nullptr; }
 
+StandsFor::StandsFor(hipStream_t recording, hipStream_t s) {
+    t_recording = recording;
+    t_stands_for = s;
+}
+StandsFor::~StandsFor() { t_recording = t_stands_for = nullptr; }
+
 bool fused_gemv_kind(const void* W, int N, int K, WeightKind* kind) {
     Entry e;
     if (!resolve("decode step", W, N, K, &e)) return false;
@@ -179,7 +188,7 @@ bool linear_argmax(hipStream_t s, int N, int K, const void* x, const void* W, vo
 int gemv_mode(hipStream_t s) {
     {
         std::lock_guard<std::mutex> lk(g_registry_mu);
-        auto it = g_stream_modes.find(s);
+        auto it = g_stream_modes.find(stood_for(s));
         if (it != g_stream_modes.end() && it->second.gemv >= 0) return it->second.gemv;
     }
     return g_gemv_mode.load(std::memory_order_relaxed);
@@ -188,7 +197,7 @@ int gemv_mode(hipStream_t s) {
 int gemm_mode(hipStream_t s) {
     {
         std::lock_guard<std::mutex> lk(g_registry_mu);
-        auto it = g_stream_modes.find(s);
+        auto it = g_stream_modes.find(stood_for(s));
         if (it != g_stream_modes.end() && it->second.gemm >= 0) return it->second.gemm;
     }
     return g_gemm_mode.load(std::memory_order_relaxed);
