@@ -1852,6 +1852,11 @@ struct StepApi {
     hipStream_t s;
     int enqueue() { return enqueue_step(d, s); }
     int replay(hipGraphExec_t exec) { return MI_HIP_OK(hipGraphLaunch(exec, s)) ? 1 : 0; }
+    // (mi_stream_destroy takes the workspace out of the table when the stream's work is over; a stream that has come
+    //  since under the same address has another workspace, or one at the same address, and then the recording fits it)
+    bool gone(const StepKey& k) { return own_stream_workspace(static_cast<hipStream_t>(const_cast<void*>(k.stream))) != k.workspace; }
+    void drain() { (void)hipStreamSynchronize(s); }
+    void drop(hipGraphExec_t exec) { (void)hipGraphExecDestroy(exec); }
     Recorded record(hipGraphExec_t* exec) {
         hipStream_t own = nullptr;
         if (hipStreamCreateWithFlags(&own, hipStreamNonBlocking) != hipSuccess) {

@@ -283,7 +283,9 @@ void* mi_stream_create(void) {
 
 int mi_stream_destroy(void* s) {
     if (!s) return 1;
-    const int ok = MI_HIP_OK(hipStreamDestroy(as_stream(s))) ? 1 : 0;    // waits for the stream's work
+    // (whoever finds the stream gone from the tables may take its work to be over)
+    if (hipStreamSynchronize(as_stream(s)) != hipSuccess) (void)hipGetLastError();
+    const int ok = MI_HIP_OK(hipStreamDestroy(as_stream(s))) ? 1 : 0;
     void* ws = nullptr;
     {
         std::lock_guard<std::mutex> lk(g_registry_mu);

@@ -60,12 +60,14 @@ int   mi_decoder_set_token(void* decoder, void* stream, int token);
 
 /* Enqueues one step: consumes the device token at the device position, writes the KV rows of that
  * position, leaves the greedy next token as the device token and advances the position.  Nothing is
- * synchronised; may be captured into a graph.  A step at position max_pos - 1 is the
+ * synchronised (but for the one case below); may be captured into a graph.  A step at position max_pos - 1 is the
  * last valid one (later steps clamp the position and overwrite that row).
  * On a stream of mi_stream_create, outside a capture, the second of two steps in a row under the same modes and
  * registered weights records the step as a graph of the decoder's own, which takes a millisecond or two and
- * is the only thing a step ever allocates; the steps after it replay that graph.  One decoder is stepped by one
- * host thread at a time. */
+ * is the only thing a step ever allocates; the steps after it replay that graph.  A decoder keeps up to eight such graphs;
+ * where there are eight, those of streams that are gone and of weights that were registered anew make room (the latter
+ * behind a wait for the stream, the only time a step waits), and without room steps are enqueued launch by launch.
+ * One decoder is stepped by one host thread at a time. */
 int   mi_decoder_step(void* decoder, void* stream);
 
 /* A prompt at once: Model::forward with seq_len = n_tokens (QW/src/model.cpp:243-376), where every

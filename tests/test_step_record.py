@@ -22,6 +22,11 @@ struct Api {
         return static_cast<Recorded>(outcome);
     }
     int replay(int exec) { ++replayed; last_exec = exec; return replay_ok; }
+    long gone_stream = 0;
+    int drained = 0, dropped = 0;                              // dropped: a bit per exec
+    bool gone(const StepKey& k) { return reinterpret_cast<long>(k.stream) == gone_stream; }
+    void drain() { ++drained; }
+    void drop(int exec) { dropped |= 1 << exec; }
 };
 static Api api;
 static StepRecordings<int>* held;
@@ -33,6 +38,8 @@ extern "C" int step(long stream, long workspace, int mode, int splits, int weigh
     k.gemv_mode = mode; k.splits = splits; k.weights = weights;
     return held->step(api, k);
 }
+extern "C" void stream_goes(long stream) { api.gone_stream = stream; }
+extern "C" void drops(int* out) { out[0] = api.drained; out[1] = api.dropped; }
 extern "C" void counts(int* out) { out[0] = api.plain; out[1] = api.recorded; out[2] = api.replayed; out[3] = api.last_exec; }
 """
 
@@ -79,6 +86,74 @@ def test_what_fails_while_it_is_recorded_is_enqueued_plainly(rule, outcome, laun
     assert rule.step(*KEY) == 1
     # refused: never tried again; otherwise the next step is recorded
     assert _counts(rule) == ([3, 1, 0, 0] if outcome == 2 else [2, 2, 1, 1])
+
+
+def _drops(rule):
+    out = (ctypes.c_int * 2)()
+    rule.drops(out)
+    return list(out)
+
+
+def _steps(rule, key, n=3):
+    """(plain steps, recordings, replays) of n steps in a row."""
+    before = _counts(rule)
+    for _ in range(n):
+        assert rule.step(*key)
+    return [b - a for a, b in zip(before, _counts(rule))][:3]
+
+
+def test_weights_registered_again_any_number_of_times(rule):
+    """Each version of the weights is recorded; of a full table the outdated ones go, behind one wait for the stream."""
+    rule.start()
+    for version in range(1, 30):
+        assert _steps(rule, (1, 2, 0, 0, version)) == [1, 1, 2], version
+        assert _drops(rule) == [(version - 1) // 8, (1 << (version - 1) // 8 * 8 + 1) - 2], version
+
+
+def test_streams_that_come_and_go(rule):
+    rule.start()
+    for stream in range(1, 9):
+        assert _steps(rule, (stream, 2, 0, 0, 1)) == [1, 1, 2]
+    assert _steps(rule, (9, 2, 0, 0, 1)) == [3, 0, 0]          # eight that live: plainly
+    rule.stream_goes(3)
+    assert _steps(rule, (9, 2, 0, 0, 1)) == [0, 1, 3]          # (again the circumstances of the step before)
+    assert _drops(rule) == [0, 1 << 3]
+    for stream in (1, 2, 4, 5, 6, 7, 8, 9):
+        assert _steps(rule, (stream, 2, 0, 0, 1)) == [1, 0, 2], stream
+
+
+def test_outdated_recordings_of_another_stream_stay(rule):
+    """Their last replay may still be running."""
+    rule.start()
+    for splits in range(8):
+        assert _steps(rule, (1, 2, 0, splits, 1)) == [1, 1, 2]
+    assert _steps(rule, (9, 2, 0, 0, 2)) == [3, 0, 0] and _drops(rule) == [0, 0]
+    assert _steps(rule, (1, 2, 0, 0, 2)) == [1, 1, 2] and _drops(rule) == [1, 0b111111110]
+    assert _steps(rule, (9, 2, 0, 0, 2)) == [1, 1, 2]
+
+
+@pytest.mark.gpu
+def test_more_circumstances_than_recordings():
+    """A weight registered again and again, and streams that come and go, replay against plain launches (two streams in turn)."""
+    import numpy as np
+
+    from helpers import mil
+    from test_step_replay_gpu import SHAPE, _pair, _same
+
+    a, b = _pair("int8")
+    for s in (a, b):
+        assert s.dec.reset(s.queues[0], 0, 5)
+    for version in range(20):
+        if version % 3 == 2:
+            a.queues = [mil.Queue()]
+        for s in (a, b):
+            scale = mil.Buffer.from_host(np.full(SHAPE[1], 0x1c00 + 16 * version, np.uint16))
+            s.keep.append(scale)
+            assert mil.nnopt_register_int8_weight(s.bufs["wgate"][1], scale, SHAPE[1], SHAPE[0])
+        print("version", version, flush=True)
+        for _ in range(3):
+            a.step(), b.step()
+        _same(a, b, version)
 
 
 @pytest.mark.gpu
