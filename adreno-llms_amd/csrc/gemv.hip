@@ -244,7 +244,7 @@ __device__ __forceinline__ Seg find_segment(const SegList& L, int rb) {
 // multiplies the current one.  Without PIPE a wavefront is expected to own one batch.
 // RB row batches are fetched together, so that narrow rows (Q4, small K) still keep enough
 // bytes in flight per wavefront.
-// first: the wavefront's first row batch (its number among the nw wavefronts of the launch), m: its row of x.
+// first: the wavefront's first row batch (its number among the nw wavefronts of the launch), one that there is; m: its row of x.
 template <int KIND, int KT, int VL, int EPI, bool PIPE, int RB, bool AM>
 __device__ __forceinline__ void fixed_k_rows(MI_HOT_PARAMS, const SegList& L, const int first, const int nw, const int m) {
     using T = WT<KIND>;
@@ -309,12 +309,6 @@ __device__ __forceinline__ void fixed_k_rows(MI_HOT_PARAMS, const SegList& L, co
     int rb = first;
     const TieRule rule{L.am_chunk};
     Cand top{kArgmaxNone, 0};                                 // AM: best row so far (lanes with g == 0)
-    if (rb >= hnbatch) {
-        if constexpr (AM) {
-            if (lane == 0) { L.am_v[first] = kArgmaxNone; L.am_i[first] = 0; }
-        }
-        return;
-    }
     constexpr int GB = PIPE ? RB : 1;
     struct Group { Batch b[GB]; };
     // A wavefront owns batches rb, rb + nw, rb + 2 nw, ...; it takes them GB at a time.  A batch
@@ -502,10 +496,24 @@ __device__ __forceinline__ void fixed_k_rows(MI_HOT_PARAMS, const SegList& L, co
     }
 }
 __device__ __forceinline__ int block_wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
+// Whether a wavefront has no row batch: it leaves "none" as its candidate.  Asked by the kernels themselves: inside the bodies,
+// which gemv_many shares, this store and the one at their end became one, with a branch around everything between.  And
+// stored by every lane: a test for lane 0 here is the one at the end, kept through the kernel in two scalar registers.
+template <bool AM>
+__device__ __forceinline__ bool no_batch(const SegList& L, const int first, const int nbatch) {
+    if (first < nbatch) return false;
+    if constexpr (AM) {
+        L.am_v[first] = kArgmaxNone;
+        L.am_i[first] = 0;
+    }
+    return true;
+}
 template <int KIND, int KT, int VL, int EPI, bool PIPE, int RB, bool AM = false>
 __global__ __launch_bounds__(kBlock) void gemv_fixed_k(MI_HOT_PARAMS, const SegList L) {
-    fixed_k_rows<KIND, KT, VL, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L,
-                                                  blockIdx.x * kWavesPerBlock + block_wave(), gridDim.x * kWavesPerBlock, blockIdx.y);
+    const int first = blockIdx.x * kWavesPerBlock + block_wave();
+    if (no_batch<AM>(L, first, hnbatch)) return;
+    fixed_k_rows<KIND, KT, VL, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L, first,
+                                                  gridDim.x * kWavesPerBlock, blockIdx.y);
 }
 
 // ---- Q4, throughput variant --------------------------------------------------------
@@ -568,12 +576,6 @@ __device__ __forceinline__ void q4_fast_rows(MI_HOT_PARAMS, const SegList& L, co
     int rb = first;
     const TieRule rule{L.am_chunk};
     Cand top{kArgmaxNone, 0};                                 // AM: best row so far (lanes with g == 0)
-    if (rb >= hnbatch) {
-        if constexpr (AM) {
-            if (lane == 0) { L.am_v[first] = kArgmaxNone; L.am_i[first] = 0; }
-        }
-        return;
-    }
     uint32_t raw[NIT][16];
     #pragma unroll
     for (int j = 0; j < NIT; ++j) {
@@ -681,8 +683,10 @@ __device__ __forceinline__ void q4_fast_rows(MI_HOT_PARAMS, const SegList& L, co
 }
 template <int KT, int EPI, bool PIPE, int RB, bool AM = false>
 __global__ __launch_bounds__(kBlock) void gemv_q4_fast(MI_HOT_PARAMS, const SegList L) {
-    q4_fast_rows<KT, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L,
-                                        blockIdx.x * kWavesPerBlock + block_wave(), gridDim.x * kWavesPerBlock, blockIdx.y);
+    const int first = blockIdx.x * kWavesPerBlock + block_wave();
+    if (no_batch<AM>(L, first, hnbatch)) return;
+    q4_fast_rows<KT, EPI, PIPE, RB, AM>(x, hN0, hnbatch, hW0, hsc0, hnorm_w, hW1, hsc1, hy0, L, first, gridDim.x * kWavesPerBlock,
+                                        blockIdx.y);
 }
 
 // Row batches a pipelined wavefront fetches at once: enough for about 3.5 KB of weights.
@@ -732,7 +736,7 @@ __global__ __launch_bounds__(kBlock, 3) void gemv_many(const ManyCalls) {
     uint16_t* y = L->c[i].y;
     const int N = L->c[i].N, nbatch = L->c[i].nbatch, waves = L->c[i].waves, code = L->c[i].code;
     const int wid = first_batch(blockIdx.x, block_wave(), L->first[i], waves, kWavesPerBlock);
-    if (wid < 0) return;
+    if (wid < 0 || wid >= nbatch) return;
     const SegList none{};
 #define MI_MANY(KT)                                                                                                     \
     case KT: {                                                                                                          \
