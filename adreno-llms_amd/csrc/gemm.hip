@@ -81,7 +81,7 @@ __device__ __forceinline__ void pick_matrix(const MoreMats& mm, int& tile, const
     tile -= first;
 }
 
-template <int BM, int BN, int WM, int WN, int KIND>
+template <int BM, int BN, int WM, int WN, int KIND, bool BANDS>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restrict__ X,
                                                         const uint8_t* __restrict__ W,
                                                         const uint16_t* __restrict__ scale,
@@ -103,18 +103,14 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restri
 
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int wm = wave / (BN / WN), wn = wave % (BN / WN);
-    // Block -> tile.  Blocks go to the 8 XCDs round-robin, each with an L2 of its own.  In the order of the tiles an XCD
-    // keeps to its share of the columns of tiles where their number is even; where it is odd it comes through all of
-    // them, and XCD x takes the x-th eighth of a list instead that runs through bands of kBand tiles along N, down M inside
-    // a band.  us, int8, tiles in order / in bands: 15 columns, 2048 x 960 x 960 16.2 / 12.2, 25, 700 x 1600 x 960 13.1 / 11.1, 9,
-    // 1200 x 576 x 1536 15.5 / 14.0; but 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.
+    // Block -> tile: see tiles_in_bands
     int tile_m, tile_n;
-    const int tiles_n = more.n ? more.tiles : (N + BN - 1) / BN;
-    if (tiles_n % 2 == 0) {                                                  // (a grid of tiles: no divisions)
+    if constexpr (!BANDS) {                                                  // (a grid of tiles: no divisions)
         tile_m = blockIdx.y;
         tile_n = blockIdx.x;
     } else {
         constexpr int kBand = 512 / BN;
+        const int tiles_n = more.n ? more.tiles : (N + BN - 1) / BN;
         const int tiles_m = (M + BM - 1) / BM, total = tiles_m * tiles_n;
         const int per_xcd = (total + 7) / 8, l = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
         if (l >= total) return;
@@ -1907,35 +1903,43 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
 
 }  // namespace skinny
 
+// Blocks go to the 8 XCDs round-robin, each with an L2 of its own.  With the tiles in their order an XCD keeps to its share
+// of the columns of tiles where their number is even; where it is odd it comes through all of them, and XCD x takes the
+// x-th eighth of a list instead that runs through bands of 512 columns of outputs, down M inside a band.  us, int8, tiles in
+// order / in bands: 15 columns of 64, 2048 x 960 x 960 16.2 / 12.2, 25, 700 x 1600 x 960 13.4 / 11.2, 45, 320 x 2880 x 576 8.4 / 7.3;
+// even: 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.  The list costs a few divisions ahead of the first load,
+// which pay from about 75 tiles on: 9 tiles, 60 x 576 x 576 5.5 / 5.7, 45, 192 x 960 x 960 9.8 / 10.0, 72, 512 x 576 x 576 6.5 / 7.0;
+// 75, 320 x 960 x 960 10.4 / 10.0, 99, 700 x 576 x 576 7.7 / 6.3.
+inline bool tiles_in_bands(long tiles_n, long tiles_m) { return tiles_n % 2 != 0 && tiles_n * tiles_m >= 75; }
+
+template <int BM, int BN, int WM, int WN, int KIND, bool BANDS>
+bool launch_tile_as(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, const dim3& grid,
+                    const MoreMats& more) {
+    constexpr size_t lds_bytes = 2u * (BM + BN) * kLd * sizeof(uint16_t);
+    auto* kern = gemm_kernel<BM, BN, WM, WN, KIND, BANDS>;
+    // more than 64 KB of LDS per block has to be asked for once per kernel
+    if (lds_bytes > 65536 &&
+        !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
+        return false;
+    hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W),
+                       static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(out), M, N, K, more);
+    return MI_HIP_OK(hipGetLastError());
+}
+
 template <int BM, int BN, int WM, int WN>
 bool launch_tile(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W,
                  const void* scale, void* out, const MoreMats& more) {
     const int tiles_n = more.n ? more.tiles : (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM;
     const long total = static_cast<long>(tiles_n) * tiles_m;
-    // see the block -> tile map in the kernel
-    const dim3 grid = tiles_n % 2 == 0 ? dim3(tiles_n, tiles_m) : dim3(static_cast<unsigned>(8 * ((total + 7) / 8)));
-    const auto* xp = static_cast<const uint16_t*>(x);
-    const auto* wp = static_cast<const uint8_t*>(W);
-    const auto* sp = static_cast<const uint16_t*>(scale);
-    auto* op = static_cast<uint16_t*>(out);
-    constexpr size_t lds_bytes = 2u * (BM + BN) * kLd * sizeof(uint16_t);
-    // more than 64 KB of LDS per block has to be asked for once per kernel
-    if (kind == WK_I8) {
-        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_I8>;
-        if (lds_bytes > 65536 &&
-            !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
-            return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
-    } else {
-        auto* kern = gemm_kernel<BM, BN, WM, WN, WK_F16>;
-        if (lds_bytes > 65536 &&
-            !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
-            return false;
-        hipLaunchKernelGGL(kern, grid, dim3(kThreads), lds_bytes, s, xp, wp, sp, op, M, N, K, more);
+    if (tiles_in_bands(tiles_n, tiles_m)) {
+        const dim3 list(static_cast<unsigned>(8 * ((total + 7) / 8)));
+        return kind == WK_I8 ? launch_tile_as<BM, BN, WM, WN, WK_I8, true>(s, M, N, K, x, W, scale, out, list, more)
+                             : launch_tile_as<BM, BN, WM, WN, WK_F16, true>(s, M, N, K, x, W, scale, out, list, more);
     }
-    return MI_HIP_OK(hipGetLastError());
+    const dim3 grid(tiles_n, tiles_m);
+    return kind == WK_I8 ? launch_tile_as<BM, BN, WM, WN, WK_I8, false>(s, M, N, K, x, W, scale, out, grid, more)
+                         : launch_tile_as<BM, BN, WM, WN, WK_F16, false>(s, M, N, K, x, W, scale, out, grid, more);
 }
 
 inline long tiles(int M, int N, int bm, int bn) {
