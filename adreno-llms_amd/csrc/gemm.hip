@@ -2146,10 +2146,12 @@ int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, cons
     const int mode = gemm_mode(s);
     if (p.kernel >= 1 && p.kernel <= 3 && p.k_slices == 1 && (mode == 0 || mode == 4) && wide_reaches(kind, M, N, K)) {
         const int terms = kind == WK_Q4 ? p.terms : 1;
+        const int cus = device_info().cus;
+        // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
+        const double uncut = p.kernel == 1 ? wide::estimate_us(kind, terms, p.tile_rows / 32, 1, M, N, K, cus) : tiled_estimate_us(M, N, K);
         int tm = 1, splits = 1;
         double us = 0.0;
-        if (wide::pick_sliced(kind, terms, M, N, K, device_info().cus, workspace_bytes, &tm, &splits, &us) &&
-            us - 2.5 < gemm_estimate_us(kind, M, N, K, workspace_bytes)) {
+        if (wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &us) && us - 2.5 < uncut) {
             p.kernel = 1;
             p.tile_rows = 32 * tm;
             p.k_slices = splits;
