@@ -1345,7 +1345,10 @@ __device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ su
 // the wide kernel), or rounded to fp16 once with TERMS = 1.
 // GLU: see launch_gemm_glu (an instance of its own: as a switch it cost the plain launch 2 % at 16 rows).
 // bx of gx blocks along N; slice by of kb slices of K, which meet as told at meet_slices.
-template <int KIND, int MT, bool XL, int TERMS, bool GLU>
+// MEET: there may be more than one slice over blocks.  An instance of its own (never with x in LDS or the SwiGLU, which come with
+// one): where it never runs, the code that meets them had fp16 rows spill 21 to 29 scalars instead of none, 5.04 -> 5.24 us at 17
+// rows of 3072 x 576, 6.66 -> 6.82 of 576 x 1536; with x in LDS 45 instead of 0, int8 73 instead of 27 at 16 rows.
+template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
 __device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
                                             const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
                                             const int K, const int ks, const int logical_blocks, float* __restrict__ partial,
@@ -1568,9 +1571,7 @@ __device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, cons
                     for (int r = 0; r < 4; ++r) acc[t][r] += v[r];
                 }
             }
-            // (x in LDS and the SwiGLU come with one slice over blocks; the code for more, where it never runs, had fp16 rows
-            //  with x in LDS spill 45 scalars instead of 0, int8 73 instead of 27 at 16 rows)
-            if constexpr (!XL && !GLU) {
+            if constexpr (MEET) {
                 if (kb > 1 &&
                     !meet_slices(acc[t], partial + (static_cast<size_t>(group) * MT + t) * kb * 256, counters + group * MT + t, by, kb, lane))
                     continue;
@@ -1614,14 +1615,14 @@ __device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, cons
     }
 }
 
-template <int KIND, int MT, bool XL, int TERMS, bool GLU>
+template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
 __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
                                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out,
                                                            int M, int N, int K, int ks, int logical_blocks,
                                                            float* __restrict__ partial, uint32_t* __restrict__ counters,
                                                            MoreMats more) {
-    skinny_rows<KIND, MT, XL, TERMS, GLU>(X, W, scale, out, M, N, K, ks, logical_blocks, partial, counters, more, blockIdx.x,
-                                              gridDim.x, blockIdx.y, gridDim.y);
+    skinny_rows<KIND, MT, XL, TERMS, GLU, MEET>(X, W, scale, out, M, N, K, ks, logical_blocks, partial, counters, more, blockIdx.x,
+                                                    gridDim.x, MEET ? blockIdx.y : 0, MEET ? gridDim.y : 1);
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -1737,9 +1738,9 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny_many(const SkinnyCall
     uint32_t* counters = L->c[q].counters;
     const int N = L->c[q].N, K = L->c[q].K, logical = L->c[q].logical, M = L->M;
     if (ks_xl & 16)
-        skinny_rows<KIND, MT, true, TERMS, false>(X, W, scale, out, M, N, K, ks, logical, nullptr, nullptr, none, at, blocks, 0, 1);
+        skinny_rows<KIND, MT, true, TERMS, false, false>(X, W, scale, out, M, N, K, ks, logical, nullptr, nullptr, none, at, blocks, 0, 1);
     else
-        skinny_rows<KIND, MT, false, TERMS, false>(X, W, scale, out, M, N, K, ks, logical, partial, counters, none, at - by * blocks, blocks, by, kb);
+        skinny_rows<KIND, MT, false, TERMS, false, true>(X, W, scale, out, M, N, K, ks, logical, partial, counters, none, at - by * blocks, blocks, by, kb);
 }
 
 // Shapes whose blocks hold a strip of the gate matrix and its strip of the up matrix, and LDS for them to meet in
@@ -1754,14 +1755,14 @@ inline long blocks_along_n(bool xl, long logical, size_t lds) {
     return logical > resident ? resident : logical;
 }
 
-template <int KIND, int MT, bool XL, int TERMS, bool GLU>
+template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
 bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
                 float* partial, const MoreMats& more) {
     const int ks = sh.ks;
     const long groups = more.n ? more.tiles : (N + 15) / 16, per_block = kWaves / ks;
     const long logical = (groups + per_block - 1) / per_block;
     const size_t lds = lds_bytes(MT, K, XL, ks);
-    auto* kern = gemm_skinny<KIND, MT, XL, TERMS, GLU>;
+    auto* kern = gemm_skinny<KIND, MT, XL, TERMS, GLU, MEET>;
     if (lds > 65536 &&
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
@@ -1777,10 +1778,11 @@ template <int KIND, int MT, int TERMS>
 bool launch_mt(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
                float* partial, const MoreMats& more, bool glu) {
     if (glu)
-        return sh.xl ? launch_one<KIND, MT, true, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                     : launch_one<KIND, MT, false, TERMS, true>(s, M, N, K, x, W, scale, out, sh, partial, more);
-    return sh.xl ? launch_one<KIND, MT, true, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                 : launch_one<KIND, MT, false, TERMS, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
+        return sh.xl ? launch_one<KIND, MT, true, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
+                     : launch_one<KIND, MT, false, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
+    if (sh.kb > 1) return launch_one<KIND, MT, false, TERMS, false, true>(s, M, N, K, x, W, scale, out, sh, partial, more);
+    return sh.xl ? launch_one<KIND, MT, true, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
+                 : launch_one<KIND, MT, false, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
 }
 
 template <int KIND, int TERMS>
