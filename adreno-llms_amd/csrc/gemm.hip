@@ -81,6 +81,15 @@ __device__ __forceinline__ void pick_matrix(const MoreMats& mm, int& tile, const
     tile -= first;
 }
 
+// Blocks go to the 8 XCDs round-robin, each with an L2 of its own.  With the tiles in their order an XCD keeps to its share
+// of the columns of tiles where their number is even; where it is odd it comes through all of them, and XCD x takes the
+// x-th eighth of a list instead that runs through bands of 512 columns of outputs, down M inside a band.  us, int8, tiles in
+// order / in bands: 15 columns of 64, 2048 x 960 x 960 16.2 / 12.2, 25, 700 x 1600 x 960 13.4 / 11.2, 45, 320 x 2880 x 576 8.4 / 7.3;
+// even: 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.  The list costs a few divisions ahead of the first load,
+// which pay from about 75 tiles on: 9 tiles, 60 x 576 x 576 5.5 / 5.7, 45, 192 x 960 x 960 9.8 / 10.0, 72, 512 x 576 x 576 6.5 / 7.0;
+// 75, 320 x 960 x 960 10.4 / 10.0, 99, 700 x 576 x 576 7.7 / 6.3.
+inline bool tiles_in_bands(long tiles_n, long tiles_m) { return tiles_n % 2 != 0 && tiles_n * tiles_m >= 75; }
+
 template <int BM, int BN, int WM, int WN, int KIND, bool BANDS>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(const uint16_t* __restrict__ X,
                                                         const uint8_t* __restrict__ W,
@@ -940,13 +949,15 @@ inline double estimate_us(int kind, int terms, int tm, int splits, int M, int N,
     //  tiles, one block per CU and twice the matrix work per byte, lose less to a full chip than the general
     //  factors say: 2048 x 4864 x 896 in 160-row tiles 34.8 us (a block alone: 27.4), 4096 x 8192 x 2048 in
     //  128-row tiles 231 us for four rounds of 48.4, against 258 us for the 64-row tiles the factors preferred.)
-    //  fp16 weights do so at any number of blocks and from 9 stages on: 1200 x 960 x 960 10.5 us, 700 x 1600 x 960 10.3,
-    //  1200 x 960 x 576 8.0, 300 x 4864 x 896 9.7, where the general factor put the 64 x 64 tiles ahead, which take 13.7,
-    //  14.0, 9.8 and 11.8.
-    const bool f16_roomy = kind == WK_F16 && splits == 1 && blocks <= cus && tm <= 2 && stages <= 48;
-    // (int8, 32-row tiles of 14 or 15 stages: 300 x 4864 x 896 10.0 us, 700 x 2560 x 960 10.5, 2048 x 960 x 960 12.1,
-    //  where the 64 x 64 tiles take 11.1, 10.2 and 12.2)
-    const bool i8_short = kind == WK_I8 && splits == 1 && tm == 1 && blocks > cus / 2 && blocks <= cus && (stages == 14 || stages == 15);
+    //  fp16 weights do so at any number of blocks and from 9 stages on: 300 x 4864 x 896 9.7 us, 416 x 5120 x 960 11.5, 917 x 3072 x
+    //  576 8.5, where the general factor put the 64 x 64 tiles ahead, which take 11.8, 12.5 and 9.3.
+    const bool bands = stages <= 16 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);      // (the 64 x 64 tiles are the faster then)
+    const bool f16_roomy = kind == WK_F16 && splits == 1 && blocks <= cus && tm <= 2 && stages <= 48 && !bands;
+    // (int8, 32-row tiles of 14 or 15 stages: 304 x 4864 x 896 9.4 us, 192 x 9728 x 896 9.6, 320 x 5120 x 960 9.9, the 64 x 64 tiles
+    //  9.6, 9.6 and 10.0, which leave the SwiGLU to a launch of its own.  Not where those go in bands: int8 2048 x 960 x 960 11.4
+    //  against 10.4, fp16 1184 x 1600 x 960 12.5 against 10.4, 1408 x 960 x 576 7.7 against 7.2; at a longer K the wide tiles keep up:
+    //  1856 x 576 x 1536 13.6 against 14.4)
+    const bool i8_short = kind == WK_I8 && splits == 1 && tm == 1 && blocks > cus / 2 && blocks <= cus && (stages == 14 || stages == 15) && !bands;
     const bool roomy = splits == 1 && blocks > cus / 2 && blocks <= cus &&
                        (tm == 2 || (tm == 1 && stages >= 16 && stages <= 48));
     const bool q4_tall = kind == WK_Q4 && terms == 2 && tm >= 3 && splits == 1;
@@ -1904,15 +1915,6 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
 }
 
 }  // namespace skinny
-
-// Blocks go to the 8 XCDs round-robin, each with an L2 of its own.  With the tiles in their order an XCD keeps to its share
-// of the columns of tiles where their number is even; where it is odd it comes through all of them, and XCD x takes the
-// x-th eighth of a list instead that runs through bands of 512 columns of outputs, down M inside a band.  us, int8, tiles in
-// order / in bands: 15 columns of 64, 2048 x 960 x 960 16.2 / 12.2, 25, 700 x 1600 x 960 13.4 / 11.2, 45, 320 x 2880 x 576 8.4 / 7.3;
-// even: 40, 700 x 2560 x 960 10.5 / 13.1, 76, 300 x 4864 x 896 11.1 / 12.0.  The list costs a few divisions ahead of the first load,
-// which pay from about 75 tiles on: 9 tiles, 60 x 576 x 576 5.5 / 5.7, 45, 192 x 960 x 960 9.8 / 10.0, 72, 512 x 576 x 576 6.5 / 7.0;
-// 75, 320 x 960 x 960 10.4 / 10.0, 99, 700 x 576 x 576 7.7 / 6.3.
-inline bool tiles_in_bands(long tiles_n, long tiles_m) { return tiles_n % 2 != 0 && tiles_n * tiles_m >= 75; }
 
 template <int BM, int BN, int WM, int WN, int KIND, bool BANDS>
 bool launch_tile_as(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, const dim3& grid,

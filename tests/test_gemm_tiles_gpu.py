@@ -39,3 +39,13 @@ def test_together_as_one_by_one(kind, rows, k, widths):
     queue = mil.Queue()
     assert mil.lib().mi_stream_set_modes(queue.handle, -1, 2)
     _together_as_one_by_one(queue, kind, rows, k, widths)
+
+
+@pytest.mark.parametrize("kind,rows,n,k,kernel", [("int8", 2048, 960, 960, 2), ("f16", 1184, 1600, 960, 2), ("f16", 1408, 960, 576, 2),
+                                                  ("int8", 320, 5120, 960, 1), ("f16", 416, 5120, 960, 1), ("f16", 704, 3072, 576, 1)])
+def test_tiles_in_bands_are_chosen_where_they_are_faster(kind, rows, n, k, kernel):
+    """Odd numbers of tile columns, 75 tiles and more, K to 1024: the 64 x 64 tiles (2); even numbers: the wide kernel (1)."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep = mil.Queue(), []
+    x, w = mil.Buffer(2 * rows * k), _weights(kind, n, k, 12, keep)
+    assert mil.linear_plan(queue, rows, n, k, x, w)[0] == kernel
