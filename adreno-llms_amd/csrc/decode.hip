@@ -1836,8 +1836,8 @@ static int enqueue_step(Decoder* d, void* stream) {
 // A step is the same launches with the same arguments at every position, and a host that enqueues them one by one spends
 // 3 to 4.5 us on each of 123 to 153 where the GPU needs less; as a recorded graph they cost one call of about 90 us and
 // follow each other at 1.6 us instead of 2.5.  So the second of two steps in a row under the same circumstances is
-// recorded (0.5 to 2 ms, once) and from then on replayed: a token of SmolLM2-135M in fp16, read back as it comes, 679 ->
-// 497 us, of Qwen2.5-0.5B in int8 602 -> 482 us.
+// recorded (0.5 to 2 ms, once) and from then on replayed: a token of SmolLM2-135M in fp16, read back as it comes, 678 ->
+// 582 us, of Qwen2.5-0.5B in int8 602 -> 482 us.
 //
 // It is recorded on a stream that nobody else knows (StandsFor), so that another thread that meanwhile waits for the step's
 // stream, or asks about it, neither fails nor breaks into the recording.
