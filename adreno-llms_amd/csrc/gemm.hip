@@ -1345,255 +1345,283 @@ __device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ su
     return true;
 }
 
-// XL: the block first copies its rows of x into LDS (rows padded by 16 bytes, which spreads the 16
-// rows a 16-byte read touches over all banks) and every wavefront reads its fragments from there;
-// blocks then live long and walk over the strips.  Without XL (x too large for LDS) the fragments
-// come from the caches with the weights, 2 MT bytes per byte of W, and the L1's few requests
-// in flight bound the rate: that form only pays for a few rows of x at a long K.
-// Q4 weights: an iteration is 128 values of K, of which a lane holds 32, exactly one scale block (16
-// bytes of nibbles and one scale per lane and iteration); the weights enter the matrix cores as
-// q * scale, exactly, in TERMS = 2 fp16 terms (scale = hi + lo with 7 and 4 significant bits, as in
-// the wide kernel), or rounded to fp16 once with TERMS = 1.
-// GLU: see launch_gemm_glu (an instance of its own: as a switch it cost the plain launch 2 % at 16 rows).
-// bx of gx blocks along N; slice by of kb slices of K, which meet as told at meet_slices.
-// MEET: there may be more than one slice over blocks.  An instance of its own (never with x in LDS or the SwiGLU, which come with
-// one): where it never runs, the code that meets them had fp16 rows spill 21 to 29 scalars instead of none, 5.04 -> 5.24 us at 17
-// rows of 3072 x 576, 6.66 -> 6.82 of 576 x 1536; with x in LDS 45 instead of 0, int8 73 instead of 27 at 16 rows.
-template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
-__device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
-                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
-                                            const int K, const int ks, const int logical_blocks, float* __restrict__ partial,
-                                            uint32_t* __restrict__ counters, const MoreMats& more, const int bx, const int gx,
-                                            const int by, const int kb) {
-    constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
-    constexpr int WV = F16 ? 2 : 1;                       // 16-byte loads of W per lane, strip and iteration
-    constexpr int kWB = F16 ? 2 : 1;                      // bytes of a row of W per 64 bytes of an iteration's weights / 64
-    constexpr int kItK = Q4 ? 128 : 64;                   // values of K per iteration
-    constexpr int XE = kItK / 32;                         // 16-byte pieces of x per lane and iteration = MFMAs per x tile and term
-    constexpr int kPerIt = 4 * WV + (Q4 ? 1 : 0) + (XL ? 0 : 4 * XE * MT);   // registers one iteration's operands take in a buffer
-    constexpr int kBudget = F16 ? 40 : 48;                // registers per buffer (with 64 the fp16 instances spill)
-    constexpr int kChunk = kBudget / kPerIt < 1 ? 1 : kBudget / kPerIt > 8 ? 8 : kBudget / kPerIt;   // iterations per buffer
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const uint32_t xrow = XL ? static_cast<uint32_t>(K) * 2u + 16u : 0u;              // bytes per row of x in LDS
-    floatx4* red = reinterpret_cast<floatx4*>(lds + 16u * MT * xrow);                 // [kWaves][MT][64]
+// Up to 64 rows of x.  A wavefront owns a tile of 16 S columns of the output (S strips of 16 rows of W) and a slice of K, and
+// works for itself: it asks for its slice of x and of W, 64 values of K at a time, by direct global -> LDS loads into a ring of
+// its own, waits for its own loads only, and multiplies.  ks wavefronts of a block share a tile; their sums meet in LDS, in
+// slice order, behind the one barrier of the kernel.
+//
+// What bounds such a launch is the way to memory, and how much of it is asked for at once: a few us of latency and one pass
+// over the weights.  So
+//  * everything a block needs is on its way before anything is used, up to 160 KB of LDS per CU and without registers;
+//  * a load instruction covers whole pieces of rows, 64 or 128 bytes of each (8 lanes to a row of x).  As fragments straight
+//    from memory neighbouring lanes are in different rows, and a load of 64 lanes is 64 lookups in the L1, for x as often
+//    as a block has strips: that bounded the launch;
+//  * the 16-byte pieces of a row are XOR-swizzled so that fragment reads are free of bank conflicts without padding.
+// us per launch, weights from HBM, with fragments (x copied to LDS first where it fitted) -> this: fp16, 37 rows of 960 x 2560 9.7 ->
+// 8.1, 1600 x 960 6.1 -> 5.3, 960 x 960 6.0 -> 4.5, 5120 x 960 with the SwiGLU 7.6 -> 6.6, 64 rows of 576 x 1536 9.8 -> 5.9; int8, 16 rows of
+// 896 x 896 4.2 -> 3.7, 9728 x 896 with the SwiGLU 7.0 -> 6.7; Q4, 24 rows of 896 x 4864 9.8 -> 7.4; the floor of a launch is 1.6.
+// An int8 weight becomes fp16 in the registers (exactly).  Q4: q * scale as two exact fp16 terms (scale = hi + lo with 7 and
+// 4 significant bits, as in the wide kernel), or rounded to fp16 once with TERMS = 1.
+// GLU: see launch_gemm_glu; the tile's two strips are the gate's and the up matrix's (S = 2).
+// MEET: kb slices of K over blocks, which meet as told at meet_slices (an instance of its own, S = 1).
+// Without MEET and with `partial` the sums go there, [slice over blocks][M][N], for a launch that adds them (N a multiple of 4).
+template <int KIND, int MT, int S>
+struct Unit {                                            // what 64 values of K take in a wavefront's ring
+    static constexpr int kX = MT * 2048;                 // rows of 128 bytes
+    static constexpr int kW = KIND == WK_F16 ? S * 2048 : KIND == WK_I8 ? S * 1024 : S * 512;
+    static constexpr int kBytes = kX + kW + (KIND == WK_Q4 ? S * 64 : 0);              // Q4: two block scales per row
+    static constexpr int kLoads = 2 * MT + (KIND == WK_F16 ? 2 * S : KIND == WK_I8 ? S : 2);
+};
+constexpr int kMaxRing = 8;                              // units in a ring
 
+template <int LOADS>
+__device__ __forceinline__ void wait_for_all_but(int units) {           // the loads of the last `units` units may be under way
+    #define MI_CASE(u) case u: MI_WAIT_VM((u) * LOADS < 63 ? (u) * LOADS : 63); break;
+    switch (units) {
+        MI_CASE(0) MI_CASE(1) MI_CASE(2) MI_CASE(3) MI_CASE(4) MI_CASE(5) MI_CASE(6)
+        default: MI_WAIT_VM(7 * LOADS < 63 ? 7 * LOADS : 63);
+    }
+    #undef MI_CASE
+}
+
+// A unit's fragments from LDS (the wait stands in the block that reads: the registers are in flight until then).
+#define MI_X1 "ds_read_b128 %[p0], %[a]\n\tds_read_b128 %[q0], %[b]\n\t"
+#define MI_X2 MI_X1 "ds_read_b128 %[p1], %[a] offset:2048\n\tds_read_b128 %[q1], %[b] offset:2048\n\t"
+#define MI_X3 MI_X2 "ds_read_b128 %[p2], %[a] offset:4096\n\tds_read_b128 %[q2], %[b] offset:4096\n\t"
+#define MI_X4 MI_X3 "ds_read_b128 %[p3], %[a] offset:6144\n\tds_read_b128 %[q3], %[b] offset:6144\n\t"
+#define MI_OX1 [p0] "=&v"(x[0][0]), [q0] "=&v"(x[0][1])
+#define MI_OX2 MI_OX1, [p1] "=&v"(x[1][0]), [q1] "=&v"(x[1][1])
+#define MI_OX3 MI_OX2, [p2] "=&v"(x[2][0]), [q2] "=&v"(x[2][1])
+#define MI_OX4 MI_OX3, [p3] "=&v"(x[3][0]), [q3] "=&v"(x[3][1])
+#define MI_F1 "ds_read_b128 %[w0], %[a] offset:%[o0]\n\tds_read_b128 %[v0], %[b] offset:%[o0]\n\t"
+#define MI_F2 MI_F1 "ds_read_b128 %[w1], %[a] offset:%[o1]\n\tds_read_b128 %[v1], %[b] offset:%[o1]\n\t"
+#define MI_OF1 [w0] "=&v"(w[0][0]), [v0] "=&v"(w[0][1])
+#define MI_OF2 MI_OF1, [w1] "=&v"(w[1][0]), [v1] "=&v"(w[1][1])
+#define MI_I1 "ds_read_b128 %[w0], %[d]\n\t"
+#define MI_I2 MI_I1 "ds_read_b128 %[w1], %[d] offset:1024\n\t"
+#define MI_OI1 [w0] "=&v"(w[0][0])
+#define MI_OI2 MI_OI1, [w1] "=&v"(w[1][0])
+#define MI_Q1 "ds_read_b64 %[w0], %[d]\n\tds_read_b32 %[v0], %[e]\n\t"
+#define MI_Q2 MI_Q1 "ds_read_b64 %[w1], %[d] offset:512\n\tds_read_b32 %[v1], %[e] offset:64\n\t"
+#define MI_OQ1 [w0] "=&v"(w4[0]), [v0] "=&v"(ws[0])
+#define MI_OQ2 MI_OQ1, [w1] "=&v"(w4[1]), [v1] "=&v"(ws[1])
+#define MI_READ_MT(MTN, WS, OWS, ...)                                                                      \
+    if constexpr (MT == MTN)                                                                               \
+        asm volatile(MI_X##MTN WS "s_waitcnt lgkmcnt(0)" : MI_OX##MTN, OWS : [a] "v"(a), [b] "v"(b), __VA_ARGS__ : "memory");
+#define MI_READ_S(SN, L, ...)                                                                              \
+    if constexpr (S == SN) {                                                                               \
+        MI_READ_MT(1, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
+        MI_READ_MT(2, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
+        MI_READ_MT(3, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
+        MI_READ_MT(4, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
+    }
+template <int KIND, int MT, int S>
+struct UnitFrags {
+    u32x4 x[MT][2];
+    u32x4 w[S][2];                                       // int8: only the first, 16 weights
+    u32x2 w4[S];                                         // Q4: 16 weights and the row's two block scales
+    uint32_t ws[S];
+    // a, b: the lane's pieces 2c and 2c + 1 of its row of the first x tile; d: of the first strip; e: its scales
+    __device__ __forceinline__ void read(uint32_t a, uint32_t b, uint32_t d, uint32_t e) {
+        if constexpr (KIND == WK_F16) {
+            MI_READ_S(1, F, [o0] "i"(MT * 2048))
+            MI_READ_S(2, F, [o0] "i"(MT * 2048), [o1] "i"(MT * 2048 + 2048))
+        } else if constexpr (KIND == WK_I8) {
+            MI_READ_S(1, I, [d] "v"(d))
+            MI_READ_S(2, I, [d] "v"(d))
+        } else {
+            MI_READ_S(1, Q, [d] "v"(d), [e] "v"(e))
+            MI_READ_S(2, Q, [d] "v"(d), [e] "v"(e))
+        }
+    }
+};
+
+template <int KIND, int MT, int S, int TERMS, bool GLU, bool MEET>
+__device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
+                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
+                                            const int K, const int ks, const int ring_units, float* __restrict__ partial,
+                                            uint32_t* __restrict__ counters, const MoreMats& more, const int bx, const int waves,
+                                            const int by, const int kb) {
+    static_assert(!GLU || S == 2, "a strip of either matrix");
+    constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
+    typedef Unit<KIND, MT, S> U;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, c = lane >> 4;
-    const int slice = wave % ks;
-    const int nit = (K + kItK - 1) / kItK;               // (Q4 at K = 64 mod 128: the upper half of the lanes sits out the last one)
-    const size_t wrowb = Q4 ? static_cast<size_t>(K) / 2 : static_cast<size_t>(K) * kWB;   // bytes of a row of W
-    // K is cut over kb blocks (a strip each, one trip through the loop below) and, inside a block, over ks wavefronts
-    const int b0 = nit * by / kb;
-    const int b1 = nit * (by + 1) / kb;
-    const int it0 = b0 + (b1 - b0) * slice / ks, it1 = b0 + (b1 - b0) * (slice + 1) / ks;
+    const int slice = wave & (ks - 1);
+    int tile = bx * (waves / ks) + wave / ks;
+    if constexpr (!GLU) pick_matrix(more, tile, W, scale, out, N);
+    const int n0 = 16 * S * tile;
+    const bool live = n0 < N;                            // (a block's last tiles may lie past the matrix: they take part in the barrier only)
+    const int nb = live ? n0 : 0;
 
-    if constexpr (XL) {
-        // Wavefront w copies rows w, w + 8, ...: a lane requests its 16-byte piece of each of the wavefront's
-        // 2 MT rows before it stores the first, so the copy is one trip to memory per 64 pieces of a row
-        // (before: a trip per 512 pieces of the tile, and a division per piece; 4864 x 896 at 16 / 32 / 48
-        // rows 4.65 / 5.8 / 6.8 -> 4.35 / 4.95 / 5.7 us).  Rows past M are read as the last row and never
-        // stored from.  Asking for the first weights ahead of this copy was measured as well: slower
-        // (4.7 / 5.4 / 6.05 us), x then arrives behind them.
-        const int per_row = K / 8;                       // 16-byte pieces per row
-        const uint8_t* Xb = reinterpret_cast<const uint8_t*>(X);
-        for (int piece = threadIdx.x & 63; piece < per_row; piece += 64) {
-            u32x4 t[2 * MT];
-            #pragma unroll
-            for (int rr = 0; rr < 2 * MT; ++rr) {
-                const int row = wave + kWaves * rr;
-                const int m = row < M ? row : M - 1;
-                t[rr] = *reinterpret_cast<const u32x4*>(Xb + static_cast<size_t>(m) * K * 2 + piece * 16);
-            }
-            #pragma unroll
-            for (int rr = 0; rr < 2 * MT; ++rr)
-                *reinterpret_cast<u32x4*>(lds + (wave + kWaves * rr) * xrow + piece * 16) = t[rr];
-        }
-        __syncthreads();
-    }
-    const uint8_t* xp[MT];                               // without XL: this lane's rows of x in memory
-    #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int m = 16 * t + i < M ? 16 * t + i : M - 1;
-        xp[t] = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(m) * K * 2 + c * (16 * XE);
-    }
-    const uint32_t xl = (16u * 0 + i) * xrow + c * (16u * XE);  // with XL: this lane's row of the first x tile in LDS
-    const uint8_t* const W0 = W;
-    const uint16_t* const scale0 = scale;
-    uint16_t* const out0 = out;
-    const int N0 = N;
+    // K is cut over kb blocks and, inside a block, over ks wavefronts
+    const int its = K / 64, b0 = its * by / kb, b1 = its * (by + 1) / kb;
+    const int it0 = b0 + (b1 - b0) * slice / ks, n = live ? b0 + (b1 - b0) * (slice + 1) / ks - it0 : 0;
 
-    for (int lb = bx; lb < logical_blocks; lb += gx) {     // (the same trips for the whole block)
-        int group = lb * (kWaves / ks) + wave / ks;                       // strip
-        if constexpr (!GLU) {
-            W = W0; scale = scale0; out = out0; N = N0;
-            pick_matrix(more, group, W, scale, out, N);
-        }
-        const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
-        const int wr = 16 * group + i < N ? 16 * group + i : N - 1;       // rows past N are read as the last row
-        const uint8_t* wp = W + static_cast<size_t>(wr) * wrowb + c * 16 * WV;
-        [[maybe_unused]] const uint16_t* sp = nullptr;                    // Q4: the row's block scales, this lane's first
-        if constexpr (Q4) sp = scale + static_cast<size_t>(wr) * (K / 32) + c;
-        floatx4 acc[MT];
+    uint32_t sc[S][4];
+    if constexpr (KIND == WK_I8) {                       // asked for first: used last
         #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-        u32x4 wb[2][kChunk][WV];
-        [[maybe_unused]] uint16_t sb[2][kChunk];
-        [[maybe_unused]] u32x4 xb[2][XL ? 1 : kChunk][XL ? 1 : MT][XE];
-        // `full`: kChunk iterations whatever the slice's end (the caller knows they exist); the number
-        // of requests is then a constant, and only then can the wait before a buffer is multiplied
-        // leave the other buffer's requests in flight
-        auto fetch = [&](auto fullc, int b, int j0) {
+        for (int s = 0; s < S; ++s)
             #pragma unroll
-            for (int u = 0; u < kChunk; ++u) {
-                const int it = j0 + u;
-                if constexpr (!decltype(fullc)::value) {
-                    if (it >= it1) break;
-                }
-                // (Q4, K = 64 mod 128: a lane without weights in the last iteration asks for the start of its rows)
-                [[maybe_unused]] const bool mine = !Q4 || kItK * it + 32 * c < K;
-                if constexpr (!XL) {
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        #pragma unroll
-                        for (int e = 0; e < XE; ++e)
-                            xb[b][u][t][e] = reinterpret_cast<const u32x4*>(
-                                xp[t] + (mine ? static_cast<ptrdiff_t>(it) * (2 * kItK) : -static_cast<ptrdiff_t>(c) * (16 * XE)))[e];
+            for (int r = 0; r < 4; ++r) {
+                const int nq = nb + 16 * s + 4 * c + r;
+                sc[s][r] = scale[nq < N ? nq : N - 1];
+            }
+    }
+
+    // --- fill side: lane l of a load writes LDS bytes [16 l, +16) of its KB ---
+    // x, fp16 W: a load covers 8 rows of 128 bytes; slot p of row r holds piece p ^ ((r >> 1) & 7)
+    // int8: 16 rows of 64 bytes, piece p ^ ((r >> 2) & 3); Q4: 16 rows of 32 bytes (S of them), piece p ^ ((r >> 3) & 1)
+    const size_t wrowb = Q4 ? static_cast<size_t>(K) / 2 : F16 ? static_cast<size_t>(K) * 2 : static_cast<size_t>(K);
+    const uint8_t* const Xb = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(it0) * 128;
+    const uint8_t* const Wb = W + static_cast<size_t>(nb) * wrowb + static_cast<size_t>(it0) * (Q4 ? 32 : F16 ? 128 : 64);
+    const int wlast = N - 1 - nb;                        // rows past N are read as the last row
+    constexpr int kWL = F16 ? 2 * S : Q4 ? 1 : S;
+    uint32_t xoff[2 * MT], woff[kWL];
+    #pragma unroll
+    for (int j = 0; j < 2 * MT; ++j) {
+        const int r = 8 * j + (lane >> 3), m = r < M ? r : M - 1;
+        xoff[j] = static_cast<uint32_t>(m) * static_cast<uint32_t>(K) * 2u + 16u * ((lane & 7) ^ ((r >> 1) & 7));
+    }
+    #pragma unroll
+    for (int j = 0; j < kWL; ++j) {
+        int r, piece;
+        if constexpr (F16) { r = 8 * j + (lane >> 3); piece = (lane & 7) ^ ((r >> 1) & 7); }
+        else if constexpr (Q4) { r = lane >> 1; piece = (lane & 1) ^ ((r >> 3) & 1); }
+        else { r = 16 * j + (lane >> 2); piece = (lane & 3) ^ ((r >> 2) & 3); }
+        woff[j] = static_cast<uint32_t>(r < wlast ? r : wlast) * static_cast<uint32_t>(wrowb) + 16u * piece;
+    }
+    [[maybe_unused]] const uint8_t* Sb = nullptr;
+    [[maybe_unused]] uint32_t soff = 0;
+    if constexpr (Q4) {
+        Sb = reinterpret_cast<const uint8_t*>(scale) + static_cast<size_t>(nb) * (K / 16) + static_cast<size_t>(it0) * 4;
+        const int r = lane & (16 * S - 1);
+        soff = static_cast<uint32_t>(r < wlast ? r : wlast) * static_cast<uint32_t>(K / 16);
+    }
+    uint8_t* const ring = lds + static_cast<size_t>(wave) * ring_units * U::kBytes;
+    auto fill = [&](int u, int slot) {                   // unit u of the slice
+        uint8_t* l = ring + slot * U::kBytes;
+        #pragma unroll
+        for (int j = 0; j < 2 * MT; ++j) wide::lds_fill16(Xb + static_cast<size_t>(u) * 128 + xoff[j], l + 1024 * j);
+        const uint8_t* w = Wb + static_cast<size_t>(u) * (Q4 ? 32 : F16 ? 128 : 64);
+        if constexpr (Q4) {
+            if (lane < 32 * S) wide::lds_fill16(w + woff[0], l + U::kX);
+            if (lane < 16 * S) wide::lds_fill4(Sb + static_cast<size_t>(u) * 4 + soff, l + U::kX + U::kW);
+        } else {
+            #pragma unroll
+            for (int j = 0; j < kWL; ++j) wide::lds_fill16(w + woff[j], l + U::kX + 1024 * j);
+        }
+    };
+    const int lead = n < ring_units ? n : ring_units;
+    for (int u = 0; u < lead; ++u) fill(u, u);
+
+    // --- read side ---
+    const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((wide::lds_u8*)ring));
+    const uint32_t xa = base + i * 128 + 16 * ((2 * c) ^ (i >> 1));
+    const uint32_t wa = base + U::kX + (Q4 ? i * 32 + 16 * ((c >> 1) ^ (i >> 3)) + 8 * (c & 1) : i * 64 + 16 * (c ^ (i >> 2)));
+    const uint32_t sa = base + U::kX + U::kW + i * 4;
+    floatx4 acc[MT][S];
+    #pragma unroll
+    for (int t = 0; t < MT; ++t)
+        #pragma unroll
+        for (int s = 0; s < S; ++s) acc[t][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    int slot = 0;
+    for (int u = 0; u < n; ++u) {
+        const int issued = u + ring_units < n ? u + ring_units : n;
+        wait_for_all_but<U::kLoads>(issued - u - 1);
+        UnitFrags<KIND, MT, S> F;
+        const uint32_t at = slot * U::kBytes;
+        F.read(xa + at, (xa + at) ^ 16u, wa + at, sa + at);
+        if (u + ring_units < n) fill(u + ring_units, slot);
+        slot = slot + 1 == ring_units ? 0 : slot + 1;
+        #pragma unroll
+        for (int s = 0; s < S; ++s) {
+            half8 a[TERMS][2];
+            if constexpr (F16) {
+                a[0][0] = __builtin_bit_cast(half8, F.w[s][0]);
+                a[0][1] = __builtin_bit_cast(half8, F.w[s][1]);
+            } else if constexpr (Q4) {
+                const uint32_t both = __builtin_amdgcn_perm(0u, F.ws[s], c >> 1 ? 0x03020302u : 0x01000100u);
+                __half2 st[TERMS];
+                if constexpr (TERMS == 2) {
+                    st[0] = __builtin_bit_cast(__half2, both & 0xFFF0FFF0u);
+                    st[1] = __hsub2(__builtin_bit_cast(__half2, both), st[0]);
+                } else {
+                    st[0] = __builtin_bit_cast(__half2, both);
                 }
                 #pragma unroll
-                for (int v = 0; v < WV; ++v)
-                    wb[b][u][v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                        wp + (mine ? static_cast<ptrdiff_t>(it) * 64 * kWB : -static_cast<ptrdiff_t>(c) * 16 * WV)) + v);
-                if constexpr (Q4) sb[b][u] = sp[mine ? 4 * it : -c];
+                for (int e = 0; e < 2; ++e)
+                    #pragma unroll
+                    for (int z = 0; z < TERMS; ++z)
+                        a[z][e] = __builtin_bit_cast(half8, u32x4{q4x2_to_h2<0>(F.w4[s][e], st[z]), q4x2_to_h2<1>(F.w4[s][e], st[z]),
+                                                                  q4x2_to_h2<2>(F.w4[s][e], st[z]), q4x2_to_h2<3>(F.w4[s][e], st[z])});
+            } else {
+                uint32_t h[8];
+                #pragma unroll
+                for (int d = 0; d < 4; ++d) i8x4_to_h4(F.w[s][0][d], h[2 * d], h[2 * d + 1]);
+                a[0][0] = __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
+                a[0][1] = __builtin_bit_cast(half8, u32x4{h[4], h[5], h[6], h[7]});
             }
-        };
-        auto multiply = [&](int b, int j0) {
             #pragma unroll
-            for (int u = 0; u < kChunk; ++u) {
-                const int it = j0 + u;
-                if (it < it1) {
-                    [[maybe_unused]] const bool mine = !Q4 || kItK * it + 32 * c < K;
-                    half8 xf[MT][XE];
+            for (int z = 0; z < TERMS; ++z)
+                #pragma unroll
+                for (int e = 0; e < 2; ++e)
                     #pragma unroll
                     for (int t = 0; t < MT; ++t)
-                        #pragma unroll
-                        for (int e = 0; e < XE; ++e) {
-                            if constexpr (XL)
-                                xf[t][e] = *reinterpret_cast<const half8*>(
-                                    lds + xl + 16u * t * xrow + (mine ? it * (2 * kItK) : -c * (16 * XE)) + 16 * e);
-                            else
-                                xf[t][e] = __builtin_bit_cast(half8, xb[b][u][t][e]);
-                        }
-                    half8 a[TERMS][XE];
-                    if constexpr (F16) {
-                        a[0][0] = __builtin_bit_cast(half8, wb[b][u][0]);
-                        a[0][1] = __builtin_bit_cast(half8, wb[b][u][1]);
-                    } else if constexpr (Q4) {
-                        // a lane that sits the iteration out multiplies by a scale of zero
-                        const uint32_t s1 = mine ? sb[b][u] : 0u;
-                        const uint32_t sboth = s1 | (s1 << 16);
-                        __half2 st[TERMS];
-                        if constexpr (TERMS == 2) {
-                            st[0] = __builtin_bit_cast(__half2, sboth & 0xFFF0FFF0u);
-                            st[1] = __hsub2(__builtin_bit_cast(__half2, sboth), st[0]);
-                        } else {
-                            st[0] = __builtin_bit_cast(__half2, sboth);
-                        }
-                        #pragma unroll
-                        for (int e = 0; e < XE; ++e) {
-                            const uint32_t v = wb[b][u][0][e];
-                            #pragma unroll
-                            for (int z = 0; z < TERMS; ++z)
-                                a[z][e] = __builtin_bit_cast(half8, u32x4{q4x2_to_h2<0>(v, st[z]), q4x2_to_h2<1>(v, st[z]),
-                                                                          q4x2_to_h2<2>(v, st[z]), q4x2_to_h2<3>(v, st[z])});
-                        }
-                    } else {
-                        uint32_t h[8];
-                        i8x4_to_h4(wb[b][u][0].x, h[0], h[1]);
-                        i8x4_to_h4(wb[b][u][0].y, h[2], h[3]);
-                        i8x4_to_h4(wb[b][u][0].z, h[4], h[5]);
-                        i8x4_to_h4(wb[b][u][0].w, h[6], h[7]);
-                        a[0][0] = __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
-                        a[0][1] = __builtin_bit_cast(half8, u32x4{h[4], h[5], h[6], h[7]});
-                    }
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        #pragma unroll
-                        for (int z = 0; z < TERMS; ++z)
-                            #pragma unroll
-                            for (int e = 0; e < XE; ++e)
-                                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][e], xf[t][e], acc[t], 0, 0, 0);
-                }
-            }
-        };
-        // buffers 0 and 1 in turn while two more whole chunks lie ahead; then what is left (one
-        // buffer that may be on its way already, and at most one more chunk)
-        int j0 = it0, cur = 0;
-        if (it1 - j0 >= 2 * kChunk) {
-            fetch(std::true_type{}, 0, j0);
-            while (true) {
-                fetch(std::true_type{}, 1, j0 + kChunk);
-                multiply(0, j0);
-                j0 += kChunk;
-                if (it1 - j0 < 2 * kChunk) { cur = 1; break; }
-                fetch(std::true_type{}, 0, j0 + kChunk);
-                multiply(1, j0);
-                j0 += kChunk;
-                if (it1 - j0 < 2 * kChunk) { cur = 0; break; }
-            }
-        } else {
-            fetch(std::false_type{}, 0, j0);
+                        acc[t][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][e], __builtin_bit_cast(half8, F.x[t][e]), acc[t][s], 0, 0, 0);
         }
-        if (cur == 0) {
-            fetch(std::false_type{}, 1, j0 + kChunk);
-            multiply(0, j0);
-            multiply(1, j0 + kChunk);
-        } else {
-            fetch(std::false_type{}, 0, j0 + kChunk);
-            multiply(1, j0);
-            multiply(0, j0 + kChunk);
-        }
+    }
 
-        // The slices' sums meet in LDS; tile t of the strip is then finished by the strip's wavefront t mod ks, which
-        // adds them in slice order (one wavefront for all tiles reads 7 x 16 values one after the other at 64 rows: a
-        // 0.5B layer of such int8 rows 35.5 us against 34.3).
-        if (ks > 1) {                                    // (the same for every wavefront of the block)
-            __syncthreads();                             // the last round's sums have been read
-            #pragma unroll
-            for (int t = 0; t < MT; ++t) red[(wave * MT + t) * 64 + lane] = acc[t];
-            __syncthreads();
-        }
-        const int nq = 16 * group + 4 * c;               // first of this lane's 4 output columns
-        float s4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-        if constexpr (KIND == WK_I8) {
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) s4[r] = h_f(scale[nq + r < N ? nq + r : N - 1]);
-        }
-        [[maybe_unused]] uint2 h[MT];
+    // The slices' sums meet in LDS, each where its wavefront's ring was; sum t S + s of the tile (GLU: both sums of rows t) is
+    // then finished by the tile's wavefront of that number mod ks, which adds them in slice order.
+    auto sums_of = [&](int w) { return reinterpret_cast<floatx4*>(lds + static_cast<size_t>(w) * ring_units * U::kBytes); };
+    if (ks > 1) {                                        // (the same for every wavefront of the block)
         #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            if ((t & (ks - 1)) != slice) continue;
+        for (int t = 0; t < MT; ++t)
+            #pragma unroll
+            for (int s = 0; s < S; ++s) sums_of(wave)[(t * S + s) * 64 + lane] = acc[t][s];
+        __syncthreads();
+    }
+    if (!live) return;
+    const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+    #pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        [[maybe_unused]] uint2 h[S];
+        #pragma unroll
+        for (int s = 0; s < S; ++s) {
+            if (((GLU ? t : t * S + s) & (ks - 1)) != slice) continue;
+            const int strip = tile * S + s;
+            if (16 * strip >= N) continue;
+            floatx4 v = acc[t][s];
             if (ks > 1) {
-                acc[t] = red[((wave - slice) * MT + t) * 64 + lane];
+                v = sums_of(wave - slice)[(t * S + s) * 64 + lane];
                 for (int z = 1; z < ks; ++z) {
-                    const floatx4 v = red[((wave - slice + z) * MT + t) * 64 + lane];
+                    const floatx4 o = sums_of(wave - slice + z)[(t * S + s) * 64 + lane];
                     #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[t][r] += v[r];
+                    for (int r = 0; r < 4; ++r) v[r] += o[r];
                 }
             }
+            const int nq = 16 * strip + 4 * c, m = 16 * t + i;           // first of this lane's 4 output columns, its row
             if constexpr (MEET) {
-                if (kb > 1 &&
-                    !meet_slices(acc[t], partial + (static_cast<size_t>(group) * MT + t) * kb * 256, counters + group * MT + t, by, kb, lane))
+                if (kb > 1 && !meet_slices(v, partial + (static_cast<size_t>(strip) * MT + t) * kb * 256, counters + strip * MT + t, by, kb, lane))
                     continue;
+            } else if constexpr (!GLU) {
+                if (partial) {                           // (N is a multiple of 4 then)
+                    if (m < M && nq < N) *reinterpret_cast<floatx4*>(partial + (static_cast<size_t>(by) * M + m) * N + nq) = v;
+                    continue;
+                }
             }
-            const uint32_t lo = wide::pack_half2(acc[t][0] * s4[0], acc[t][1] * s4[1]);
-            const uint32_t hi = wide::pack_half2(acc[t][2] * s4[2], acc[t][3] * s4[3]);
+            if constexpr (KIND == WK_I8) {
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] *= h_f(static_cast<uint16_t>(sc[s][r]));
+            }
+            const uint32_t lo = wide::pack_half2(v[0], v[1]), hi = wide::pack_half2(v[2], v[3]);
             if constexpr (GLU) {
-                h[t] = uint2{lo, hi};
+                h[s] = uint2{lo, hi};
                 continue;
             }
-            const int m = 16 * t + i;
             if (m >= M || nq >= N) continue;
             uint16_t* dst = out + static_cast<size_t>(m) * N + nq;
             if (cols4 && nq + 3 < N) {
@@ -1605,98 +1633,82 @@ __device__ __forceinline__ void skinny_rows(const uint16_t* __restrict__ X, cons
             }
         }
         if constexpr (GLU) {
-            // odd strips belong to the up matrix, the strip below to the same columns of the gate matrix (see
-            // launch_gemm_glu) and to the wavefronts before these: the up values cross through LDS
-            __syncthreads();                             // the sums have been read
-            uint2* cross = reinterpret_cast<uint2*>(red);
-            #pragma unroll
-            for (int t = 0; t < MT; ++t)
-                if ((t & (ks - 1)) == slice && group % 2) cross[(wave * MT + t) * 64 + lane] = h[t];
-            __syncthreads();
-            #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const int m = 16 * t + i;
-                if ((t & (ks - 1)) == slice && group % 2 == 0 && nq < N && m < M) {
-                    const uint2 up = cross[((wave + ks) * MT + t) * 64 + lane];
-                    *reinterpret_cast<uint2*>(out + static_cast<size_t>(m) * (N / 2) + 8 * group + 4 * c) =
-                        uint2{swiglu_h2(h[t].x, up.x), swiglu_h2(h[t].y, up.y)};
-                }
-            }
+            if ((t & (ks - 1)) == slice && 16 * t + i < M)
+                *reinterpret_cast<uint2*>(out + static_cast<size_t>(16 * t + i) * (N / 2) + 16 * tile + 4 * c) =
+                    uint2{swiglu_h2(h[0].x, h[1].x), swiglu_h2(h[0].y, h[1].y)};
         }
     }
 }
 
-template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
+template <int KIND, int MT, int S, int TERMS, bool GLU, bool MEET>
 __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
                                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out,
-                                                           int M, int N, int K, int ks, int logical_blocks,
-                                                           float* __restrict__ partial, uint32_t* __restrict__ counters,
-                                                           MoreMats more) {
-    skinny_rows<KIND, MT, XL, TERMS, GLU, MEET>(X, W, scale, out, M, N, K, ks, logical_blocks, partial, counters, more, blockIdx.x,
-                                                    gridDim.x, MEET ? blockIdx.y : 0, MEET ? gridDim.y : 1);
+                                                           int M, int N, int K, int ks, int ring_units, float* __restrict__ partial,
+                                                           uint32_t* __restrict__ counters, MoreMats more) {
+    skinny_tile<KIND, MT, S, TERMS, GLU, MEET>(X, W, scale, out, M, N, K, ks, ring_units, partial, counters, more, blockIdx.x,
+                                               blockDim.x >> 6, blockIdx.y, gridDim.y);
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
-// bytes of LDS a block takes: the rows of x (XL) and the buffer in which K-slices meet
-inline size_t lds_bytes(int mt, int K, bool xl, int ks) {
-    return (xl ? static_cast<size_t>(16) * mt * (2 * static_cast<size_t>(K) + 16) : 0) +
-           (ks > 1 ? static_cast<size_t>(kWaves) * mt * 4 * 64 * 4 : 0);
+inline size_t unit_bytes(int kind, int mt, int S) {      // Unit::kBytes
+    return static_cast<size_t>(mt) * 2048 + (kind == WK_F16 ? S * 2048 : kind == WK_I8 ? S * 1024 : S * 576);
 }
 
 // bytes of partial sums that kb slices of K over blocks leave in the workspace (meet_slices)
 inline size_t partial_bytes(int mt, int N, int kb) { return static_cast<size_t>((N + 15) / 16) * kb * mt * 1024; }
 
-struct Shape { int ks; bool xl; int kb; };
-// Slices of K per strip inside a block (1, 2, 4, 8: the fewest that give the chip four wavefronts
-// per CU; measured at 4864 x 896: 4 slices 4.5 us, 8 slices 6.7 us), x in LDS where it fits, and
-// slices of K over blocks (kb) where one block per strip still leaves most CUs idle and what a
-// single CU can pull bounds the launch (896 x 4864: 56 strips): their sums go through the
-// workspace, where the last block to arrive adds them in order.  One strip per wavefront: two and four were measured slower at every shape tried (fewer wavefronts; the reads of x they
-// save are not the bound).
+// ks: wavefronts that share a tile, the fewest of 4 and 8 that give the chip four wavefronts per CU (4 at least: with two, 9728 x 896 at
+// 16 rows 7.2 us, with four 6.7); 8 only where a ring holds two units then (fp16 at more than 48 rows: 3072 x 576 5.2 us in 4
+// slices, 6.0 in 8).  kb: slices over blocks where one block per tile still leaves most CUs idle and the trip of the sums
+// through memory, 2.5 us, is less than what it saves (896 x 4864 at 16 rows: 8.7 us in 8 slices, 7.1 in 8 x 4).  S: two
+// strips per wavefront where one per wavefront is more blocks than CUs: x is fetched half as often (4864 x 896 at 48 int8 rows
+// 6.7 -> 6.1 us); fewer blocks than CUs with two lose (1152 x 896 at 16 rows 3.7 against 4.1).
+struct Shape { int ks, kb, S; };
 inline Shape pick_shape(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
     const int mt = (M + 15) / 16;
     const long strips = (N + 15) / 16;
-    const int its = kind == WK_Q4 ? (K + 127) / 128 : K / 64;        // iterations over K
-    Shape sh{1, false, 1};
-    while (sh.ks < kWaves && strips * sh.ks < 4L * cus && its >= 2 * sh.ks) sh.ks *= 2;
-    // (a block whose eight wavefronts share one strip reads every byte of x once either way: no LDS then)
-    sh.xl = sh.ks < kWaves && lds_bytes(mt, K, true, sh.ks) <= kLdsLimit;
-    if (sh.ks == kWaves) {
+    const int its = K / 64;
+    Shape sh{1, 1, strips > cus && mt > 1 ? 2 : 1};
+    const long tiles = (strips + sh.S - 1) / sh.S;
+    const int most = 2 * kWaves * unit_bytes(kind, mt, 2) <= kLdsLimit ? kWaves : kWaves / 2;
+    while (sh.ks < most && (sh.ks < 4 || tiles * sh.ks < (sh.S == 2 ? 5L : 4L) * cus) && its >= 2 * sh.ks) sh.ks *= 2;
+    if (sh.ks == most) {
         while (sh.kb < 8 && strips * sh.kb * 2 <= cus && its >= 2 * sh.ks * sh.kb * 2 && strips * mt <= kSliceCounters &&
                partial_bytes(mt, N, 2 * sh.kb) <= workspace_bytes)
             sh.kb *= 2;
     }
     return sh;
 }
-
-// Where the streaming kernel is the library's own choice (measured against the tiles above, warm
-// weights, us).
-//  - With x in LDS, or one strip per block: up to 48 rows (int8 4864 x 896: 4.4 / 5.0 / 5.7 at 16 / 32 / 48
-//    rows against 6.3 to 6.5 for the 64 x 64 tiles, 6.65 against 6.5 at 64; 2560 x 1024: 4.4 / 5.4 / 6.5
-//    against 8.2 to 9.1); up to 64 where K is cut over blocks as well (896 x 4864: 6.9 / 8.0 / 10.5 at 16 /
-//    32 / 64 rows against 25 and more unsliced, 12 to 14 as the wide kernel was chosen in slices).
-//  - x in LDS, Q4 or fp16 weights of a few MB: up to 64 rows (Q4 4864 x 896 at 64 rows 8.55 against
-//    11.8 for the wide kernel, 9728 x 896 10.5 against 12.4; fp16 4864 x 896 7.5 against 8.0).
-//  - x from the caches and shared by several strips per block: only up to 16 rows (8192 x 2048 at 48
-//    rows: 28 us against 17).  Q4 then holds twice the x per iteration in registers: one strip per
-//    block is good for 48 rows (2560 x 1024: 7.5 against 10.7, 3072 x 1024: 7.6 against 10.9), K over
-//    blocks as well for 32 (896 x 4864: 10.3 / 14.0 / 26.5 at 32 / 48 / 64 rows against 12.7 to 12.9).
-//  - No more than 13.5 MB of weights: beyond that the launch is long enough for the wide kernel's
-//    higher streaming rate to win (a wavefront here loads a strip, waits, multiplies).  int8 14 592 x
-//    896 (13.1 MB) 6.4 / 7.0 / 7.9 at 16 / 32 / 48 rows against 8.5, but 19 456 x 896 8.8 / 9.6 / 10.5 against
-//    8.6 / 8.7 / 9.0, 49 152 x 576 11.2 against 7.3 and fp16 49 152 x 576 16.7 against 10.8; an lm_head of
-//    151 936 rows streams at 4.0 TB/s here against 4.8 TB/s there.
-inline bool preferred(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
-    const Shape sh = pick_shape(kind, M, N, K, cus, workspace_bytes);
-    const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
-    int rows = sh.xl || sh.ks == kWaves ? (sh.kb > 1 ? 64 : 48) : 16;
-    if (kind == WK_Q4 && !sh.xl) rows = sh.ks == kWaves && sh.kb == 1 ? 48 : rows > 32 ? 32 : rows;
-    if (kind == WK_F16 && rows == 48) rows = 56;         // (fp16 2560 x 1024 at 49 / 56 rows: 7.45 / 7.7 against 9.4 / 8.8 us)
-    if (kind != WK_I8 && sh.xl && w_bytes <= (kind == WK_Q4 ? 6.0e6 : 9.0e6)) rows = 64;
-    return M <= rows && w_bytes <= 13.5e6 && (N + 15) / 16 <= 16L * cus;
+// The slices of a launch whose sums another launch adds: as many over blocks as give every CU one, 4 in a block (us at kb = 1 /
+// these / twice as many: fp16, 37 rows of 960 x 2560 8.8 / 4.9 / 5.0, 960 x 960 4.6 / 3.6 / 3.8, int8, 16 rows of 896 x 4864 8.9 / 4.6 / 4.5).
+// kb = 1: none, the launch would save nothing.
+inline Shape pick_apart(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
+    const long strips = (N + 15) / 16;
+    const int its = K / 64;
+    Shape sh{4, 1, 1};
+    while (sh.kb < 8 && strips * (sh.kb + 1) <= cus && its >= sh.ks * (sh.kb + 1) &&
+           static_cast<size_t>(sh.kb + 1) * M * N * 4 <= workspace_bytes)
+        ++sh.kb;
+    return sh;
 }
 
-// Estimated time (us), fitted to the same measurements.
+// Where the streaming kernel is the library's own choice, against the tiles above (us, weights from HBM).
+//  - Up to 64 rows: 2560 x 1024 at 24 / 40 / 64 rows 4.4 / 4.7 / 5.2 (fp16 5.0 / 5.6 / 6.2) against 8.7 to 9.6 for the 64 x 64 tiles, 896 x
+//    4864 at 64 fp16 rows 9.1 against 14 (the wide kernel in slices), 8192 x 2048 12.6 against 16.2.  (int8 of a K up to 512
+//    only to 48 rows, a plan that is promised, though 1024 x 512 at 64 takes 4.1 against 5.9.)
+//  - fp16 of more than 8192 rows of W only up to 32: 9728 x 896 at 32 / 48 / 64 rows 8.5 / 9.6 / 10.5 against 8.8 / 9.3 / 9.7 (the tiles fetch
+//    x once per 64 rows of W); int8 9728 x 896 at 48 8.5 against 8.8, 19 456 x 896 11.2 against 11.5.
+//  - Not beyond 36 MB of weights or 80 rows of W per CU: the wide kernel's higher streaming rate wins there (int8 49 152 x 576 at
+//    16 rows 11.2 against 7.3).
+inline bool preferred(int kind, int M, int N, int K, int cus) {
+    const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
+    const long strips = (N + 15) / 16;
+    return M <= (kind == WK_I8 && K <= 512 ? 48 : kind == WK_F16 && strips > 2L * cus ? 32 : 64) && w_bytes <= 36.0e6 && strips <= 5L * cus;
+}
+
+// Estimated time (us): what decides between this kernel and rows of GEMV below 16 rows.  (Fitted to the kernel that took
+// fragments from memory, and 0.3 to 1 us too high: a line that moved would take prompts of a few tokens off the reference's
+// order, in which their attention goes with the projections.)
 inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
     const Shape sh = pick_shape(kind, M, N, K, cus, workspace_bytes);
     const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
@@ -1705,7 +1717,8 @@ inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspa
     // (x from the caches: 0.07 us per row where several strips of a block read it, 0.03 where the block's
     //  eight wavefronts share one strip, 0.06 with K over blocks as well)
     const double xg_us = sh.kb > 1 ? 5.4 + 0.06 * M : sh.ks == kWaves ? 3.6 + 0.03 * M : 3.6 + 0.07 * M;
-    return q4_us + (sh.xl ? 3.75 + 0.035 * M : xg_us) + w_bytes / 8.0e6;
+    // (more than 13.5 MB: 19 456 x 896 at 8 int8 rows 8.6)
+    return q4_us + (sh.ks < kWaves ? 3.75 + 0.035 * M : xg_us) + w_bytes / 8.0e6 + (w_bytes > 13.5e6 ? 2.4 : 0.0);
 }
 
 // ---- calls that share no x, in one launch ----
@@ -1713,10 +1726,11 @@ inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspa
 // Calls of a batch that cannot observe one another's results (the batch's host code checks that) and that the streaming
 // kernel serves, each as its own plan has it (the same slices of K in the same order: the same bits as a launch of its
 // own), a block per call and group of strips.  A launch of a few hundred rows of W takes 4 to 5 us whatever its size:
-// the seven int8 projections of a 0.5B layer at 16 rows, four launches and one for the slices' sums, 26.6 -> 14.0 us.
+// the seven int8 projections of a 0.5B layer at 16 rows, four launches and one for the slices' sums, 26.6 -> 14.0 us (7.5 since
+// the kernel loads by rows).
 constexpr int kMaxManyGemm = 32;
 struct SkinnyCalls {
-    int n = 0, M = 0;
+    int n = 0, M = 0, ring = 1;
     uint16_t first[kMaxManyGemm] = {};                   // a call's first block
     struct Call {
         const uint16_t* X;
@@ -1725,9 +1739,9 @@ struct SkinnyCalls {
         uint16_t* out;
         float* partial;
         uint32_t* counters;
-        int N, K, logical;
+        int N, K;
         uint16_t blocks;                                 // blocks along N; kb times as many in all
-        uint8_t ks_xl, kb;                               // slices inside a block, + 16 with x in LDS; slices over blocks
+        uint8_t ks, kb;                                  // slices inside a block and over blocks
     } c[kMaxManyGemm] = {};
 };
 static_assert(sizeof(SkinnyCalls) <= 4096, "kernel arguments");
@@ -1739,82 +1753,72 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny_many(const SkinnyCall
     const int lane = threadIdx.x & 63, n = L->n, b = blockIdx.x;
     const int mine = L->first[lane < kMaxManyGemm ? lane : 0];
     const int q = __popcll(__ballot(lane < n && b >= mine)) - 1;
-    const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb, ks_xl = L->c[q].ks_xl, ks = ks_xl & 15;
-    const int by = kb > 1 ? at / blocks : 0;
+    const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb, by = kb > 1 ? at / blocks : 0;
     const MoreMats none{};
-    const uint16_t *X = L->c[q].X, *scale = L->c[q].scale;
-    const uint8_t* W = L->c[q].W;
-    uint16_t* out = L->c[q].out;
-    float* partial = L->c[q].partial;
-    uint32_t* counters = L->c[q].counters;
-    const int N = L->c[q].N, K = L->c[q].K, logical = L->c[q].logical, M = L->M;
-    if (ks_xl & 16)
-        skinny_rows<KIND, MT, true, TERMS, false, false>(X, W, scale, out, M, N, K, ks, logical, nullptr, nullptr, none, at, blocks, 0, 1);
-    else
-        skinny_rows<KIND, MT, false, TERMS, false, true>(X, W, scale, out, M, N, K, ks, logical, partial, counters, none, at - by * blocks, blocks, by, kb);
+    skinny_tile<KIND, MT, 1, TERMS, false, true>(L->c[q].X, L->c[q].W, L->c[q].scale, L->c[q].out, L->M, L->c[q].N, L->c[q].K, L->c[q].ks,
+                                                 L->ring, L->c[q].partial, L->c[q].counters, none, at - by * blocks, kWaves, by, kb);
 }
 
-// Shapes whose blocks hold a strip of the gate matrix and its strip of the up matrix, and LDS for them to meet in
-inline bool glu_shape(const Shape& sh) { return sh.kb == 1 && (sh.ks == 2 || sh.ks == 4); }
-
-// Blocks along N for `logical` groups of strips.  With x in LDS a block is worth keeping: as many as fit a CU at once
-// (by LDS; at most 4), each walking over the groups.
-inline long blocks_along_n(bool xl, long logical, size_t lds) {
-    if (!xl) return logical;
-    const long per_cu = lds == 0 ? 4 : static_cast<long>(kLdsLimit / lds) < 4 ? static_cast<long>(kLdsLimit / lds) : 4;
-    const long resident = static_cast<long>(device_info().cus) * (per_cu < 1 ? 1 : per_cu);
-    return logical > resident ? resident : logical;
+// Units of K in a wavefront's ring: its whole slice where `per_cu` such blocks fit the LDS of a CU.
+inline int ring_units(size_t unit, int waves, long per_cu, int K, int ks, int kb) {
+    const int its = (K / 64 + kb - 1) / kb, most = (its + ks - 1) / ks;
+    int ring = static_cast<int>(kLdsLimit / static_cast<size_t>(per_cu < 1 ? 1 : per_cu > 4 ? 4 : per_cu) / (waves * unit));
+    if (ring > kMaxRing) ring = kMaxRing;
+    if (ring > most) ring = most;
+    return ring < 1 ? 1 : ring;
 }
 
-template <int KIND, int MT, bool XL, int TERMS, bool GLU, bool MEET>
+template <int KIND, int MT, int S, int TERMS, bool GLU, bool MEET>
 bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-                float* partial, const MoreMats& more) {
-    const int ks = sh.ks;
-    const long groups = more.n ? more.tiles : (N + 15) / 16, per_block = kWaves / ks;
-    const long logical = (groups + per_block - 1) / per_block;
-    const size_t lds = lds_bytes(MT, K, XL, ks);
-    auto* kern = gemm_skinny<KIND, MT, XL, TERMS, GLU, MEET>;
+                float* partial, uint32_t* counters, const MoreMats& more) {
+    const int ks = sh.ks, waves = ks < 4 ? 4 : ks;
+    const long tiles = more.n ? more.tiles : (N + 16 * S - 1) / (16 * S), per_block = waves / ks;
+    const long blocks = (tiles + per_block - 1) / per_block;
+    const int cus = device_info().cus;
+    constexpr size_t unit = Unit<KIND, MT, S>::kBytes;
+    const int ring = ring_units(unit, waves, (blocks * sh.kb + cus - 1) / cus, K, ks, sh.kb);
+    const size_t lds = waves * ring * unit;
+    auto* kern = gemm_skinny<KIND, MT, S, TERMS, GLU, MEET>;
     if (lds > 65536 &&
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
         return false;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks_along_n(XL, logical, lds)), static_cast<unsigned>(sh.kb)),
-                       dim3(64 * kWaves), lds, s, static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W),
-                       static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(out), M, N, K, ks, static_cast<int>(logical),
-                       sh.kb > 1 ? partial : nullptr, sh.kb > 1 ? slice_counters(partial) : nullptr, more);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(sh.kb)), dim3(64 * waves), lds, s,
+                       static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
+                       static_cast<uint16_t*>(out), M, N, K, ks, ring, partial, counters, more);
     return MI_HIP_OK(hipGetLastError());
 }
 
+// glu, or sums for another launch (`apart`), or neither
 template <int KIND, int MT, int TERMS>
 bool launch_mt(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-               float* partial, const MoreMats& more, bool glu) {
-    if (glu)
-        return sh.xl ? launch_one<KIND, MT, true, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                     : launch_one<KIND, MT, false, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
-    if (sh.kb > 1) return launch_one<KIND, MT, false, TERMS, false, true>(s, M, N, K, x, W, scale, out, sh, partial, more);
-    return sh.xl ? launch_one<KIND, MT, true, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, partial, more)
-                 : launch_one<KIND, MT, false, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, partial, more);
+               float* partial, const MoreMats& more, bool glu, bool apart) {
+    if (glu) return launch_one<KIND, MT, 2, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, nullptr, nullptr, more);
+    if (sh.kb > 1 && !apart)
+        return launch_one<KIND, MT, 1, TERMS, false, true>(s, M, N, K, x, W, scale, out, sh, partial, slice_counters(partial), more);
+    float* sums = apart ? partial : nullptr;
+    return sh.S == 2 ? launch_one<KIND, MT, 2, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, sums, nullptr, more)
+                     : launch_one<KIND, MT, 1, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, sums, nullptr, more);
 }
 
 template <int KIND, int TERMS>
 bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, Shape sh,
-            void* workspace, size_t workspace_bytes, const MoreMats& more, bool glu) {
-    if (M < 1 || M > kMaxM || !(sh.ks == 1 || sh.ks == 2 || sh.ks == 4 || sh.ks == 8) ||
-        lds_bytes((M + 15) / 16, K, sh.xl, sh.ks) > kLdsLimit || sh.kb < 1 || (sh.kb > 1 && (sh.xl || more.n)) ||
-        (glu && !glu_shape(sh)) ||
-        (sh.kb > 1 && (sh.ks != kWaves || !workspace || partial_bytes((M + 15) / 16, N, sh.kb) > workspace_bytes ||
+            void* workspace, size_t workspace_bytes, const MoreMats& more, bool glu, bool apart = false) {
+    if (M < 1 || M > kMaxM || !(sh.ks == 1 || sh.ks == 2 || sh.ks == 4 || sh.ks == 8) || sh.kb < 1 || (sh.kb > 1 && more.n) ||
+        (glu && sh.kb > 1) || (apart && (!workspace || static_cast<size_t>(sh.kb) * M * N * 4 > workspace_bytes)) ||
+        (sh.kb > 1 && !apart && (!workspace || partial_bytes((M + 15) / 16, N, sh.kb) > workspace_bytes ||
                        (N + 15) / 16 * ((M + 15) / 16) > kSliceCounters))) {
-        MI_ERROR_FMT("gemm: the streaming kernel takes up to %d rows of x, 1, 2, 4 or 8 slices of K per block, %zu bytes of LDS "
-                     "and a workspace for slices over blocks (M=%d K=%d, %d slices, x in LDS %d, %d slices over blocks, %zu bytes)",
-                     kMaxM, kLdsLimit, M, K, sh.ks, static_cast<int>(sh.xl), sh.kb, workspace_bytes);
+        MI_ERROR_FMT("gemm: the streaming kernel takes up to %d rows of x, 1, 2, 4 or 8 slices of K per block "
+                     "and a workspace for slices over blocks (M=%d K=%d, %d slices, %d slices over blocks, %zu bytes)",
+                     kMaxM, M, K, sh.ks, sh.kb, workspace_bytes);
         return false;
     }
     auto* partial = static_cast<float*>(workspace);
     switch ((M + 15) / 16) {
-        case 1: return launch_mt<KIND, 1, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
-        case 2: return launch_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
-        case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
-        default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu);
+        case 1: return launch_mt<KIND, 1, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
+        case 2: return launch_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
+        case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
+        default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
     }
 }
 
@@ -1840,49 +1844,41 @@ bool launch_calls_mt(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_
 }
 
 // n calls of one M <= kMaxM and weight kind in as few launches as hold them.  Calls whose slices meet in memory go
-// first, so that their last blocks' trips run under the others' work.  A launch takes the LDS of the call that needs
-// most, for all its blocks: calls of more than half a CU's (x of many rows in LDS) share launches of their own, with
-// no more blocks than the chip holds at once, dealt out to the calls by their strips: a block is then worth its copy of
-// x (a 0.5B layer's calls at 37 / 64 Q4 rows 34.6 / 39.8 -> 24.4 / 29.5 us; gate and up at 64 fp16 rows with a block per two strips, more
-// than fit at once, made the layer 41.8 us instead of 39.7).
+// first, so that their last blocks' trips run under the others' work.
 bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* workspace, size_t workspace_bytes) {
     const int M = calls[0].M, mt = (M + 15) / 16;
     const WeightKind kind = calls[0].kind;
+    const size_t unit = unit_bytes(kind, mt, 1);
     SkinnyCalls L;
     long blocks = 0;
-    size_t lds = 0, sums = 0;
+    size_t sums = 0;
     int counters = 0;
     auto flush = [&]() {
         if (L.n == 0) return true;
         L.M = M;
+        const int cus = device_info().cus;
+        for (int j = 0; j < L.n; ++j) {
+            const int ring = ring_units(unit, kWaves, (blocks + cus - 1) / cus, L.c[j].K, L.c[j].ks, L.c[j].kb);
+            if (ring > L.ring) L.ring = ring;
+        }
         const auto nb = static_cast<unsigned>(blocks);
+        const size_t lds = kWaves * L.ring * unit;
         const bool ok = kind == WK_Q4 ? (terms == 1 ? launch_calls_mt<WK_Q4, 1>(s, L, nb, lds) : launch_calls_mt<WK_Q4, 2>(s, L, nb, lds))
                       : kind == WK_F16 ? launch_calls_mt<WK_F16, 1>(s, L, nb, lds) : launch_calls_mt<WK_I8, 1>(s, L, nb, lds);
         L = SkinnyCalls{};
         blocks = 0;
-        lds = sums = 0;
+        sums = 0;
         counters = 0;
         return ok;
     };
-    long crowd = 0;                                      // blocks the calls of much LDS would like
-    auto is_big = [&](size_t need) { return need > kLdsLimit / 2; };
-    for (int i = 0; i < n; ++i) {
-        const Shape sh = pick_shape(kind, M, calls[i].N, calls[i].K, device_info().cus, workspace_bytes);
-        const long strips = (calls[i].N + 15) / 16, per_block = kWaves / sh.ks;
-        if (is_big(lds_bytes(mt, calls[i].K, sh.xl, sh.ks))) crowd += (strips + per_block - 1) / per_block;
-    }
-    for (int pass = 0; pass < 3; ++pass) {               // slices over blocks; the others; those of much LDS
-        if (pass == 2 && !flush()) return false;
+    for (int pass = 0; pass < 2; ++pass) {               // slices over blocks; the others
         for (int i = 0; i < n; ++i) {
             const GemvCall& c = calls[i];
             const Shape sh = pick_shape(kind, M, c.N, c.K, device_info().cus, workspace_bytes);
-            const size_t need = lds_bytes(mt, c.K, sh.xl, sh.ks);
-            if (pass != (is_big(need) ? 2 : sh.kb > 1 ? 0 : 1)) continue;
-            const int strips = (c.N + 15) / 16, per_block = kWaves / sh.ks, logical = (strips + per_block - 1) / per_block;
-            long along_n = blocks_along_n(sh.xl, logical, need);
-            if (pass == 2 && crowd > device_info().cus) along_n = (static_cast<long>(logical) * device_info().cus + crowd - 1) / crowd;
-            const long nb = along_n * sh.kb;
-            if (need > kLdsLimit || nb > 65535) {
+            if (pass != (sh.kb > 1 ? 0 : 1)) continue;
+            const int strips = (c.N + 15) / 16, per_block = kWaves / sh.ks;
+            const long along_n = (strips + per_block - 1) / per_block, nb = along_n * sh.kb;
+            if (nb > 65535) {
                 MI_ERROR_FMT("gemm: a call beyond a launch of several (M=%d N=%d K=%d)", M, c.N, c.K);
                 return false;
             }
@@ -1896,9 +1892,9 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
             d.W = static_cast<const uint8_t*>(c.W);
             d.scale = static_cast<const uint16_t*>(c.scale);
             d.out = static_cast<uint16_t*>(c.y);
-            d.N = c.N; d.K = c.K; d.logical = logical;
+            d.N = c.N; d.K = c.K;
             d.blocks = static_cast<uint16_t>(along_n);
-            d.ks_xl = static_cast<uint8_t>(sh.ks + (sh.xl ? 16 : 0));
+            d.ks = static_cast<uint8_t>(sh.ks);
             d.kb = static_cast<uint8_t>(sh.kb);
             if (bytes) {
                 d.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + sums);
@@ -1908,7 +1904,6 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
             }
             L.first[L.n++] = static_cast<uint16_t>(blocks);
             blocks += nb;
-            if (need > lds) lds = need;
         }
     }
     return flush();
@@ -1991,7 +1986,7 @@ double gemm_estimate_us(WeightKind kind, int M, int N, int K, size_t workspace_b
     int tm = 1, splits = 1;
     if (wide_reaches(kind, M, N, K))
         wide::pick_shape(kind, terms, M, N, K, device_info().cus, workspace_bytes, &tm, &splits, &wide_us);
-    if (M <= skinny::kMaxM && skinny::preferred(kind, M, N, K, device_info().cus, workspace_bytes))
+    if (M <= skinny::kMaxM && skinny::preferred(kind, M, N, K, device_info().cus))
         return skinny::estimate_us(kind, M, N, K, device_info().cus, workspace_bytes);
     if (kind == WK_Q4) return wide_us;
     const double tiled_us = tiled_estimate_us(M, N, K);
@@ -2015,7 +2010,7 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         // two fp16 terms.
         if (mode == 2) return p;
         p.terms = mode == 4 ? 1 : 2;
-        if (M <= skinny::kMaxM && (mode == 5 || ((mode == 0 || mode == 4) && skinny::preferred(WK_Q4, M, N, K, cus, workspace_bytes)))) {
+        if (M <= skinny::kMaxM && (mode == 5 || ((mode == 0 || mode == 4) && skinny::preferred(WK_Q4, M, N, K, cus)))) {
             const skinny::Shape sh = skinny::pick_shape(WK_Q4, M, N, K, cus, workspace_bytes);
             p.kernel = 4; p.tile_rows = 16 * ((M + 15) / 16); p.k_slices = sh.ks * sh.kb;
             return p;
@@ -2042,7 +2037,7 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
     }
     if (mode == 30) return p;
     // int8 and fp16, a few rows of x: the streaming kernel (mode 5 asks for it by name, up to 64 rows)
-    if (M <= skinny::kMaxM && (mode == 5 || (mode == 0 && skinny::preferred(kind, M, N, K, cus, workspace_bytes)))) {
+    if (M <= skinny::kMaxM && (mode == 5 || (mode == 0 && skinny::preferred(kind, M, N, K, cus)))) {
         const skinny::Shape sh = skinny::pick_shape(kind, M, N, K, cus, workspace_bytes);
         p.kernel = 4; p.tile_rows = 16 * ((M + 15) / 16); p.k_slices = sh.ks * sh.kb;
         return p;
@@ -2132,7 +2127,7 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
     const size_t ws_bytes = workspace ? workspace_bytes : 0;
     const GemmPlan p = plan_gemm(s, kind, M, N, K, ws_bytes);
     if (!(p.kernel == 1 ||
-          (p.kernel == 4 && skinny::glu_shape(skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes)))))
+          (p.kernel == 4 && skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes).kb == 1)))
         return 0;
     return launch_planned(s, p, kind, M, N, K, x, W, scale, out, workspace, ws_bytes, MoreMats{}, true) ? 1 : -1;
 }
@@ -2148,6 +2143,18 @@ int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, cons
     if (!workspace || !gemm_supported(kind, M, N, K, x, W, scale)) return 0;
     GemmPlan p = plan_gemm(s, kind, M, N, K, workspace_bytes);
     const int mode = gemm_mode(s);
+    // (a few rows: the streaming kernel's own slices, whatever the plan for a launch by itself.  Prompts of 10 / 24 / 37 / 64
+    //  tokens, int8 0.5B, int8 360M, fp16 360M, int8 0.5B, with its new loads in all: 973 / 1354 / 1514 / 1338 -> 927 / 1186 / 1208 / 1104 us)
+    if (M <= skinny::kMaxM && (mode == 0 || mode == 4)) {
+        const skinny::Shape sh = skinny::pick_apart(kind, M, N, K, device_info().cus, workspace_bytes);
+        if (sh.kb > 1) {
+            const bool ok = kind == WK_Q4 ? (p.terms == 1 ? skinny::launch<WK_Q4, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true)
+                                                          : skinny::launch<WK_Q4, 2>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true))
+                          : kind == WK_F16 ? skinny::launch<WK_F16, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true)
+                                           : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true);
+            return ok ? sh.kb : -1;
+        }
+    }
     if (p.kernel >= 1 && p.kernel <= 3 && p.k_slices == 1 && (mode == 0 || mode == 4) && wide_reaches(kind, M, N, K)) {
         const int terms = kind == WK_Q4 ? p.terms : 1;
         const int cus = device_info().cus;
@@ -2177,7 +2184,7 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
     skinny::Shape sh{};
     if (p.kernel == 4) sh = skinny::pick_shape(kind, M, mat[0].N, K, cus, ws_bytes);
     if (!(p.kernel == 2 || p.kernel == 3 || (p.kernel == 1 && p.k_slices == 1) || (p.kernel == 4 && sh.kb == 1))) return 0;
-    const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : 16;
+    const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : 16 * sh.S;
     auto tiles_of = [&](int N) { return N / width + (N % width != 0); };
     MoreMats more;
     more.tiles = tiles_of(mat[0].N);
@@ -2189,7 +2196,7 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
         if (q.kernel != p.kernel || q.terms != p.terms || q.k_slices != p.k_slices) break;
         if (p.kernel == 4) {
             const skinny::Shape t = skinny::pick_shape(kind, M, c.N, K, cus, ws_bytes);
-            if (t.ks != sh.ks || t.xl != sh.xl || t.kb != 1) break;
+            if (t.ks != sh.ks || t.S != sh.S || t.kb != 1) break;
         }
         if (static_cast<long>(more.tiles) + tiles_of(c.N) > 65535) break;
         more.m[g - 1].W = static_cast<const uint8_t*>(c.W);

@@ -209,8 +209,7 @@ int mi_stream_set_modes(void* stream, int gemv_mode, int gemm_mode);
  * *k_slices slices (more than one slice: fp32 partial sums in the stream's workspace and a
  * reduction launch), 2 / 3 = the 64 x 64 / 128 x 128 tile kernel, 4 = the streaming kernel for up
  * to 64 rows of x (*tile_rows = M rounded up to 16, *k_slices = wavefronts, over one or several
- * blocks, that share one strip of 16 rows of W; slices over several blocks also end in a reduction
- * launch), 5 = the MFMA kernel with 256 x 256 blocks (int8 weights), -1 = bad arguments.  For tests and tuning; tile_rows and k_slices
+ * blocks, that share 16 or 32 rows of W; slices over several blocks meet inside the launch), 5 = the MFMA kernel with 256 x 256 blocks (int8 weights), -1 = bad arguments.  For tests and tuning; tile_rows and k_slices
  * may be NULL. */
 int mi_linear_plan(void* stream, int M, int N, int K, const void* x, const void* W, int* tile_rows, int* k_slices);
 

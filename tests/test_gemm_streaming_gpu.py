@@ -1,0 +1,69 @@
+"""The streaming kernel (named by mode 5) and its sums for another launch (linear_slices), on integers: every product and
+sum is exact in fp32 whatever the order, so the result is integer arithmetic's, bit for bit.  Rows around the 16-row
+tiles; strips that end inside a tile of one and of two; K of one unit of 64, of fewer and of more units than wavefronts
+share it, and of more than a ring holds (32 768: 64 units a wavefront with 8 wavefronts)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from helpers import mil
+from test_prefill_slices_mode4_gpu import _slices
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 64), (15, 128), (17, 576), (33, 896), (130, 1536), (4132, 320), (48, 32768)]
+
+
+def _weights(kind, n, k, rng, keep):
+    """-> device weights, their integer values, the scale they are to be multiplied with (a power of two per row)"""
+    if kind == "f16":
+        q = rng.integers(-8, 9, (n, k))
+        keep.append(mil.Buffer.from_host(q.astype(np.float16)))
+        return keep[-1], q, np.ones(n)
+    scale = 2.0 ** rng.integers(-9, -5, n)
+    if kind == "int8":
+        q, stored, scales = rng.integers(-127, 128, (n, k)), None, scale
+        stored = q.astype(np.int8)
+    else:
+        nib = rng.integers(0, 16, (n, k))
+        q, stored = nib - 8, (nib[:, 0::2] | (nib[:, 1::2] << 4)).astype(np.uint8)
+        scales = np.repeat(scale[:, None], k // 32, axis=1)
+    w, s = mil.Buffer.from_host(stored), mil.Buffer.from_host(scales.astype(np.float16))
+    keep += [w, s]
+    assert (mil.nnopt_register_int8_weight if kind == "int8" else mil.nnopt_register_q4_weight)(w, s, n, k)
+    return w, q, scale
+
+
+@pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
+@pytest.mark.parametrize("rows", [2, 16, 17, 33, 49, 64])
+def test_exact_on_integers(kind, rows):
+    assert mil.lib().mi_init(0) == 1
+    queue, keep, rng = mil.Queue(), [], np.random.default_rng(rows)
+    for n, k in SHAPES:
+        w, q, scale = _weights(kind, n, k, rng, keep)
+        x = rng.integers(-3, 4, (rows, k))
+        xb, out = mil.Buffer.from_host(x.astype(np.float16)), mil.Buffer.from_host(np.full(rows * n + 8, 0x7bff, np.uint16))
+        print(f"{kind} rows {rows} N {n} K {k}", flush=True)
+        total = (x @ q.T).astype(np.float64)
+        assert np.abs(total).max() < 2 ** 24
+        assert mil.lib().mi_stream_set_modes(queue.handle, -1, 5)
+        assert mil.linear_plan(queue, rows, n, k, xb, w)[0] == 4
+        assert mil.pytorch_linear(queue, rows, n, k, xb, w, out)
+        queue.finish()
+        got = out.read(np.uint16, (rows * n + 8,))
+        assert np.all(got[-8:] == 0x7bff)
+        with np.errstate(over="ignore"):
+            want = (total * scale).astype(np.float32).astype(np.float16)
+        assert np.array_equal(got[:-8].view(np.float16).reshape(rows, n), want), (n, k)
+        assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
+        sums, scales = ctypes.c_void_p(), ctypes.c_void_p()
+        slices = _slices()(queue.handle, rows, n, k, xb.ptr, w.ptr, ctypes.byref(sums), ctypes.byref(scales))
+        assert slices >= 0
+        if slices:
+            assert n % 4 == 0 and k >= 64 * 4 * slices
+            host = np.empty((slices, rows, n), np.float32)
+            queue.finish()
+            assert mil.lib().mi_memcpy_d2h(host.ctypes.data, sums.value, host.nbytes, queue.handle)
+            want = total if kind != "q4" else total * scale
+            assert np.array_equal(host.astype(np.float64).sum(0), want), (n, k, slices)
