@@ -1370,6 +1370,7 @@ struct Unit {                                            // what 64 values of K 
     static constexpr int kX = MT * 2048;                 // rows of 128 bytes
     static constexpr int kW = KIND == WK_F16 ? S * 2048 : KIND == WK_I8 ? S * 1024 : S * 512;
     static constexpr int kBytes = kX + kW + (KIND == WK_Q4 ? S * 64 : 0);              // Q4: two block scales per row
+    static constexpr int kSums = MT * S * 1024;          // the tile's fp32 sums, which take the place of the ring
     static constexpr int kLoads = 2 * MT + (KIND == WK_F16 ? 2 * S : KIND == WK_I8 ? S : 2);
 };
 constexpr int kMaxRing = 8;                              // units in a ring
@@ -1395,12 +1396,17 @@ __device__ __forceinline__ void wait_for_all_but(int units) {           // the l
 #define MI_OX4 MI_OX3, [p3] "=&v"(x[3][0]), [q3] "=&v"(x[3][1])
 #define MI_F1 "ds_read_b128 %[w0], %[a] offset:%[o0]\n\tds_read_b128 %[v0], %[b] offset:%[o0]\n\t"
 #define MI_F2 MI_F1 "ds_read_b128 %[w1], %[a] offset:%[o1]\n\tds_read_b128 %[v1], %[b] offset:%[o1]\n\t"
+#define MI_F4 MI_F2 "ds_read_b128 %[w2], %[a] offset:%[o2]\n\tds_read_b128 %[v2], %[b] offset:%[o2]\n\t" \
+              "ds_read_b128 %[w3], %[a] offset:%[o3]\n\tds_read_b128 %[v3], %[b] offset:%[o3]\n\t"
 #define MI_OF1 [w0] "=&v"(w[0][0]), [v0] "=&v"(w[0][1])
 #define MI_OF2 MI_OF1, [w1] "=&v"(w[1][0]), [v1] "=&v"(w[1][1])
+#define MI_OF4 MI_OF2, [w2] "=&v"(w[2][0]), [v2] "=&v"(w[2][1]), [w3] "=&v"(w[3][0]), [v3] "=&v"(w[3][1])
 #define MI_I1 "ds_read_b128 %[w0], %[d]\n\t"
 #define MI_I2 MI_I1 "ds_read_b128 %[w1], %[d] offset:1024\n\t"
+#define MI_I4 MI_I2 "ds_read_b128 %[w2], %[d] offset:2048\n\tds_read_b128 %[w3], %[d] offset:3072\n\t"
 #define MI_OI1 [w0] "=&v"(w[0][0])
 #define MI_OI2 MI_OI1, [w1] "=&v"(w[1][0])
+#define MI_OI4 MI_OI2, [w2] "=&v"(w[2][0]), [w3] "=&v"(w[3][0])
 #define MI_Q1 "ds_read_b64 %[w0], %[d]\n\tds_read_b32 %[v0], %[e]\n\t"
 #define MI_Q2 MI_Q1 "ds_read_b64 %[w1], %[d] offset:512\n\tds_read_b32 %[v1], %[e] offset:64\n\t"
 #define MI_OQ1 [w0] "=&v"(w4[0]), [v0] "=&v"(ws[0])
@@ -1426,9 +1432,11 @@ struct UnitFrags {
         if constexpr (KIND == WK_F16) {
             MI_READ_S(1, F, [o0] "i"(MT * 2048))
             MI_READ_S(2, F, [o0] "i"(MT * 2048), [o1] "i"(MT * 2048 + 2048))
+            MI_READ_S(4, F, [o0] "i"(MT * 2048), [o1] "i"(MT * 2048 + 2048), [o2] "i"(MT * 2048 + 4096), [o3] "i"(MT * 2048 + 6144))
         } else if constexpr (KIND == WK_I8) {
             MI_READ_S(1, I, [d] "v"(d))
             MI_READ_S(2, I, [d] "v"(d))
+            MI_READ_S(4, I, [d] "v"(d))
         } else {
             MI_READ_S(1, Q, [d] "v"(d), [e] "v"(e))
             MI_READ_S(2, Q, [d] "v"(d), [e] "v"(e))
@@ -1441,8 +1449,8 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
                                             const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
                                             const int K, const int ks, const int ring_units, float* __restrict__ partial,
                                             uint32_t* __restrict__ counters, const MoreMats& more, const int bx, const int waves,
-                                            const int by, const int kb) {
-    static_assert(!GLU || S == 2, "a strip of either matrix");
+                                            const int by, const int kb, const int bz) {
+    static_assert(!GLU || S % 2 == 0, "strips of either matrix");
     constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
     typedef Unit<KIND, MT, S> U;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -1452,7 +1460,7 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
     const int slice = wave & (ks - 1);
     int tile = bx * (waves / ks) + wave / ks;
     if constexpr (!GLU) pick_matrix(more, tile, W, scale, out, N);
-    const int n0 = 16 * S * tile;
+    const int n0 = 16 * S * tile, m0 = 16 * MT * bz;
     const bool live = n0 < N;                            // (a block's last tiles may lie past the matrix: they take part in the barrier only)
     const int nb = live ? n0 : 0;
 
@@ -1475,14 +1483,14 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
     // x, fp16 W: a load covers 8 rows of 128 bytes; slot p of row r holds piece p ^ ((r >> 1) & 7)
     // int8: 16 rows of 64 bytes, piece p ^ ((r >> 2) & 3); Q4: 16 rows of 32 bytes (S of them), piece p ^ ((r >> 3) & 1)
     const size_t wrowb = Q4 ? static_cast<size_t>(K) / 2 : F16 ? static_cast<size_t>(K) * 2 : static_cast<size_t>(K);
-    const uint8_t* const Xb = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(it0) * 128;
+    const uint8_t* const Xb = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(m0) * K * 2 + static_cast<size_t>(it0) * 128;
     const uint8_t* const Wb = W + static_cast<size_t>(nb) * wrowb + static_cast<size_t>(it0) * (Q4 ? 32 : F16 ? 128 : 64);
-    const int wlast = N - 1 - nb;                        // rows past N are read as the last row
+    const int wlast = N - 1 - nb, xlast = M - 1 - m0;    // rows past N and M are read as the last row
     constexpr int kWL = F16 ? 2 * S : Q4 ? 1 : S;
     uint32_t xoff[2 * MT], woff[kWL];
     #pragma unroll
     for (int j = 0; j < 2 * MT; ++j) {
-        const int r = 8 * j + (lane >> 3), m = r < M ? r : M - 1;
+        const int r = 8 * j + (lane >> 3), m = r < xlast ? r : xlast;
         xoff[j] = static_cast<uint32_t>(m) * static_cast<uint32_t>(K) * 2u + 16u * ((lane & 7) ^ ((r >> 1) & 7));
     }
     #pragma unroll
@@ -1500,7 +1508,8 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
         const int r = lane & (16 * S - 1);
         soff = static_cast<uint32_t>(r < wlast ? r : wlast) * static_cast<uint32_t>(K / 16);
     }
-    uint8_t* const ring = lds + static_cast<size_t>(wave) * ring_units * U::kBytes;
+    const int stride = ring_units * U::kBytes > U::kSums ? ring_units * U::kBytes : U::kSums;
+    uint8_t* const ring = lds + wave * stride;
     auto fill = [&](int u, int slot) {                   // unit u of the slice
         uint8_t* l = ring + slot * U::kBytes;
         #pragma unroll
@@ -1576,7 +1585,7 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
 
     // The slices' sums meet in LDS, each where its wavefront's ring was; sum t S + s of the tile (GLU: both sums of rows t) is
     // then finished by the tile's wavefront of that number mod ks, which adds them in slice order.
-    auto sums_of = [&](int w) { return reinterpret_cast<floatx4*>(lds + static_cast<size_t>(w) * ring_units * U::kBytes); };
+    auto sums_of = [&](int w) { return reinterpret_cast<floatx4*>(lds + w * stride); };
     if (ks > 1) {                                        // (the same for every wavefront of the block)
         #pragma unroll
         for (int t = 0; t < MT; ++t)
@@ -1603,9 +1612,10 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
                     for (int r = 0; r < 4; ++r) v[r] += o[r];
                 }
             }
-            const int nq = 16 * strip + 4 * c, m = 16 * t + i;           // first of this lane's 4 output columns, its row
+            const int nq = 16 * strip + 4 * c, m = m0 + 16 * t + i;      // first of this lane's 4 output columns, its row
             if constexpr (MEET) {
-                if (kb > 1 && !meet_slices(v, partial + (static_cast<size_t>(strip) * MT + t) * kb * 256, counters + strip * MT + t, by, kb, lane))
+                const int met = (bz * ((N + 15) / 16) + strip) * MT + t;
+                if (kb > 1 && !meet_slices(v, partial + static_cast<size_t>(met) * kb * 256, counters + met, by, kb, lane))
                     continue;
             } else if constexpr (!GLU) {
                 if (partial) {                           // (N is a multiple of 4 then)
@@ -1633,9 +1643,13 @@ __device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, cons
             }
         }
         if constexpr (GLU) {
-            if ((t & (ks - 1)) == slice && 16 * t + i < M)
-                *reinterpret_cast<uint2*>(out + static_cast<size_t>(16 * t + i) * (N / 2) + 16 * tile + 4 * c) =
-                    uint2{swiglu_h2(h[0].x, h[1].x), swiglu_h2(h[0].y, h[1].y)};
+            if ((t & (ks - 1)) == slice && m0 + 16 * t + i < M) {
+                #pragma unroll
+                for (int s = 0; s < S; s += 2)
+                    if (n0 + 16 * s < N)
+                        *reinterpret_cast<uint2*>(out + static_cast<size_t>(m0 + 16 * t + i) * (N / 2) + (n0 + 16 * s) / 2 + 4 * c) =
+                            uint2{swiglu_h2(h[s].x, h[s + 1].x), swiglu_h2(h[s].y, h[s + 1].y)};
+            }
         }
     }
 }
@@ -1646,7 +1660,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __res
                                                            int M, int N, int K, int ks, int ring_units, float* __restrict__ partial,
                                                            uint32_t* __restrict__ counters, MoreMats more) {
     skinny_tile<KIND, MT, S, TERMS, GLU, MEET>(X, W, scale, out, M, N, K, ks, ring_units, partial, counters, more, blockIdx.x,
-                                               blockDim.x >> 6, blockIdx.y, gridDim.y);
+                                               blockDim.x >> 6, blockIdx.y, gridDim.y, blockIdx.z);
 }
 
 constexpr size_t kLdsLimit = 160 * 1024;
@@ -1706,6 +1720,74 @@ inline bool preferred(int kind, int M, int N, int K, int cus) {
     return M <= (kind == WK_I8 && K <= 512 ? 48 : kind == WK_F16 && strips > 2L * cus ? 32 : 64) && w_bytes <= 36.0e6 && strips <= 5L * cus;
 }
 
+// ---- more rows of x than a tile holds: tiles of 16 mt rows by 16 S columns ----
+//
+// us per launch, weights from HBM, the 64 x 64 tiles or the wide kernel -> these: int8 100 / 300 / 600 rows of 1152 x 896 8.6 / 9.3 / 9.4 ->
+// 4.7 / 5.6 / 7.2, 100 rows of 9728 x 896 with the SwiGLU 10.8 -> 9.8, Q4 300 rows of 896 x 896 12.0 -> 5.7, of 9728 x 896 with the SwiGLU
+// 17.8 -> 15.8, 100 fp16 rows of 896 x 4864 14.2 -> 8.2.  From about 600 rows on by many columns the wide kernel's larger tiles
+// win: a block here pulls 1 byte into LDS for 25 to 60 multiplications, there for 140.
+//
+//
+// A launch takes 4.1 us and, per block on a CU, what it pulls into LDS and its share of multiplying: fitted to 2341 launches of 65
+// to 2048 rows (8 % rms; the shape it picks is 2 % behind the best one in the mean).  Blocks beyond one per CU come in rounds, a
+// last round that is not full at 0.7 of its price (the blocks in it have the L2s to themselves).  Four strips to a wavefront leave
+// a CU with one block: 1.15 to 1.3 times as long; with Q4 never the best.
+struct RowShape { int mt = 0, S = 1, ks = 4, kb = 1; double us = 1e30; };
+inline double rows_us(int kind, int mt, int S, int kb, int M, int N, int K, int cus) {
+    const long blocks = static_cast<long>((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * S - 1) / (16 * S)) * kb;
+    const double unit = static_cast<double>(unit_bytes(kind, mt, S));
+    const double unit_us = kind == WK_F16 ? (unit / 118.0e3 + mt * S * 0.0053) * (S == 4 ? 1.15 : 1.0)
+                         : kind == WK_I8  ? (unit / 94.0e3 + mt * S * 0.0027) * (S == 4 ? 1.33 : S == 1 ? 0.88 : 1.0)
+                                          : unit / 57.0e3 * (S == 1 ? 0.72 : 1.0);
+    const double mean = static_cast<double>(blocks) / cus;
+    const long full = (blocks + cus - 1) / cus;
+    return 4.1 + (full == 1 ? 1.0 : 0.7 * full + 0.3 * mean) * (K / 64.0 / kb) * unit_us;
+}
+// Slices of K inside a block, by what a launch by itself, one among several matrices and one with the SwiGLU have in
+// common, since they decide the order of the sums.
+inline int rows_ks(int M, int N, int K) {
+    int ks = N > 8192 ? 2 : N > 1536 || M > 400 ? 4 : 8;
+    while (ks > 1 && K / 64 < ks) ks /= 2;
+    return ks;
+}
+inline bool rows_fit(int kind, int mt, int S, int ks) {
+    const size_t unit = unit_bytes(kind, mt, S), sums = static_cast<size_t>(mt) * S * 1024;
+    return (ks < 4 ? 4 : ks) * (unit > sums ? unit : sums) <= kLdsLimit;
+}
+inline RowShape pick_rows(int kind, int M, int N, int K, int cus, bool glu) {
+    RowShape best;
+    for (int mt = 2; mt <= 4; ++mt)
+        for (int S = 1; S <= 4; S *= 2) {
+            const int ks = rows_ks(M, N, K);
+            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || (glu && S == 1) || !rows_fit(kind, mt, S, ks)) continue;
+            const double us = rows_us(kind, mt, S, 1, M, N, K, cus);
+            if (us < best.us) best = RowShape{mt, S, ks, 1, us};
+        }
+    return best;
+}
+// Where they are the choice over the wide kernel, by its estimate (which is 4 to 7 us too high for slices of K, 1200 x 896 x 4864
+// in three 25.6 us, estimated at 32.6, and 1 too low for a few rows of fp16, 300 x 5120 x 960 12.5 against 10.7 here), and not for many rows of W (see preferred) or many of both: 600 x 3072 x 576 int8 9.0 against
+// 8.2, 600 x 5120 x 960 17.5 against 14.1; Q4 450 x 3072 x 576 8.6 against 10.2, but 900 x 3072 x 576 13.3 against 11.9; fp16 2048 x
+// 896 x 896 11.6 against 10.1, 1200 x 896 x 896 8.1 against 9.9.
+inline bool rows_preferred(int kind, const RowShape& r, double wide_us, int wide_slices, int M, int N, int cus) {
+    return (N + 15) / 16 <= 5L * cus && !(N > 2560 && M > (kind == WK_Q4 ? 512 : 304)) && !(kind == WK_F16 && M > 1280) && r.us < (wide_slices == 1 ? 1.0 : M <= 1024 ? 0.85 : 0.7) * wide_us + (kind == WK_F16 && M <= 304 ? 0.8 : 0.0);
+}
+// The same cut into slices over blocks for a launch that adds them (mt = 0: not worth it).
+inline RowShape pick_rows_apart(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
+    RowShape best;
+    const int its = K / 64;
+    if (its < 14 || static_cast<long>((M + 47) / 48) * ((N + 31) / 32) > cus * 9L / 5) return best;
+    for (int mt = 2; mt <= 4; ++mt)
+        for (int S = 1; S <= 4; S *= 2) {
+            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || !rows_fit(kind, mt, S, 4)) continue;
+            for (int kb = 2; kb <= 6 && its >= 4 * kb && static_cast<size_t>(kb) * M * N * 4 <= workspace_bytes; ++kb) {
+                const double us = rows_us(kind, mt, S, kb, M, N, K, cus) + kb * 4.0e-6 * M * N / 4.0;
+                if (us < best.us) best = RowShape{mt, S, 4, kb, us};
+            }
+        }
+    return best;
+}
+
 // Estimated time (us): what decides between this kernel and rows of GEMV below 16 rows.  (Fitted to the kernel that took
 // fragments from memory, and 0.3 to 1 us too high: a line that moved would take prompts of a few tokens off the reference's
 // order, in which their attention goes with the projections.)
@@ -1756,7 +1838,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_skinny_many(const SkinnyCall
     const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb, by = kb > 1 ? at / blocks : 0;
     const MoreMats none{};
     skinny_tile<KIND, MT, 1, TERMS, false, true>(L->c[q].X, L->c[q].W, L->c[q].scale, L->c[q].out, L->M, L->c[q].N, L->c[q].K, L->c[q].ks,
-                                                 L->ring, L->c[q].partial, L->c[q].counters, none, at - by * blocks, kWaves, by, kb);
+                                                 L->ring, L->c[q].partial, L->c[q].counters, none, at - by * blocks, kWaves, by, kb, 0);
 }
 
 // Units of K in a wavefront's ring: its whole slice where `per_cu` such blocks fit the LDS of a CU.
@@ -1776,14 +1858,15 @@ bool launch_one(hipStream_t s, int M, int N, int K, const void* x, const void* W
     const long blocks = (tiles + per_block - 1) / per_block;
     const int cus = device_info().cus;
     constexpr size_t unit = Unit<KIND, MT, S>::kBytes;
-    const int ring = ring_units(unit, waves, (blocks * sh.kb + cus - 1) / cus, K, ks, sh.kb);
-    const size_t lds = waves * ring * unit;
+    const long tiles_m = (M + 16 * MT - 1) / (16 * MT);
+    const int ring = ring_units(unit, waves, (blocks * sh.kb * tiles_m + cus - 1) / cus, K, ks, sh.kb);
+    const size_t lds = waves * (ring * unit > Unit<KIND, MT, S>::kSums ? ring * unit : Unit<KIND, MT, S>::kSums);
     auto* kern = gemm_skinny<KIND, MT, S, TERMS, GLU, MEET>;
     if (lds > 65536 &&
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
         return false;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(sh.kb)), dim3(64 * waves), lds, s,
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(sh.kb), static_cast<unsigned>(tiles_m)), dim3(64 * waves), lds, s,
                        static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W), static_cast<const uint16_t*>(scale),
                        static_cast<uint16_t*>(out), M, N, K, ks, ring, partial, counters, more);
     return MI_HIP_OK(hipGetLastError());
@@ -1819,6 +1902,30 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
         case 2: return launch_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
         case 3: return launch_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
         default: return launch_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, sh, partial, more, glu, apart);
+    }
+}
+
+template <int KIND, int MT, int TERMS>
+bool launch_rows_mt(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, int S, Shape sh,
+                    float* sums, const MoreMats& more, bool glu) {
+    if constexpr (MT > 2 && KIND != WK_Q4) {
+        if (S == 4)
+            return glu ? launch_one<KIND, MT, 4, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, nullptr, nullptr, more)
+                       : launch_one<KIND, MT, 4, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, sums, nullptr, more);
+    }
+    if (glu) return launch_one<KIND, MT, 2, TERMS, true, false>(s, M, N, K, x, W, scale, out, sh, nullptr, nullptr, more);
+    return S == 2 ? launch_one<KIND, MT, 2, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, sums, nullptr, more)
+                  : launch_one<KIND, MT, 1, TERMS, false, false>(s, M, N, K, x, W, scale, out, sh, sums, nullptr, more);
+}
+// sums: null, or where the sums of kb slices go (for a launch that adds them)
+template <int KIND, int TERMS>
+bool launch_rows(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out, const RowShape& r,
+                 float* sums, const MoreMats& more, bool glu) {
+    const Shape sh{r.ks, r.kb, r.S};
+    switch (r.mt) {
+        case 2: return launch_rows_mt<KIND, 2, TERMS>(s, M, N, K, x, W, scale, out, r.S, sh, sums, more, glu);
+        case 3: return launch_rows_mt<KIND, 3, TERMS>(s, M, N, K, x, W, scale, out, r.S, sh, sums, more, glu);
+        default: return launch_rows_mt<KIND, 4, TERMS>(s, M, N, K, x, W, scale, out, r.S, sh, sums, more, glu);
     }
 }
 
@@ -2017,7 +2124,15 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         }
         if (!wide_fits || mode == 5) return p;
         const bool may_slice = mode == 0 || mode == 4;
-        wide::pick_shape(WK_Q4, p.terms, M, N, K, cus, may_slice ? workspace_bytes : 0, &tm, &splits, nullptr);
+        double wide_us = 0.0;
+        wide::pick_shape(WK_Q4, p.terms, M, N, K, cus, may_slice ? workspace_bytes : 0, &tm, &splits, &wide_us);
+        if (may_slice || mode == 6) {
+            const skinny::RowShape r = skinny::pick_rows(kind, M, N, K, cus, false);
+            if (mode == 6 || skinny::rows_preferred(kind, r, wide_us, splits, M, N, cus)) {
+                p.kernel = 6; p.tile_rows = 16 * r.mt; p.ks = r.ks; p.strips = r.S;
+                return p;
+            }
+        }
         if (mode >= 11 && mode <= 15) tm = mode - 10;
         if (pin_splits) splits = pin_splits;
         p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;
@@ -2043,6 +2158,13 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         return p;
     }
     if (mode == 5) return p;
+    // the same in tiles of rows, where its estimated time beats that of the other two
+    const skinny::RowShape r = mode == 0 || mode == 6 ? skinny::pick_rows(kind, M, N, K, cus, false) : skinny::RowShape{};
+    auto rows = [&]() {
+        p.kernel = 6; p.tile_rows = 16 * r.mt; p.ks = r.ks; p.strips = r.S;
+        return p;
+    };
+    if (mode == 6) return rows();
     // the wide kernel where its estimated time beats that of the 64 x 64 tiles
     if (wide_fits && (mode == 0 || mode == 3 || (mode >= 11 && mode <= 15))) {
         double wide_us = 0.0;
@@ -2050,7 +2172,12 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         wide::pick_shape(kind, 1, M, N, K, cus, mode == 0 ? workspace_bytes : 0, &tm, &splits, &wide_us);
         if (mode >= 11) tm = mode - 10;
         if (pin_splits) splits = pin_splits;
-        if (mode != 0 || wide_us < tiled_estimate_us(M, N, K)) {
+        const double tiled_us = tiled_estimate_us(M, N, K);
+        // (the 64 x 64 tiles' estimate is for weights in the caches: 1.5 to 2.5 us less than from HBM, as they come in a model)
+        // (many rows in tiles that go in bands keep those, a plan that is promised: 2048 x 960 x 960 int8 11.6 us against 12.2 here)
+        const bool banded = M > (K < 896 ? 1280 : 1024) && N >= 960 && K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);
+        if (mode == 0 && !banded && skinny::rows_preferred(kind, r, wide_us, splits, M, N, cus) && r.us < tiled_us + 1.5) return rows();
+        if (mode != 0 || wide_us < tiled_us) {
             p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;
             return p;
         }
@@ -2088,6 +2215,14 @@ bool launch_planned(hipStream_t s, const GemmPlan& p, WeightKind kind, int M, in
                                   : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, out, sh, workspace, ws_bytes, more, glu);
         }
         case 5: return quad::launch(s, M, N, K, x, W, scale, out);
+        case 6: {
+            const skinny::RowShape r{p.tile_rows / 16, p.strips, p.ks, 1, 0.0};
+            if (kind == WK_Q4)
+                return p.terms == 1 ? skinny::launch_rows<WK_Q4, 1>(s, M, N, K, x, W, scale, out, r, nullptr, more, glu)
+                                    : skinny::launch_rows<WK_Q4, 2>(s, M, N, K, x, W, scale, out, r, nullptr, more, glu);
+            return kind == WK_F16 ? skinny::launch_rows<WK_F16, 1>(s, M, N, K, x, W, scale, out, r, nullptr, more, glu)
+                                  : skinny::launch_rows<WK_I8, 1>(s, M, N, K, x, W, scale, out, r, nullptr, more, glu);
+        }
         case 2: return launch_tile<64, 64, 32, 32>(s, kind, M, N, K, x, W, scale, out, more);
         case 3: return launch_tile<128, 128, 64, 64>(s, kind, M, N, K, x, W, scale, out, more);
         default:
@@ -2125,8 +2260,12 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
                     void* out, void* workspace, size_t workspace_bytes) {
     if (N % 32 || reinterpret_cast<uintptr_t>(out) % 16 || !gemm_supported(kind, M, N, K, x, W, scale)) return 0;
     const size_t ws_bytes = workspace ? workspace_bytes : 0;
-    const GemmPlan p = plan_gemm(s, kind, M, N, K, ws_bytes);
-    if (!(p.kernel == 1 ||
+    GemmPlan p = plan_gemm(s, kind, M, N, K, ws_bytes);
+    if (p.kernel == 6) {                                 // (the slices of K as planned: they are the order of the sums)
+        const skinny::RowShape r = skinny::pick_rows(kind, M, N, K, device_info().cus, true);
+        p.tile_rows = 16 * r.mt; p.strips = r.S;
+    }
+    if (!(p.kernel == 1 || p.kernel == 6 ||
           (p.kernel == 4 && skinny::pick_shape(kind, M, N, K, device_info().cus, ws_bytes).kb == 1)))
         return 0;
     return launch_planned(s, p, kind, M, N, K, x, W, scale, out, workspace, ws_bytes, MoreMats{}, true) ? 1 : -1;
@@ -2155,11 +2294,27 @@ int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, cons
             return ok ? sh.kb : -1;
         }
     }
-    if (p.kernel >= 1 && p.kernel <= 3 && p.k_slices == 1 && (mode == 0 || mode == 4) && wide_reaches(kind, M, N, K)) {
-        const int terms = kind == WK_Q4 ? p.terms : 1;
-        const int cus = device_info().cus;
+    const int terms = kind == WK_Q4 ? p.terms : 1, cus = device_info().cus;
+    if ((mode == 0 || mode == 4) && p.kernel >= 1 && p.kernel != 5) {
+        // (against what would run otherwise: the plan, or the wide kernel's slices)
+        const skinny::RowShape r = skinny::pick_rows_apart(kind, M, N, K, cus, workspace_bytes);
+        int tm = 1, splits = 1;
+        double cut = 1e30;
+        if (wide_reaches(kind, M, N, K)) wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &cut);
+        if (r.mt && r.us < cut - 2.5) {
+            auto* sums = static_cast<float*>(workspace);
+            const bool ok = kind == WK_Q4 ? (terms == 1 ? skinny::launch_rows<WK_Q4, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false)
+                                                        : skinny::launch_rows<WK_Q4, 2>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false))
+                          : kind == WK_F16 ? skinny::launch_rows<WK_F16, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false)
+                                           : skinny::launch_rows<WK_I8, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false);
+            return ok ? r.kb : -1;
+        }
+    }
+    if (p.kernel >= 1 && p.kernel != 4 && p.kernel != 5 && (p.kernel != 1 || p.k_slices == 1) && (mode == 0 || mode == 4) && wide_reaches(kind, M, N, K)) {
         // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
-        const double uncut = p.kernel == 1 ? wide::estimate_us(kind, terms, p.tile_rows / 32, 1, M, N, K, cus) : tiled_estimate_us(M, N, K);
+        const double uncut = p.kernel == 1   ? wide::estimate_us(kind, terms, p.tile_rows / 32, 1, M, N, K, cus)
+                             : p.kernel == 6 ? skinny::rows_us(kind, p.tile_rows / 16, p.strips, 1, M, N, K, cus)
+                                             : tiled_estimate_us(M, N, K);
         int tm = 1, splits = 1;
         double us = 0.0;
         if (wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &us) && us - 2.5 < uncut) {
@@ -2183,8 +2338,14 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
     GemmPlan p = plan_gemm(s, kind, M, mat[0].N, K, ws_bytes);
     skinny::Shape sh{};
     if (p.kernel == 4) sh = skinny::pick_shape(kind, M, mat[0].N, K, cus, ws_bytes);
-    if (!(p.kernel == 2 || p.kernel == 3 || (p.kernel == 1 && p.k_slices == 1) || (p.kernel == 4 && sh.kb == 1))) return 0;
-    const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : 16 * sh.S;
+    if (p.kernel == 6) {
+        long all = 0;
+        for (int j = 0; j < n; ++j) all += mat[j].N;
+        const skinny::RowShape r = skinny::pick_rows(kind, M, all < (1 << 30) ? static_cast<int>(all) : mat[0].N, K, cus, false);
+        if (skinny::rows_fit(kind, r.mt, r.S, p.ks)) { p.tile_rows = 16 * r.mt; p.strips = r.S; }
+    }
+    if (!(p.kernel == 2 || p.kernel == 3 || p.kernel == 6 || (p.kernel == 1 && p.k_slices == 1) || (p.kernel == 4 && sh.kb == 1))) return 0;
+    const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : p.kernel == 6 ? 16 * p.strips : 16 * sh.S;
     auto tiles_of = [&](int N) { return N / width + (N % width != 0); };
     MoreMats more;
     more.tiles = tiles_of(mat[0].N);
@@ -2193,7 +2354,7 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
         const GemmMat& c = mat[g];
         if (!gemm_supported(kind, M, c.N, K, x, c.W, c.scale)) break;
         const GemmPlan q = plan_gemm(s, kind, M, c.N, K, ws_bytes);
-        if (q.kernel != p.kernel || q.terms != p.terms || q.k_slices != p.k_slices) break;
+        if (q.kernel != p.kernel || q.terms != p.terms || q.k_slices != p.k_slices || q.ks != p.ks) break;
         if (p.kernel == 4) {
             const skinny::Shape t = skinny::pick_shape(kind, M, c.N, K, cus, ws_bytes);
             if (t.ks != sh.ks || t.S != sh.S || t.kb != 1) break;

@@ -67,3 +67,31 @@ def test_exact_on_integers(kind, rows):
             assert mil.lib().mi_memcpy_d2h(host.ctypes.data, sums.value, host.nbytes, queue.handle)
             want = total if kind != "q4" else total * scale
             assert np.array_equal(host.astype(np.float64).sum(0), want), (n, k, slices)
+
+
+@pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
+@pytest.mark.parametrize("rows", [2, 65, 96, 97, 300, 1200])
+def test_tiles_of_rows_exact_on_integers(kind, rows):
+    """Mode 6: tiles of 32, 48 and 64 rows with a last one that is not full, of 16, 32 and 64 columns likewise, K in 2, 4 and 8
+    slices; and the library's own choice at the same calls."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep, rng = mil.Queue(), [], np.random.default_rng(rows)
+    for n, k in [(1, 64), (130, 576), (904, 960), (896, 4864), (1700, 128), (3080, 192), (9728, 128)]:
+        w, q, scale = _weights(kind, n, k, rng, keep)
+        x = rng.integers(-3, 4, (rows, k))
+        xb = mil.Buffer.from_host(x.astype(np.float16))
+        total = x.astype(np.float64) @ q.T.astype(np.float64)
+        assert np.abs(total).max() < 2 ** 24
+        with np.errstate(over="ignore"):
+            want = (total * scale).astype(np.float32).astype(np.float16)
+        for mode in (6, -1):
+            out = mil.Buffer.from_host(np.full(rows * n + 8, 0x7bff, np.uint16))
+            assert mil.lib().mi_stream_set_modes(queue.handle, -1, mode)
+            plan = mil.linear_plan(queue, rows, n, k, xb, w)
+            print(f"{kind} rows {rows} N {n} K {k} mode {mode} plan {plan}", flush=True)
+            assert mode != 6 or plan[0] == 6
+            assert mil.pytorch_linear(queue, rows, n, k, xb, w, out)
+            queue.finish()
+            got = out.read(np.uint16, (rows * n + 8,))
+            assert np.all(got[-8:] == 0x7bff)
+            assert np.array_equal(got[:-8].view(np.float16).reshape(rows, n), want), (n, k, mode)
