@@ -13,6 +13,7 @@
 // exactness against the CPU restatement (same operations in the same order, so that the token
 // lists can be compared for identity), and are launch-bound at batch 1 whatever they do.
 #include "common.h"
+#include <type_traits>
 #include "device_math.h"
 #include "step_record.h"
 #include "../../include/mi_decode.h"
@@ -260,9 +261,9 @@ __global__ __launch_bounds__(256) void rope_attention_kernel(const uint16_t* __r
 // The same launch for head widths known at compile time (64 and 128): one block of 512 threads per query
 // head, the arithmetic and its order those of rope_attention_kernel.
 //
-// What bounds it at a long context are the two serial chains that order leaves: the sum of the exponentials
-// and, per output element, the sum over the keys.  A dependent addition takes 8 shader cycles (3.55 ns)
-// whatever else the CU does, so the launch cannot be faster than 7.1 ns per position.  Everything else is kept off
+// What bounds it at a long context are the two serial chains that order leaves: the sum of the exponentials (to 900 positions;
+// beyond, ordered_sum) and, per output element, the sum over the keys.  A dependent addition takes 8 shader cycles (3.55 ns)
+// whatever else the CU does, so the launch cannot be faster than 7.1 (3.6) ns per position.  Everything else is kept off
 // the chains' path:
 //  * scores, exponentials and probabilities are spread over all eight wavefronts (a key per thread, from a
 //    tile of key rows in LDS; the next tile is requested while one is worked on);
@@ -292,6 +293,113 @@ constexpr int kMaxPositions = 8192;                      // longest context a de
 // short context kShort rows of either.
 constexpr int kTileData = 65536;
 constexpr size_t tile_area(int D) { return static_cast<size_t>(kTileData) / (2 * D) * (2 * D + 16); }
+
+// A value of the lane `SH` below inside a row of 16, of the last lane of the row below, of lane 31 (DPP moves); a lane
+// without one keeps its own.
+template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t from_below(uint32_t a) {
+    return __builtin_amdgcn_update_dpp(static_cast<int>(a), static_cast<int>(a), CTRL, ROWS, 0xf, false);
+}
+// f(step): for every step of a scan over the 64 lanes, from_below's controls and the lowest lane its value covers last
+template <typename F> __device__ __forceinline__ void scan_steps(F&& f, int lane) {
+    f(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}, (lane & 15) >= 1 ? lane - 1 : -1);      // row_shr:1
+    f(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{}, (lane & 15) >= 2 ? lane - 2 : -1);
+    f(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}, (lane & 15) >= 4 ? lane - 4 : -1);
+    f(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{}, (lane & 15) >= 8 ? lane - 8 : -1);
+    f(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}, lane & 16 ? (lane & 48) - 1 : -1);      // row_bcast:15
+    f(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}, lane & 32 ? 31 : -1);                   // row_bcast:31
+}
+
+// The sum of ex[0 .. n) in index order, as one chain of fp32 additions from 0 gives it bit for bit, by a wavefront whose
+// lanes each hold a run of the terms; n a multiple of 4 and at most 256 * QUADS, terms not negative, the result in every lane.
+//
+// A running sum S >= 0 that stays in its binade, S = m u with u the unit in its last place, grows by a multiple of u
+// with every term: fp32(S + e) - S depends on e and, where e / u ends in exactly a half, on whether m is even.  So a
+// lane adds its terms to two stand-ins for the sum in front of them, an even and an odd one of the same binade (a plain sum
+// of everything ahead tells which that is); what either gained is what the true sum gains, in units of u the
+// difference of the bit patterns.  Gains of neighbouring lanes in one binade are put together by a scan: "from an even
+// sum k0 units, from an odd one k1".  Runs in which the sum passes into the next binade, seven or so of 64, are added
+// term by term, and so is everything whose binade turns out another when the true sum gets there: nothing rests on the plain sum.
+// 8 steps of the decoder, int8 0.5B at position 1030 / 1900 6028 / 7690 -> 5850 / 6990 us, Q4 360M at 2400 11 560 -> 10 470, fp16 0.5B at
+// 3800 12 070 -> 10 490.  (With its lanes' terms read from LDS where they are used and its scans through LDS: no gain at 1900.)
+template <int QUADS>
+__device__ __forceinline__ float ordered_sum(const float* ex, const int n) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const f32x4* e4 = reinterpret_cast<const f32x4*>(ex);
+    const int lane = threadIdx.x & 63;
+    // quadruples of terms per lane (an odd number: 16-byte reads that far apart fall on all banks); of all; this lane's
+    const int run = ((n + 255) / 256) | 1, quads = n / 4;
+    const int q0 = lane * run, mine = q0 + run <= quads ? run : q0 < quads ? quads - q0 : 0;
+    f32x4 e[QUADS];
+    #pragma unroll
+    for (int j = 0; j < QUADS; ++j) {
+        e[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (j < mine) e[j] = e4[q0 + j];
+    }
+    f32x4 a = e[0];
+    #pragma unroll
+    for (int j = 1; j < QUADS; ++j) a += e[j];
+    float upto = (a[0] + a[1]) + (a[2] + a[3]);                // a plain sum of the terms up to the run's end, then of those ahead of it
+    scan_steps([&](auto ctrl, auto rows, int last) {
+        const float o = __uint_as_float(from_below<decltype(ctrl)::value, decltype(rows)::value>(__float_as_uint(upto)));
+        upto += last >= 0 ? o : 0.0f;
+    }, lane);
+    const float before = __shfl_up(upto, 1, 64);
+    // (it is off by less than 2^-10 of itself: n is at most 2^13)
+    const float lo = before * (1.0f - 0x1p-10f), hi = upto * (1.0f + 0x1p-10f);
+    const uint32_t binade = __float_as_uint(lo) >> 23;
+    bool steady = lane > 0 && mine > 0 && lo > 1e-30f && hi < 1e30f && binade == __float_as_uint(hi) >> 23;
+    const uint32_t even = __float_as_uint(before) & ~1u;
+    float s0 = __uint_as_float(even), s1 = __uint_as_float(even | 1u);
+    #pragma unroll
+    for (int j = 0; j < QUADS; ++j)
+        #pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s0 = s0 + e[j][r];
+            s1 = s1 + e[j][r];
+        }
+    uint32_t k0 = __float_as_uint(s0) - even, k1 = __float_as_uint(s1) - (even | 1u);
+    steady = steady && __float_as_uint(s0) >> 23 == binade && __float_as_uint(s1) >> 23 == binade;
+    // runs of neighbouring steady lanes of one binade, in one piece each: a head is a lane that does not go on with the one below
+    const uint32_t below = __shfl_up(steady ? binade : 0u, 1, 64);
+    const uint64_t heads = __ballot(lane == 0 || !steady || below != binade);
+    const int from = 63 - __clzll(heads & (~0ull >> (63 - lane)));
+    scan_steps([&](auto ctrl, auto rows, int last) {
+        const uint32_t p0 = from_below<decltype(ctrl)::value, decltype(rows)::value>(k0), p1 = from_below<decltype(ctrl)::value, decltype(rows)::value>(k1);
+        const uint32_t n0 = p0 + (p0 & 1u ? k1 : k0), n1 = p1 + (p1 & 1u ? k0 : k1);
+        if (last >= from) { k0 = n0; k1 = n1; }
+    }, lane);
+    // from head to head with the true sum (lanes that hold terms are the lowest ones)
+    const uint64_t steadies = __ballot(steady);
+    const int lanes = (quads + run - 1) / run;
+    uint64_t left = heads & (~0ull >> (64 - lanes));
+    float sum = 0.0f;
+    while (left) {
+        const int first = __ffsll(static_cast<unsigned long long>(left)) - 1;
+        left &= left - 1;
+        const int next = left ? __ffsll(static_cast<unsigned long long>(left)) - 1 : lanes;
+        if (steadies >> first & 1) {
+            const uint32_t b = __builtin_amdgcn_readlane(binade, first), g0 = __builtin_amdgcn_readlane(k0, next - 1),
+                           g1 = __builtin_amdgcn_readlane(k1, next - 1);
+            const uint32_t at = __builtin_amdgcn_readfirstlane(__float_as_uint(sum)), to = at + (at & 1u ? g1 : g0);
+            if (at >> 23 == b && to >> 23 == b) {
+                sum = __uint_as_float(to);
+                continue;
+            }
+        }
+        for (int l = first; l < next; ++l) {                   // every lane goes on with its own terms, lane l's is the sum
+            float t = sum;
+            #pragma unroll
+            for (int j = 0; j < QUADS; ++j)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) t = t + e[j][r];
+            sum = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(t), l));
+        }
+    }
+    return sum;
+}
+// Positions (in whole batches) from which on the sum is spread over the lanes (even at about 800), and the most of them (what a
+// lane holds in registers).
+constexpr int kSpreadFrom = 928, kSpreadQuads = 17, kSpreadMost = 256 * (kSpreadQuads - 1);
 
 template <int D>
 // (Arguments in the order of need: the first 14 dwords arrive in registers with the wavefront, and the
@@ -632,7 +740,9 @@ __global__ __launch_bounds__(kAttnThreads) void rope_attention_tiled(uint16_t* _
         if (vtiles > 1) { request_tile(1); keep_tile(1); }
         if (vtiles > 2) request_tile(2);
     } else if (wave == 0) {
-        const float inv = rcp_rn(sum_in_order() + 1e-20f);
+        const float sum = padded < kSpreadFrom || padded > kSpreadMost ? sum_in_order()
+                        : padded <= 2048                              ? ordered_sum<9>(ex, padded) : ordered_sum<kSpreadQuads>(ex, padded);
+        const float inv = rcp_rn(sum + 1e-20f);
         if (tid == 0) red[0] = inv;
     }
     __syncthreads();                                           // the sum
