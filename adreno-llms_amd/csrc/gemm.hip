@@ -16,6 +16,7 @@
 #include "common.h"
 #include "device_math.h"
 #include <hip/hip_fp16.h>
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1822,23 +1823,26 @@ struct SkinnyCalls {
         float* partial;
         uint32_t* counters;
         int N, K;
-        uint16_t blocks;                                 // blocks along N; kb times as many in all
+        uint16_t blocks;                                 // blocks along N; for every slice over blocks and tile of rows as many
         uint8_t ks, kb;                                  // slices inside a block and over blocks
     } c[kMaxManyGemm] = {};
 };
 static_assert(sizeof(SkinnyCalls) <= 4096, "kernel arguments");
 
-template <int KIND, int MT, int TERMS>
+// S = 1: up to 64 rows of x, slices over blocks may meet; S = 2: tiles of rows.
+template <int KIND, int MT, int S, int TERMS>
 __global__ __launch_bounds__(64 * kWaves) void gemm_skinny_many(const SkinnyCalls) {
     // (the argument is read where it lies: indexed by a run-time number it would be copied to scratch first)
     const auto* L = (const __attribute__((address_space(4))) SkinnyCalls*)__builtin_amdgcn_kernarg_segment_ptr();
     const int lane = threadIdx.x & 63, n = L->n, b = blockIdx.x;
     const int mine = L->first[lane < kMaxManyGemm ? lane : 0];
     const int q = __popcll(__ballot(lane < n && b >= mine)) - 1;
-    const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb, by = kb > 1 ? at / blocks : 0;
+    const int blocks = L->c[q].blocks, at = b - L->first[q], kb = L->c[q].kb;
+    const int piece = S == 2 || kb > 1 ? at / blocks : 0;                // slice over blocks, or tile of rows
     const MoreMats none{};
-    skinny_tile<KIND, MT, 1, TERMS, false, true>(L->c[q].X, L->c[q].W, L->c[q].scale, L->c[q].out, L->M, L->c[q].N, L->c[q].K, L->c[q].ks,
-                                                 L->ring, L->c[q].partial, L->c[q].counters, none, at - by * blocks, kWaves, by, kb, 0);
+    skinny_tile<KIND, MT, S, TERMS, false, S == 1>(L->c[q].X, L->c[q].W, L->c[q].scale, L->c[q].out, L->M, L->c[q].N, L->c[q].K, L->c[q].ks,
+                                                   L->ring, L->c[q].partial, L->c[q].counters, none, at - piece * blocks, kWaves,
+                                                   S == 1 ? piece : 0, kb, S == 1 ? 0 : piece);
 }
 
 // Units of K in a wavefront's ring: its whole slice where `per_cu` such blocks fit the LDS of a CU.
@@ -1930,9 +1934,9 @@ bool launch_rows(hipStream_t s, int M, int N, int K, const void* x, const void* 
 }
 
 // The calls of L as one launch with `lds` bytes per block.
-template <int KIND, int MT, int TERMS>
+template <int KIND, int MT, int S, int TERMS>
 bool launch_calls(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_t lds) {
-    auto* kern = gemm_skinny_many<KIND, MT, TERMS>;
+    auto* kern = gemm_skinny_many<KIND, MT, S, TERMS>;
     if (lds > 65536 &&
         !MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsLimit)))))
@@ -1941,21 +1945,27 @@ bool launch_calls(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_t l
     return MI_HIP_OK(hipGetLastError());
 }
 template <int KIND, int TERMS>
-bool launch_calls_mt(hipStream_t s, const SkinnyCalls& L, unsigned blocks, size_t lds) {
-    switch ((L.M + 15) / 16) {
-        case 1: return launch_calls<KIND, 1, TERMS>(s, L, blocks, lds);
-        case 2: return launch_calls<KIND, 2, TERMS>(s, L, blocks, lds);
-        case 3: return launch_calls<KIND, 3, TERMS>(s, L, blocks, lds);
-        default: return launch_calls<KIND, 4, TERMS>(s, L, blocks, lds);
+bool launch_calls_mt(hipStream_t s, const SkinnyCalls& L, int mt, unsigned blocks, size_t lds) {
+    if (L.M > kMaxM) return mt == 3 ? launch_calls<KIND, 3, 2, TERMS>(s, L, blocks, lds) : launch_calls<KIND, 4, 2, TERMS>(s, L, blocks, lds);
+    switch (mt) {
+        case 1: return launch_calls<KIND, 1, 1, TERMS>(s, L, blocks, lds);
+        case 2: return launch_calls<KIND, 2, 1, TERMS>(s, L, blocks, lds);
+        case 3: return launch_calls<KIND, 3, 1, TERMS>(s, L, blocks, lds);
+        default: return launch_calls<KIND, 4, 1, TERMS>(s, L, blocks, lds);
     }
 }
 
-// n calls of one M <= kMaxM and weight kind in as few launches as hold them.  Calls whose slices meet in memory go
-// first, so that their last blocks' trips run under the others' work.
+// n calls of one M and weight kind in as few launches as hold them.  Calls whose slices meet in memory go first, so that
+// their last blocks' trips run under the others' work.  More than 64 rows: in the fewest tiles of at most 64 (fp16: 48) rows, 32
+// columns wide, the longest K first, and as much LDS as lets two blocks share a CU, one's loads under the other's products (one
+// block per CU: 130 int8 rows of 0.5B 21.1 against 15.5, 200 Q4 rows of 360M 25.9 against 21.0; fp16 in tiles of 64: 400 rows of 0.5B 35.9
+// against 33.4).  us per layer, launches of their own -> together: 80 fp16 rows of 135M 17.4 -> 8.0, 130 int8 rows of 0.5B 27.9 -> 15.5,
+// 700 int8 rows of 360M 49.8 -> 38.9, 2048 int8 rows of 0.5B (q, k, v and o) 105.0 -> 99.1.
 bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* workspace, size_t workspace_bytes) {
-    const int M = calls[0].M, mt = (M + 15) / 16;
+    const int M = calls[0].M, tiles_m = (M + kMaxM - 1) / kMaxM, mt_even = ((M + tiles_m - 1) / tiles_m + 15) / 16;
+    const int mt = tiles_m > 1 && (mt_even < 3 || calls[0].kind == WK_F16) ? 3 : mt_even, S = tiles_m > 1 ? 2 : 1, rows_m = (M + 16 * mt - 1) / (16 * mt);
     const WeightKind kind = calls[0].kind;
-    const size_t unit = unit_bytes(kind, mt, 1);
+    const size_t unit = std::max(unit_bytes(kind, mt, S), static_cast<size_t>(mt) * S * 1024);
     SkinnyCalls L;
     long blocks = 0;
     size_t sums = 0;
@@ -1965,26 +1975,28 @@ bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* w
         L.M = M;
         const int cus = device_info().cus;
         for (int j = 0; j < L.n; ++j) {
-            const int ring = ring_units(unit, kWaves, (blocks + cus - 1) / cus, L.c[j].K, L.c[j].ks, L.c[j].kb);
+            const int ring = ring_units(unit, kWaves, S == 2 ? 2 : (blocks + cus - 1) / cus, L.c[j].K, L.c[j].ks, L.c[j].kb);
             if (ring > L.ring) L.ring = ring;
         }
         const auto nb = static_cast<unsigned>(blocks);
         const size_t lds = kWaves * L.ring * unit;
-        const bool ok = kind == WK_Q4 ? (terms == 1 ? launch_calls_mt<WK_Q4, 1>(s, L, nb, lds) : launch_calls_mt<WK_Q4, 2>(s, L, nb, lds))
-                      : kind == WK_F16 ? launch_calls_mt<WK_F16, 1>(s, L, nb, lds) : launch_calls_mt<WK_I8, 1>(s, L, nb, lds);
+        const bool ok = kind == WK_Q4 ? (terms == 1 ? launch_calls_mt<WK_Q4, 1>(s, L, mt, nb, lds) : launch_calls_mt<WK_Q4, 2>(s, L, mt, nb, lds))
+                      : kind == WK_F16 ? launch_calls_mt<WK_F16, 1>(s, L, mt, nb, lds) : launch_calls_mt<WK_I8, 1>(s, L, mt, nb, lds);
         L = SkinnyCalls{};
         blocks = 0;
         sums = 0;
         counters = 0;
         return ok;
     };
-    for (int pass = 0; pass < 2; ++pass) {               // slices over blocks; the others
+    int longest = 0;
+    for (int i = 0; i < n; ++i) longest = calls[i].K > longest ? calls[i].K : longest;
+    for (int pass = 0; pass < 2; ++pass) {               // slices over blocks, or the longest K; the others
         for (int i = 0; i < n; ++i) {
             const GemvCall& c = calls[i];
-            const Shape sh = pick_shape(kind, M, c.N, c.K, device_info().cus, workspace_bytes);
-            if (pass != (sh.kb > 1 ? 0 : 1)) continue;
+            const Shape sh = M > kMaxM ? Shape{rows_ks(M, c.N, c.K), 1, S} : pick_shape(kind, M, c.N, c.K, device_info().cus, workspace_bytes);
+            if (pass != (sh.kb > 1 || (M > kMaxM && c.K == longest) ? 0 : 1)) continue;
             const int strips = (c.N + 15) / 16, per_block = kWaves / sh.ks;
-            const long along_n = (strips + per_block - 1) / per_block, nb = along_n * sh.kb;
+            const long along_n = ((c.N + 16 * S - 1) / (16 * S) + per_block - 1) / per_block, nb = along_n * sh.kb * (S == 2 ? rows_m : 1);
             if (nb > 65535) {
                 MI_ERROR_FMT("gemm: a call beyond a launch of several (M=%d N=%d K=%d)", M, c.N, c.K);
                 return false;
@@ -2100,9 +2112,25 @@ double gemm_estimate_us(WeightKind kind, int M, int N, int K, size_t workspace_b
     return wide_us < tiled_us ? wide_us : tiled_us;
 }
 
+static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t workspace_bytes);
+
+// A plan follows from these numbers alone and takes a host 1 to 2 us to make, most of it estimates of the wide kernel's
+// shapes, where a layer's calls come again and again: each thread keeps the last 64 it made, by their numbers.
 GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t workspace_bytes) {
+    const int set = gemm_mode(s), mode = set == 4 && kind != WK_Q4 ? 0 : set;   // mode 4 only concerns Q4 weights
+    struct Made { int mode = -1, kind = 0, M = 0, N = 0, K = 0; size_t bytes = 0; GemmPlan plan; };
+    constexpr unsigned kMade = 64;
+    thread_local Made made[kMade];
+    const unsigned h = (static_cast<unsigned>(N) * 2654435761u + static_cast<unsigned>(K) * 40503u + static_cast<unsigned>(M) * 97u +
+                        static_cast<unsigned>(kind)) >> 7;
+    Made& m = made[h % kMade];
+    if (m.mode != mode || m.kind != kind || m.M != M || m.N != N || m.K != K || m.bytes != workspace_bytes)
+        m = Made{mode, kind, M, N, K, workspace_bytes, make_plan(mode, kind, M, N, K, workspace_bytes)};
+    return m.plan;
+}
+
+static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t workspace_bytes) {
     GemmPlan p;
-    int mode = gemm_mode(s) == 4 && kind != WK_Q4 ? 0 : gemm_mode(s);   // mode 4 only concerns Q4 weights
     // 100 s + 10 + t: the wide kernel pinned to 32 t rows of x per block and s slices of K
     int pin_splits = 0;
     if (mode >= 111) { pin_splits = mode / 100; mode %= 100; }
@@ -2175,7 +2203,7 @@ GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t w
         const double tiled_us = tiled_estimate_us(M, N, K);
         // (the 64 x 64 tiles' estimate is for weights in the caches: 1.5 to 2.5 us less than from HBM, as they come in a model)
         // (many rows in tiles that go in bands keep those, a plan that is promised: 2048 x 960 x 960 int8 11.6 us against 12.2 here)
-        const bool banded = M > (K < 896 ? 1280 : 1024) && N >= 960 && K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);
+        const bool banded = M > (K < 896 ? 1280 : 1024) && (N >= 960 || K >= 896) && K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);
         if (mode == 0 && !banded && skinny::rows_preferred(kind, r, wide_us, splits, M, N, cus) && r.us < tiled_us + 1.5) return rows();
         if (mode != 0 || wide_us < tiled_us) {
             p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;
@@ -2377,15 +2405,20 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
     return launch_planned(s, p, kind, M, mat[0].N, K, x, mat[0].W, mat[0].scale, mat[0].out, workspace, ws_bytes, more) ? g : -1;
 }
 
+// Rows of x up to which calls in tiles of rows go out together (beyond, few calls are in tiles of rows).
+constexpr int kMostShared = 2048;
+
 GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
     if (!gemm_supported(c.kind, c.M, c.N, c.K, c.x, c.W, c.scale)) return GemmRoute::kRefused;
     const int mode = gemm_mode(s);
-    if (c.M > skinny::kMaxM && (mode == 0 || mode == 4))      // (without a plan: only the wide kernel's reach is missing for Q4)
+    if (c.M > kMostShared && (mode == 0 || mode == 4))        // (without a plan: only the wide kernel's reach is missing for Q4)
         return c.kind != WK_Q4 || wide_reaches(c.kind, c.M, c.N, c.K) ? GemmRoute::kAlone : GemmRoute::kRefused;
     const GemmPlan p = plan_gemm(s, c.kind, c.M, c.N, c.K, workspace_bytes);
     if (p.kernel < 1 || (p.kernel == 1 && p.k_slices > 1 && !wide::slices_fit(p.k_slices, c.M, c.N, c.K, workspace_bytes)))
         return GemmRoute::kRefused;
-    return p.kernel == 4 && (c.N + 15) / 16 <= 8191 ? GemmRoute::kShares : GemmRoute::kAlone;
+    // (tiles of rows: as many as a launch of several counts, in the slices that launch_many takes)
+    const bool rows = p.kernel == 6 && c.M > skinny::kMaxM && p.ks == skinny::rows_ks(c.M, c.N, c.K);
+    return (p.kernel == 4 || rows) && (c.N + 15) / 16 <= 8191 ? GemmRoute::kShares : GemmRoute::kAlone;
 }
 
 bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes) {

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from helpers import mil
+from test_gemm_many_gpu import _check, _weight
 from test_prefill_slices_mode4_gpu import _slices
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,20 @@ def test_tiles_of_rows_exact_on_integers(kind, rows):
             got = out.read(np.uint16, (rows * n + 8,))
             assert np.all(got[-8:] == 0x7bff)
             assert np.array_equal(got[:-8].view(np.float16).reshape(rows, n), want), (n, k, mode)
+
+
+@pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
+@pytest.mark.parametrize("rows", [65, 97, 128, 300, 513])
+def test_calls_in_tiles_of_rows_together_as_one_by_one(kind, rows):
+    """Independent calls of different x and K beyond 64 rows: one launch for those in tiles of rows, 2, 4 and 8 slices of K
+    side by side, ragged widths, a call of another kernel between them; each output bit for bit that of the call alone."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep, calls = mil.Queue(), [], []
+    for j, (k, n) in enumerate([(896, 1152), (896, 130), (576, 9728), (4864, 896), (64, 1), (960, 2560), (128, 4864), (2560, 17)]):
+        x = mil.Buffer.from_host(mil.synth_normal_f16(3 + j, 1.0, (rows, k)))
+        keep.append(x)
+        calls.append((rows, n, k, x, _weight(kind, n, k, 60 + j, keep)))
+    plans = {mil.linear_plan(queue, *c)[0] for c in calls}
+    print(f"{kind} rows {rows} plans {plans}", flush=True)
+    assert 6 in plans
+    _check(queue, calls, 3)
