@@ -99,12 +99,7 @@ __global__ __launch_bounds__(64) void rmsnorm_kernel(const uint16_t* __restrict_
         const float v = h_f(x[c]);
         acc = fmaf(v, v, acc);
     }
-    #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const float o = __shfl_down(acc, s, 64);      // work-item t adds work-item t + s
-        acc = acc + o;
-    }
-    const float total = __shfl(acc, 0, 64);
+    const float total = wave_tree_sum(acc);
     // sqrtf is the correctly rounded one (-fhip-fp32-correctly-rounded-divide-sqrt); the
     // __fsqrt_rn intrinsic is not, despite its name: it is off by an ulp for one input in six
     const float inv = rcp_rn(sqrtf(__fdiv_rn(total, static_cast<float>(cols)) + eps));
@@ -1386,12 +1381,7 @@ __global__ __launch_bounds__(64) void add_rmsnorm_rows_kernel(uint16_t* __restri
             acc = acc + d;
         }
     }
-    #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const float o = __shfl_down(acc, s, 64);
-        acc = acc + o;
-    }
-    const float total = __shfl(acc, 0, 64);
+    const float total = wave_tree_sum(acc);
     const float inv = rcp_rn(sqrtf(__fdiv_rn(total, static_cast<float>(cols)) + eps));
     #pragma unroll
     for (int g = 0; g < kGroups; ++g) {
@@ -1468,12 +1458,7 @@ __global__ __launch_bounds__(512) void slices_add_rmsnorm_kernel(const float* __
     __syncthreads();
     float acc = 0.0f;
     for (int g = 0; g < groups; ++g) acc = acc + sq[64 * g + lane];
-    #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const float o = __shfl_down(acc, s, 64);
-        acc = acc + o;
-    }
-    const float total = __shfl(acc, 0, 64);
+    const float total = wave_tree_sum(acc);
     const float inv = rcp_rn(sqrtf(__fdiv_rn(total, static_cast<float>(cols)) + eps));
     u16x4 o;
     #pragma unroll

@@ -50,6 +50,21 @@ __device__ __forceinline__ float wave_max(float m) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
 }
 
+// Lane 0's sum of the tree "work-item t adds work-item t + s", s = 32 .. 1, over a wavefront, in every lane (the same moves; a
+// trip through the LDS crossbar per step made a row's norm 0.3 us longer).
+template <int SH> __device__ __forceinline__ float add_from_above(float a) {
+    return a + __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(a), __float_as_int(a), 0x100 + SH, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float wave_tree_sum(float a) {
+    a = a + lane_plus32(a);
+    a = a + lane_plus16(a);
+    a = add_from_above<8>(a);
+    a = add_from_above<4>(a);
+    a = add_from_above<2>(a);
+    a = add_from_above<1>(a);
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a)));
+}
+
 // exp() of the SwiGLU epilogue: range reduction by ln2 in two parts and a degree-7 Horner
 // polynomial, built from fma/rint/ldexp only so that a host evaluation of the same
 // formula gives the same bits (the reference's native_exp has no defined precision,

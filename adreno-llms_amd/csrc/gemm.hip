@@ -2417,7 +2417,8 @@ GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
     if (p.kernel < 1 || (p.kernel == 1 && p.k_slices > 1 && !wide::slices_fit(p.k_slices, c.M, c.N, c.K, workspace_bytes)))
         return GemmRoute::kRefused;
     // (tiles of rows: as many as a launch of several counts, in the slices that launch_many takes)
-    const bool rows = p.kernel == 6 && c.M > skinny::kMaxM && p.ks == skinny::rows_ks(c.M, c.N, c.K);
+    const bool rows = p.kernel == 6 && c.M > skinny::kMaxM && p.ks == skinny::rows_ks(c.M, c.N, c.K) &&
+                      static_cast<long>((c.N + 31) / 32) * ((c.M + 47) / 48) <= 65535;
     return (p.kernel == 4 || rows) && (c.N + 15) / 16 <= 8191 ? GemmRoute::kShares : GemmRoute::kAlone;
 }
 
