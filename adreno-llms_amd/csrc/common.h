@@ -177,7 +177,7 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
 // by itself, or the streaming kernel serves it, which launch_gemm_many can have serve several.
 enum class GemmRoute { kRefused, kAlone, kShares };
 GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes);
-// n calls of one M and weight kind and of GemmRoute::kShares, of any x, K and N, none of which reads or writes what
+// n calls of one M and weight kind and of GemmRoute::kShares (up to 64 rows, or in tiles of rows), of any x, K and N, none of which reads or writes what
 // another one writes: in one launch where they fit it, each result what launch_gemm gives.
 bool launch_gemm_many(hipStream_t s, const GemvCall* calls, int n, void* workspace, size_t workspace_bytes);
 // A stream's workspace holds kWorkspaceBytes for whatever a launch puts there and, behind them, kSliceCounters

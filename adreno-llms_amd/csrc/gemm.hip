@@ -1346,7 +1346,7 @@ __device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ su
     return true;
 }
 
-// Up to 64 rows of x.  A wavefront owns a tile of 16 S columns of the output (S strips of 16 rows of W) and a slice of K, and
+// Up to 64 rows of x, or tiles of as many.  A wavefront owns a tile of 16 S columns of the output (S strips of 16 rows of W) and a slice of K, and
 // works for itself: it asks for its slice of x and of W, 64 values of K at a time, by direct global -> LDS loads into a ring of
 // its own, waits for its own loads only, and multiplies.  ks wavefronts of a block share a tile; their sums meet in LDS, in
 // slice order, behind the one barrier of the kernel.
@@ -1363,7 +1363,7 @@ __device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ su
 // 896 x 896 4.2 -> 3.7, 9728 x 896 with the SwiGLU 7.0 -> 6.7; Q4, 24 rows of 896 x 4864 9.8 -> 7.4; the floor of a launch is 1.6.
 // An int8 weight becomes fp16 in the registers (exactly).  Q4: q * scale as two exact fp16 terms (scale = hi + lo with 7 and
 // 4 significant bits, as in the wide kernel), or rounded to fp16 once with TERMS = 1.
-// GLU: see launch_gemm_glu; the tile's two strips are the gate's and the up matrix's (S = 2).
+// GLU: see launch_gemm_glu; the tile's strips are the gate's and the up matrix's in turn (S = 2, 4).
 // MEET: kb slices of K over blocks, which meet as told at meet_slices (an instance of its own, S = 1).
 // Without MEET and with `partial` the sums go there, [slice over blocks][M][N], for a launch that adds them (N a multiple of 4).
 template <int KIND, int MT, int S>
@@ -2277,8 +2277,8 @@ bool launch_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, const void
 
 // The SwiGLU of a stacked gate | up projection in the projection's own launch (or in the launch that adds its slices of
 // K).  W holds 16 rows of the gate matrix, the same 16 of the up matrix, the next 16 of the gate matrix, and so on: a
-// lane of the wide kernel then holds gate and up of a column in one accumulator, and the streaming kernel has them in
-// neighbouring wavefronts.  Both are rounded to fp16 as launch_gemm stores them, and the operations are swiglu_h's: the
+// lane of the wide kernel then holds gate and up of a column in one accumulator, and a wavefront of the streaming kernel
+// has them in neighbouring strips.  Both are rounded to fp16 as launch_gemm stores them, and the operations are swiglu_h's: the
 // result is that of the two launches bit for bit.  What it saves is the trip of 2 x inter columns through memory:
 // 2048 rows of 4864 + 4864 columns, 40 MB written and read again.
 // Measured: a 2048-token int8 prompt 4253 -> 4147 us, 300 Q4 tokens behind 900 2206 -> 2172, 37 fp16 tokens 1661 -> 1609;

@@ -574,7 +574,7 @@ static int launch_run(hipStream_t s, const GemvCall* c, int n, bool gemm) {
 // call of the window writes.  No order among them can be observed, so the runs of a window that one launch can hold go
 // out together: GEMVs of one M and weight kind (launch_gemv_many), GEMMs of one M and weight kind that the streaming
 // kernel serves (launch_gemm_many); the others as launches of their own.  One token's projections of SmolLM2-135M in
-// fp16, seven calls of four runs, 16.6 -> 4.8 us; of the 0.5B model at 16 int8 rows 26.6 -> 14.0 us; the 169 of Qwen2.5-0.5B in int8, each layer
+// fp16, seven calls of four runs, 16.6 -> 4.8 us; of the 0.5B model at 16 int8 rows 26.6 -> 7.4 us (launches and kernel); the 169 of Qwen2.5-0.5B in int8, each layer
 // with buffers of its own and so independent, 320 -> 93 us (three launches; a decode step in which attention stands
 // between them has its runs alone).
 int mi_linear_batch(void* stream, const mi_linear_call* calls, int n) {
