@@ -1677,13 +1677,14 @@ inline size_t partial_bytes(int mt, int N, int kb) { return static_cast<size_t>(
 // slices, 6.0 in 8).  kb: slices over blocks where one block per tile still leaves most CUs idle and the trip of the sums
 // through memory, 2.5 us, is less than what it saves (896 x 4864 at 16 rows: 8.7 us in 8 slices, 7.1 in 8 x 4).  S: two
 // strips per wavefront where one per wavefront is more blocks than CUs: x is fetched half as often (4864 x 896 at 48 int8 rows
-// 6.7 -> 6.1 us); fewer blocks than CUs with two lose (1152 x 896 at 16 rows 3.7 against 4.1).
+// 6.7 -> 6.1 us), up to 16 rows only from five blocks per CU on (Q4 32 000 x 320 8.0 with one); fewer blocks than CUs with two
+// lose (1152 x 896 at 16 rows 3.7 against 4.1).
 struct Shape { int ks, kb, S; };
 inline Shape pick_shape(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
     const int mt = (M + 15) / 16;
     const long strips = (N + 15) / 16;
     const int its = K / 64;
-    Shape sh{1, 1, strips > cus && mt > 1 ? 2 : 1};
+    Shape sh{1, 1, strips > cus && (mt > 1 || strips > 5L * cus) ? 2 : 1};
     const long tiles = (strips + sh.S - 1) / sh.S;
     const int most = 2 * kWaves * unit_bytes(kind, mt, 2) <= kLdsLimit ? kWaves : kWaves / 2;
     while (sh.ks < most && (sh.ks < 4 || tiles * sh.ks < (sh.S == 2 ? 5L : 4L) * cus) && its >= 2 * sh.ks) sh.ks *= 2;
@@ -1713,12 +1714,13 @@ inline Shape pick_apart(int kind, int M, int N, int K, int cus, size_t workspace
 //    only to 48 rows, a plan that is promised, though 1024 x 512 at 64 takes 4.1 against 5.9.)
 //  - fp16 of more than 8192 rows of W only up to 32: 9728 x 896 at 32 / 48 / 64 rows 8.5 / 9.6 / 10.5 against 8.8 / 9.3 / 9.7 (the tiles fetch
 //    x once per 64 rows of W); int8 9728 x 896 at 48 8.5 against 8.8, 19 456 x 896 11.2 against 11.5.
-//  - Not beyond 36 MB of weights or 80 rows of W per CU: the wide kernel's higher streaming rate wins there (int8 49 152 x 576 at
-//    16 rows 11.2 against 7.3).
+//  - Not beyond 36 MB of weights, nor, above 13.5 MB, 80 rows of W per CU: the wide kernel's higher streaming rate wins there (int8
+//    49 152 x 576 at 16 rows 11.2 against 7.3).
 inline bool preferred(int kind, int M, int N, int K, int cus) {
     const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
     const long strips = (N + 15) / 16;
-    return M <= (kind == WK_I8 && K <= 512 ? 48 : kind == WK_F16 && strips > 2L * cus ? 32 : 64) && w_bytes <= 36.0e6 && strips <= 5L * cus;
+    return M <= (kind == WK_I8 && K <= 512 ? 48 : kind == WK_F16 && strips > 2L * cus ? 32 : 64) &&
+           (w_bytes <= 13.5e6 ? strips <= (M > 48 ? 10L : 16L) * cus : w_bytes <= 36.0e6 && strips <= 5L * cus);
 }
 
 // ---- more rows of x than a tile holds: tiles of 16 mt rows by 16 S columns ----
