@@ -1730,21 +1730,23 @@ inline bool preferred(int kind, int M, int N, int K, int cus) {
 // 17.8 -> 15.8, 100 fp16 rows of 896 x 4864 14.2 -> 8.2.  From about 600 rows on by many columns the wide kernel's larger tiles
 // win: a block here pulls 1 byte into LDS for 25 to 60 multiplications, there for 140.
 //
-//
-// A launch takes 4.1 us and, per block on a CU, what it pulls into LDS and its share of multiplying: fitted to 2341 launches of 65
-// to 2048 rows (8 % rms; the shape it picks is 2 % behind the best one in the mean).  Blocks beyond one per CU come in rounds, a
-// last round that is not full at 0.7 of its price (the blocks in it have the L2s to themselves).  Four strips to a wavefront leave
-// a CU with one block: 1.15 to 1.3 times as long; with Q4 never the best.
+// A launch takes 3.5 us and more the larger the tile, and for every round of blocks on the CUs the tile's end and what a block pulls
+// into LDS: int8 and fp16 fitted to 4600 launches of 65 to 2048 rows, every tile at each of 310 calls (8 % rms; the tile it picks is 1 %
+// behind the best one in the mean), Q4 to 1300 (10 %).  Blocks beyond one per CU come in rounds, a last round that is not full
+// at about 0.6 of its price (the blocks in it have the L2s to themselves).  Tiles of 64 columns leave a CU with one block and wait
+// for more before they begin, which a short K does not pay back (512 rows of 1536 x 576 fp16 7.5 us, with 32 columns 6.5); with Q4 never the best.
 struct RowShape { int mt = 0, S = 1, ks = 4, kb = 1; double us = 1e30; };
 inline double rows_us(int kind, int mt, int S, int kb, int M, int N, int K, int cus) {
     const long blocks = static_cast<long>((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * S - 1) / (16 * S)) * kb;
-    const double unit = static_cast<double>(unit_bytes(kind, mt, S));
-    const double unit_us = kind == WK_F16 ? (unit / 118.0e3 + mt * S * 0.0053) * (S == 4 ? 1.15 : 1.0)
-                         : kind == WK_I8  ? (unit / 94.0e3 + mt * S * 0.0027) * (S == 4 ? 1.33 : S == 1 ? 0.88 : 1.0)
-                                          : unit / 57.0e3 * (S == 1 ? 0.72 : 1.0);
-    const double mean = static_cast<double>(blocks) / cus;
+    const double unit = static_cast<double>(unit_bytes(kind, mt, S)), its = K / 64.0 / kb, mean = static_cast<double>(blocks) / cus;
     const long full = (blocks + cus - 1) / cus;
-    return 4.1 + (full == 1 ? 1.0 : 0.7 * full + 0.3 * mean) * (K / 64.0 / kb) * unit_us;
+    auto rounds = [&](double f) { return full == 1 ? 1.0 : f * full + (1.0 - f) * mean; };
+    if (kind == WK_Q4) return 4.1 + rounds(0.7) * its * unit / 57.0e3 * (S == 1 ? 0.72 : 1.0);
+    if (kind == WK_F16)
+        return 3.43 + 0.047 * mt * S + (S == 4 ? 0.25 : 0.0) +
+               rounds(0.58) * (0.043 * mt * S + its * unit / 80.4e3 * (S == 4 ? 1.16 : S == 1 ? 0.92 : 1.0));
+    return 3.51 + 0.047 * mt * S + (S == 4 ? 0.6 : 0.0) +
+           rounds(0.64) * (0.022 * mt * S + its * unit / 74.6e3 * (S == 4 ? 1.26 : S == 1 ? 0.85 : 1.0));
 }
 // Slices of K inside a block, by what a launch by itself, one among several matrices and one with the SwiGLU have in
 // common, since they decide the order of the sums.
@@ -1768,12 +1770,30 @@ inline RowShape pick_rows(int kind, int M, int N, int K, int cus, bool glu) {
         }
     return best;
 }
-// Where they are the choice over the wide kernel, by its estimate (which is 4 to 7 us too high for slices of K, 1200 x 896 x 4864
-// in three 25.6 us, estimated at 32.6, and 1 too low for a few rows of fp16, 300 x 5120 x 960 12.5 against 10.7 here), and not for many rows of W (see preferred) or many of both: 600 x 3072 x 576 int8 9.0 against
-// 8.2, 600 x 5120 x 960 17.5 against 14.1; Q4 450 x 3072 x 576 8.6 against 10.2, but 900 x 3072 x 576 13.3 against 11.9; fp16 2048 x
-// 896 x 896 11.6 against 10.1, 1200 x 896 x 896 8.1 against 9.9.
-inline bool rows_preferred(int kind, const RowShape& r, double wide_us, int wide_slices, int M, int N, int cus) {
-    return (N + 15) / 16 <= 5L * cus && !(N > 2560 && M > (kind == WK_Q4 ? 512 : 304)) && !(kind == WK_F16 && M > 1280) && r.us < (wide_slices == 1 ? 1.0 : M <= 1024 ? 0.85 : 0.7) * wide_us + (kind == WK_F16 && M <= 304 ? 0.8 : 0.0);
+// Where they are the choice over the kernels above, by the estimates of all (us, weights from HBM, tiles of rows / the other).
+//  - Up to 64 rows of W per CU with Q4, 48 otherwise: beyond, the others stream better (80 int8 rows of 19 456 x 896 14.9 / 12.1, 100
+//    Q4 rows 18.2 / 16.1, 56 fp16 rows of 14 592 x 896 13.6 / 10.3).
+//  - Up to 8192 outputs per CU, about five rounds of tiles, from where 140 multiplications per byte pulled into LDS beat 25 to 60 (int8 512
+//    rows of 4096 x 512 7.7 / 6.7); 9600 with Q4, which the wide kernel multiplies twice (3072 rows of 1536 x 576 20.4 / 16.2, 2600 of
+//    1152 x 896 18.9 / 16.6), and at a long K up to 2e7 products per CU (600 rows of 2048 x 8192 67 / 51; 2560 x 2560 at 600 / 800 rows
+//    25 / 27 and 37 / 32).  Many columns, the gate and up matrices of a prompt, whose SwiGLU rides in the launch: 300 x 9728 x 896 Q4 17.6 / 16.1
+//    without it, but the prompt of 300 tokens 1477 / 1545.  Fewer rows for them: 600 x 3072 x 576 int8 9.0 / 8.2, 600 x 5120 x 960 17.5 / 14.1.
+//    fp16 to 1280 rows (2048 x 896 x 896 11.6 / 10.1), int8 to 3072 (4096 x 333 x 1920 24.1 / 20.9).
+//  - The estimates' own errors: the wide kernel's is 5 to 10 % too low without slices of K and 20 to 50 % too high with them (1200 x 896 x
+//    4864 in three 25.6 us, estimated at 32.6; fp16 130 x 2048 x 8192 20.1, at 24.4), for a few rows of fp16 0.5 us too low on top (300 x
+//    5120 x 960 12.5 against 10.7 here); the 64 x 64 tiles' is for weights in the caches, from HBM up to 1.5 us too low, the less the
+//    shorter K (200 rows of 4096 x 256 6.0 / 4.4 as they were chosen with 1.5 for any K); this one's 8 % too low for int8 beyond 8192 rows of W,
+//    in two slices of K.
+// Of 2016 calls (30 shapes of W, 40 to 4096 rows, every kind) 20 are 3 to 16 % slower than with the kernels above alone, by 0.2 to 1.5 us: int8 1200 x
+// 1536 x 576 8.8 / 7.6, fp16 300 x 3072 x 576 7.1 / 6.5, int8 600 x 1536 x 576 6.9 / 6.5.  Their layers, calls together, and prompts are
+// the faster for them (a layer of 600 int8 rows 17.9 / 23.0 us, of 1200 29.4 / 32.8, 30 layers of 300 fp16 rows 1230 / 1360).
+inline bool rows_preferred(int kind, const RowShape& r, double wide_us, int wide_slices, double tiled_us, int M, int N, int K, int cus) {
+    const double outs = static_cast<double>(M) * N, us = r.us * (kind == WK_I8 && N > 8192 ? 1.08 : 1.0);
+    if (N > (kind == WK_Q4 ? 64L : 48L) * cus || outs > (kind != WK_Q4 ? 8192.0 : N > 2560 ? 16000.0 : 9600.0) * cus || (kind == WK_Q4 && outs * K > 2.0e7 * cus)) return false;
+    if ((N > 2560 && M > (kind == WK_Q4 ? 512 : 304)) || M > (kind == WK_F16 ? 1280 : kind == WK_I8 ? 3072 : 1 << 30)) return false;
+    if (wide_slices > 1) wide_us *= kind == WK_F16 ? 0.82 : M <= 1024 ? 0.85 : 0.7;
+    else if (kind != WK_Q4) wide_us = kind == WK_I8 ? 1.05 * wide_us : 1.1 * wide_us + (M <= 304 ? 0.5 : 0.0);
+    return us < wide_us && (kind == WK_Q4 || us < tiled_us + (K < 640 ? (K - 128) / 345.0 : 1.5));
 }
 // The same cut into slices over blocks for a launch that adds them (mt = 0: not worth it).
 inline RowShape pick_rows_apart(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
@@ -2158,7 +2178,7 @@ static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t
         wide::pick_shape(WK_Q4, p.terms, M, N, K, cus, may_slice ? workspace_bytes : 0, &tm, &splits, &wide_us);
         if (may_slice || mode == 6) {
             const skinny::RowShape r = skinny::pick_rows(kind, M, N, K, cus, false);
-            if (mode == 6 || skinny::rows_preferred(kind, r, wide_us, splits, M, N, cus)) {
+            if (mode == 6 || skinny::rows_preferred(kind, r, wide_us, splits, 0.0, M, N, K, cus)) {
                 p.kernel = 6; p.tile_rows = 16 * r.mt; p.ks = r.ks; p.strips = r.S;
                 return p;
             }
@@ -2203,10 +2223,9 @@ static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t
         if (mode >= 11) tm = mode - 10;
         if (pin_splits) splits = pin_splits;
         const double tiled_us = tiled_estimate_us(M, N, K);
-        // (the 64 x 64 tiles' estimate is for weights in the caches: 1.5 to 2.5 us less than from HBM, as they come in a model)
         // (many rows in tiles that go in bands keep those, a plan that is promised: 2048 x 960 x 960 int8 11.6 us against 12.2 here)
         const bool banded = M > (K < 896 ? 1280 : 1024) && (N >= 960 || K >= 896) && K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);
-        if (mode == 0 && !banded && skinny::rows_preferred(kind, r, wide_us, splits, M, N, cus) && r.us < tiled_us + 1.5) return rows();
+        if (mode == 0 && !banded && skinny::rows_preferred(kind, r, wide_us, splits, tiled_us, M, N, K, cus)) return rows();
         if (mode != 0 || wide_us < tiled_us) {
             p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;
             return p;
