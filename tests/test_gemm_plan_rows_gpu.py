@@ -32,3 +32,18 @@ def test_the_choice_is_near_the_fastest_pinned_kernel(queue, kind, M, N, K):  # 
         if worst[0] <= BEHIND:
             return
     assert False, f"{kind} M={M} N={N} K={K}: plan {worst[1]} takes {worst[0]:.2f} times what mode {worst[2]} does"
+
+
+@pytest.mark.parametrize("kind,M,N,K,plan", [
+    ("f16", 16, 1536, 576, (4, 16, 4)), ("int8", 24, 960, 704, (4, 32, 4)), ("q4", 16, 576, 576, (4, 16, 4)),       # a short K: 4 slices,
+    ("int8", 24, 960, 768, (4, 32, 8)), ("q4", 24, 1600, 960, (4, 32, 8)),                                          # 8 from 768 on
+    ("q4", 8, 2048, 2048, (4, 16, 8)), ("int8", 16, 2048, 2048, (4, 16, 8)),                                        # one block per strip,
+    ("int8", 16, 2048, 2112, (4, 16, 16)), ("int8", 16, 896, 4864, (4, 16, 32)),                                    # over blocks beyond 4 units each
+    ("int8", 32, 32000, 320, (4, 32, 4)), ("int8", 33, 32000, 320, (2, 64, 1)),                                     # many rows of W
+    ("int8", 48, 14592, 896, (4, 48, 4)), ("int8", 49, 14592, 896, (2, 64, 1)), ("int8", 64, 9728, 896, (4, 64, 8))])
+def test_slices_of_the_streaming_kernel_where_they_measured_faster(kind, M, N, K, plan):
+    """Both sides of the lines of pick_shape and preferred for up to 64 rows."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep = mil.Queue(), []
+    x, w = mil.Buffer(2 * M * K), _weights(kind, N, K, 73, keep)
+    assert mil.linear_plan(queue, M, N, K, x, w) == plan
