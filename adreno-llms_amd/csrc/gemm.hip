@@ -1820,902 +1820,6 @@ inline RowShape pick_rows_apart(int kind, int M, int N, int K, int cus, size_t w
 // Estimated time (us): what decides between this kernel and rows of GEMV below 16 rows.  Fitted to the kernel that took fragments
 // from memory, with its slices, and 0.3 to 1 us too high: 8 to 15 rows of a small matrix stay rows of GEMV, whose results are the
 // reference's order bit for bit, though 16 rows of a 0.5B layer take 7.4 us here and 8 rows 12 there.
-inline double estimate_us(int kind, int terms, int tm, int splits, int M, int N, int K, int cus) {
-    const long blocks = static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + kBN - 1) / kBN) * splits;
-    const int stages = (K / 64 + splits - 1) / splits;
-    const double stage_us = kind == WK_Q4 ? (terms == 2 ? 0.49 + 0.22 * tm : 0.56 + 0.10 * tm)
-                          : kind == WK_F16 ? 0.35 + 0.10 * tm : 0.27 + 0.10 * tm;
-    // two blocks on one CU take about 1.4 times as long each as one alone (the dispatcher puts a
-    // second block on a CU only when every CU has one)
-    const int per_cu = blocks > cus ? blocks_per_cu(kind, tm) : 1;
-    const double block_us = (2.6 + 0.5 * tm + stages * stage_us) * (per_cu == 2 ? 1.4 : 1.0);
-    const long slots = static_cast<long>(cus) * per_cu;
-    const long full = (blocks - 1) / slots, rem = blocks - full * slots;     // the last round, full or not, is `rem`
-    // (64-row tiles of int8 / fp16 weights, unsliced, on more than half of the CUs and at most one per CU,
-    //  run nearly as on an empty chip: 512 x 4864 x 896 in 11.2 us where the general factor says 13.6 and the
-    //  64 x 64 tiles, estimated at 13.5, take 13.2; 2048 x 1152 x 896 13.2 against 15.9, 512 x 4608 x 1024 12.1
-    //  against 14.5, 4096 x 576 x 1536 18.9 against 33.5.  With fewer blocks the long serial K of such
-    //  shapes decides and the general factor holds: 2048 x 896 x 4864 unsliced 47 against 37 us in two slices.
-    //  32-row tiles likewise at a K of 1280 to 3072, where the 64 x 64 tiles slow down as soon as a CU holds
-    //  two of them: 1536 x 576 x 1536 19.2 -> 14.6 us, 1024 x 2048 x 2048 23.2 -> 18.4, 192 x 8192 x 2048 21.6 ->
-    //  17.3, fp16 1536 x 1024 x 2560 29.6 -> 22.7, and from K = 1024 on (2048 x 1024 x 1024: 12.2 against 14.5 us);
-    //  at a shorter K the 64 x 64 tiles stay ahead (1536 x 1152 x 896 10.2 against 11.2), at a longer one
-    //  slices do (1536 x 896 x 4864 32.6 against 37.7).
-    //  Q4 weights in two terms behave the same there (1024 x 2048 x 2048 in 32-row tiles 29.1 us against 34.0
-    //  in two slices, 256 x 8192 x 2048 29.2 against 35.0, 2048 x 576 x 1536 21.7 against 24.2), and their tall
-    //  tiles, one block per CU and twice the matrix work per byte, lose less to a full chip than the general
-    //  factors say: 2048 x 4864 x 896 in 160-row tiles 34.8 us (a block alone: 27.4), 4096 x 8192 x 2048 in
-    //  128-row tiles 231 us for four rounds of 48.4, against 258 us for the 64-row tiles the factors preferred.)
-    //  fp16 weights do so at any number of blocks and from 9 stages on: 300 x 4864 x 896 9.7 us, 416 x 5120 x 960 11.5, 917 x 3072 x
-    //  576 8.5, where the general factor put the 64 x 64 tiles ahead, which take 11.8, 12.5 and 9.3.
-    const bool bands = stages <= 16 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);      // (the 64 x 64 tiles are the faster then)
-    const bool f16_roomy = kind == WK_F16 && splits == 1 && blocks <= cus && tm <= 2 && stages <= 48 && !bands;
-    // (int8, 32-row tiles of 14 or 15 stages: 304 x 4864 x 896 9.4 us, 192 x 9728 x 896 9.6, 320 x 5120 x 960 9.9, the 64 x 64 tiles
-    //  9.6, 9.6 and 10.0, which leave the SwiGLU to a launch of its own.  Not where those go in bands: int8 2048 x 960 x 960 11.4
-    //  against 10.4, fp16 1184 x 1600 x 960 12.5 against 10.4, 1408 x 960 x 576 7.7 against 7.2; at a longer K the wide tiles keep up:
-    //  1856 x 576 x 1536 13.6 against 14.4)
-    const bool i8_short = kind == WK_I8 && splits == 1 && tm == 1 && blocks > cus / 2 && blocks <= cus && (stages == 14 || stages == 15) && !bands;
-    const bool roomy = splits == 1 && blocks > cus / 2 && blocks <= cus &&
-                       (tm == 2 || (tm == 1 && stages >= 16 && stages <= 48));
-    const bool q4_tall = kind == WK_Q4 && terms == 2 && tm >= 3 && splits == 1;
-    const double crowd = f16_roomy ? (blocks * 5 > slots * 4 ? 0.2 : 0.05) : i8_short ? 0.4 : roomy ? 0.2 : q4_tall ? 0.3 : 0.56;
-    const double round = q4_tall ? 1.25 : 1.56;
-    double t = full * round * block_us + (rem ? (1.0 + crowd * rem / slots) * block_us : 0.0);
-    // every row of tiles streams W again: not faster than that many bytes at about 6.8 TB/s, or,
-    // for a W that stays in the memory-side cache (40 MB taken as the limit: fp16 8192 x 2048, 33.5 MB, still
-    // runs eight rows of tiles in 25.9 us, and the choices at 50 MB and more are right as they are), 2.2 times that for
-    // the reads after the first
-    const double w_once = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_I8 ? 1.0 : 0.5625);
-    const int tiles_m = (M + 32 * tm - 1) / (32 * tm);
-    const double w_bytes = w_once <= 40.0e6 ? w_once * (1.0 + (tiles_m - 1) / 2.2) : w_once * tiles_m;
-    if (t < 2.5 + w_bytes / 6.8e6) t = 2.5 + w_bytes / 6.8e6;
-    if (splits > 1) t += 2.5 + 2.0 * splits * M * static_cast<double>(N) * 4 / 4.0e6;   // ~4 TB/s there and back
-    return t;
-}
-
-// Rows of x per block (in units of 32) and slices of K with the smallest estimated time; slices
-// only as far as their fp32 partial sums fit the workspace.
-inline void pick_shape(int kind, int terms, int M, int N, int K, int cus, size_t workspace_bytes, int* tm_out,
-                       int* splits_out, double* best_us) {
-    static const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
-    double best_t = 1e30;
-    for (int tm = 1; tm <= 5; ++tm) {
-        if (32 * (tm - 1) >= M) break;                   // no tile taller than x needs (16 x 49 152 x 576: 7.8 against 8.7 us)
-        for (int sp : kSplits) {
-            if (sp > 1 && (K / 64 < 2 * sp || static_cast<double>(sp) * M * N * 4 > static_cast<double>(workspace_bytes)))
-                continue;
-            const double t = estimate_us(kind, terms, tm, sp, M, N, K, cus);
-            if (t < best_t) { best_t = t; *tm_out = tm; *splits_out = sp; }
-        }
-    }
-    if (best_us) *best_us = best_t;
-}
-
-// The same among two slices and more: false where none fits.
-inline bool pick_sliced(int kind, int terms, int M, int N, int K, int cus, size_t workspace_bytes, int* tm_out, int* splits_out,
-                        double* best_us) {
-    *best_us = 1e30;
-    for (int tm = 1; tm <= 5 && 32 * (tm - 1) < M; ++tm)
-        for (int sp : {2, 3, 4, 6, 8, 12, 16, 24}) {
-            if (!slices_fit(sp, M, N, K, workspace_bytes)) continue;
-            const double t = estimate_us(kind, terms, tm, sp, M, N, K, cus);
-            if (t < *best_us) { *best_us = t; *tm_out = tm; *splits_out = sp; }
-        }
-    return *best_us < 1e30;
-}
-
-template <int KIND, int TERMS>
-bool launch_any(int tm, hipStream_t s, int M, int N, int K, const void* x, const void* W,
-                const void* scale, void* out, float* partial, size_t partial_bytes, int splits, const MoreMats& more,
-                bool glu) {
-    switch (tm) {
-        case 1: return launch<1, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more, glu);
-        case 2: return launch<2, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more, glu);
-        case 3: return launch<3, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more, glu);
-        case 4: return launch<4, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more, glu);
-        default: return launch<5, KIND, TERMS>(s, M, N, K, x, W, scale, out, partial, partial_bytes, splits, more, glu);
-    }
-}
-
-}  // namespace wide
-
-// ---- 256 x 256 blocks, 128 x 128 per wavefront (int8 weights) --------------------------------------
-//
-// The wide kernel above gives a wavefront 64 rows of W against up to 160 rows of x: per MFMA it reads
-// (2 + 2 TM) / (4 TM) fragments from LDS, and at 160 rows that traffic (133 KB per stage of K = 64) takes
-// the LDS four fifths as long as the MFMAs take the matrix cores, overlapped by less than half.  Here the
-// four wavefronts sit two along x by two along W and each owns 128 x 128 of the block's 256 x 256 outputs:
-// sixteen 32 x 32 accumulators (all 256 AGPRs), four fragments of W and four of x per 16 MFMAs, 37 % less
-// LDS read traffic and 19 % less fill traffic per MFMA.  Same LDS layout, swizzles, K permutation, fills
-// and barrier scheme as the wide kernel; three stages of 48 KB.  It needs whole rounds of 256-row tiles to
-// pay: a few hundred tiles at least, and a long K (each block's prologue and epilogue stand alone on its CU).
-namespace quad {
-
-constexpr int kBM = 256, kBN = 256, kStages = 3;
-constexpr int kXStage = kBM * 128, kWStage = kBN * 64, kStage = kXStage + kWStage;
-constexpr int kXLoads = 8, kWLoads = 4, kLoads = kXLoads + kWLoads;   // 1 KB loads per wavefront and stage
-constexpr int kReads = 12, kConv = 16, kMfmas = 32;                   // per half stage (K = 32)
-constexpr int kERow = 272;                                            // epilogue: 128 columns of fp16 + 16 bytes
-
-struct Frags {
-    u32x4 w[4];                // 16 int8 weights of four 32-row fragments of W
-    uint32_t wf[4][2][4];      // the same as fp16: [fragment][MFMA of the pair][4 dwords = 8 halves]
-    u32x4 x[2][4];             // [MFMA of the pair][32-row fragment of x]
-};
-
-using wide::lds_fill16;
-using wide::static_for;
-using wide::pack_half2;
-
-__global__ __launch_bounds__(256) void gemm_quad(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
-                                                 const uint16_t* __restrict__ scale, uint16_t* __restrict__ out,
-                                                 int M, int N, int K) {
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wr = w >> 1, wc = w & 1;                  // this wavefront's 128 rows of x, 128 rows of W
-    const int g = lane >> 5, li = lane & 31;
-    // block -> tile: as in the wide kernel (an XCD takes a contiguous eighth of the list, bands of 4 tiles along N)
-    int tile_m, tile_n;
-    {
-        const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN, total = tiles_m * tiles_n;
-        const int per_xcd = (total + 7) / 8;
-        const int l = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-        if (blockIdx.x >= 8 * per_xcd || l >= total) return;          // whole block, before any barrier
-        constexpr int kBand = 4;
-        const int band = l / (kBand * tiles_m);
-        const int width = tiles_n - band * kBand < kBand ? tiles_n - band * kBand : kBand;
-        const int in_band = l - band * kBand * tiles_m;
-        tile_m = in_band / width;
-        tile_n = band * kBand + in_band % width;
-    }
-    const int m0 = tile_m * kBM, n0 = tile_n * kBN;
-    const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((wide::lds_u8*)lds));
-
-    // fill side: x load j covers rows 8 (w + 4 j) .. + 7 of the tile (128 bytes each, chunk p of row r in slot
-    // p ^ ((r >> 1) & 7)); W load j rows 16 (4 w + j) .. + 15 (64 bytes each, slot p ^ ((r >> 2) & 3))
-    uint32_t xsrc[kXLoads], wsrc[kWLoads];
-    #pragma unroll
-    for (int j = 0; j < kXLoads; ++j) {
-        const int r = 8 * (w + 4 * j) + (lane >> 3);
-        const int c = (lane & 7) ^ ((r >> 1) & 7);
-        const int m = m0 + r < M ? m0 + r : M - 1;
-        xsrc[j] = static_cast<uint32_t>(m) * K * 2u + c * 16u;
-    }
-    #pragma unroll
-    for (int j = 0; j < kWLoads; ++j) {
-        const int r = 16 * (4 * w + j) + (lane >> 2);
-        const int c = (lane & 3) ^ ((r >> 2) & 3);
-        const int n = n0 + r < N ? n0 + r : N - 1;
-        wsrc[j] = static_cast<uint32_t>(n) * K + c * 16u;
-    }
-    const uint8_t* Xb = reinterpret_cast<const uint8_t*>(X);
-    auto fill_one = [&](int stage_k, int slot, auto jc) {
-        constexpr int j = decltype(jc)::value;
-        uint8_t* xs = lds + slot * kStage;
-        if constexpr (j < kXLoads)
-            lds_fill16(Xb + static_cast<size_t>(stage_k) * 128 + xsrc[j], xs + 1024 * (w + 4 * j));
-        else
-            lds_fill16(W + static_cast<size_t>(stage_k) * 64 + wsrc[j - kXLoads], xs + kXStage + 1024 * (4 * w + (j - kXLoads)));
-    };
-    auto fill_stage = [&](int stage_k, int slot) {
-        static_for<kLoads>([&](auto jc) { fill_one(stage_k, slot, jc); });
-    };
-
-    // read side: pair S of a stage, MFMA e of the pair: x chunk 4 S + 2 g + e, W chunk 2 S + g
-    const uint32_t xrow = lbase + (128u * wr + li) * 128u, xq = (2u * g) ^ ((li >> 1) & 7u);
-    const uint32_t wrow = lbase + kXStage + (128u * wc + li) * 64u, wq = g ^ ((li >> 2) & 3u);
-    uint32_t xoff[2][2], woff[2];
-    #pragma unroll
-    for (int S = 0; S < 2; ++S) {
-        #pragma unroll
-        for (int e = 0; e < 2; ++e) xoff[S][e] = xrow + (((4u * S + e) ^ xq) << 4);
-        woff[S] = wrow + (((2u * S) ^ wq) << 4);
-    }
-    // read j of a set: the four W fragments first, then x for the first and the second MFMA of the pair
-    auto read_one = [&](Frags& F, uint32_t slot_bytes, auto Sc, auto jc) {
-        constexpr int S = decltype(Sc)::value, j = decltype(jc)::value;
-        if constexpr (j < 4) {
-            const uint32_t a = woff[S] + slot_bytes;
-            MI_LDS_READ16(F.w[j], a, j * 32 * 64);
-        } else {
-            constexpr int e = (j - 4) / 4, t = (j - 4) % 4;
-            const uint32_t a = xoff[S][e] + slot_bytes;
-            MI_LDS_READ16(F.x[e][t], a, t * 4096);
-        }
-    };
-    auto convert_one = [&](Frags& F, auto jc) {
-        constexpr int j = decltype(jc)::value, u = j / 4, d = j % 4;
-        i8x4_to_h4(F.w[u][d], F.wf[u][d / 2][2 * (d % 2)], F.wf[u][d / 2][2 * (d % 2) + 1]);
-    };
-
-    floatx16 acc[4][4];
-    #pragma unroll
-    for (int u = 0; u < 4; ++u)
-        #pragma unroll
-        for (int t = 0; t < 4; ++t)
-            #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[u][t][r] = 0.0f;
-
-    auto mfma_one = [&](const Frags& F, auto nc) {
-        constexpr int n = decltype(nc)::value, e = n / 16, u = (n / 4) % 4, t = n % 4;
-        const u32x4 wv = u32x4{F.wf[u][e][0], F.wf[u][e][1], F.wf[u][e][2], F.wf[u][e][3]};
-        acc[u][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, wv),
-                                                          __builtin_bit_cast(half8, F.x[e][t]), acc[u][t], 0, 0, 0);
-    };
-
-    // one half stage: the fills of a later stage, the reads and conversions of the next fragments, dealt out
-    // between the MFMAs of the current ones
-    auto half_stage = [&](Frags& C, Frags& Nx, uint32_t next_bytes, auto NSc, auto fillc, int fill_k, int fill_slot) {
-        constexpr bool FILL = decltype(fillc)::value;
-        constexpr int nF = FILL ? kLoads : 0;
-        constexpr int A = nF + kReads + 1 + kConv;
-        static_for<kMfmas>([&](auto nc) {
-            constexpr int n = decltype(nc)::value;
-            mfma_one(C, nc);
-            MI_SCHED_FENCE();
-            constexpr int a0 = n * A / kMfmas, a1 = (n + 1) * A / kMfmas;
-            static_for<a1 - a0>([&](auto kc) {
-                constexpr int a = a0 + decltype(kc)::value;
-                if constexpr (a < nF) {
-                    fill_one(fill_k, fill_slot, std::integral_constant<int, a>{});
-                } else if constexpr (a < nF + kReads) {
-                    read_one(Nx, next_bytes, NSc, std::integral_constant<int, a - nF>{});
-                } else if constexpr (a == nF + kReads) {
-                    // LDS returns in order: with the eight x reads outstanding, the four W reads are back
-                    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(Nx.w[0]), "+v"(Nx.w[1]), "+v"(Nx.w[2]), "+v"(Nx.w[3]) : : "memory");
-                    MI_SCHED_FENCE();
-                } else {
-                    convert_one(Nx, std::integral_constant<int, a - nF - kReads - 1>{});
-                }
-            });
-            MI_SCHED_FENCE();
-        });
-        MI_WAIT_LGKM(0);
-        MI_SCHED_FENCE();
-    };
-    // at most `stages` (0 or 1) of this wavefront's stage fills still in flight
-    auto wait_fills = [&](int stages) {
-        if (stages >= 1) MI_WAIT_VM(kLoads); else MI_WAIT_VM(0);
-    };
-
-    const int nk = K / 64;
-    Frags FA, FB;
-    #pragma unroll
-    for (int st = 0; st < kStages - 1; ++st)
-        if (st < nk) fill_stage(st, st);
-    wait_fills((nk < kStages - 1 ? nk : kStages - 1) - 1);          // stage 0 has landed
-    __builtin_amdgcn_s_barrier();
-    MI_SCHED_FENCE();
-    static_for<kReads>([&](auto jc) { read_one(FA, 0u, std::integral_constant<int, 0>{}, jc); });
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(FA.w[0]), "+v"(FA.w[1]), "+v"(FA.w[2]), "+v"(FA.w[3]) : : "memory");
-    MI_SCHED_FENCE();
-    static_for<kConv>([&](auto jc) { convert_one(FA, jc); });
-
-    auto stage = [&](int i, int slot, auto fillc) {
-        const int next = slot + 1 == kStages ? 0 : slot + 1;
-        const int prev = slot == 0 ? kStages - 1 : slot - 1;
-        half_stage(FA, FB, static_cast<uint32_t>(slot) * kStage, std::integral_constant<int, 1>{}, std::false_type{}, 0, 0);
-        MI_SCHED_FENCE();
-        const int last = i + kStages - 2 < nk - 1 ? i + kStages - 2 : nk - 1;   // newest stage requested so far
-        wait_fills(last - (i + 1));
-        __builtin_amdgcn_s_barrier();
-        MI_SCHED_FENCE();
-        half_stage(FB, FA, static_cast<uint32_t>(next) * kStage, std::integral_constant<int, 0>{}, fillc, i + kStages - 1, prev);
-        MI_SCHED_FENCE();
-    };
-    int slot = 0, i = 0;
-    for (; i + kStages - 1 < nk; ++i) {
-        stage(i, slot, std::true_type{});
-        slot = slot + 1 == kStages ? 0 : slot + 1;
-    }
-    for (; i < nk; ++i) {
-        stage(i, slot, std::false_type{});
-        slot = slot + 1 == kStages ? 0 : slot + 1;
-    }
-
-    // epilogue: D[i][j], i = 8 (r / 4) + 4 g + r % 4 a row of W (an output column), j = li a row of x.  The scaled
-    // fp16 values go through LDS (this wavefront's own 128 x 128 patch, rows padded to 272 bytes) so that the
-    // stores are 16 bytes per lane, 256 consecutive bytes per 16 lanes.
-    MI_WAIT_LGKM(0);
-    __builtin_amdgcn_s_barrier();                        // nobody reads operands from LDS any more
-    MI_SCHED_FENCE();
-    uint8_t* ebase = lds + w * (128 * kERow);
-    const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(scale) % 8 == 0;
-    #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        #pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-            const int nq = n0 + 128 * wc + 32 * u + 8 * rq + 4 * g;
-            uint32_t h[4];
-            if (cols4 && nq + 3 < N) {
-                const uint2 v = *reinterpret_cast<const uint2*>(scale + nq);
-                h[0] = v.x & 0xFFFFu; h[1] = v.x >> 16; h[2] = v.y & 0xFFFFu; h[3] = v.y >> 16;
-            } else {
-                #pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = scale[nq + e < N ? nq + e : N - 1];
-            }
-            float s4[4];
-            #pragma unroll
-            for (int e = 0; e < 4; ++e) s4[e] = __half2float(__ushort_as_half(static_cast<uint16_t>(h[e])));
-            #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint32_t lo = pack_half2(acc[u][t][4 * rq] * s4[0], acc[u][t][4 * rq + 1] * s4[1]);
-                const uint32_t hi = pack_half2(acc[u][t][4 * rq + 2] * s4[2], acc[u][t][4 * rq + 3] * s4[3]);
-                *reinterpret_cast<uint2*>(ebase + (32 * t + li) * kERow + (32 * u + 8 * rq + 4 * g) * 2) = uint2{lo, hi};
-            }
-        }
-    }
-    // each wavefront reads back only what it wrote itself
-    const int ncol = n0 + 128 * wc + 8 * (lane & 15);    // first of this lane's 8 output columns
-    const bool cols8 = (N % 8) == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    #pragma unroll 4
-    for (int j = 0; j < 32; ++j) {
-        const int row = 4 * j + (lane >> 4);
-        const u32x4 v = *reinterpret_cast<const u32x4*>(ebase + row * kERow + (lane & 15) * 16);
-        const int m = m0 + 128 * wr + row;
-        if (m >= M) continue;
-        uint16_t* dst = out + static_cast<size_t>(m) * N + ncol;
-        if (cols8 && ncol + 7 < N) {
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
-        } else {
-            #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (ncol + e < N) dst[e] = static_cast<uint16_t>(v[e / 2] >> (16 * (e % 2)));
-        }
-    }
-}
-
-bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, const void* scale, void* out) {
-    constexpr size_t lds_bytes = static_cast<size_t>(kStages) * kStage;
-    static_assert(4 * 128 * kERow <= kStages * kStage, "the epilogue's patches fit the operand stages");
-    if (!MI_ONCE_OK(MI_HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_quad),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes))))
-        return false;
-    const long total = static_cast<long>((N + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
-    hipLaunchKernelGGL(gemm_quad, dim3(static_cast<unsigned>(8 * ((total + 7) / 8))), dim3(256), lds_bytes, s,
-                       static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(W),
-                       static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(out), M, N, K);
-    return MI_HIP_OK(hipGetLastError());
-}
-
-}  // namespace quad
-
-// ---- a few rows of x (M <= 64): the weights stream once, as in the GEMV ------------------------
-//
-// With up to 64 rows of x the contraction is bound by the weights' bytes, like the GEMV, not by
-// the matrix cores, and the tiles above leave most of the chip idle (19 tiles at N = 4864).  Here a
-// wavefront takes a strip of 16 rows of W and streams it through v_mfma_f32_16x16x32_f16 against
-// the 16 MT rows of x:
-//   A = W strip: lane l supplies row l % 16, 8 values of K starting at 16 (l / 16) + 8 s of the
-//       iteration's 64 (s = 0, 1: the two MFMAs of an iteration), i.e. one 16-byte load of int8
-//       weights per lane and iteration, 64 contiguous bytes per row;
-//   B = x^T: lane l supplies row l % 16 of the x tile at the same 16 values of K, 32 contiguous
-//       bytes (x is small and comes from the caches);
-//   D[i][j] (lane l: i = 4 (l / 16) + r, j = l % 16) = out[row j of the x tile][row i of the strip]:
-//       four consecutive output columns per lane.
-// K is cut into ks slices over the wavefronts of a block where N alone gives too few strips to
-// fill the chip; their sums meet in LDS and are added in slice order.  Iterations go through two
-// register buffers, one in flight while the other is multiplied.
-namespace skinny {
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-constexpr int kMaxM = 64;
-constexpr int kWaves = 8;                // wavefronts per block
-
-// The sums of a 16 x 16 tile's kb slices of K, each in one wavefront of a block of its own, meet in memory: the
-// wavefront that arrives last takes all of them in slice order (a lane the sums of the lanes of its number) and goes
-// on with their total; the others return false.  Sums and counter travel as agent-scope accesses, which pass the
-// XCDs' own L2s: a store that has been acknowledged (vmcnt) is where every other CU's such load looks for it.  No
-// block waits for another.  The counter starts at 0 (add_workspace) and is left at 0; launches on a stream are ordered.
-// What it replaces is a second launch over 1 KB per tile and slice, which in a prompt or a batch waits for this one and
-// holds up the next: a prompt of 37 fp16 tokens 1618 -> 1576 us in 32 layers (960 x 2560 each); at 64 rows equal.
-__device__ __forceinline__ bool meet_slices(floatx4& acc, float* __restrict__ sums, uint32_t* __restrict__ counter, const int by,
-                                            const int kb, const int lane) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    auto* at = reinterpret_cast<uint64_t*>(sums) + lane;                 // [kb][2][64] pairs
-    #pragma unroll
-    for (int h = 0; h < 2; ++h)
-        __hip_atomic_store(at + (by * 2 + h) * 64, __builtin_bit_cast(uint64_t, f32x2{acc[2 * h], acc[2 * h + 1]}),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    uint32_t before = 0;
-    if (lane == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    before = __builtin_amdgcn_readfirstlane(before);
-    if (before + 1 != static_cast<uint32_t>(kb)) return false;
-    asm volatile("" ::: "memory");
-    if (lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    constexpr int kMost = 8;                                             // slices over blocks (pick_shape), asked for together
-    f32x2 v[kMost][2];
-    #pragma unroll
-    for (int y = 0; y < kMost; ++y)
-        #pragma unroll
-        for (int h = 0; h < 2; ++h)
-            v[y][h] = __builtin_bit_cast(f32x2, __hip_atomic_load(at + ((y < kb ? y : 0) * 2 + h) * 64, __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_AGENT));
-    #pragma unroll
-    for (int y = 0; y < kMost; ++y)
-        if (y < kb) {
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] = y == 0 ? v[y][r / 2][r % 2] : acc[r] + v[y][r / 2][r % 2];
-        }
-    return true;
-}
-
-// Up to 64 rows of x, or tiles of as many.  A wavefront owns a tile of 16 S columns of the output (S strips of 16 rows of W) and a slice of K, and
-// works for itself: it asks for its slice of x and of W, 64 values of K at a time, by direct global -> LDS loads into a ring of
-// its own, waits for its own loads only, and multiplies.  ks wavefronts of a block share a tile; their sums meet in LDS, in
-// slice order, behind the one barrier of the kernel.
-//
-// What bounds such a launch is the way to memory, and how much of it is asked for at once: a few us of latency and one pass
-// over the weights.  So
-//  * everything a block needs is on its way before anything is used, up to 160 KB of LDS per CU and without registers;
-//  * a load instruction covers whole pieces of rows, 64 or 128 bytes of each (8 lanes to a row of x).  As fragments straight
-//    from memory neighbouring lanes are in different rows, and a load of 64 lanes is 64 lookups in the L1, for x as often
-//    as a block has strips: that bounded the launch;
-//  * the 16-byte pieces of a row are XOR-swizzled so that fragment reads are free of bank conflicts without padding.
-// us per launch, weights from HBM, with fragments (x copied to LDS first where it fitted) -> this: fp16, 37 rows of 960 x 2560 9.7 ->
-// 8.1, 1600 x 960 6.1 -> 5.3, 960 x 960 6.0 -> 4.5, 5120 x 960 with the SwiGLU 7.6 -> 6.6, 64 rows of 576 x 1536 9.8 -> 5.9; int8, 16 rows of
-// 896 x 896 4.2 -> 3.7, 9728 x 896 with the SwiGLU 7.0 -> 6.7; Q4, 24 rows of 896 x 4864 9.8 -> 7.4; the floor of a launch is 1.6.
-// An int8 weight becomes fp16 in the registers (exactly).  Q4: q * scale as two exact fp16 terms (scale = hi + lo with 7 and
-// 4 significant bits, as in the wide kernel), or rounded to fp16 once with TERMS = 1.
-// GLU: see launch_gemm_glu; the tile's strips are the gate's and the up matrix's in turn (S = 2, 4).
-// MEET: kb slices of K over blocks, which meet as told at meet_slices (an instance of its own, S = 1).
-// Without MEET and with `partial` the sums go there, [slice over blocks][M][N], for a launch that adds them (N a multiple of 4).
-template <int KIND, int MT, int S>
-struct Unit {                                            // what 64 values of K take in a wavefront's ring
-    static constexpr int kX = MT * 2048;                 // rows of 128 bytes
-    static constexpr int kW = KIND == WK_F16 ? S * 2048 : KIND == WK_I8 ? S * 1024 : S * 512;
-    static constexpr int kBytes = kX + kW + (KIND == WK_Q4 ? S * 64 : 0);              // Q4: two block scales per row
-    static constexpr int kSums = MT * S * 1024;          // the tile's fp32 sums, which take the place of the ring
-    static constexpr int kLoads = 2 * MT + (KIND == WK_F16 ? 2 * S : KIND == WK_I8 ? S : 2);
-};
-constexpr int kMaxRing = 8;                              // units in a ring
-
-template <int LOADS>
-__device__ __forceinline__ void wait_for_all_but(int units) {           // the loads of the last `units` units may be under way
-    #define MI_CASE(u) case u: MI_WAIT_VM((u) * LOADS < 63 ? (u) * LOADS : 63); break;
-    switch (units) {
-        MI_CASE(0) MI_CASE(1) MI_CASE(2) MI_CASE(3) MI_CASE(4) MI_CASE(5) MI_CASE(6)
-        default: MI_WAIT_VM(7 * LOADS < 63 ? 7 * LOADS : 63);
-    }
-    #undef MI_CASE
-}
-
-// A unit's fragments from LDS (the wait stands in the block that reads: the registers are in flight until then).
-#define MI_X1 "ds_read_b128 %[p0], %[a]\n\tds_read_b128 %[q0], %[b]\n\t"
-#define MI_X2 MI_X1 "ds_read_b128 %[p1], %[a] offset:2048\n\tds_read_b128 %[q1], %[b] offset:2048\n\t"
-#define MI_X3 MI_X2 "ds_read_b128 %[p2], %[a] offset:4096\n\tds_read_b128 %[q2], %[b] offset:4096\n\t"
-#define MI_X4 MI_X3 "ds_read_b128 %[p3], %[a] offset:6144\n\tds_read_b128 %[q3], %[b] offset:6144\n\t"
-#define MI_OX1 [p0] "=&v"(x[0][0]), [q0] "=&v"(x[0][1])
-#define MI_OX2 MI_OX1, [p1] "=&v"(x[1][0]), [q1] "=&v"(x[1][1])
-#define MI_OX3 MI_OX2, [p2] "=&v"(x[2][0]), [q2] "=&v"(x[2][1])
-#define MI_OX4 MI_OX3, [p3] "=&v"(x[3][0]), [q3] "=&v"(x[3][1])
-#define MI_F1 "ds_read_b128 %[w0], %[a] offset:%[o0]\n\tds_read_b128 %[v0], %[b] offset:%[o0]\n\t"
-#define MI_F2 MI_F1 "ds_read_b128 %[w1], %[a] offset:%[o1]\n\tds_read_b128 %[v1], %[b] offset:%[o1]\n\t"
-#define MI_F4 MI_F2 "ds_read_b128 %[w2], %[a] offset:%[o2]\n\tds_read_b128 %[v2], %[b] offset:%[o2]\n\t" \
-              "ds_read_b128 %[w3], %[a] offset:%[o3]\n\tds_read_b128 %[v3], %[b] offset:%[o3]\n\t"
-#define MI_OF1 [w0] "=&v"(w[0][0]), [v0] "=&v"(w[0][1])
-#define MI_OF2 MI_OF1, [w1] "=&v"(w[1][0]), [v1] "=&v"(w[1][1])
-#define MI_OF4 MI_OF2, [w2] "=&v"(w[2][0]), [v2] "=&v"(w[2][1]), [w3] "=&v"(w[3][0]), [v3] "=&v"(w[3][1])
-#define MI_I1 "ds_read_b128 %[w0], %[d]\n\t"
-#define MI_I2 MI_I1 "ds_read_b128 %[w1], %[d] offset:1024\n\t"
-#define MI_I4 MI_I2 "ds_read_b128 %[w2], %[d] offset:2048\n\tds_read_b128 %[w3], %[d] offset:3072\n\t"
-#define MI_OI1 [w0] "=&v"(w[0][0])
-#define MI_OI2 MI_OI1, [w1] "=&v"(w[1][0])
-#define MI_OI4 MI_OI2, [w2] "=&v"(w[2][0]), [w3] "=&v"(w[3][0])
-#define MI_Q1 "ds_read_b64 %[w0], %[d]\n\tds_read_b32 %[v0], %[e]\n\t"
-#define MI_Q2 MI_Q1 "ds_read_b64 %[w1], %[d] offset:512\n\tds_read_b32 %[v1], %[e] offset:64\n\t"
-#define MI_OQ1 [w0] "=&v"(w4[0]), [v0] "=&v"(ws[0])
-#define MI_OQ2 MI_OQ1, [w1] "=&v"(w4[1]), [v1] "=&v"(ws[1])
-#define MI_READ_MT(MTN, WS, OWS, ...)                                                                      \
-    if constexpr (MT == MTN)                                                                               \
-        asm volatile(MI_X##MTN WS "s_waitcnt lgkmcnt(0)" : MI_OX##MTN, OWS : [a] "v"(a), [b] "v"(b), __VA_ARGS__ : "memory");
-#define MI_READ_S(SN, L, ...)                                                                              \
-    if constexpr (S == SN) {                                                                               \
-        MI_READ_MT(1, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
-        MI_READ_MT(2, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
-        MI_READ_MT(3, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
-        MI_READ_MT(4, MI_##L##SN, MI_O##L##SN, __VA_ARGS__)                                                \
-    }
-template <int KIND, int MT, int S>
-struct UnitFrags {
-    u32x4 x[MT][2];
-    u32x4 w[S][2];                                       // int8: only the first, 16 weights
-    u32x2 w4[S];                                         // Q4: 16 weights and the row's two block scales
-    uint32_t ws[S];
-    // a, b: the lane's pieces 2c and 2c + 1 of its row of the first x tile; d: of the first strip; e: its scales
-    __device__ __forceinline__ void read(uint32_t a, uint32_t b, uint32_t d, uint32_t e) {
-        if constexpr (KIND == WK_F16) {
-            MI_READ_S(1, F, [o0] "i"(MT * 2048))
-            MI_READ_S(2, F, [o0] "i"(MT * 2048), [o1] "i"(MT * 2048 + 2048))
-            MI_READ_S(4, F, [o0] "i"(MT * 2048), [o1] "i"(MT * 2048 + 2048), [o2] "i"(MT * 2048 + 4096), [o3] "i"(MT * 2048 + 6144))
-        } else if constexpr (KIND == WK_I8) {
-            MI_READ_S(1, I, [d] "v"(d))
-            MI_READ_S(2, I, [d] "v"(d))
-            MI_READ_S(4, I, [d] "v"(d))
-        } else {
-            MI_READ_S(1, Q, [d] "v"(d), [e] "v"(e))
-            MI_READ_S(2, Q, [d] "v"(d), [e] "v"(e))
-        }
-    }
-};
-
-template <int KIND, int MT, int S, int TERMS, bool GLU, bool MEET>
-__device__ __forceinline__ void skinny_tile(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
-                                            const uint16_t* __restrict__ scale, uint16_t* __restrict__ out, const int M, int N,
-                                            const int K, const int ks, const int ring_units, float* __restrict__ partial,
-                                            uint32_t* __restrict__ counters, const MoreMats& more, const int bx, const int waves,
-                                            const int by, const int kb, const int bz) {
-    static_assert(!GLU || S % 2 == 0, "strips of either matrix");
-    constexpr bool F16 = KIND == WK_F16, Q4 = KIND == WK_Q4;
-    typedef Unit<KIND, MT, S> U;
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = lane & 15, c = lane >> 4;
-    const int slice = wave & (ks - 1);
-    int tile = bx * (waves / ks) + wave / ks;
-    if constexpr (!GLU) pick_matrix(more, tile, W, scale, out, N);
-    const int n0 = 16 * S * tile, m0 = 16 * MT * bz;
-    const bool live = n0 < N;                            // (a block's last tiles may lie past the matrix: they take part in the barrier only)
-    const int nb = live ? n0 : 0;
-
-    // K is cut over kb blocks and, inside a block, over ks wavefronts
-    const int its = K / 64, b0 = its * by / kb, b1 = its * (by + 1) / kb;
-    const int it0 = b0 + (b1 - b0) * slice / ks, n = live ? b0 + (b1 - b0) * (slice + 1) / ks - it0 : 0;
-
-    uint32_t sc[S][4];
-    if constexpr (KIND == WK_I8) {                       // asked for first: used last
-        #pragma unroll
-        for (int s = 0; s < S; ++s)
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int nq = nb + 16 * s + 4 * c + r;
-                sc[s][r] = scale[nq < N ? nq : N - 1];
-            }
-    }
-
-    // --- fill side: lane l of a load writes LDS bytes [16 l, +16) of its KB ---
-    // x, fp16 W: a load covers 8 rows of 128 bytes; slot p of row r holds piece p ^ ((r >> 1) & 7)
-    // int8: 16 rows of 64 bytes, piece p ^ ((r >> 2) & 3); Q4: 16 rows of 32 bytes (S of them), piece p ^ ((r >> 3) & 1)
-    const size_t wrowb = Q4 ? static_cast<size_t>(K) / 2 : F16 ? static_cast<size_t>(K) * 2 : static_cast<size_t>(K);
-    const uint8_t* const Xb = reinterpret_cast<const uint8_t*>(X) + static_cast<size_t>(m0) * K * 2 + static_cast<size_t>(it0) * 128;
-    const uint8_t* const Wb = W + static_cast<size_t>(nb) * wrowb + static_cast<size_t>(it0) * (Q4 ? 32 : F16 ? 128 : 64);
-    const int wlast = N - 1 - nb, xlast = M - 1 - m0;    // rows past N and M are read as the last row
-    constexpr int kWL = F16 ? 2 * S : Q4 ? 1 : S;
-    uint32_t xoff[2 * MT], woff[kWL];
-    #pragma unroll
-    for (int j = 0; j < 2 * MT; ++j) {
-        const int r = 8 * j + (lane >> 3), m = r < xlast ? r : xlast;
-        xoff[j] = static_cast<uint32_t>(m) * static_cast<uint32_t>(K) * 2u + 16u * ((lane & 7) ^ ((r >> 1) & 7));
-    }
-    #pragma unroll
-    for (int j = 0; j < kWL; ++j) {
-        int r, piece;
-        if constexpr (F16) { r = 8 * j + (lane >> 3); piece = (lane & 7) ^ ((r >> 1) & 7); }
-        else if constexpr (Q4) { r = lane >> 1; piece = (lane & 1) ^ ((r >> 3) & 1); }
-        else { r = 16 * j + (lane >> 2); piece = (lane & 3) ^ ((r >> 2) & 3); }
-        woff[j] = static_cast<uint32_t>(r < wlast ? r : wlast) * static_cast<uint32_t>(wrowb) + 16u * piece;
-    }
-    [[maybe_unused]] const uint8_t* Sb = nullptr;
-    [[maybe_unused]] uint32_t soff = 0;
-    if constexpr (Q4) {
-        Sb = reinterpret_cast<const uint8_t*>(scale) + static_cast<size_t>(nb) * (K / 16) + static_cast<size_t>(it0) * 4;
-        const int r = lane & (16 * S - 1);
-        soff = static_cast<uint32_t>(r < wlast ? r : wlast) * static_cast<uint32_t>(K / 16);
-    }
-    const int stride = ring_units * U::kBytes > U::kSums ? ring_units * U::kBytes : U::kSums;
-    uint8_t* const ring = lds + wave * stride;
-    auto fill = [&](int u, int slot) {                   // unit u of the slice
-        uint8_t* l = ring + slot * U::kBytes;
-        #pragma unroll
-        for (int j = 0; j < 2 * MT; ++j) wide::lds_fill16(Xb + static_cast<size_t>(u) * 128 + xoff[j], l + 1024 * j);
-        const uint8_t* w = Wb + static_cast<size_t>(u) * (Q4 ? 32 : F16 ? 128 : 64);
-        if constexpr (Q4) {
-            if (lane < 32 * S) wide::lds_fill16(w + woff[0], l + U::kX);
-            if (lane < 16 * S) wide::lds_fill4(Sb + static_cast<size_t>(u) * 4 + soff, l + U::kX + U::kW);
-        } else {
-            #pragma unroll
-            for (int j = 0; j < kWL; ++j) wide::lds_fill16(w + woff[j], l + U::kX + 1024 * j);
-        }
-    };
-    const int lead = n < ring_units ? n : ring_units;
-    for (int u = 0; u < lead; ++u) fill(u, u);
-
-    // --- read side ---
-    const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((wide::lds_u8*)ring));
-    const uint32_t xa = base + i * 128 + 16 * ((2 * c) ^ (i >> 1));
-    const uint32_t wa = base + U::kX + (Q4 ? i * 32 + 16 * ((c >> 1) ^ (i >> 3)) + 8 * (c & 1) : i * 64 + 16 * (c ^ (i >> 2)));
-    const uint32_t sa = base + U::kX + U::kW + i * 4;
-    floatx4 acc[MT][S];
-    #pragma unroll
-    for (int t = 0; t < MT; ++t)
-        #pragma unroll
-        for (int s = 0; s < S; ++s) acc[t][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    int slot = 0;
-    for (int u = 0; u < n; ++u) {
-        const int issued = u + ring_units < n ? u + ring_units : n;
-        wait_for_all_but<U::kLoads>(issued - u - 1);
-        UnitFrags<KIND, MT, S> F;
-        const uint32_t at = slot * U::kBytes;
-        F.read(xa + at, (xa + at) ^ 16u, wa + at, sa + at);
-        if (u + ring_units < n) fill(u + ring_units, slot);
-        slot = slot + 1 == ring_units ? 0 : slot + 1;
-        #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            half8 a[TERMS][2];
-            if constexpr (F16) {
-                a[0][0] = __builtin_bit_cast(half8, F.w[s][0]);
-                a[0][1] = __builtin_bit_cast(half8, F.w[s][1]);
-            } else if constexpr (Q4) {
-                const uint32_t both = __builtin_amdgcn_perm(0u, F.ws[s], c >> 1 ? 0x03020302u : 0x01000100u);
-                __half2 st[TERMS];
-                if constexpr (TERMS == 2) {
-                    st[0] = __builtin_bit_cast(__half2, both & 0xFFF0FFF0u);
-                    st[1] = __hsub2(__builtin_bit_cast(__half2, both), st[0]);
-                } else {
-                    st[0] = __builtin_bit_cast(__half2, both);
-                }
-                #pragma unroll
-                for (int e = 0; e < 2; ++e)
-                    #pragma unroll
-                    for (int z = 0; z < TERMS; ++z)
-                        a[z][e] = __builtin_bit_cast(half8, u32x4{q4x2_to_h2<0>(F.w4[s][e], st[z]), q4x2_to_h2<1>(F.w4[s][e], st[z]),
-                                                                  q4x2_to_h2<2>(F.w4[s][e], st[z]), q4x2_to_h2<3>(F.w4[s][e], st[z])});
-            } else {
-                uint32_t h[8];
-                #pragma unroll
-                for (int d = 0; d < 4; ++d) i8x4_to_h4(F.w[s][0][d], h[2 * d], h[2 * d + 1]);
-                a[0][0] = __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
-                a[0][1] = __builtin_bit_cast(half8, u32x4{h[4], h[5], h[6], h[7]});
-            }
-            #pragma unroll
-            for (int z = 0; z < TERMS; ++z)
-                #pragma unroll
-                for (int e = 0; e < 2; ++e)
-                    #pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        acc[t][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][e], __builtin_bit_cast(half8, F.x[t][e]), acc[t][s], 0, 0, 0);
-        }
-    }
-
-    // The slices' sums meet in LDS, each where its wavefront's ring was; sum t S + s of the tile (GLU: both sums of rows t) is
-    // then finished by the tile's wavefront of that number mod ks, which adds them in slice order.
-    auto sums_of = [&](int w) { return reinterpret_cast<floatx4*>(lds + w * stride); };
-    if (ks > 1) {                                        // (the same for every wavefront of the block)
-        #pragma unroll
-        for (int t = 0; t < MT; ++t)
-            #pragma unroll
-            for (int s = 0; s < S; ++s) sums_of(wave)[(t * S + s) * 64 + lane] = acc[t][s];
-        __syncthreads();
-    }
-    if (!live) return;
-    const bool cols4 = (N % 4) == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
-    #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        [[maybe_unused]] uint2 h[S];
-        #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            if (((GLU ? t : t * S + s) & (ks - 1)) != slice) continue;
-            const int strip = tile * S + s;
-            if (16 * strip >= N) continue;
-            floatx4 v = acc[t][s];
-            if (ks > 1) {
-                v = sums_of(wave - slice)[(t * S + s) * 64 + lane];
-                for (int z = 1; z < ks; ++z) {
-                    const floatx4 o = sums_of(wave - slice + z)[(t * S + s) * 64 + lane];
-                    #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] += o[r];
-                }
-            }
-            const int nq = 16 * strip + 4 * c, m = m0 + 16 * t + i;      // first of this lane's 4 output columns, its row
-            if constexpr (MEET) {
-                const int met = (bz * ((N + 15) / 16) + strip) * MT + t;
-                if (kb > 1 && !meet_slices(v, partial + static_cast<size_t>(met) * kb * 256, counters + met, by, kb, lane))
-                    continue;
-            } else if constexpr (!GLU) {
-                if (partial) {                           // (N is a multiple of 4 then)
-                    if (m < M && nq < N) *reinterpret_cast<floatx4*>(partial + (static_cast<size_t>(by) * M + m) * N + nq) = v;
-                    continue;
-                }
-            }
-            if constexpr (KIND == WK_I8) {
-                #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] *= h_f(static_cast<uint16_t>(sc[s][r]));
-            }
-            const uint32_t lo = wide::pack_half2(v[0], v[1]), hi = wide::pack_half2(v[2], v[3]);
-            if constexpr (GLU) {
-                h[s] = uint2{lo, hi};
-                continue;
-            }
-            if (m >= M || nq >= N) continue;
-            uint16_t* dst = out + static_cast<size_t>(m) * N + nq;
-            if (cols4 && nq + 3 < N) {
-                *reinterpret_cast<uint2*>(dst) = uint2{lo, hi};
-            } else {
-                #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (nq + r < N) dst[r] = static_cast<uint16_t>((r / 2 ? hi : lo) >> (16 * (r % 2)));
-            }
-        }
-        if constexpr (GLU) {
-            if ((t & (ks - 1)) == slice && m0 + 16 * t + i < M) {
-                #pragma unroll
-                for (int s = 0; s < S; s += 2)
-                    if (n0 + 16 * s < N)
-                        *reinterpret_cast<uint2*>(out + static_cast<size_t>(m0 + 16 * t + i) * (N / 2) + (n0 + 16 * s) / 2 + 4 * c) =
-                            uint2{swiglu_h2(h[s].x, h[s + 1].x), swiglu_h2(h[s].y, h[s + 1].y)};
-            }
-        }
-    }
-}
-
-template <int KIND, int MT, int S, int TERMS, bool GLU, bool MEET>
-__global__ __launch_bounds__(64 * kWaves) void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
-                                                           const uint16_t* __restrict__ scale, uint16_t* __restrict__ out,
-                                                           int M, int N, int K, int ks, int ring_units, float* __restrict__ partial,
-                                                           uint32_t* __restrict__ counters, MoreMats more) {
-    skinny_tile<KIND, MT, S, TERMS, GLU, MEET>(X, W, scale, out, M, N, K, ks, ring_units, partial, counters, more, blockIdx.x,
-                                               blockDim.x >> 6, blockIdx.y, gridDim.y, blockIdx.z);
-}
-
-constexpr size_t kLdsLimit = 160 * 1024;
-inline size_t unit_bytes(int kind, int mt, int S) {      // Unit::kBytes
-    return static_cast<size_t>(mt) * 2048 + (kind == WK_F16 ? S * 2048 : kind == WK_I8 ? S * 1024 : S * 576);
-}
-
-// bytes of partial sums that kb slices of K over blocks leave in the workspace (meet_slices)
-inline size_t partial_bytes(int mt, int N, int kb) { return static_cast<size_t>((N + 15) / 16) * kb * mt * 1024; }
-
-// ks: wavefronts that share a tile, the fewest of 4 and 8 that give the chip four wavefronts per CU (4 at least: with two, 9728 x 896 at
-// 16 rows 7.2 us, with four 6.7); 8 only where a ring holds two units then (fp16 at more than 48 rows: 3072 x 576 5.2 us in 4
-// slices, 6.0 in 8) and, one strip to a wavefront, from a K of 768 on: below, a wavefront has one unit or two, and more of them only
-// meet later (int8, 16 rows of 1536 x 576 3.8 in 4 slices, 4.0 in 8; of 960 x 576 3.5 / 3.8; 1600 x 960 as fast either way).  kb: slices over
-// blocks where one block per tile still leaves most CUs idle and the trip of the sums through memory, 2.5 us, is less than
-// what it saves, from more than 4 units per wavefront on (896 x 4864 at 16 rows: 8.7 us in 8 slices, 7.1 in 8 x 4; 2048 x 2048 at 8 Q4 rows
-// 5.6 in 8, 6.6 in 8 x 2, int8 5.5 / 6.5).  S: two strips per wavefront where one per wavefront is more blocks than CUs: x is
-// fetched half as often (4864 x 896 at 48 int8 rows 6.7 -> 6.1 us), up to 16 rows only from five blocks per CU on (Q4 32 000 x 320 8.0 with one, 6.0
-// with two); fewer blocks than CUs with two lose (1152 x 896 at 16 rows 3.7 against 4.1).
-struct Shape { int ks, kb, S; };
-// before: the slices that estimate_us was fitted with
-inline Shape pick_shape(int kind, int M, int N, int K, int cus, size_t workspace_bytes, bool before = false) {
-    const int mt = (M + 15) / 16;
-    const long strips = (N + 15) / 16;
-    const int its = K / 64;
-    Shape sh{1, 1, strips > cus && (mt > 1 || strips > 5L * cus) ? 2 : 1};
-    const long tiles = (strips + sh.S - 1) / sh.S;
-    const int most = 2 * kWaves * unit_bytes(kind, mt, 2) <= kLdsLimit ? kWaves : kWaves / 2;
-    while (sh.ks < most && (sh.ks < 4 || tiles * sh.ks < (sh.S == 2 ? 5L : 4L) * cus) && its >= 2 * sh.ks) sh.ks *= 2;
-    if (sh.S == 1 && sh.ks == 8 && its < 12 && !before) sh.ks = 4;
-    if (sh.ks == most) {
-        while (sh.kb < 8 && strips * sh.kb * 2 <= cus && its >= 4 * sh.ks * sh.kb + !before && strips * mt <= kSliceCounters &&
-               partial_bytes(mt, N, 2 * sh.kb) <= workspace_bytes)
-            sh.kb *= 2;
-    }
-    return sh;
-}
-// The slices of a launch whose sums another launch adds: as many over blocks as give every CU one, 4 in a block (us at kb = 1 /
-// these / twice as many: fp16, 37 rows of 960 x 2560 8.8 / 4.9 / 5.0, 960 x 960 4.6 / 3.6 / 3.8, int8, 16 rows of 896 x 4864 8.9 / 4.6 / 4.5).
-// kb = 1: none, the launch would save nothing.
-inline Shape pick_apart(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
-    const long strips = (N + 15) / 16;
-    const int its = K / 64;
-    Shape sh{4, 1, 1};
-    while (sh.kb < 8 && strips * (sh.kb + 1) <= cus && its >= sh.ks * (sh.kb + 1) &&
-           static_cast<size_t>(sh.kb + 1) * M * N * 4 <= workspace_bytes)
-        ++sh.kb;
-    return sh;
-}
-
-// Where the streaming kernel is the library's own choice, against the tiles above (us, weights from HBM).
-//  - Up to 64 rows: 2560 x 1024 at 24 / 40 / 64 rows 4.4 / 4.7 / 5.2 (fp16 5.0 / 5.6 / 6.2) against 8.7 to 9.6 for the 64 x 64 tiles, 896 x
-//    4864 at 64 fp16 rows 9.1 against 14 (the wide kernel in slices), 8192 x 2048 12.6 against 16.2.
-//  - Fewer of many rows of W, where the tiles fetch x once per 64 of them: fp16 up to 32 beyond 8192 (9728 x 896 at 32 / 48 / 64 rows 8.5 / 9.6 /
-//    10.5 against 8.8 / 9.3 / 9.7); int8 up to 48 beyond 12 288 (64 rows of 14 592 x 896 9.7 / 9.4, 19 456 x 896 12.4 / 11.9), 32 beyond 24 576
-//    (48 of 32 000 x 320 7.6 / 6.9).  int8 of a K up to 512 beyond 48 rows goes in tiles of 32 rows, 16 columns each: 64 rows of 1024 x 512 3.6
-//    against 4.0 here.
-//  - Not beyond 36 MB of weights, nor, above 13.5 MB, 80 rows of W per CU: the wide kernel's higher streaming rate wins there (int8
-//    49 152 x 576 at 16 rows 11.2 against 7.3).
-inline bool preferred(int kind, int M, int N, int K, int cus) {
-    const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
-    const long strips = (N + 15) / 16;
-    const int rows = kind == WK_F16 ? (strips > 2L * cus ? 32 : 64)
-                   : kind == WK_I8 ? (strips > 6L * cus ? 32 : strips > 3L * cus || K <= 512 ? 48 : 64) : 64;
-    return M <= rows && (w_bytes <= 13.5e6 ? strips <= (M > 48 ? 10L : 16L) * cus : w_bytes <= 36.0e6 && strips <= 5L * cus);
-}
-
-// ---- more rows of x than a tile holds: tiles of 16 mt rows by 16 S columns ----
-//
-// us per launch, weights from HBM, the 64 x 64 tiles or the wide kernel -> these: int8 100 / 300 / 600 rows of 1152 x 896 8.6 / 9.3 / 9.4 ->
-// 4.7 / 5.6 / 7.2, 100 rows of 9728 x 896 with the SwiGLU 10.8 -> 9.8, Q4 300 rows of 896 x 896 12.0 -> 5.7, of 9728 x 896 with the SwiGLU
-// 17.8 -> 15.8, 100 fp16 rows of 896 x 4864 14.2 -> 8.2.  From about 600 rows on by many columns the wide kernel's larger tiles
-// win: a block here pulls 1 byte into LDS for 25 to 60 multiplications, there for 140.
-//
-// A launch takes 3.5 us and more the larger the tile, and for every round of blocks on the CUs the tile's end and what a block pulls
-// into LDS: int8 and fp16 fitted to 4600 launches of 65 to 2048 rows, every tile at each of 310 calls (8 % rms; the tile it picks is 1 %
-// behind the best one in the mean), Q4 to 1300 (10 %).  Blocks beyond one per CU come in rounds, a last round that is not full
-// at about 0.6 of its price (the blocks in it have the L2s to themselves).  Tiles of 64 columns leave a CU with one block and wait
-// for more before they begin, which a short K does not pay back (512 rows of 1536 x 576 fp16 7.5 us, with 32 columns 6.5); with Q4 never the best.
-struct RowShape { int mt = 0, S = 1, ks = 4, kb = 1; double us = 1e30; };
-inline double rows_us(int kind, int mt, int S, int kb, int M, int N, int K, int cus) {
-    const long blocks = static_cast<long>((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * S - 1) / (16 * S)) * kb;
-    const double unit = static_cast<double>(unit_bytes(kind, mt, S)), its = K / 64.0 / kb, mean = static_cast<double>(blocks) / cus;
-    const long full = (blocks + cus - 1) / cus;
-    auto rounds = [&](double f) { return full == 1 ? 1.0 : f * full + (1.0 - f) * mean; };
-    if (kind == WK_Q4) return 4.1 + rounds(0.7) * its * unit / 57.0e3 * (S == 1 ? 0.72 : 1.0);
-    if (kind == WK_F16)
-        return 3.43 + 0.047 * mt * S + (S == 4 ? 0.25 : 0.0) +
-               rounds(0.58) * (0.043 * mt * S + its * unit / 80.4e3 * (S == 4 ? 1.16 : S == 1 ? 0.92 : 1.0));
-    return 3.51 + 0.047 * mt * S + (S == 4 ? 0.6 : 0.0) +
-           rounds(0.64) * (0.022 * mt * S + its * unit / 74.6e3 * (S == 4 ? 1.26 : S == 1 ? 0.85 : 1.0));
-}
-// Slices of K inside a block, by what a launch by itself, one among several matrices and one with the SwiGLU have in
-// common, since they decide the order of the sums.
-inline int rows_ks(int M, int N, int K) {
-    int ks = N > 8192 ? 2 : N > 1536 || M > 400 ? 4 : 8;
-    while (ks > 1 && K / 64 < ks) ks /= 2;
-    return ks;
-}
-inline bool rows_fit(int kind, int mt, int S, int ks) {
-    const size_t unit = unit_bytes(kind, mt, S), sums = static_cast<size_t>(mt) * S * 1024;
-    return (ks < 4 ? 4 : ks) * (unit > sums ? unit : sums) <= kLdsLimit;
-}
-inline RowShape pick_rows(int kind, int M, int N, int K, int cus, bool glu) {
-    RowShape best;
-    for (int mt = 2; mt <= 4; ++mt)
-        for (int S = 1; S <= 4; S *= 2) {
-            const int ks = rows_ks(M, N, K);
-            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || (glu && S == 1) || !rows_fit(kind, mt, S, ks)) continue;
-            const double us = rows_us(kind, mt, S, 1, M, N, K, cus);
-            if (us < best.us) best = RowShape{mt, S, ks, 1, us};
-        }
-    return best;
-}
-// Where they are the choice over the kernels above, by the estimates of all (us, weights from HBM, tiles of rows / the other).
-//  - Up to 64 rows of W per CU with Q4, 48 otherwise: beyond, the others stream better (80 int8 rows of 19 456 x 896 14.9 / 12.1, 100
-//    Q4 rows 18.2 / 16.1, 56 fp16 rows of 14 592 x 896 13.6 / 10.3).
-//  - Up to 8192 outputs per CU, about five rounds of tiles, from where 140 multiplications per byte pulled into LDS beat 25 to 60 (int8 512
-//    rows of 4096 x 512 7.7 / 6.7); 9600 with Q4, which the wide kernel multiplies twice (3072 rows of 1536 x 576 20.4 / 16.2, 2600 of
-//    1152 x 896 18.9 / 16.6), and at a long K up to 2e7 products per CU (600 rows of 2048 x 8192 67 / 51; 2560 x 2560 at 600 / 800 rows
-//    25 / 27 and 37 / 32).  Many columns, the gate and up matrices of a prompt, whose SwiGLU rides in the launch: 300 x 9728 x 896 Q4 17.6 / 16.1
-//    without it, but the prompt of 300 tokens 1477 / 1545.  Fewer rows for them: 600 x 3072 x 576 int8 9.0 / 8.2, 600 x 5120 x 960 17.5 / 14.1.
-//    fp16 to 1280 rows (2048 x 896 x 896 11.6 / 10.1), int8 to 3072 (4096 x 333 x 1920 24.1 / 20.9).
-//  - The estimates' own errors: the wide kernel's is 5 to 10 % too low without slices of K and 20 to 50 % too high with them (1200 x 896 x
-//    4864 in three 25.6 us, estimated at 32.6; fp16 130 x 2048 x 8192 20.1, at 24.4), for a few rows of fp16 0.5 us too low on top (300 x
-//    5120 x 960 12.5 against 10.7 here); the 64 x 64 tiles' is for weights in the caches, from HBM up to 1.5 us too low, the less the
-//    shorter K (200 rows of 4096 x 256 6.0 / 4.4 as they were chosen with 1.5 for any K); this one's 8 % too low for int8 beyond 8192 rows of W,
-//    in two slices of K.
-// Of 2016 calls (30 shapes of W, 40 to 4096 rows, every kind) 20 are 3 to 16 % slower than with the kernels above alone, by 0.2 to 1.5 us: int8 1200 x
-// 1536 x 576 8.8 / 7.6, fp16 300 x 3072 x 576 7.1 / 6.5, int8 600 x 1536 x 576 6.9 / 6.5.  Their layers, calls together, and prompts are
-// the faster for them (a layer of 600 int8 rows 17.9 / 23.0 us, of 1200 29.4 / 32.8, 30 layers of 300 fp16 rows 1230 / 1360).
-inline bool rows_preferred(int kind, const RowShape& r, double wide_us, int wide_slices, double tiled_us, int M, int N, int K, int cus) {
-    const double outs = static_cast<double>(M) * N, us = r.us * (kind == WK_I8 && N > 8192 ? 1.08 : 1.0);
-    if (N > (kind == WK_Q4 ? 64L : 48L) * cus || outs > (kind != WK_Q4 ? 8192.0 : N > 2560 ? 16000.0 : 9600.0) * cus || (kind == WK_Q4 && outs * K > 2.0e7 * cus)) return false;
-    if ((N > 2560 && M > (kind == WK_Q4 ? 512 : 304)) || M > (kind == WK_F16 ? 1280 : kind == WK_I8 ? 3072 : 1 << 30)) return false;
-    if (wide_slices > 1) wide_us *= kind == WK_F16 ? 0.82 : M <= 1024 ? 0.85 : 0.7;
-    else if (kind != WK_Q4) wide_us = kind == WK_I8 ? 1.05 * wide_us : 1.1 * wide_us + (M <= 304 ? 0.5 : 0.0);
-    return us < wide_us && (kind == WK_Q4 || us < tiled_us + (K < 640 ? (K - 128) / 345.0 : 1.5));
-}
-// The same cut into slices over blocks for a launch that adds them (mt = 0: not worth it).
-inline RowShape pick_rows_apart(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
-    RowShape best;
-    const int its = K / 64;
-    if (its < 14 || static_cast<long>((M + 47) / 48) * ((N + 31) / 32) > cus * 9L / 5) return best;
-    for (int mt = 2; mt <= 4; ++mt)
-        for (int S = 1; S <= 4; S *= 2) {
-            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || !rows_fit(kind, mt, S, 4)) continue;
-            for (int kb = 2; kb <= 6 && its >= 4 * kb && static_cast<size_t>(kb) * M * N * 4 <= workspace_bytes; ++kb) {
-                const double us = rows_us(kind, mt, S, kb, M, N, K, cus) + kb * 4.0e-6 * M * N / 4.0;
-                if (us < best.us) best = RowShape{mt, S, 4, kb, us};
-            }
-        }
-    return best;
-}
-
-// Estimated time (us): what decides between this kernel and rows of GEMV below 16 rows.  (Fitted to the kernel that took
-// fragments from memory, and 0.3 to 1 us too high: a line that moved would take prompts of a few tokens off the reference's
-// order, in which their attention goes with the projections.)
 inline double estimate_us(int kind, int M, int N, int K, int cus, size_t workspace_bytes) {
     const Shape sh = pick_shape(kind, M, N, K, cus, workspace_bytes, true);
     const double w_bytes = static_cast<double>(N) * K * (kind == WK_F16 ? 2.0 : kind == WK_Q4 ? 0.5625 : 1.0);
