@@ -1989,10 +1989,13 @@ bool launch_calls_mt(hipStream_t s, const SkinnyCalls& L, int mt, unsigned block
 // block per CU: 130 int8 rows of 0.5B 21.1 against 15.5, 200 Q4 rows of 360M 25.9 against 21.0; fp16 in tiles of 64: 400 rows of 0.5B 35.9
 // against 33.4).  us per layer, launches of their own -> together: 80 fp16 rows of 135M 17.4 -> 8.0, 130 int8 rows of 0.5B 27.9 -> 15.5,
 // 700 int8 rows of 360M 49.8 -> 38.9, 2048 int8 rows of 0.5B (q, k, v and o) 105.0 -> 99.1.
+inline int many_mt(int kind, int M) {
+    const int tiles_m = (M + kMaxM - 1) / kMaxM, mt = ((M + tiles_m - 1) / tiles_m + 15) / 16;
+    return tiles_m > 1 && (mt < 3 || kind == WK_F16) ? 3 : mt;
+}
 bool launch_many(hipStream_t s, const GemvCall* calls, int n, int terms, void* workspace, size_t workspace_bytes) {
-    const int M = calls[0].M, tiles_m = (M + kMaxM - 1) / kMaxM, mt_even = ((M + tiles_m - 1) / tiles_m + 15) / 16;
-    const int mt = tiles_m > 1 && (mt_even < 3 || calls[0].kind == WK_F16) ? 3 : mt_even, S = tiles_m > 1 ? 2 : 1, rows_m = (M + 16 * mt - 1) / (16 * mt);
     const WeightKind kind = calls[0].kind;
+    const int M = calls[0].M, mt = many_mt(kind, M), S = M > kMaxM ? 2 : 1, rows_m = (M + 16 * mt - 1) / (16 * mt);
     const size_t unit = std::max(unit_bytes(kind, mt, S), static_cast<size_t>(mt) * S * 1024);
     SkinnyCalls L;
     long blocks = 0;
@@ -2432,20 +2435,19 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
     return launch_planned(s, p, kind, M, mat[0].N, K, x, mat[0].W, mat[0].scale, mat[0].out, workspace, ws_bytes, more) ? g : -1;
 }
 
-// Rows of x up to which calls in tiles of rows go out together (beyond, few calls are in tiles of rows).
-constexpr int kMostShared = 2048;
-
 GemmRoute gemm_route(hipStream_t s, const GemvCall& c, size_t workspace_bytes) {
     if (!gemm_supported(c.kind, c.M, c.N, c.K, c.x, c.W, c.scale)) return GemmRoute::kRefused;
-    const int mode = gemm_mode(s);
-    if (c.M > kMostShared && (mode == 0 || mode == 4))        // (without a plan: only the wide kernel's reach is missing for Q4)
-        return c.kind != WK_Q4 || wide_reaches(c.kind, c.M, c.N, c.K) ? GemmRoute::kAlone : GemmRoute::kRefused;
     const GemmPlan p = plan_gemm(s, c.kind, c.M, c.N, c.K, workspace_bytes);
     if (p.kernel < 1 || (p.kernel == 1 && p.k_slices > 1 && !wide::slices_fit(p.k_slices, c.M, c.N, c.K, workspace_bytes)))
         return GemmRoute::kRefused;
-    // (tiles of rows: as many as a launch of several counts, in the slices that launch_many takes)
-    const bool rows = p.kernel == 6 && c.M > skinny::kMaxM && p.ks == skinny::rows_ks(c.M, c.N, c.K) &&
-                      static_cast<long>((c.N + 31) / 32) * ((c.M + 47) / 48) <= 65535;
+    // Tiles of rows: as many as a launch of several counts, in its slices.  They take its tile there, 32 columns wide: a call that fills the
+    // chip more than twice over with them goes alone where its own tile saves the time of a launch, 3.4 us (the down projection of 0.5B
+    // in int8: with q and o the layer of 2304 rows takes 131 us, alone 120; of 600 rows 44.5, alone 46).
+    const int cus = device_info().cus, mt = skinny::many_mt(c.kind, c.M);
+    const long blocks = static_cast<long>((c.N + 31) / 32) * ((c.M + 16 * mt - 1) / (16 * mt));
+    const bool rows = p.kernel == 6 && c.M > skinny::kMaxM && p.ks == skinny::rows_ks(c.M, c.N, c.K) && blocks <= 65535 &&
+                      (blocks <= 2L * cus || skinny::rows_us(c.kind, mt, 2, 1, c.M, c.N, c.K, cus) <
+                                                 skinny::rows_us(c.kind, p.tile_rows / 16, p.strips, 1, c.M, c.N, c.K, cus) + 3.4);
     return (p.kernel == 4 || rows) && (c.N + 15) / 16 <= 8191 ? GemmRoute::kShares : GemmRoute::kAlone;
 }
 

@@ -7,6 +7,7 @@ import pytest
 from helpers import mil
 from test_gemm_plan_gpu import _time_us, queue  # noqa: F401
 from test_gemm_group_gpu import _weights
+from test_gemm_many_gpu import _check
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,55 @@ def test_slices_of_the_streaming_kernel_where_they_measured_faster(kind, M, N, K
     queue, keep = mil.Queue(), []
     x, w = mil.Buffer(2 * M * K), _weights(kind, N, K, 73, keep)
     assert mil.linear_plan(queue, M, N, K, x, w) == plan
+
+
+def _layer(kind, rows, shapes, keep):
+    calls = []
+    for j, (n, k) in enumerate(shapes):
+        x = mil.Buffer.from_host(mil.synth_normal_f16(80 + j, 1.0, (rows, k)))
+        keep.append(x)
+        calls.append((rows, n, k, x, _weights(kind, n, k, 90 + j, keep)))
+    return calls
+
+
+@pytest.mark.parametrize("kind,rows,shapes", [
+    ("int8", 2049, [(576, 576), (192, 576), (576, 576), (576, 1536)]), ("q4", 2305, [(576, 576), (192, 576), (576, 1536)]),
+    ("f16", 900, [(896, 896), (128, 896), (896, 4864)]), ("int8", 2304, [(896, 896), (128, 896), (896, 4864)])])
+def test_batches_beyond_2048_rows_and_long_calls_that_go_alone(kind, rows, shapes):
+    """Tiles of rows at any number of rows share a launch but for the call that fills the chip and has a better tile of its
+    own (the last one of the last two cases): each output bit for bit that of the call by itself."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep = mil.Queue(), []
+    calls = _layer(kind, rows, shapes, keep)
+    print(f"{kind} rows {rows} plans {[mil.linear_plan(queue, *c) for c in calls]}", flush=True)
+    assert all(mil.linear_plan(queue, *c)[0] == 6 for c in calls)
+    _check(queue, calls, 2)
+
+
+def test_a_row_more_than_2048_costs_no_launch(queue):  # noqa: F811
+    """Five small calls, which go out together: 2049 rows within 8 % of 2048 (1.5 times as long while they went one by one)."""
+    keep, us = [], {}
+    shapes = [(576, 576), (192, 576), (192, 576), (576, 576), (576, 1536)]
+    for attempt in range(3):
+        for rows in (2048, 2049):
+            calls = _layer("int8", rows, shapes, keep)
+            outs = [mil.Buffer(2 * rows * c[1]) for c in calls]
+            keep += outs                                 # (the calls hold addresses only)
+            arr = mil.make_calls([(*c, o) for c, o in zip(calls, outs)])
+            assert mil.linear_batch(queue, arr) == len(calls)
+            queue.finish()
+            with mil.Graph(queue) as g:
+                for _ in range(8):
+                    assert mil.linear_batch(queue, arr) == len(calls)
+            e0, e1, got = mil.Event(), mil.Event(), []
+            for _ in range(9):
+                e0.record(queue)
+                g.launch()
+                e1.record(queue)
+                e1.synchronize()
+                got.append(e0.elapsed_ms(e1) * 125)
+            us[rows] = sorted(got)[4]
+        print(us, flush=True)
+        if us[2049] <= 1.08 * us[2048]:
+            return
+    assert False, us
