@@ -2354,12 +2354,18 @@ int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, cons
     }
     const int terms = kind == WK_Q4 ? p.terms : 1, cus = device_info().cus;
     if ((mode == 0 || mode == 4) && p.kernel >= 1 && p.kernel != 5) {
-        // (against what would run otherwise: the plan, or the wide kernel's slices)
-        const skinny::RowShape r = skinny::pick_rows_apart(kind, M, N, K, cus, workspace_bytes);
+        // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
+        const double uncut = p.kernel == 1   ? wide::estimate_us(kind, terms, p.tile_rows / 32, p.k_slices, M, N, K, cus)
+                             : p.kernel == 6 ? skinny::rows_us(kind, p.tile_rows / 16, p.strips, 1, M, N, K, cus)
+                             : p.kernel == 4 ? 1e30 : tiled_estimate_us(M, N, K);
         int tm = 1, splits = 1;
         double cut = 1e30;
         if (wide_reaches(kind, M, N, K)) wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &cut);
-        if (r.mt && r.us < cut - 2.5) {
+        // Tiles of rows: against the wide kernel's slices and the plan, which also leaves the next launch a pass over its fp16 result,
+        // 1 us per 400 rows: 400 tokens of 0.5B int8 / fp16, whose q | k | v is estimated 1.1 / 1.25 us longer in slices, 1628 / 1726 us with them, 1577 /
+        // 1676 without; 500 Q4 tokens of 360M, o 0.9 longer, 2138 / 2184.
+        const skinny::RowShape r = skinny::pick_rows_apart(kind, M, N, K, cus, workspace_bytes);
+        if (r.mt && r.us < cut - 2.5 && r.us < uncut + M / 400.0) {
             auto* sums = static_cast<float*>(workspace);
             const bool ok = kind == WK_Q4 ? (terms == 1 ? skinny::launch_rows<WK_Q4, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false)
                                                         : skinny::launch_rows<WK_Q4, 2>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false))
@@ -2367,15 +2373,7 @@ int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, cons
                                            : skinny::launch_rows<WK_I8, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false);
             return ok ? r.kb : -1;
         }
-    }
-    if (p.kernel >= 1 && p.kernel != 4 && p.kernel != 5 && (p.kernel != 1 || p.k_slices == 1) && (mode == 0 || mode == 4) && wide_reaches(kind, M, N, K)) {
-        // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
-        const double uncut = p.kernel == 1   ? wide::estimate_us(kind, terms, p.tile_rows / 32, 1, M, N, K, cus)
-                             : p.kernel == 6 ? skinny::rows_us(kind, p.tile_rows / 16, p.strips, 1, M, N, K, cus)
-                                             : tiled_estimate_us(M, N, K);
-        int tm = 1, splits = 1;
-        double us = 0.0;
-        if (wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &us) && us - 2.5 < uncut) {
+        if (p.kernel != 4 && !(p.kernel == 1 && p.k_slices > 1) && cut - 2.5 < uncut) {
             p.kernel = 1;
             p.tile_rows = 32 * tm;
             p.k_slices = splits;
