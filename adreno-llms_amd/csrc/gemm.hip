@@ -15,6 +15,7 @@
 // accumulators of 32 x 32.
 #include "common.h"
 #include "device_math.h"
+#include "plan_keep.h"
 #include <hip/hip_fp16.h>
 #include <algorithm>
 #include <type_traits>
@@ -2145,19 +2146,10 @@ double gemm_estimate_us(WeightKind kind, int M, int N, int K, size_t workspace_b
 
 static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t workspace_bytes);
 
-// A plan follows from these numbers alone and takes a host 1 to 2 us to make, most of it estimates of the wide kernel's
-// shapes, where a layer's calls come again and again: each thread keeps the last 64 it made, by their numbers.
 GemmPlan plan_gemm(hipStream_t s, WeightKind kind, int M, int N, int K, size_t workspace_bytes) {
     const int set = gemm_mode(s), mode = set == 4 && kind != WK_Q4 ? 0 : set;   // mode 4 only concerns Q4 weights
-    struct Made { int mode = -1, kind = 0, M = 0, N = 0, K = 0; size_t bytes = 0; GemmPlan plan; };
-    constexpr unsigned kMade = 64;
-    thread_local Made made[kMade];
-    const unsigned h = (static_cast<unsigned>(N) * 2654435761u + static_cast<unsigned>(K) * 40503u + static_cast<unsigned>(M) * 97u +
-                        static_cast<unsigned>(kind)) >> 7;
-    Made& m = made[h % kMade];
-    if (m.mode != mode || m.kind != kind || m.M != M || m.N != N || m.K != K || m.bytes != workspace_bytes)
-        m = Made{mode, kind, M, N, K, workspace_bytes, make_plan(mode, kind, M, N, K, workspace_bytes)};
-    return m.plan;
+    return kept_plan<GemmPlan>(PlanKey{mode, device_info().cus, kind, M, N, K, workspace_bytes},
+                               [&] { return make_plan(mode, kind, M, N, K, workspace_bytes); });
 }
 
 static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t workspace_bytes) {
