@@ -2321,6 +2321,54 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
     return launch_planned(s, p, kind, M, N, K, x, W, scale, out, workspace, ws_bytes, MoreMats{}, true) ? 1 : -1;
 }
 
+namespace {
+
+// kernel 4 (shape few), 6 (shape rows) or 1 (wide: `plan`) in slices; 0: none
+struct SlicePlan { int kernel = 0, terms = 1; skinny::Shape few{}; skinny::RowShape rows{}; GemmPlan plan{}; };
+
+SlicePlan make_slice_plan(int mode, GemmPlan p, WeightKind kind, int M, int N, int K, size_t workspace_bytes) {
+    SlicePlan sp;
+    sp.terms = kind == WK_Q4 ? p.terms : 1;
+    const int cus = device_info().cus;
+    const bool own = mode == 0 || mode == 4;
+    // (a few rows: the streaming kernel's own slices, whatever the plan for a launch by itself.  Prompts of 10 / 24 / 37 / 64
+    //  tokens, int8 0.5B, int8 360M, fp16 360M, int8 0.5B, with its new loads in all: 973 / 1354 / 1514 / 1338 -> 927 / 1186 / 1208 / 1104 us)
+    if (M <= skinny::kMaxM && own) {
+        sp.few = skinny::pick_apart(kind, M, N, K, cus, workspace_bytes);
+        if (sp.few.kb > 1) { sp.kernel = 4; return sp; }
+    }
+    if (own && p.kernel >= 1 && p.kernel != 5) {
+        // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
+        const double uncut = p.kernel == 1   ? wide::estimate_us(kind, sp.terms, p.tile_rows / 32, p.k_slices, M, N, K, cus)
+                             : p.kernel == 6 ? skinny::rows_us(kind, p.tile_rows / 16, p.strips, 1, M, N, K, cus)
+                             : p.kernel == 4 ? 1e30 : tiled_estimate_us(M, N, K);
+        int tm = 1, splits = 1;
+        double cut = 1e30;
+        if (wide_reaches(kind, M, N, K)) wide::pick_sliced(kind, sp.terms, M, N, K, cus, workspace_bytes, &tm, &splits, &cut);
+        // Tiles of rows: against the wide kernel's slices and the plan, which also leaves the next launch a pass over its fp16 result,
+        // 1 us per 400 rows: 400 tokens of 0.5B int8 / fp16, whose q | k | v is estimated 1.1 / 1.25 us longer in slices, 1628 / 1726 us with them, 1577 /
+        // 1676 without; 500 Q4 tokens of 360M, o 0.9 longer, 2138 / 2184.
+        sp.rows = skinny::pick_rows_apart(kind, M, N, K, cus, workspace_bytes);
+        if (sp.rows.mt && sp.rows.us < cut - 2.5 && sp.rows.us < uncut + M / 400.0) { sp.kernel = 6; return sp; }
+        if (p.kernel != 4 && !(p.kernel == 1 && p.k_slices > 1) && cut - 2.5 < uncut) {
+            p.kernel = 1;
+            p.tile_rows = 32 * tm;
+            p.k_slices = splits;
+        }
+    }
+    if (p.kernel == 1 && p.k_slices > 1) { sp.kernel = 1; sp.plan = p; }
+    return sp;
+}
+
+template <int KIND, int TERMS>
+bool launch_streaming_slices(hipStream_t s, const SlicePlan& sp, int M, int N, int K, const void* x, const void* W, const void* scale,
+                             void* workspace, size_t workspace_bytes) {
+    if (sp.kernel == 6) return skinny::launch_rows<KIND, TERMS>(s, M, N, K, x, W, scale, nullptr, sp.rows, static_cast<float*>(workspace), MoreMats{}, false);
+    return skinny::launch<KIND, TERMS>(s, M, N, K, x, W, scale, nullptr, sp.few, workspace, workspace_bytes, MoreMats{}, false, true);
+}
+
+}  // namespace
+
 // A GEMM with K cut into slices, up to their sums: fp32 [slices][M][N] at the start of the workspace, for a launch that
 // adds them in index order and goes on with the result (decode.hip).  As launch_gemm would cut it, or, where that has no
 // slices, as many as pay without the launch that would add them: that launch is counted as 2.5 us in the estimate.
@@ -2330,49 +2378,18 @@ int launch_gemm_glu(hipStream_t s, WeightKind kind, int M, int N, int K, const v
 int launch_gemm_slices(hipStream_t s, WeightKind kind, int M, int N, int K, const void* x, const void* W, const void* scale,
                        void* workspace, size_t workspace_bytes) {
     if (!workspace || !gemm_supported(kind, M, N, K, x, W, scale)) return 0;
-    GemmPlan p = plan_gemm(s, kind, M, N, K, workspace_bytes);
+    const GemmPlan p = plan_gemm(s, kind, M, N, K, workspace_bytes);
     const int mode = gemm_mode(s);
-    // (a few rows: the streaming kernel's own slices, whatever the plan for a launch by itself.  Prompts of 10 / 24 / 37 / 64
-    //  tokens, int8 0.5B, int8 360M, fp16 360M, int8 0.5B, with its new loads in all: 973 / 1354 / 1514 / 1338 -> 927 / 1186 / 1208 / 1104 us)
-    if (M <= skinny::kMaxM && (mode == 0 || mode == 4)) {
-        const skinny::Shape sh = skinny::pick_apart(kind, M, N, K, device_info().cus, workspace_bytes);
-        if (sh.kb > 1) {
-            const bool ok = kind == WK_Q4 ? (p.terms == 1 ? skinny::launch<WK_Q4, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true)
-                                                          : skinny::launch<WK_Q4, 2>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true))
-                          : kind == WK_F16 ? skinny::launch<WK_F16, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true)
-                                           : skinny::launch<WK_I8, 1>(s, M, N, K, x, W, scale, nullptr, sh, workspace, workspace_bytes, MoreMats{}, false, true);
-            return ok ? sh.kb : -1;
-        }
-    }
-    const int terms = kind == WK_Q4 ? p.terms : 1, cus = device_info().cus;
-    if ((mode == 0 || mode == 4) && p.kernel >= 1 && p.kernel != 5) {
-        // (of this very plan: gemm_estimate_us counts two terms for Q4 weights in every mode)
-        const double uncut = p.kernel == 1   ? wide::estimate_us(kind, terms, p.tile_rows / 32, p.k_slices, M, N, K, cus)
-                             : p.kernel == 6 ? skinny::rows_us(kind, p.tile_rows / 16, p.strips, 1, M, N, K, cus)
-                             : p.kernel == 4 ? 1e30 : tiled_estimate_us(M, N, K);
-        int tm = 1, splits = 1;
-        double cut = 1e30;
-        if (wide_reaches(kind, M, N, K)) wide::pick_sliced(kind, terms, M, N, K, cus, workspace_bytes, &tm, &splits, &cut);
-        // Tiles of rows: against the wide kernel's slices and the plan, which also leaves the next launch a pass over its fp16 result,
-        // 1 us per 400 rows: 400 tokens of 0.5B int8 / fp16, whose q | k | v is estimated 1.1 / 1.25 us longer in slices, 1628 / 1726 us with them, 1577 /
-        // 1676 without; 500 Q4 tokens of 360M, o 0.9 longer, 2138 / 2184.
-        const skinny::RowShape r = skinny::pick_rows_apart(kind, M, N, K, cus, workspace_bytes);
-        if (r.mt && r.us < cut - 2.5 && r.us < uncut + M / 400.0) {
-            auto* sums = static_cast<float*>(workspace);
-            const bool ok = kind == WK_Q4 ? (terms == 1 ? skinny::launch_rows<WK_Q4, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false)
-                                                        : skinny::launch_rows<WK_Q4, 2>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false))
-                          : kind == WK_F16 ? skinny::launch_rows<WK_F16, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false)
-                                           : skinny::launch_rows<WK_I8, 1>(s, M, N, K, x, W, scale, nullptr, r, sums, MoreMats{}, false);
-            return ok ? r.kb : -1;
-        }
-        if (p.kernel != 4 && !(p.kernel == 1 && p.k_slices > 1) && cut - 2.5 < uncut) {
-            p.kernel = 1;
-            p.tile_rows = 32 * tm;
-            p.k_slices = splits;
-        }
-    }
-    if (p.kernel != 1 || p.k_slices < 2) return 0;
-    return launch_planned(s, p, kind, M, N, K, x, W, scale, nullptr, workspace, workspace_bytes, MoreMats{}) ? p.k_slices : -1;
+    const SlicePlan sp = kept_plan<SlicePlan>(PlanKey{mode, device_info().cus, kind, M, N, K, workspace_bytes},
+                                              [&] { return make_slice_plan(mode, p, kind, M, N, K, workspace_bytes); });
+    if (sp.kernel == 0) return 0;
+    if (sp.kernel == 1)
+        return launch_planned(s, sp.plan, kind, M, N, K, x, W, scale, nullptr, workspace, workspace_bytes, MoreMats{}) ? sp.plan.k_slices : -1;
+    const bool ok = kind == WK_Q4 ? (sp.terms == 1 ? launch_streaming_slices<WK_Q4, 1>(s, sp, M, N, K, x, W, scale, workspace, workspace_bytes)
+                                                   : launch_streaming_slices<WK_Q4, 2>(s, sp, M, N, K, x, W, scale, workspace, workspace_bytes))
+                  : kind == WK_F16 ? launch_streaming_slices<WK_F16, 1>(s, sp, M, N, K, x, W, scale, workspace, workspace_bytes)
+                                   : launch_streaming_slices<WK_I8, 1>(s, sp, M, N, K, x, W, scale, workspace, workspace_bytes);
+    return !ok ? -1 : sp.kernel == 6 ? sp.rows.kb : sp.few.kb;
 }
 
 // One launch serves the leading matrices whose own plans sum K in the same order, so that each result is what
