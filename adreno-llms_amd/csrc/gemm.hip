@@ -1762,7 +1762,9 @@ inline int rows_ks(int M, int N, int K) {
     while (ks > 1 && K / 64 < ks) ks /= 2;
     return ks;
 }
-inline bool rows_fit(int kind, int mt, int S, int ks) {
+// (a grid counts 65 535 tiles of rows)
+inline bool rows_fit(int kind, int mt, int S, int ks, int M) {
+    if ((static_cast<long>(M) + 16 * mt - 1) / (16 * mt) > 65535) return false;
     const size_t unit = unit_bytes(kind, mt, S), sums = static_cast<size_t>(mt) * S * 1024;
     return (ks < 4 ? 4 : ks) * (unit > sums ? unit : sums) <= kLdsLimit;
 }
@@ -1771,7 +1773,7 @@ inline RowShape pick_rows(int kind, int M, int N, int K, int cus, bool glu) {
     for (int mt = 2; mt <= 4; ++mt)
         for (int S = 1; S <= 4; S *= 2) {
             const int ks = rows_ks(M, N, K);
-            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || (glu && S == 1) || !rows_fit(kind, mt, S, ks)) continue;
+            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || (glu && S == 1) || !rows_fit(kind, mt, S, ks, M)) continue;
             const double us = rows_us(kind, mt, S, 1, M, N, K, cus);
             if (us < best.us) best = RowShape{mt, S, ks, 1, us};
         }
@@ -1809,7 +1811,7 @@ inline RowShape pick_rows_apart(int kind, int M, int N, int K, int cus, size_t w
     if (its < 14 || static_cast<long>((M + 47) / 48) * ((N + 31) / 32) > cus * 9L / 5) return best;
     for (int mt = 2; mt <= 4; ++mt)
         for (int S = 1; S <= 4; S *= 2) {
-            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || !rows_fit(kind, mt, S, 4)) continue;
+            if ((S == 4 && (mt == 2 || kind == WK_Q4)) || !rows_fit(kind, mt, S, 4, M)) continue;
             for (int kb = 2; kb <= 6 && its >= 4 * kb && static_cast<size_t>(kb) * M * N * 4 <= workspace_bytes; ++kb) {
                 const double us = rows_us(kind, mt, S, kb, M, N, K, cus) + kb * 4.0e-6 * M * N / 4.0;
                 if (us < best.us) best = RowShape{mt, S, 4, kb, us};
@@ -2179,6 +2181,7 @@ static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t
         wide::pick_shape(WK_Q4, p.terms, M, N, K, cus, may_slice ? workspace_bytes : 0, &tm, &splits, &wide_us);
         if (may_slice || mode == 6) {
             const skinny::RowShape r = skinny::pick_rows(kind, M, N, K, cus, false);
+            if (mode == 6 && !r.mt) return p;            // more rows than the grid counts
             if (mode == 6 || skinny::rows_preferred(kind, r, wide_us, splits, 0.0, M, N, K, cus)) {
                 p.kernel = 6; p.tile_rows = 16 * r.mt; p.ks = r.ks; p.strips = r.S;
                 return p;
@@ -2215,7 +2218,7 @@ static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t
         p.kernel = 6; p.tile_rows = 16 * r.mt; p.ks = r.ks; p.strips = r.S;
         return p;
     };
-    if (mode == 6) return rows();
+    if (mode == 6) return r.mt ? rows() : p;               // (none: more rows than the grid counts)
     // the wide kernel where its estimated time beats that of the 64 x 64 tiles
     if (wide_fits && (mode == 0 || mode == 3 || (mode >= 11 && mode <= 15))) {
         double wide_us = 0.0;
@@ -2407,7 +2410,7 @@ int launch_gemm_group(hipStream_t s, WeightKind kind, int n, const GemmMat* mat,
         long all = 0;
         for (int j = 0; j < n; ++j) all += mat[j].N;
         const skinny::RowShape r = skinny::pick_rows(kind, M, all < (1 << 30) ? static_cast<int>(all) : mat[0].N, K, cus, false);
-        if (skinny::rows_fit(kind, r.mt, r.S, p.ks)) { p.tile_rows = 16 * r.mt; p.strips = r.S; }
+        if (r.mt && skinny::rows_fit(kind, r.mt, r.S, p.ks, M)) { p.tile_rows = 16 * r.mt; p.strips = r.S; }
     }
     if (!(p.kernel == 2 || p.kernel == 3 || p.kernel == 6 || (p.kernel == 1 && p.k_slices == 1) || (p.kernel == 4 && sh.kb == 1))) return 0;
     const int width = p.kernel == 1 ? wide::kBN : p.kernel == 2 ? 64 : p.kernel == 3 ? 128 : p.kernel == 6 ? 16 * p.strips : 16 * sh.S;

@@ -181,7 +181,7 @@ int   mi_graph_destroy(void* graph);
  * slices' fp32 sums do not fit the stream's workspace), 30 = the kernel with 256 x 256 blocks (int8 weights only; mode 0
  * takes it by itself for contractions of several rounds of such blocks at K >= 2048), 5 = the streaming kernel for up to 64 rows of x (every kind of weights takes
  * it by itself in mode 0 up to 32 to 64 rows, depending on the shape, where it is the faster one; fails for
- * more than 64 rows), 6 = the same in tiles of up to 64 rows, any number of them (mode 0 takes it where it is the faster one).
+ * more than 64 rows), 6 = the same in tiles of up to 64 rows, up to 65 535 of them (mode 0 takes it where it is the faster one).
  * Q4 weights: a weight q * scale (4 and 11 significant bits) is not an fp16 number in general.
  * Every mode but 4 feeds it to the matrix cores exactly, as two fp16 terms q * hi + q * lo with
  * scale = hi + lo, and stays within one fp16 step of the batched GEMV.  Mode 4 = as 0, but each

@@ -2,6 +2,7 @@
 tests/test_gemm_plan_gpu.py holds the choice among those: no more than 20 % behind the fastest pinned one.  Calls on
 both sides of every line that rows_preferred draws: many columns, a short K, many outputs, a long K with the wide
 kernel in slices (mode 100 s + 10 + t), and calls of some hundred rows, which the tiles of rows win."""
+import numpy as np
 import pytest
 
 from helpers import mil
@@ -100,3 +101,29 @@ def test_a_row_more_than_2048_costs_no_launch(queue):  # noqa: F811
         if us[2049] <= 1.08 * us[2048]:
             return
     assert False, us
+
+
+@pytest.mark.parametrize("kind", ["f16", "int8", "q4"])
+def test_more_tiles_of_rows_than_a_grid_counts(kind):
+    """65 535 in its third dimension: beyond 65 535 x 32 rows in taller tiles, beyond 65 535 x 64 not at all."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep, n, k = mil.Queue(), [], 16, 64
+    rows = 65535 * 32 + 1
+    w = _weights(kind, n, k, 74, keep)
+    x, out, row = mil.Buffer(2 * rows * k), mil.Buffer(2 * rows * n), mil.synth_normal_f16(75, 1.0, (1, k))
+    assert mil.lib().mi_memset(x.ptr, 0, 2 * rows * k, queue.handle)
+    last = mil.Buffer.from_host(row)
+    assert mil.lib().mi_memcpy_d2d(x.ptr + 2 * (rows - 1) * k, last.ptr, 2 * k, queue.handle)
+    assert mil.lib().mi_stream_set_modes(queue.handle, -1, 6)
+    for m, tile in ((rows, 48), (65535 * 64, 64), (65535 * 64 + 1, 0)):
+        plan = mil.linear_plan(queue, m, n, k, x, w)
+        print(f"{kind} {m} rows plan {plan}", flush=True)
+        assert plan[0] == (6 if tile else -1) and plan[1] >= tile
+    assert mil.pytorch_linear(queue, rows, n, k, x, w, out)
+    two, want = mil.Buffer.from_host(np.concatenate([row, row])), mil.Buffer(4 * n)      # (the same slices of K: the same bits)
+    assert mil.linear_plan(queue, 2, n, k, two, w)[0] == 6 and mil.pytorch_linear(queue, 2, n, k, two, w, want)
+    queue.finish()
+    got = out.read(np.uint16, (rows, n))
+    assert np.array_equal(got[-1], want.read(np.uint16, (2, n))[0]) and got[-1].any()
+    assert not got[:-1].any()
+    assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
