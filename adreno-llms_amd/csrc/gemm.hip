@@ -2227,8 +2227,11 @@ static GemmPlan make_plan(int mode, WeightKind kind, int M, int N, int K, size_t
         if (mode >= 11) tm = mode - 10;
         if (pin_splits) splits = pin_splits;
         const double tiled_us = tiled_estimate_us(M, N, K);
-        // (many rows in tiles that go in bands keep those, a plan that is promised: 2048 x 960 x 960 int8 11.6 us against 12.2 here)
-        const bool banded = M > (K < 896 ? 1280 : 1024) && (N >= 960 || K >= 896) && K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64);
+        // (64 x 64 tiles in bands keep up from fewer outputs on: 2048 x 960 x 960 int8 12.2 us there, 12.3 in tiles of rows, 1200 x 1600 x 960 fp16
+        // 12.6 / 13.0; but 1500 x 960 x 960 int8 11.9 / 10.5, 1200 rows 11.7 / 8.9, fp16 12.4 / 9.5.  Where 960 columns keep them, fewer columns
+        // by such a K do too, which may go out with them: the layer of 360M at 2048 int8 rows 91.8 us, with k and v apart from q 95.3.)
+        const bool banded = K <= 1024 && tiles_in_bands((N + 63) / 64, (M + 63) / 64) &&
+                            (static_cast<double>(M) * N > 7000.0 * cus || (K >= 768 && M > 7 * cus));
         if (mode == 0 && !banded && skinny::rows_preferred(kind, r, wide_us, splits, tiled_us, M, N, K, cus)) return rows();
         if (mode != 0 || wide_us < tiled_us) {
             p.kernel = 1; p.tile_rows = 32 * tm; p.k_slices = splits;

@@ -127,3 +127,13 @@ def test_more_tiles_of_rows_than_a_grid_counts(kind):
     assert np.array_equal(got[-1], want.read(np.uint16, (2, n))[0]) and got[-1].any()
     assert not got[:-1].any()
     assert mil.lib().mi_stream_set_modes(queue.handle, -1, -1)
+
+
+@pytest.mark.parametrize("kind,M,N,K,kernel", [("int8", 1200, 960, 960, 6), ("f16", 1200, 960, 960, 6), ("int8", 1600, 320, 960, 6),
+                                               ("int8", 2048, 320, 960, 2), ("int8", 2048, 576, 576, 6), ("f16", 1200, 1600, 960, 2)])
+def test_tiles_of_rows_beside_64_x_64_tiles_in_bands(kind, M, N, K, kernel):
+    """Odd numbers of columns of 64 x 64 tiles: the tiles of rows up to 7000 outputs per CU, by a K of 768 and more up to 7 rows."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep = mil.Queue(), []
+    x, w = mil.Buffer(2 * M * K), _weights(kind, N, K, 76, keep)
+    assert mil.linear_plan(queue, M, N, K, x, w)[0] == kernel
