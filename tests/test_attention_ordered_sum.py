@@ -47,3 +47,25 @@ def test_steps_equal_the_prompt(sigma):
         assert mil.lib().mi_memcpy_d2h(got.ctypes.data, dec.logits_ptr, 2 * VOCAB, queue.handle)
         queue.finish()
         assert np.array_equal(got, want), pos
+
+
+@pytest.mark.parametrize("sigma", [0.0, 0.02, 0.3])
+def test_steps_equal_the_prompt_where_a_lane_holds_more_quadruples(sigma):
+    """9 of them to 2304 positions, 17 beyond."""
+    assert mil.lib().mi_init(0) == 1
+    queue, keep = mil.Queue(), []
+    dec = _decoder(sigma, keep)
+    ids = [int(t) for t in np.random.default_rng(6).integers(0, VOCAB, MOST)]
+    assert mil.lib().mi_stream_set_modes(queue.handle, -1, 1)
+    for pos in (2051, 2176, 2271, 2287, 2303, 2304, 2320, 2560):
+        print(f"sigma {sigma} position {pos}", flush=True)
+        got, want = np.empty(VOCAB, np.uint16), np.empty(VOCAB, np.uint16)
+        assert dec.prefill(queue, ids[:pos + 1])
+        first = dec.read(queue)
+        assert mil.lib().mi_memcpy_d2h(want.ctypes.data, dec.logits_ptr, 2 * VOCAB, queue.handle)
+        queue.finish()
+        assert dec.reset(queue, pos, ids[pos]) and dec.step(queue)
+        assert dec.read(queue) == first
+        assert mil.lib().mi_memcpy_d2h(got.ctypes.data, dec.logits_ptr, 2 * VOCAB, queue.handle)
+        queue.finish()
+        assert np.array_equal(got, want), pos
