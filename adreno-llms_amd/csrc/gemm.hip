@@ -1286,22 +1286,17 @@ bool launch(hipStream_t s, int M, int N, int K, const void* x, const void* W, co
 
 }  // namespace quad
 
-// ---- a few rows of x (M <= 64): the weights stream once, as in the GEMV ------------------------
+// ---- a few rows of x, and tiles of as many: the weights stream past them, as in the GEMV --------
 //
-// With up to 64 rows of x the contraction is bound by the weights' bytes, like the GEMV, not by
-// the matrix cores, and the tiles above leave most of the chip idle (19 tiles at N = 4864).  Here a
-// wavefront takes a strip of 16 rows of W and streams it through v_mfma_f32_16x16x32_f16 against
-// the 16 MT rows of x:
-//   A = W strip: lane l supplies row l % 16, 8 values of K starting at 16 (l / 16) + 8 s of the
-//       iteration's 64 (s = 0, 1: the two MFMAs of an iteration), i.e. one 16-byte load of int8
-//       weights per lane and iteration, 64 contiguous bytes per row;
-//   B = x^T: lane l supplies row l % 16 of the x tile at the same 16 values of K, 32 contiguous
-//       bytes (x is small and comes from the caches);
+// With up to 64 rows of x the contraction is bound by the weights' bytes, like the GEMV, not by the matrix cores, and the
+// tiles above leave most of the chip idle (19 tiles at N = 4864).  Here a wavefront takes strips of 16 rows of W through
+// v_mfma_f32_16x16x32_f16 against 16 MT rows of x, 64 values of K (a unit) at a time:
+//   A = W strip: lane l supplies row l % 16, 8 values of K starting at 16 (l / 16) + 8 s of the unit's 64 (s = 0, 1: the two
+//       MFMAs of a unit);
+//   B = x^T: lane l supplies row l % 16 of the x tile at the same values of K;
 //   D[i][j] (lane l: i = 4 (l / 16) + r, j = l % 16) = out[row j of the x tile][row i of the strip]:
 //       four consecutive output columns per lane.
-// K is cut into ks slices over the wavefronts of a block where N alone gives too few strips to
-// fill the chip; their sums meet in LDS and are added in slice order.  Iterations go through two
-// register buffers, one in flight while the other is multiplied.
+// How both get there, and how K is shared out: skinny_tile.
 namespace skinny {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
